@@ -1134,10 +1134,9 @@ int gic_raw_stream(gic_context *c, unsigned long seed, uint32_t *host_out, size_
   return guarded(c, [&] {
     RngPlan plan;
     rng_plan(seed, n / 2 + 1, plan);
-    c->work.ensure(rng_workspace_bytes(plan));
     DevBuf out;
     out.ensure(n * 4);
-    rng_raw(plan, (uint32_t *)out.p, n, c->work.p, c->work.bytes, c->st);
+    rng_raw(plan, (uint32_t *)out.p, n, c->st);
     GIC_HIP(hipMemcpyAsync(host_out, out.p, n * 4, hipMemcpyDeviceToHost, c->st));
     GIC_HIP(hipStreamSynchronize(c->st));
   });

@@ -462,7 +462,7 @@ void do_batch(gic_context *c, int nreal, const uint64_t *seeds, int ncons, const
   // every realisation's RNG plan in device memory: the recorded work holds
   // no seed, so one instantiated graph serves every batch of this shape
   std::vector<RngPlan> plans(nreal);
-  const size_t pb = (rng_dev_bytes() + 255) / 256 * 256;
+  const size_t pb = (rng_dev_bytes(plan0) + 255) / 256 * 256;
   std::vector<char> hplans(size_t(nreal) * pb, 0);
   for (int r = 0; r < nreal; ++r) {
     rng_plan(seeds[r], n3, plans[r]);
@@ -480,7 +480,7 @@ void do_batch(gic_context *c, int nreal, const uint64_t *seeds, int ncons, const
     };
     auto q = [&](const void *ptr) { key.push_back(uint64_t(uintptr_t(ptr))); };
     for (long v : {long(sizeof(T)), long(n), long(nreal), long(ncons), long(nlanes), long(boxes), long(wl), nrows,
-                   long(np), plans[0].nchunks, long(plans[0].kc)})
+                   long(np), plans[0].nseg, long(plans[0].kclog)})
       key.push_back(uint64_t(v));
     for (double v : {g.dx, g.ox, g.oy, g.oz, g.periodic, g.kmin()}) u(v);
     for (const void *ptr : std::initializer_list<const void *>{out, B.cons.p, B.flags.p, B.win.p, B.plans.p, L.sqrtp.p,
@@ -515,7 +515,7 @@ void do_batch(gic_context *c, int nreal, const uint64_t *seeds, int ncons, const
       const double *rc = dcons + size_t(r) * ncons * 5;
       // the white noise, then its spectrum with Re(w_0) = 0 (randomfieldgenerator.hpp:194-195)
       std::vector<RngLevelOut> outs{{ln.w.p, n, n3}};
-      rng_draw_real<T>(plans[r], outs, ln.ws.p, ln.ws.bytes, st, nullptr, 1.0, dflags + r,
+      rng_draw_real<T>(plans[r], outs, ln.ws.p, ln.ws.bytes, st, nullptr, 1.0, dflags + r, 0,
                        (const char *)B.plans.p + size_t(r) * pb);
       fft_r2c_post<T>(w, n, nullptr, st, nullptr);
       fill<T>(w, 1, T(0), st);

@@ -10,19 +10,26 @@ struct U576 {
   uint64_t w[9];
 };
 
-// Host-side set-up of one real-space draw: the seeded RANLUX state and the
-// table of jump multipliers b^{-397*KC*2^i} mod m (b = 2^48, m = b^12-b^5+1).
-struct RngPlan {
-  static constexpr int MAXBITS = 32;
-  int kc = 64;                             // ranlxs2 blocks (24 numbers) per chunk: 4..64, set by rng_plan
-  int ch() const { return kc * 24; }       // raw numbers per chunk
-  uint64_t seed_words[12];                 // the 12 seeded 48-bit words, oldest first
-  U576 y0;                                 // LCG state 11 steps past the seeded state, times ... (see rng.hip)
-  U576 jump[MAXBITS];
-  long nchunks = 0;
+// One stream of a draw: its seed, the Gaussians wanted, and where the first
+// of them goes, counted in the order of the draw's targets.
+struct RngStream {
+  unsigned long seed;
+  size_t count;
+  size_t out0;
 };
 
-void rng_plan(unsigned long seed, size_t n_gaussians, RngPlan &plan);
+// Host-side set-up of one real-space draw: its streams, the chunk length and
+// how many wavefronts of 64 chunks each stream takes.
+struct RngPlan {
+  std::vector<RngStream> streams;
+  int kclog = 6;                             // log2 of the ranlxs2 blocks (24 numbers) per chunk: 0..6
+  int ch() const { return 24 << kclog; }     // raw numbers per chunk
+  std::vector<long> seg0;                    // each stream's first wavefront
+  long nseg = 0;                             // wavefronts in all
+};
+
+void rng_plan(const std::vector<RngStream> &streams, RngPlan &plan);
+void rng_plan(unsigned long seed, size_t n_gaussians, RngPlan &plan);   // one stream from the start of the targets
 
 // Draw the stream's Gaussians into the listed targets in order, as the
 // reference's serial loop does: a padded real field (n > 0, count n^3, cell
@@ -36,19 +43,19 @@ struct RngLevelOut {
 template <typename T>
 void rng_draw_real(const RngPlan &plan, const std::vector<RngLevelOut> &levels, void *workspace, size_t ws_bytes,
                    hipStream_t st, struct TimingHook *hook, double scale = 1.0, uint32_t *cover_flag = nullptr,
-                   const void *dev_plan = nullptr);
+                   int flag_stride = 0, const void *dev_plan = nullptr);
 // With cover_flag the draw has no host synchronisation: a device check sets
-// *cover_flag to 1 if the stream held too few Gaussians (the cells past the
-// end are then left as they were), instead of the host raising an error.
+// cover_flag[i * flag_stride] to 1 if stream i held too few Gaussians (the
+// cells past the end are then left as they were); without, the call waits
+// for the draw and raises an error.
 // dev_plan: the plan already in device memory (rng_dev_pack'd, rng_dev_bytes
-// long, copied there by the caller); otherwise a kernel writes it into the
-// workspace, so that the draw's launches carry no seed-dependent arguments
-// past that one.
-size_t rng_dev_bytes();
+// long, copied there by the caller); otherwise the call puts it into the
+// workspace.
+size_t rng_dev_bytes(const RngPlan &plan);
 void rng_dev_pack(const RngPlan &plan, void *host_dst);
 size_t rng_workspace_bytes(const RngPlan &plan);
-// uploads the ziggurat tables (once, synchronously) ahead of draws that a
-// graph records
+// uploads the ziggurat and jump tables (once, synchronously) ahead of draws
+// that a graph records
 void rng_prepare();
 
 // Draws into a caller's device array with the fixed per-device workspace:
@@ -60,7 +67,7 @@ size_t rng_noalloc_max_gaussians();
 void rng_gaussians_noalloc(int device, unsigned long seed, double *dev_out, size_t n, hipStream_t st);
 
 // Raw 24-bit stream (testing / bit-exactness checks): the first n numbers.
-void rng_raw(const RngPlan &plan, uint32_t *d_out, size_t n, void *workspace, size_t ws_bytes, hipStream_t st);
+void rng_raw(const RngPlan &plan, uint32_t *d_out, size_t n, hipStream_t st);
 
 // Host reference pieces used by tests of the jump arithmetic.
 void u576_mulmod_host(const U576 &a, const U576 &b, U576 &r);

@@ -17,13 +17,20 @@
 //
 // gsl_ran_gaussian_ziggurat consumes 2 numbers per accepted iteration and
 // 3 or 4 on the rare edge/tail tests, so the Gaussian index of a chunk is
-// data dependent.  Pass 1 generates every chunk and parses it from the 4
-// possible entry offsets (the parses merge after a few iterations), pass 2
-// scans the entry->(exit, count) maps, pass 3 parses each chunk again from
-// its true entry and writes the Gaussians to their cells.  Pass 1 stores the
-// chunk's raw 24-bit numbers (4 bytes each, about 2.05 per Gaussian) for
-// pass 3 to read back, so the generator runs once; within a pass the parse
-// reads them from a per-thread LDS ring.
+// data dependent.  Pass 1 generates every chunk, parses it from the 4
+// possible entry offsets (the parses merge after a few iterations) and scans
+// the entry->(exit, count) maps across its wavefront; pass 2 scans the
+// wavefronts' maps; pass 3 generates each chunk again, parses it from its
+// true entry and writes the Gaussians to their cells.
+//
+// Generating twice is cheaper than keeping the numbers: a block of 24
+// numbers takes about 3200 issue cycles of a wavefront (two instructions per
+// recurrence step), writing and reading back its 64 x 24 words about 6100
+// cycles of that SIMD's share of the memory bandwidth.
+//
+// One launch draws any number of independent streams (the shells of a
+// Fourier-space draw, the realisations of a batch); every wavefront works on
+// 64 consecutive chunks of one stream.
 #include "rng.h"
 #include "fft.h"
 #include <cstring>
@@ -209,57 +216,116 @@ __host__ __device__ inline void decode_state(const uint64_t *V, uint64_t *x) {
   for (int j = 0; j < 5; ++j) x[7 + j] = get48(B, 48 * j);
 }
 
-// one subtract-with-borrow step on the ring: x[i] <- x[j] - x[i] - c
-#define SWB(i, j)                              \
-  {                                            \
-    int64_t d = (int64_t)x[j] - (int64_t)x[i] - c; \
-    c = (int64_t)((uint64_t)d >> 63);          \
-    x[i] = (uint64_t)d & MASK48;               \
-  }
-
-// 397 recurrence steps (33 rounds of 12 plus one), keeping x[0] as the
-// oldest word afterwards by rotating the registers once.
-__device__ __forceinline__ void ranlux_block(uint64_t *x, int64_t &c) {
-  for (int r = 0; r < 33; ++r) {
-    SWB(0, 7) SWB(1, 8) SWB(2, 9) SWB(3, 10) SWB(4, 11) SWB(5, 0)
-    SWB(6, 1) SWB(7, 2) SWB(8, 3) SWB(9, 4) SWB(10, 5) SWB(11, 6)
-  }
-  SWB(0, 7)
-  uint64_t t0 = x[0];
-#pragma unroll
-  for (int i = 0; i < 11; ++i) x[i] = x[i + 1];
-  x[11] = t0;
-}
-
-struct RngDev {
-  uint64_t seed_words[12];
-  U576 y0;
-  U576 jump[RngPlan::MAXBITS];
-  int kc;   // ranlxs2 blocks per chunk
+// The generator's 12 words, oldest first, as 32 + 16 bits each: 48-bit words
+// split this way need no masks (see swb_round)
+struct Lux {
+  uint32_t lo[12], hi[12];
+  uint32_t c;   // borrow, 0 or 1
 };
 
-__device__ void chunk_start_state(const RngDev &p, long t, uint64_t *x, int64_t &c) {
-  c = 0;
-  if (t == 0) {
-    for (int i = 0; i < 12; ++i) x[i] = p.seed_words[i];
-    return;
-  }
-  uint64_t acc[9];
-  for (int i = 0; i < 9; ++i) acc[i] = p.y0.w[i];
-  for (int b = 0; b < RngPlan::MAXBITS; ++b) {
-    if ((t >> b) & 1) {
-      uint64_t r[9];
-      u576_mulmod(acc, p.jump[b].w, r);
-      for (int i = 0; i < 9; ++i) acc[i] = r[i];
-    }
-  }
-  decode_state(acc, x);
-  // 12 steps resolve the carry ambiguity and land on the chunk's start
-  SWB(0, 7) SWB(1, 8) SWB(2, 9) SWB(3, 10) SWB(4, 11) SWB(5, 0)
-  SWB(6, 1) SWB(7, 2) SWB(8, 3) SWB(9, 4) SWB(10, 5) SWB(11, 6)
+// One subtract-with-borrow step x[i] <- x[j] - x[i] - c in two instructions:
+// the borrow stays in VCC, and the upper half is a 32-bit subtraction of
+// zero-extended 16-bit values (SDWA), whose borrow is that of the 48-bit
+// word and whose result is cut to 16 bits on the way out.  From the 64-bit
+// C expression the compiler makes six.  gfx950 wants two wait states between
+// a VALU write of VCC and its use as a carry, hence the s_nop.  Written for
+// one wavefront the waits show; four wavefronts per SIMD fill them.
+#define LUX_STEP(i, j)                                              \
+  "v_subb_co_u32 %[l" #i "], vcc, %[l" #j "], %[l" #i "], vcc\n\t"  \
+  "s_nop 1\n\t"                                                     \
+  "v_subb_co_u32_sdwa %[h" #i "], vcc, %[h" #j "], %[h" #i "], vcc" \
+  " dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_0\n\t" \
+  "s_nop 1\n\t"
+#define LUX_IO(x)                                                                                            \
+  [l0] "+v"(x.lo[0]), [l1] "+v"(x.lo[1]), [l2] "+v"(x.lo[2]), [l3] "+v"(x.lo[3]), [l4] "+v"(x.lo[4]),        \
+      [l5] "+v"(x.lo[5]), [l6] "+v"(x.lo[6]), [l7] "+v"(x.lo[7]), [l8] "+v"(x.lo[8]), [l9] "+v"(x.lo[9]),    \
+      [l10] "+v"(x.lo[10]), [l11] "+v"(x.lo[11]), [h0] "+v"(x.hi[0]), [h1] "+v"(x.hi[1]), [h2] "+v"(x.hi[2]), \
+      [h3] "+v"(x.hi[3]), [h4] "+v"(x.hi[4]), [h5] "+v"(x.hi[5]), [h6] "+v"(x.hi[6]), [h7] "+v"(x.hi[7]),    \
+      [h8] "+v"(x.hi[8]), [h9] "+v"(x.hi[9]), [h10] "+v"(x.hi[10]), [h11] "+v"(x.hi[11]), [c] "+v"(x.c)
+#define LUX_BEGIN "v_cmp_ne_u32 vcc, 0, %[c]\n\ts_nop 1\n\t"
+#define LUX_END "v_cndmask_b32 %[c], 0, 1, vcc\n\ts_nop 1\n\t"
+
+// 12 steps: every word is replaced once, x[0] stays the oldest
+__device__ __forceinline__ void lux_round(Lux &x) {
+  asm volatile(LUX_BEGIN LUX_STEP(0, 7) LUX_STEP(1, 8) LUX_STEP(2, 9) LUX_STEP(3, 10) LUX_STEP(4, 11) LUX_STEP(5, 0)
+                   LUX_STEP(6, 1) LUX_STEP(7, 2) LUX_STEP(8, 3) LUX_STEP(9, 4) LUX_STEP(10, 5) LUX_STEP(11, 6) LUX_END
+               : LUX_IO(x)
+               :
+               : "vcc");
+}
+__device__ __forceinline__ void lux_step0(Lux &x) {
+  asm volatile(LUX_BEGIN LUX_STEP(0, 7) LUX_END : LUX_IO(x) : : "vcc");
 }
 
-// ---- ziggurat iteration ---------------------------------------------------------
+// 397 steps (33 rounds of 12 plus one), the words rotated once at the end so
+// that x[0] is the oldest again
+__device__ __forceinline__ void lux_block(Lux &x) {
+#pragma unroll 1
+  for (int r = 0; r < 33; ++r) lux_round(x);
+  lux_step0(x);
+  uint32_t l = x.lo[0], h = x.hi[0];
+#pragma unroll
+  for (int i = 0; i < 11; ++i) {
+    x.lo[i] = x.lo[i + 1];
+    x.hi[i] = x.hi[i + 1];
+  }
+  x.lo[11] = l;
+  x.hi[11] = h;
+}
+// the two 24-bit numbers of word k, in stream order
+__device__ __forceinline__ uint32_t lux_first(const Lux &x, int k) { return x.lo[k] & 0xFFFFFFu; }
+__device__ __forceinline__ uint32_t lux_second(const Lux &x, int k) {
+  return __builtin_amdgcn_alignbit(x.hi[k], x.lo[k], 24);
+}
+
+// The jump multipliers b^{-397 kc d 64^l} mod m for kc = 2^q blocks per
+// chunk, digit d at base-64 position l of the chunk index: a chunk's start
+// is at most RNG_DIGITS modular products from the stream's (a table of
+// squarings takes one per bit set in any lane's index).  They depend on
+// neither seed nor size.
+constexpr int RNG_KC_LOG = 7;    // kc = 1 .. 64
+constexpr int RNG_DIGITS = 4;    // 64^4 chunks
+static __device__ uint64_t d_jump[RNG_KC_LOG][RNG_DIGITS][64][9];
+
+// One stream of a draw
+struct RngDev {
+  uint64_t seed_words[12];
+  U576 y0;          // the LCG state 12 steps before the stream's start
+  uint64_t seg0;    // its first wavefront (64 chunks each)
+  uint64_t nseg;
+  uint64_t out0;    // where its first Gaussian goes, counted in the targets' order
+  uint64_t total;   // Gaussians wanted
+};
+
+__device__ __forceinline__ void lux_set(Lux &x, const uint64_t *w) {
+#pragma unroll
+  for (int i = 0; i < 12; ++i) {
+    x.lo[i] = uint32_t(w[i]);
+    x.hi[i] = uint32_t(w[i] >> 32);
+  }
+  x.c = 0;
+}
+
+__device__ __forceinline__ void chunk_start_state(const RngDev &p, int kclog, long t, Lux &x) {
+  uint64_t acc[9];
+  for (int i = 0; i < 9; ++i) acc[i] = p.y0.w[i];
+#pragma unroll 1
+  for (int l = 0; l < RNG_DIGITS; ++l) {
+    long up = t >> (6 * l);
+    if (l > 0 && up == 0) break;
+    uint64_t r[9];
+    u576_mulmod(acc, d_jump[kclog][l][up & 63], r);
+    for (int i = 0; i < 9; ++i) acc[i] = r[i];
+  }
+  uint64_t w[12];
+  decode_state(acc, w);
+  lux_set(x, w);
+  // 12 steps resolve the carry ambiguity and land on the chunk's start
+  lux_round(x);
+  if (t == 0) lux_set(x, p.seed_words);
+}
+
+// ---- ziggurat -------------------------------------------------------------------
 // The ziggurat tables in LDS: the lookups are indexed by random bytes, so
 // each lane reads a different entry (constant memory serves one address per
 // wavefront)
@@ -278,221 +344,264 @@ __device__ __forceinline__ void zig_tabs_load(ZigTabs &z) {
   __syncthreads();
 }
 
-// One loop iteration of gsl_ran_gaussian_ziggurat starting at stream position
-// pos: returns the number of numbers consumed (2, 3 or 4) and whether it
-// accepted; *val receives the Gaussian when accepted.
-template <class Get>
-__device__ __forceinline__ int zig_iter(Get get, long pos, bool &accept, double &val, const ZigTabs &zt) {
-  const double PARAM_R = 3.44428647676;
-  uint32_t k1 = get(pos), k2 = get(pos + 1);
-  uint32_t i = k1 & 0xFF, j = k2 & 0xFFFFFF;
-  double sign = (i & 0x80) ? 1.0 : -1.0;
-  i &= 0x7f;
-  double x = j * zt.w[i];
-  if (j < zt.k[i]) {
-    accept = true;
-    val = sign * x;
-    return 2;
+// A chunk is parsed window by window: with block q of the chunk come its 24
+// numbers, and the iterations that may start at the 24 positions s = 0..23
+// beginning 3 numbers before them can be finished (an iteration reads at
+// most 4 numbers).  The 3 numbers before the first block are the newest ones
+// of the chunk's start state.  So a chunk covers the starts from 3 numbers
+// before its first block to 4 before its end, the parse enters it at s = 0,
+// 1, 2 or 3, and the stream itself starts at s = 3 of chunk 0.
+constexpr int ZIG_WIN = 27;   // numbers a window's iterations read
+constexpr int ZIG_START = 3;
+
+// An iteration of gsl_ran_gaussian_ziggurat starting at s reads number s
+// (layer and sign) and s + 1 (abscissa); nearly always the abscissa lies in
+// the layer's inner part and the iteration accepts with 2 numbers read.  Bit
+// s of the result: it does.  No branches: the others are resolved after.
+__device__ __forceinline__ uint32_t zig_fast(const uint32_t (&num)[ZIG_WIN], const ZigTabs &zt) {
+  uint32_t f = 0;
+#pragma unroll
+  for (int s = 23; s >= 0; --s) {
+    uint32_t d = num[s + 1] - zt.k[num[s] & 0x7Fu];   // both below 2^25: the sign bit is the comparison
+    f = __builtin_amdgcn_alignbit(f, d, 31);
   }
+  return f;
+}
+
+// the iteration's magnitude when it is accepted by the layer's own abscissa
+__device__ __forceinline__ double zig_abscissa(uint32_t k1, uint32_t k2, const ZigTabs &zt) {
+  return double(k2) * zt.w[k1 & 0x7Fu];
+}
+
+// An iteration that is not accepted at once: k1..k4 are the numbers from its
+// start on.  Whether it accepts; x receives its magnitude.  It reads 4
+// numbers in the tail (layer 127), otherwise 3.
+__device__ __forceinline__ bool zig_slow(uint32_t k1, uint32_t k2, uint32_t k3, uint32_t k4, const ZigTabs &zt,
+                                         double &x) {
+  const double PARAM_R = 3.44428647676;
+  uint32_t i = k1 & 0x7Fu;
   double y;
-  int used;
   if (i < 127) {
+    x = zig_abscissa(k1, k2, zt);
     double y0 = zt.y[i], y1 = zt.y[i + 1];
-    double U1 = get(pos + 2) / 16777216.0;
+    double U1 = k3 / 16777216.0;
     y = y1 + (y0 - y1) * U1;
-    used = 3;
   } else {
-    double U1 = 1.0 - get(pos + 2) / 16777216.0;
-    double U2 = get(pos + 3) / 16777216.0;
+    double U1 = 1.0 - k3 / 16777216.0;
+    double U2 = k4 / 16777216.0;
     x = PARAM_R - log(U1) / PARAM_R;
     y = exp(-PARAM_R * (x - 0.5 * PARAM_R)) * U2;
-    used = 4;
   }
-  accept = y < exp(-0.5 * x * x);
-  val = sign * x;
-  return used;
+  return y < exp(-0.5 * x * x);
 }
 
-// Chunks are parsed straight out of the generator: each thread keeps the
-// newest 48 numbers of its chunk in an LDS ring (slot-major, so a wave's
-// threads touch consecutive banks) and advances its ziggurat cursors while
-// an iteration is guaranteed to fit in the numbers generated so far.
-constexpr int RING = 48;
-
-template <int SLOTS> struct RingT {
-  uint32_t *base;
-  int stride;
-  // positions within a chunk are non-negative and below 2^31
-  __device__ __forceinline__ uint32_t get(long pos) const { return base[int(uint32_t(pos) % SLOTS) * stride]; }
-  __device__ __forceinline__ void put(long pos, uint32_t v) const { base[int(uint32_t(pos) % SLOTS) * stride] = v; }
-};
-using Ring = RingT<RING>;
-
-template <class R> __device__ __forceinline__ void push_block(const R &r, long at, const uint64_t *x) {
+// the window's numbers: the 3 kept from the block before, then this block's
+__device__ __forceinline__ void zig_window(const Lux &x, uint32_t (&num)[ZIG_WIN]) {
+  num[0] = num[24];
+  num[1] = num[25];
+  num[2] = num[26];
 #pragma unroll
   for (int k = 0; k < 12; ++k) {
-    r.put(at + 2 * k, uint32_t(x[k] & 0xFFFFFF));
-    r.put(at + 2 * k + 1, uint32_t(x[k] >> 24));
+    num[3 + 2 * k] = lux_first(x, k);
+    num[4 + 2 * k] = lux_second(x, k);
   }
 }
-
-// Raw numbers of the summary pass, kept for the emit pass: block q, number k
-// of chunk t at ((t/64)*rawb + q*24 + k)*64 + t%64 with rawb = (kc+1)*24, so a
-// wavefront's 64 chunks store and load each number as one contiguous 256-byte
-// segment.
-__device__ __forceinline__ size_t raw_at(long t, int q, int k, int rawb) {
-  return (size_t(t >> 6) * rawb + q * 24 + k) * 64 + (t & 63);
+// before the first block: the start state's newest numbers
+__device__ __forceinline__ void zig_before(const Lux &x, uint32_t (&num)[ZIG_WIN]) {
+  num[24] = lux_second(x, 10);
+  num[25] = lux_first(x, 11);
+  num[26] = lux_second(x, 11);
 }
+// length of the run of accepted 2-number iterations from s, in numbers; it
+// stops at 24 or 25 at the latest
+__device__ __forceinline__ int zig_run(uint32_t fast, int s) { return __ffs(int(~(fast >> s) & 0x55555555u)) - 1; }
 
-// Pass 1: per chunk, the exit offset and Gaussian count for each of the four
-// possible entry offsets.  Once the four cursors sit on the same position
-// they share the rest of the parse, so only one is advanced and its later
-// acceptances are added to all four.
-__global__ __launch_bounds__(256) void k_rng_summary(const RngDev *__restrict__ pp, long nchunks,
-                                                    uint32_t *__restrict__ summary,
-                                                    uint32_t *__restrict__ raw) {
-  extern __shared__ uint32_t ring_mem[];
-  __shared__ ZigTabs zt;
-  zig_tabs_load(zt);
-  long t = long(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t >= nchunks) return;
-  Ring ring{ring_mem + threadIdx.x, int(blockDim.x)};
-  const RngDev &p = *pp;
-  const int kc = p.kc, ch = kc * 24, rawb = (kc + 1) * 24;
-  uint64_t x[12];
-  int64_t c;
-  chunk_start_state(p, t, x, c);
-  auto get = [&](long pos) { return ring.get(pos); };
-  long cur[4] = {0, 1, 2, 3};
-  uint32_t cnt[4] = {0, 0, 0, 0};
-  uint32_t shared_cnt = 0;   // acceptances after the cursors merged
-  bool merged = false;
-  long avail = 0;
-  for (int q = 0; q <= kc; ++q) {
-    ranlux_block(x, c);
-    push_block(ring, avail, x);
-#pragma unroll
-    for (int k = 0; k < 12; ++k) {
-      raw[raw_at(t, q, 2 * k, rawb)] = uint32_t(x[k] & 0xFFFFFF);
-      raw[raw_at(t, q, 2 * k + 1, rawb)] = uint32_t(x[k] >> 24);
-    }
-    avail += 24;
-    if (merged) {
-      long pos = cur[0];
-      while (pos < ch && pos + 4 <= avail) {
-        bool acc;
-        double v;
-        pos += zig_iter(get, pos, acc, v, zt);
-        shared_cnt += acc;
-      }
-      cur[0] = pos;
-      if (pos >= ch) break;
-    } else {
-      bool done = true;
-      for (int e = 0; e < 4; ++e) {
-        long pos = cur[e];
-        while (pos < ch && pos + 4 <= avail) {
-          bool acc;
-          double v;
-          pos += zig_iter(get, pos, acc, v, zt);
-          cnt[e] += acc;
-        }
-        cur[e] = pos;
-        done &= pos >= ch;
-      }
-      merged = cur[0] == cur[1] && cur[0] == cur[2] && cur[0] == cur[3];
-      if (done) break;
-    }
-  }
-  uint32_t ex = 0;
-  for (int e = 0; e < 4; ++e) {
-    long end = merged ? cur[0] : cur[e];
-    ex |= uint32_t(end - ch) << (2 * e);
-    summary[t * 5 + 1 + e] = cnt[e] + (merged ? shared_cnt : 0);
-  }
-  summary[t * 5] = ex;
-}
+constexpr int RNG_THREADS = 256;   // four wavefronts, each 64 consecutive chunks of one stream
+constexpr int RNG_SEGS = RNG_THREADS / 64;
 
-// Pass 2a: compose the maps of SEG consecutive chunks.
+// entry offset -> exit offset (2 bits each in ex) and accepted count
 struct Map4 {
-  uint8_t ex[4];
+  uint32_t ex;
   uint32_t cnt[4];
 };
-__device__ __forceinline__ Map4 compose(const Map4 &a, const Map4 &b) {
+__device__ __forceinline__ uint32_t pick4(const uint32_t (&v)[4], uint32_t e) {
+  // all four read first: selected by address they would live in memory
+  const uint32_t a = v[0], b = v[1], c = v[2], d = v[3];
+  const uint32_t lo = e & 1u ? b : a, hi = e & 1u ? d : c;
+  return e & 2u ? hi : lo;
+}
+__device__ __forceinline__ Map4 compose(const Map4 &a, const Map4 &b) {   // a, then b
   Map4 r;
+  r.ex = 0;
+#pragma unroll
   for (int e = 0; e < 4; ++e) {
-    r.ex[e] = b.ex[a.ex[e]];
-    r.cnt[e] = a.cnt[e] + b.cnt[a.ex[e]];
+    uint32_t m = (a.ex >> (2 * e)) & 3u;
+    r.ex |= ((b.ex >> (2 * m)) & 3u) << (2 * e);
+    r.cnt[e] = a.cnt[e] + pick4(b.cnt, m);
   }
   return r;
 }
+constexpr uint32_t MAP_ID = 0xE4u;   // e -> e
 __device__ __forceinline__ Map4 load_map(const uint32_t *s, long t) {
   Map4 m;
-  uint32_t ex = s[t * 5];
-  for (int e = 0; e < 4; ++e) {
-    m.ex[e] = (ex >> (2 * e)) & 3;
-    m.cnt[e] = s[t * 5 + 1 + e];
-  }
+  m.ex = s[t * 5];
+  for (int e = 0; e < 4; ++e) m.cnt[e] = s[t * 5 + 1 + e];
   return m;
 }
-__device__ __forceinline__ Map4 identity_map() {
+__device__ __forceinline__ void store_map(uint32_t *s, long t, const Map4 &m) {
+  s[t * 5] = m.ex;
+  for (int e = 0; e < 4; ++e) s[t * 5 + 1 + e] = m.cnt[e];
+}
+// Words 0..23 of chunk t's start state, 64 chunks side by side; the borrow
+// rides in the free half of the first upper word
+__device__ __forceinline__ size_t state_at(long seg, int k, int lane) { return (size_t(seg) * 24 + k) * 64 + lane; }
+
+// Pass 1: per chunk the map from each of the four entry offsets, composed
+// with those of the wavefront's earlier chunks (maps), per wavefront the
+// whole (segmaps), and the chunk's start state for pass 3.  Bound by integer
+// issue (the recurrence), four wavefronts per SIMD by registers.
+// 1.1e9 Gaussians: 4.4 ms, where the 64-bit recurrence with an iteration at
+// a time parsed from all entries, storing the numbers, took 10.6 ms; 20011
+// Gaussians: 22 us against 125 us.
+__global__ __launch_bounds__(RNG_THREADS) void k_rng_summary(const RngDev *__restrict__ streams,
+                                                             const uint32_t *__restrict__ seg_stream, long nseg,
+                                                             int kclog, uint32_t *__restrict__ state,
+                                                             uint32_t *__restrict__ maps,
+                                                             uint32_t *__restrict__ segmaps) {
+  __shared__ uint32_t ring[ZIG_WIN * RNG_THREADS];   // a lane's numbers, for the slow iterations' indexed reads
+  __shared__ ZigTabs zt;
+  zig_tabs_load(zt);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const long seg = long(blockIdx.x) * RNG_SEGS + __builtin_amdgcn_readfirstlane(tid >> 6);
+  if (seg >= nseg) return;
+  const RngDev &p = streams[seg_stream ? seg_stream[seg] : 0u];
+  Lux x;
+  chunk_start_state(p, kclog, (seg - long(p.seg0)) * 64 + lane, x);
+#pragma unroll
+  for (int k = 0; k < 12; ++k) {
+    state[state_at(seg, k, lane)] = x.lo[k];
+    state[state_at(seg, 12 + k, lane)] = k == 0 ? x.hi[k] | x.c << 16 : x.hi[k];
+  }
+  uint32_t num[ZIG_WIN];
+  zig_before(x, num);
+  int cur[4] = {0, 1, 2, 3};
+  uint32_t cnt[4] = {0, 0, 0, 0};
+  bool merged = false;   // one cursor is left: its acceptances count for all
+  uint32_t shared_cnt = 0;
+  const int kc = 1 << kclog;
+#pragma unroll 1
+  for (int q = 0; q < kc; ++q) {
+    lux_block(x);
+    zig_window(x, num);
+#pragma unroll
+    for (int s = 0; s < ZIG_WIN; ++s) ring[s * RNG_THREADS + tid] = num[s];
+    const uint32_t fast = zig_fast(num, zt);
+    // every start of the window that is not accepted at once, on a cursor's
+    // way or not: about one in 42
+    uint32_t acc = fast, four = 0;
+    for (uint32_t z = ~fast & 0xFFFFFFu; z; z &= z - 1) {
+      int s = __ffs(int(z)) - 1;
+      const uint32_t *r = ring + s * RNG_THREADS + tid;
+      uint32_t k1 = r[0];
+      double v;
+      if (zig_slow(k1, r[RNG_THREADS], r[2 * RNG_THREADS], r[3 * RNG_THREADS], zt, v)) acc |= 1u << s;
+      if ((k1 & 0x7Fu) == 127u) four |= 1u << s;
+    }
+    auto walk = [&](int &pos) {
+      uint32_t n = 0;
+      int s = pos;
+      while (s < 24) {
+        int r = zig_run(fast, s);
+        n += r >> 1;
+        s += r;
+        if (s >= 24) break;
+        n += (acc >> s) & 1u;
+        s += 3 + int((four >> s) & 1u);
+      }
+      pos = s - 24;
+      return n;
+    };
+    if (merged) {
+      shared_cnt += walk(cur[0]);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) cnt[e] += walk(cur[e]);
+      merged = cur[0] == cur[1] && cur[0] == cur[2] && cur[0] == cur[3];
+    }
+  }
   Map4 m;
+  m.ex = 0;
+#pragma unroll
   for (int e = 0; e < 4; ++e) {
-    m.ex[e] = e;
-    m.cnt[e] = 0;
+    const uint32_t own = uint32_t(cur[e]), one = uint32_t(cur[0]);
+    m.ex |= (merged ? one : own) << (2 * e);
+    m.cnt[e] = cnt[e] + shared_cnt;
   }
-  return m;
-}
-constexpr int SEG = 64;
-
-__global__ __launch_bounds__(256) void k_rng_seg_compose(const uint32_t *__restrict__ summary, long nchunks, long nseg,
-                                                         uint32_t *__restrict__ segmaps) {
-  long s = long(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (s >= nseg) return;
-  Map4 acc = identity_map();
-  long b0 = s * SEG, b1 = min(nchunks, b0 + SEG);
-  for (long t = b0; t < b1; ++t) acc = compose(acc, load_map(summary, t));
-  uint32_t ex = 0;
-  for (int e = 0; e < 4; ++e) {
-    ex |= uint32_t(acc.ex[e]) << (2 * e);
-    segmaps[s * 5 + 1 + e] = acc.cnt[e];
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    Map4 a;
+    a.ex = __shfl_up(m.ex, off);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) a.cnt[e] = __shfl_up(m.cnt[e], off);
+    if (lane >= off) m = compose(a, m);
   }
-  segmaps[s * 5] = ex;
+  if (lane == 63) store_map(segmaps, seg, m);
+  Map4 before;
+  before.ex = __shfl_up(m.ex, 1);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) before.cnt[e] = __shfl_up(m.cnt[e], 1);
+  if (lane == 0) before = Map4{MAP_ID, {0, 0, 0, 0}};
+  store_map(maps, seg * 64 + lane, before);
 }
 
-// Pass 2b: one workgroup scans the segment maps; segstart[s] = (base << 2) | entry.
-__global__ __launch_bounds__(1024) void k_rng_seg_scan(const uint32_t *__restrict__ segmaps, long nseg,
-                                                      uint64_t *__restrict__ segstart) {
-  __shared__ Map4 sm[1024];
-  int tid = threadIdx.x;
-  long per = (nseg + 1023) / 1024;
-  long b0 = tid * per, b1 = min(nseg, b0 + per);
-  Map4 acc = identity_map();
-  for (long t = b0; t < b1; ++t) acc = compose(acc, load_map(segmaps, t));
-  sm[tid] = acc;
+// Pass 2: one workgroup per stream scans its wavefronts' maps; segstart[s] =
+// (index of the stream's Gaussian the wavefront starts with << 2) | entry.
+// *flag gets 1 if a stream holds fewer Gaussians than are wanted.
+__global__ __launch_bounds__(1024) void k_rng_seg_scan(const RngDev *__restrict__ streams,
+                                                       const uint32_t *__restrict__ segmaps,
+                                                       uint64_t *__restrict__ segstart, uint32_t *__restrict__ flag,
+                                                       int flag_stride) {
+  __shared__ Map4 wave[16];
+  const RngDev &p = streams[blockIdx.x];
+  const long nseg = long(p.nseg), s0 = long(p.seg0);
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const long per = (nseg + 1023) / 1024;
+  const long b0 = min(nseg, tid * per), b1 = min(nseg, b0 + per);
+  Map4 m{MAP_ID, {0, 0, 0, 0}};
+  for (long t = b0; t < b1; ++t) m = compose(m, load_map(segmaps, s0 + t));
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    Map4 a;
+    a.ex = __shfl_up(m.ex, off);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) a.cnt[e] = __shfl_up(m.cnt[e], off);
+    if (lane >= off) m = compose(a, m);
+  }
+  if (lane == 63) wave[w] = m;
+  Map4 before;
+  before.ex = __shfl_up(m.ex, 1);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) before.cnt[e] = __shfl_up(m.cnt[e], 1);
   __syncthreads();
-  for (int off = 1; off < 1024; off <<= 1) {
-    Map4 v = sm[tid];
-    if (tid >= off) v = compose(sm[tid - off], v);
-    __syncthreads();
-    sm[tid] = v;
-    __syncthreads();
-  }
-  int e = 0;
+  uint32_t e = ZIG_START;
   uint64_t base = 0;
-  if (tid > 0) {
-    e = sm[tid - 1].ex[0];
-    base = sm[tid - 1].cnt[0];
+  for (int i = 0; i < w; ++i) {
+    base += pick4(wave[i].cnt, e);
+    e = (wave[i].ex >> (2 * e)) & 3u;
+  }
+  if (lane > 0) {
+    base += pick4(before.cnt, e);
+    e = (before.ex >> (2 * e)) & 3u;
   }
   for (long t = b0; t < b1; ++t) {
-    segstart[t] = (base << 2) | uint64_t(e);
-    Map4 m = load_map(segmaps, t);
-    base += m.cnt[e];
-    e = m.ex[e];
+    segstart[s0 + t] = (base << 2) | uint64_t(e);
+    Map4 a = load_map(segmaps, s0 + t);
+    base += pick4(a.cnt, e);
+    e = (a.ex >> (2 * e)) & 3u;
   }
+  if (b1 == nseg && (b0 < b1 || nseg == 0) && base < p.total) flag[size_t(blockIdx.x) * flag_stride] = 1u;
 }
 
-// Pass 3: regenerate each chunk, parse from its true entry, write Gaussians.
 struct LevelTargets {
   void *f[4];
   int n[4];        // grid size of a padded real field; 0 for a dense array
@@ -500,178 +609,180 @@ struct LevelTargets {
   double scale;    // every value is stored as T(v * scale)
 };
 
-// Pass 3 works one wavefront per workgroup.  Each lane parses its chunk from
-// the stored raw numbers (read through an LDS ring, one coalesced block at a
-// time) and stages its Gaussians in LDS; lanes holding 32 or more flush
-// them cooperatively, two lanes' runs of 32 consecutive cells per store
-// instruction, so every store writes whole 128-byte lines.
-constexpr int EMIT_RING = 32;
-// staged Gaussians per lane: a flush leaves fewer than EMIT_FLUSH and one
-// block of 24 numbers (plus up to 3 left over) adds at most 13
-constexpr int EMIT_FLUSH = 32;   // flushing 16 at a time ran slower at 1024^3 (more barriers than occupancy gained)
-constexpr int EMIT_STAGE = 48;
-static_assert(EMIT_FLUSH - 1 + 13 <= EMIT_STAGE, "staging overflow");
+// Where a lane's next Gaussian goes: its cell and the cells left in its row
+// (a dense target is one row)
+template <typename T> struct CellCursor {
+  T *p;
+  uint64_t g;       // index of that Gaussian in the targets' order
+  uint64_t end;     // end of the target it lies in
+  uint32_t left;    // cells of the row from p on
+  uint32_t n;
+  __device__ __forceinline__ void seek(const LevelTargets &lt, uint64_t at) {
+    g = at;
+    int L = g < lt.cum[0] ? 0 : g < lt.cum[1] ? 1 : g < lt.cum[2] ? 2 : 3;
+    size_t i = g - (L ? lt.cum[L - 1] : 0);
+    end = lt.cum[L];
+    n = uint32_t(lt.n[L]);
+    if (n == 0) {
+      p = reinterpret_cast<T *>(lt.f[L]) + i;
+      left = uint32_t(min(uint64_t(0xFFFFFFFFu), end - g));
+      return;
+    }
+    size_t row = i / n, z = i - row * n;
+    p = reinterpret_cast<T *>(lt.f[L]) + row * (n + 2) + z;
+    left = n - uint32_t(z);
+  }
+  // past m cells of the row (m <= left)
+  __device__ __forceinline__ void step(const LevelTargets &lt, uint32_t m, uint64_t total) {
+    p += m;
+    g += m;
+    left -= m;
+    if (left == 0) {
+      if (n != 0 && g < end) {
+        p += 2;
+        left = n;
+      } else if (g < total) {
+        seek(lt, g);
+      }
+    }
+  }
+};
 
+// Pass 3 stages a lane's Gaussians in LDS and stores them four at a time as
+// they complete (16 or 32 bytes a lane: a store of single values takes one
+// address per lane, and four times as many).  A window adds at most 12 to
+// the at most 3 left over.
+constexpr int EMIT_STAGE = 16;
+template <typename T> struct __attribute__((packed, aligned(sizeof(T)))) Four {
+  T v[4];
+};
+
+// Pass 3: generate each chunk again, parse it from its true entry, write the
+// Gaussians.  Bound by integer issue like pass 1, three wavefronts per SIMD
+// (FP32) by LDS.  1.1e9 Gaussians in FP32: 5.4 ms, where reading stored
+// numbers back, parsing an iteration at a time and storing runs
+// cooperatively took 11.0 ms; 20011 Gaussians: 12 us against 56 us.
 template <typename T>
-__device__ __forceinline__ T *cell_ptr(const LevelTargets &lt, uint64_t g) {
-  int L = g < lt.cum[0] ? 0 : g < lt.cum[1] ? 1 : g < lt.cum[2] ? 2 : 3;
-  size_t i = g - (L ? lt.cum[L - 1] : 0);
-  int n = lt.n[L];
-  if (n == 0) return reinterpret_cast<T *>(lt.f[L]) + i;
-  size_t nn = size_t(n) * n;
-  size_t xx = i / nn, r = i - xx * nn, y = r / n, z = r - y * n;
-  return reinterpret_cast<T *>(lt.f[L]) + (xx * n + y) * (n + 2) + z;
-}
-
-// Level and (x, y, z) of global Gaussian index g; n[L] == 0 (a dense target)
-// leaves the coordinates unused
-__device__ __forceinline__ void cell_coords(const LevelTargets &lt, uint64_t g, int &L, uint32_t &x, uint32_t &y,
-                                            uint32_t &z) {
-  L = g < lt.cum[0] ? 0 : g < lt.cum[1] ? 1 : g < lt.cum[2] ? 2 : 3;
-  size_t i = g - (L ? lt.cum[L - 1] : 0);
-  int n = lt.n[L];
-  x = y = z = 0;
-  if (n == 0) return;
-  size_t nn = size_t(n) * n;
-  size_t xx = i / nn, r = i - xx * nn, yy = r / n;
-  x = uint32_t(xx);
-  y = uint32_t(yy);
-  z = uint32_t(r - yy * n);
-}
-
-template <typename T>
-__global__ __launch_bounds__(64) void k_rng_emit(const uint32_t *__restrict__ raw, long nchunks,
-                                                const uint32_t *__restrict__ summary,
-                                                const uint64_t *__restrict__ segstart, LevelTargets lt,
-                                                size_t total, int kc) {
-  __shared__ uint32_t ring_mem[EMIT_RING * 64];
-  __shared__ T stage_mem[EMIT_STAGE * 64];
+__global__ __launch_bounds__(RNG_THREADS) void k_rng_emit(const RngDev *__restrict__ streams,
+                                                          const uint32_t *__restrict__ seg_stream, long nseg,
+                                                          int kclog, const uint32_t *__restrict__ state,
+                                                          const uint32_t *__restrict__ maps,
+                                                          const uint64_t *__restrict__ segstart, LevelTargets lt) {
+  __shared__ uint32_t ring[ZIG_WIN * RNG_THREADS];
+  __shared__ T stage[EMIT_STAGE * RNG_THREADS];
   __shared__ ZigTabs zt;
   zig_tabs_load(zt);
-  const int lane = threadIdx.x;
-  long t = long(blockIdx.x) * 64 + lane;
-  bool active = t < nchunks;
-  uint64_t g = 0;
-  int e = 0;
-  if (active) {
-    long s = t / SEG;
-    uint64_t ss = segstart[s];
-    g = ss >> 2;
-    e = int(ss & 3);
-    for (long u = s * SEG; u < t; ++u) {
-      // the map's entry e only (no per-thread array indexed by e)
-      uint32_t exw = summary[u * 5];
-      g += summary[u * 5 + 1 + e];
-      e = int((exw >> (2 * e)) & 3u);
-    }
-    if (g >= total) active = false;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const long seg = long(blockIdx.x) * RNG_SEGS + __builtin_amdgcn_readfirstlane(tid >> 6);
+  if (seg >= nseg) return;
+  const RngDev &p = streams[seg_stream ? seg_stream[seg] : 0u];
+  const uint64_t ss = segstart[seg];
+  Map4 before = load_map(maps, seg * 64 + lane);
+  const uint32_t e = uint32_t(ss & 3u);
+  // indexes in the targets' order from here on
+  const uint64_t total = p.out0 + p.total;
+  uint64_t g = p.out0 + (ss >> 2) + pick4(before.cnt, e);
+  int pos = int((before.ex >> (2 * e)) & 3u);
+  bool live = g < total;
+  if (!__any(live)) return;
+  Lux x;
+#pragma unroll
+  for (int k = 0; k < 12; ++k) {
+    x.lo[k] = state[state_at(seg, k, lane)];
+    x.hi[k] = state[state_at(seg, 12 + k, lane)];
   }
-  RingT<EMIT_RING> ring{ring_mem + lane, 64};
-  auto get = [&](long pos) { return ring.get(pos); };
-  long pos = e;
-  long avail = 0;
-  int fill = 0;
-  uint64_t gstage = g;   // global index of staged slot 0
-  auto flush = [&](bool final) {
-    __syncthreads();
-    int want = final ? fill : (fill >= EMIT_FLUSH ? EMIT_FLUSH : 0);
-    unsigned long long mask = __ballot(want > 0);
-    // each lane locates its own run's first cell once; the 32 lanes storing
-    // a run step from there (no divisions per stored value)
-    int myL = 0;
-    uint32_t mx = 0, my = 0, mz = 0;
-    if (want > 0) cell_coords(lt, gstage, myL, mx, my, mz);
-    while (mask) {
-      int s0 = __ffsll((long long)mask) - 1;
-      mask &= mask - 1;
-      int s1 = -1;
-      if (mask) {
-        s1 = __ffsll((long long)mask) - 1;
-        mask &= mask - 1;
+  x.c = x.hi[0] >> 16;
+  x.hi[0] &= 0xFFFFu;
+  CellCursor<T> cell;
+  if (live) cell.seek(lt, g);
+  uint32_t num[ZIG_WIN];
+  zig_before(x, num);
+  int head = 0, fill = 0;   // staged Gaussians: slots head .. head + fill - 1 (mod EMIT_STAGE)
+  auto slot = [&](int i) -> T & { return stage[((head + i) & (EMIT_STAGE - 1)) * RNG_THREADS + tid]; };
+  const int kc = 1 << kclog;
+#pragma unroll 1
+  for (int q = 0; q < kc; ++q) {
+    if (!__any(live)) break;
+    lux_block(x);
+    zig_window(x, num);
+#pragma unroll
+    for (int s = 0; s < ZIG_WIN; ++s) ring[s * RNG_THREADS + tid] = num[s];
+    const uint32_t fast = zig_fast(num, zt);
+    // the accepted starts on the way (all), and those of them whose value is
+    // the layer's abscissa (plain); the tail's values are staged here
+    uint32_t all = 0, plain = 0;
+    int s = live ? pos : 24;
+    while (s < 24) {
+      int r = zig_run(fast, s);
+      uint32_t run = (0x555555u & ((1u << r) - 1u)) << s;
+      all |= run;
+      plain |= run;
+      s += r;
+      if (s >= 24) break;
+      const uint32_t *k = ring + s * RNG_THREADS + tid;
+      uint32_t k1 = k[0];
+      bool tail = (k1 & 0x7Fu) == 127u;
+      double v;
+      if (zig_slow(k1, k[RNG_THREADS], k[2 * RNG_THREADS], k[3 * RNG_THREADS], zt, v)) {
+        if (tail) slot(fill + __popc(all)) = T(((k1 & 0x80u) ? v : -v) * lt.scale);
+        else plain |= 1u << s;
+        all |= 1u << s;
       }
-      int src = lane < 32 ? s0 : s1;
-      int j = lane & 31;
-      int sl = src < 0 ? 0 : src;
-      int w = __shfl(want, sl);
-      uint64_t gs = __shfl(gstage, sl);
-      int L = __shfl(myL, sl);
-      uint32_t x = __shfl(mx, sl), y = __shfl(my, sl), z = __shfl(mz, sl);
-      if (src >= 0 && j < w) {
-        T *ptr;
-        int n = lt.n[L];
-        if (n != 0 && gs + j < lt.cum[L]) {
-          uint32_t zz = z + j, yy = y, xx = x;
-          while (zz >= uint32_t(n)) {   // at most once when n >= 32
-            zz -= n;
-            if (++yy == uint32_t(n)) {
-              yy = 0;
-              ++xx;
-            }
+      s += tail ? 4 : 3;
+    }
+    pos = s - 24;
+    // at most one of the starts 2k, 2k + 1 is on the way
+#pragma unroll
+    for (int k = 0; k < 12; ++k) {
+      uint32_t b = (plain >> (2 * k)) & 3u;
+      uint32_t k1 = b & 2u ? num[2 * k + 1] : num[2 * k], k2 = b & 2u ? num[2 * k + 2] : num[2 * k + 1];
+      double v = zig_abscissa(k1, k2, zt);
+      if (b) slot(fill + __popc(all & ((1u << (2 * k)) - 1u))) = T(((k1 & 0x80u) ? v : -v) * lt.scale);
+    }
+    fill += __popc(all);
+    while (fill >= 4 && live) {
+      T v[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = slot(i);
+      if (cell.left >= 4 && total - cell.g >= 4) {
+        *reinterpret_cast<Four<T> *>(cell.p) = Four<T>{{v[0], v[1], v[2], v[3]}};
+        cell.step(lt, 4, total);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (cell.g < total) {
+            *cell.p = v[i];
+            cell.step(lt, 1, total);
           }
-          ptr = reinterpret_cast<T *>(lt.f[L]) + (size_t(xx) * n + yy) * (n + 2) + zz;
-        } else {
-          ptr = cell_ptr<T>(lt, gs + j);   // a dense target, or a run that crosses into the next level
-        }
-        *ptr = stage_mem[j * 64 + src];
       }
+      head += 4;
+      fill -= 4;
+      live = cell.g < total;
     }
-    __syncthreads();
-    if (want > 0) {
-      for (int j = 0; j + want < fill; ++j) stage_mem[j * 64 + lane] = stage_mem[(j + want) * 64 + lane];
-      fill -= want;
-      gstage += want;
-    }
-    __syncthreads();
-  };
-  const int ch = kc * 24, rawb = (kc + 1) * 24;
-  // the next block's numbers are loaded while this block is parsed (every
-  // block q <= kc of a chunk lies inside the raw buffer)
-  uint32_t nxt[24];
-  if (active) {
-#pragma unroll
-    for (int k = 0; k < 24; ++k) nxt[k] = raw[raw_at(t, 0, k, rawb)];
   }
-  for (int q = 0; q <= kc; ++q) {
-    bool busy = active && pos < ch && g < total;
-    if (!__any(busy)) break;
-    if (busy) {
-#pragma unroll
-      for (int k = 0; k < 24; ++k) ring.put(avail + k, nxt[k]);
-      avail += 24;
-      if (q < kc) {
-#pragma unroll
-        for (int k = 0; k < 24; ++k) nxt[k] = raw[raw_at(t, q + 1, k, rawb)];
-      }
-      while (pos < ch && pos + 4 <= avail && g < total) {
-        bool acc;
-        double v;
-        pos += zig_iter(get, pos, acc, v, zt);
-        if (acc) {
-          stage_mem[fill * 64 + lane] = T(v * lt.scale);
-          ++fill;
-          ++g;
-        }
-      }
+  if (live)
+    for (int i = 0; i < fill && cell.g < total; ++i) {
+      *cell.p = slot(i);
+      cell.step(lt, 1, total);
     }
-    flush(false);
-  }
-  flush(true);
 }
 
 // Raw 24-bit numbers in stream order (for bit-exactness checks).
-__global__ __launch_bounds__(256) void k_rng_raw(RngDev p, long nchunks, uint32_t *__restrict__ out, size_t n) {
+__global__ __launch_bounds__(256) void k_rng_raw(RngDev p, int kclog, long nchunks, uint32_t *__restrict__ out,
+                                                 size_t n) {
   long t = long(blockIdx.x) * blockDim.x + threadIdx.x;
   if (t >= nchunks) return;
-  uint64_t x[12];
-  int64_t c;
-  chunk_start_state(p, t, x, c);
-  size_t base = size_t(t) * (p.kc * 24);
-  for (int q = 0; q < p.kc; ++q) {
-    ranlux_block(x, c);
+  Lux x;
+  chunk_start_state(p, kclog, t, x);
+  const int kc = 1 << kclog;
+  size_t base = size_t(t) * (kc * 24);
+  for (int q = 0; q < kc; ++q) {
+    lux_block(x);
+#pragma unroll
     for (int k = 0; k < 12; ++k) {
       size_t i = base + q * 24 + 2 * k;
-      if (i < n) out[i] = uint32_t(x[k] & 0xFFFFFF);
-      if (i + 1 < n) out[i + 1] = uint32_t(x[k] >> 24);
+      if (i < n) out[i] = lux_first(x, k);
+      if (i + 1 < n) out[i + 1] = lux_second(x, k);
     }
   }
 }
@@ -725,37 +836,17 @@ static void u576_powmod(const uint64_t *base, u128 e_lo, uint64_t *r) {
   memcpy(r, acc, sizeof acc);
 }
 
-void rng_plan(unsigned long seed, size_t n_gaussians, RngPlan &plan) {
-  seed_words(seed, plan.seed_words);
-  // A = sum_j x_j b^j (12 words), B = sum_j x_{7+j} b^j (5 words)
-  uint64_t A[9], B[9];
-  u576_from_words(plan.seed_words, 12, A);
-  u576_from_words(plan.seed_words + 7, 5, B);
-  // reduce A mod m (A < 2^576 but may exceed m)
-  while (u576_geq_m(A)) u576_sub_m(A);
-  // V_0 = A - B (mod m) is the LCG state one step past the seed (carry 0)
-  uint64_t V[9];
-  {
-    uint64_t borrow = 0;
-    for (int i = 0; i < 9; ++i) {
-      u128 d = (u128)A[i] - B[i] - borrow;
-      V[i] = (uint64_t)d;
-      borrow = (uint64_t)(d >> 64) & 1;
-    }
-    if (borrow) {
-      // add m back
-      const uint64_t m[9] = {1, 0, 0, 0xFFFF000000000000ull, ~0ull, ~0ull, ~0ull, ~0ull, ~0ull};
-      u128 c = 0;
-      for (int i = 0; i < 9; ++i) {
-        u128 t = (u128)V[i] + m[i] + c;
-        V[i] = (uint64_t)t;
-        c = t >> 64;
-      }
-    }
-  }
-  // b^{-1} = m - b^11 + b^4 ; b^12 = b^5 - 1 (mod m)
-  uint64_t binv[9];
-  {
+// The constants of the jumps: b^12 and the device table d_jump, computed
+// once per process (about 1800 modular products)
+struct JumpTable {
+  uint64_t b12[9];
+  std::vector<uint64_t> w;   // as d_jump
+  JumpTable() : w(size_t(RNG_KC_LOG) * RNG_DIGITS * 64 * 9) {
+    uint64_t one_b[9] = {0};
+    put48(one_b, 48, 1);   // b
+    u576_powmod(one_b, 12, b12);
+    // b^{-1} = m - b^11 + b^4 (b^12 = b^5 - 1 mod m)
+    uint64_t binv[9];
     const uint64_t m[9] = {1, 0, 0, 0xFFFF000000000000ull, ~0ull, ~0ull, ~0ull, ~0ull, ~0ull};
     uint64_t b11[9] = {0}, b4[9] = {0};
     put48(b11, 48 * 11, 1);
@@ -772,69 +863,133 @@ void rng_plan(unsigned long seed, size_t n_gaussians, RngPlan &plan) {
       binv[i] = (uint64_t)t;
       c = t >> 64;
     }
+    for (int q = 0; q < RNG_KC_LOG; ++q) {
+      uint64_t step[9];   // one unit of the digit
+      u576_powmod(binv, (u128)397 << q, step);
+      for (int l = 0; l < RNG_DIGITS; ++l) {
+        uint64_t v[9] = {1, 0, 0, 0, 0, 0, 0, 0, 0}, t[9];
+        for (int d = 0; d < 64; ++d) {
+          memcpy(&w[((size_t(q) * RNG_DIGITS + l) * 64 + d) * 9], v, sizeof v);
+          u576_mulmod(v, step, t);
+          memcpy(v, t, sizeof v);
+        }
+        memcpy(step, v, sizeof step);   // step^64
+      }
+    }
   }
-  // raw numbers needed: 2 per Gaussian plus rejections (~1.2% of iterations
-  // take 3-4 numbers and may repeat); 2.2x plus slack is never exceeded in
-  // practice and is checked after the scan.  Chunks of kc blocks: long
-  // chunks amortise the jump to each chunk's start, and a small draw takes
-  // shorter ones (down to four blocks) so that it still has about 64k
-  // chunks (a wavefront per SIMD) to run on; shorter chunks than that spend
-  // more on the jumps than they gain in parallelism.
-  double need = 2.2 * double(n_gaussians) + 4096.0;
-  plan.kc = 64;
-  while (plan.kc > 4 && need / (plan.kc * 24.0) < 65536.0) plan.kc /= 2;
-  // The chunk-t start state is step T_t = 397*kc*t; the device decodes the
-  // LCG state V_{T-12} = Z_{T-11} = b^{-(T-12)} V_0 and runs 12 steps.
-  // y0 = b^{12} V_0 ;  jump[i] = b^{-397*kc*2^i}.
-  uint64_t b12[9];
-  {
-    uint64_t one_b[9] = {0};
-    put48(one_b, 48, 1);        // b
-    u576_powmod(one_b, 12, b12);
-  }
-  u576_mulmod(b12, V, plan.y0.w);
-  uint64_t step[9];
-  u576_powmod(binv, (u128)397 * plan.kc, step);
-  for (int i = 0; i < RngPlan::MAXBITS; ++i) {
-    memcpy(plan.jump[i].w, step, sizeof step);
-    uint64_t t[9];
-    u576_mulmod(step, step, t);
-    memcpy(step, t, sizeof t);
-  }
-  plan.nchunks = long(need / plan.ch()) + 2;
+};
+static const JumpTable &jump_table() {
+  static const JumpTable t;
+  return t;
 }
 
-static size_t raw_bytes(long nc, int kc) { return size_t((nc + 63) / 64) * 64 * size_t(kc + 1) * 24 * 4; }
+// The LCG state 12 steps before the stream's start: b^12 V_0, V_0 the state
+// one step past the seed (carry 0).  The device decodes V at 12 steps before
+// a chunk's start and runs 12 steps.
+static void start_value(const uint64_t *words, U576 &y0) {
+  // A = sum_j x_j b^j (12 words), B = sum_j x_{7+j} b^j (5 words), V_0 = A - B (mod m)
+  uint64_t A[9], B[9], V[9];
+  u576_from_words(words, 12, A);
+  u576_from_words(words + 7, 5, B);
+  while (u576_geq_m(A)) u576_sub_m(A);   // A < 2^576 but may exceed m
+  uint64_t borrow = 0;
+  for (int i = 0; i < 9; ++i) {
+    u128 d = (u128)A[i] - B[i] - borrow;
+    V[i] = (uint64_t)d;
+    borrow = (uint64_t)(d >> 64) & 1;
+  }
+  if (borrow) {
+    const uint64_t m[9] = {1, 0, 0, 0xFFFF000000000000ull, ~0ull, ~0ull, ~0ull, ~0ull, ~0ull};
+    u128 c = 0;
+    for (int i = 0; i < 9; ++i) {
+      u128 t = (u128)V[i] + m[i] + c;
+      V[i] = (uint64_t)t;
+      c = t >> 64;
+    }
+  }
+  u576_mulmod(jump_table().b12, V, y0.w);
+}
 
+// Raw numbers to have ready for n Gaussians: 2 per Gaussian plus rejections
+// (~1.2% of iterations take 3-4 numbers and may repeat); 2.2x plus slack is
+// never exceeded in practice and is checked after the scan.
+static double raw_needed(size_t n) { return 2.2 * double(n) + 4096.0; }
+
+void rng_plan(const std::vector<RngStream> &streams, RngPlan &plan) {
+  if (streams.empty()) throw std::runtime_error("RNG: no streams");
+  plan.streams = streams;
+  plan.seg0.clear();
+  double need = 0;
+  for (auto &s : streams) need += raw_needed(s.count);
+  // Chunks of kc blocks: long chunks amortise the jump to each chunk's start
+  // (about four blocks' time), and a small draw takes shorter ones so that
+  // it still has about 64k chunks (a wavefront per SIMD) to run on.
+  plan.kclog = RNG_KC_LOG - 1;
+  while (plan.kclog > 0 && need / (24.0 * (1 << plan.kclog)) < 65536.0) --plan.kclog;
+  plan.nseg = 0;
+  for (auto &s : streams) {
+    plan.seg0.push_back(plan.nseg);
+    long chunks = long(raw_needed(s.count) / plan.ch()) + 2;
+    plan.nseg += (chunks + 63) / 64;
+  }
+  if (plan.nseg > (1L << (6 * (RNG_DIGITS - 1)))) throw std::runtime_error("RNG: draw too large");
+}
+void rng_plan(unsigned long seed, size_t n_gaussians, RngPlan &plan) {
+  rng_plan(std::vector<RngStream>{{seed, n_gaussians, 0}}, plan);
+}
+
+static size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
+
+// Per chunk its start state (24 words) and map (5), per wavefront its map
+// and start; then the streams, and for several of them each wavefront's.
 size_t rng_workspace_bytes(const RngPlan &plan) {
-  long nc = plan.nchunks;
-  long nseg = (nc + SEG - 1) / SEG;
-  return (size_t(nc) * 5 * 4 + 255) / 256 * 256 + (size_t(nseg) * 5 * 4 + 255) / 256 * 256 +
-         (size_t(nseg) * 8 + 255) / 256 * 256 + raw_bytes(nc, plan.kc) + (sizeof(RngDev) + 255) / 256 * 256 + 256;
+  size_t ns = size_t(plan.nseg);
+  return align256(ns * 64 * 24 * 4) + align256(ns * 64 * 5 * 4) + align256(ns * 5 * 4) + align256(ns * 8) +
+         rng_dev_bytes(plan) + 256;
+}
+size_t rng_dev_bytes(const RngPlan &plan) {
+  size_t n = plan.streams.size();
+  return align256(n * sizeof(RngDev)) + (n > 1 ? align256(size_t(plan.nseg) * 4) : 0);
+}
+static RngDev to_dev(const RngPlan &plan, size_t i) {
+  RngDev d;
+  seed_words(plan.streams[i].seed, d.seed_words);
+  start_value(d.seed_words, d.y0);
+  d.seg0 = uint64_t(plan.seg0[i]);
+  d.nseg = uint64_t((i + 1 < plan.seg0.size() ? plan.seg0[i + 1] : plan.nseg) - plan.seg0[i]);
+  d.out0 = plan.streams[i].out0;
+  d.total = plan.streams[i].count;
+  return d;
+}
+void rng_dev_pack(const RngPlan &plan, void *host_dst) {
+  size_t n = plan.streams.size();
+  RngDev *d = (RngDev *)host_dst;
+  for (size_t i = 0; i < n; ++i) d[i] = to_dev(plan, i);
+  if (n == 1) return;
+  uint32_t *of = (uint32_t *)((char *)host_dst + align256(n * sizeof(RngDev)));
+  for (size_t i = 0; i < n; ++i)
+    for (uint64_t k = 0; k < d[i].nseg; ++k) of[d[i].seg0 + k] = uint32_t(i);
 }
 
 struct RngBufs {
-  RngDev *dev;   // the plan, read by the summary pass
-  uint32_t *summary, *segmaps, *raw;
+  uint32_t *state, *maps, *segmaps;
   uint64_t *segstart;
-  long nseg;
+  char *dev;
 };
 static RngBufs carve(const RngPlan &plan, void *ws, size_t bytes) {
-  long nc = plan.nchunks;
-  long nseg = (nc + SEG - 1) / SEG;
+  size_t ns = size_t(plan.nseg);
   char *p = (char *)ws;
   auto take = [&](size_t b) {
     char *r = p;
-    p += (b + 255) & ~size_t(255);
+    p += align256(b);
     return r;
   };
   RngBufs r;
-  r.summary = (uint32_t *)take(size_t(nc) * 5 * 4);
-  r.segmaps = (uint32_t *)take(size_t(nseg) * 5 * 4);
-  r.segstart = (uint64_t *)take(size_t(nseg) * 8);
-  r.raw = (uint32_t *)take(raw_bytes(nc, plan.kc));
-  r.dev = (RngDev *)take(sizeof(RngDev));
-  r.nseg = nseg;
+  r.state = (uint32_t *)take(ns * 64 * 24 * 4);
+  r.maps = (uint32_t *)take(ns * 64 * 5 * 4);
+  r.segmaps = (uint32_t *)take(ns * 5 * 4);
+  r.segstart = (uint64_t *)take(ns * 8);
+  r.dev = take(rng_dev_bytes(plan));
   if ((size_t)(p - (char *)ws) > bytes) throw std::runtime_error("RNG workspace too small");
   return r;
 }
@@ -843,8 +998,8 @@ constexpr int RNG_MAX_DEVICES = 64;
 static std::mutex g_tables_mu;
 static bool g_tables_done[RNG_MAX_DEVICES];
 
-// the ziggurat tables into the constant memory of the current device (each
-// device has its own copy), once per device
+// the ziggurat and jump tables into the current device's memory (each device
+// has its own copy), once per device
 static void upload_tables() {
   int dev = 0;
   GIC_HIP(hipGetDevice(&dev));
@@ -854,69 +1009,29 @@ static void upload_tables() {
   GIC_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_ytab), ZIG_YTAB, sizeof ZIG_YTAB));
   GIC_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_wtab), ZIG_WTAB, sizeof ZIG_WTAB));
   GIC_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_ktab), ZIG_KTAB, sizeof ZIG_KTAB));
+  GIC_HIP(hipMemcpyToSymbol(HIP_SYMBOL(d_jump), jump_table().w.data(), sizeof(uint64_t) * jump_table().w.size()));
   g_tables_done[dev] = true;
 }
 
 void rng_prepare() { upload_tables(); }
 
-static RngDev to_dev(const RngPlan &plan) {
-  RngDev d;
-  memcpy(d.seed_words, plan.seed_words, sizeof d.seed_words);
-  d.y0 = plan.y0;
-  memcpy(d.jump, plan.jump, sizeof d.jump);
-  d.kc = plan.kc;
-  return d;
-}
-
-// the device-side form of the coverage check below
-__global__ void k_rng_cover(const uint64_t *__restrict__ last_start, const uint32_t *__restrict__ last_map,
-                            uint64_t total, uint32_t *__restrict__ flag) {
-  if (threadIdx.x != 0) return;
-  uint64_t last = *last_start;
-  uint64_t produced = (last >> 2) + last_map[1 + (last & 3)];
-  if (produced < total) *flag = 1u;
-}
-
-// the plan's device copy, written by a kernel from its arguments
-__global__ void k_rng_put_plan(RngDev d, RngDev *__restrict__ dst) {
+// a stream's device copy, written by a kernel from its arguments
+__global__ void k_rng_put_plan(RngDev d, RngDev *__restrict__ dst, uint32_t *__restrict__ flag) {
   const uint64_t *s = reinterpret_cast<const uint64_t *>(&d);
   uint64_t *o = reinterpret_cast<uint64_t *>(dst);
   for (int i = threadIdx.x; i < int(sizeof(RngDev) / 8); i += blockDim.x) o[i] = s[i];
+  if (flag && threadIdx.x == 0) *flag = 0;
 }
 static_assert(sizeof(RngDev) % 8 == 0, "RngDev is copied as 64-bit words");
 
-size_t rng_dev_bytes() { return sizeof(RngDev); }
-void rng_dev_pack(const RngPlan &plan, void *host_dst) {
-  RngDev d = to_dev(plan);
-  memcpy(host_dst, &d, sizeof d);
-}
-
 template <typename T>
 static void draw_real_list(const RngPlan &plan, const RngLevelOut *levels, size_t nlev, void *ws, size_t ws_bytes,
-                           hipStream_t st, TimingHook *hook, double scale, uint32_t *cover_flag, const void *dev_plan) {
+                           hipStream_t st, TimingHook *hook, double scale, uint32_t *cover_flag, int flag_stride,
+                           const void *dev_plan) {
   if (nlev < 1 || nlev > 4) throw std::runtime_error("real-space draw supports 1 to 4 levels");
   upload_tables();
   RngBufs b = carve(plan, ws, ws_bytes);
-  long nc = plan.nchunks;
-  const int TB = 256;
-  size_t ring_bytes = size_t(RING) * TB * 4;
-  const RngDev *pd = static_cast<const RngDev *>(dev_plan);
-  if (!pd) {
-    hipLaunchKernelGGL(k_rng_put_plan, dim3(1), dim3(64), 0, st, to_dev(plan), b.dev);
-    GIC_HIP(hipGetLastError());
-    pd = b.dev;
-  }
-  if (hook) hook->begin("rng_summary", st);
-  hipLaunchKernelGGL(k_rng_summary, dim3((nc + TB - 1) / TB), dim3(TB), ring_bytes, st, pd, nc, b.summary, b.raw);
-  GIC_HIP(hipGetLastError());
-  if (hook) hook->end("rng_summary", st);
-  if (hook) hook->begin("rng_scan", st);
-  hipLaunchKernelGGL(k_rng_seg_compose, dim3((b.nseg + 255) / 256), dim3(256), 0, st, b.summary, nc, b.nseg,
-                     b.segmaps);
-  GIC_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_rng_seg_scan, dim3(1), dim3(1024), 0, st, b.segmaps, b.nseg, b.segstart);
-  GIC_HIP(hipGetLastError());
-  if (hook) hook->end("rng_scan", st);
+  const size_t n = plan.streams.size();
   LevelTargets lt;
   size_t acc = 0;
   for (size_t i = 0; i < 4; ++i) {
@@ -926,42 +1041,71 @@ static void draw_real_list(const RngPlan &plan, const RngLevelOut *levels, size_
     lt.cum[i] = acc;
   }
   lt.scale = scale;
-  size_t total = acc;
-  // coverage: the stream must hold at least `total` Gaussians
-  if (cover_flag) {
-    hipLaunchKernelGGL(k_rng_cover, dim3(1), dim3(64), 0, st, (const uint64_t *)(b.segstart + (b.nseg - 1)),
-                       (const uint32_t *)(b.segmaps + 5 * (b.nseg - 1)), uint64_t(total), cover_flag);
-    GIC_HIP(hipGetLastError());
-  } else {
-    uint64_t last = 0;
-    uint32_t lastmap[5];
-    GIC_HIP(hipMemcpyAsync(&last, b.segstart + (b.nseg - 1), 8, hipMemcpyDeviceToHost, st));
-    GIC_HIP(hipMemcpyAsync(lastmap, b.segmaps + 5 * (b.nseg - 1), 20, hipMemcpyDeviceToHost, st));
-    GIC_HIP(hipStreamSynchronize(st));
-    uint64_t produced = (last >> 2) + lastmap[1 + (last & 3)];
-    if (produced < total) throw std::runtime_error("internal error: RNG plan produced too few Gaussians");
+  for (auto &s : plan.streams)
+    if (s.out0 > acc || s.count > acc - s.out0) throw std::runtime_error("RNG: a stream runs past the targets");
+  // coverage: every stream must hold the Gaussians wanted of it; without a
+  // caller's flag the check is this call's own, after the work
+  uint32_t *flag = cover_flag;
+  if (!flag) flag = (uint32_t *)(b.dev + rng_dev_bytes(plan));   // carve's slack
+  const RngDev *pd = static_cast<const RngDev *>(dev_plan);
+  std::vector<char> host;
+  if (!pd) {
+    pd = (const RngDev *)b.dev;
+    if (n == 1) {
+      hipLaunchKernelGGL(k_rng_put_plan, dim3(1), dim3(64), 0, st, to_dev(plan, 0), (RngDev *)b.dev,
+                         cover_flag ? nullptr : flag);
+      GIC_HIP(hipGetLastError());
+    } else {
+      // (host outlives the copy: without a caller's flag the call ends with a wait)
+      if (cover_flag) throw std::runtime_error("internal error: several streams and a flag need a packed plan");
+      host.resize(rng_dev_bytes(plan) + 4, 0);   // the flag follows
+      rng_dev_pack(plan, host.data());
+      GIC_HIP(hipMemcpyAsync(b.dev, host.data(), host.size(), hipMemcpyHostToDevice, st));
+    }
+  } else if (!cover_flag) {
+    throw std::runtime_error("internal error: a draw from a packed plan needs a flag");
   }
+  const uint32_t *of = n > 1 ? (const uint32_t *)((const char *)pd + align256(n * sizeof(RngDev))) : nullptr;
+  const unsigned nblk = unsigned((plan.nseg + RNG_SEGS - 1) / RNG_SEGS);
+  if (hook) hook->begin("rng_summary", st);
+  hipLaunchKernelGGL(k_rng_summary, dim3(nblk), dim3(RNG_THREADS), 0, st, pd, of, plan.nseg, plan.kclog, b.state,
+                     b.maps, b.segmaps);
+  GIC_HIP(hipGetLastError());
+  if (hook) hook->end("rng_summary", st);
+  if (hook) hook->begin("rng_scan", st);
+  hipLaunchKernelGGL(k_rng_seg_scan, dim3(unsigned(n)), dim3(1024), 0, st, pd, b.segmaps, b.segstart, flag,
+                     cover_flag ? flag_stride : 0);
+  GIC_HIP(hipGetLastError());
+  if (hook) hook->end("rng_scan", st);
   if (hook) hook->begin("rng_emit", st);
-  hipLaunchKernelGGL(k_rng_emit<T>, dim3((nc + 63) / 64), dim3(64), 0, st, b.raw, nc, b.summary, b.segstart, lt,
-                     total, plan.kc);
+  hipLaunchKernelGGL(k_rng_emit<T>, dim3(nblk), dim3(RNG_THREADS), 0, st, pd, of, plan.nseg, plan.kclog, b.state,
+                     b.maps, b.segstart, lt);
   GIC_HIP(hipGetLastError());
   if (hook) hook->end("rng_emit", st);
+  if (!cover_flag) {
+    uint32_t few = 0;
+    GIC_HIP(hipMemcpyAsync(&few, flag, 4, hipMemcpyDeviceToHost, st));
+    GIC_HIP(hipStreamSynchronize(st));
+    if (few) throw std::runtime_error("internal error: RNG plan produced too few Gaussians");
+  }
 }
 
 template <typename T>
 void rng_draw_real(const RngPlan &plan, const std::vector<RngLevelOut> &levels, void *ws, size_t ws_bytes,
-                   hipStream_t st, TimingHook *hook, double scale, uint32_t *cover_flag, const void *dev_plan) {
-  draw_real_list<T>(plan, levels.data(), levels.size(), ws, ws_bytes, st, hook, scale, cover_flag, dev_plan);
+                   hipStream_t st, TimingHook *hook, double scale, uint32_t *cover_flag, int flag_stride,
+                   const void *dev_plan) {
+  draw_real_list<T>(plan, levels.data(), levels.size(), ws, ws_bytes, st, hook, scale, cover_flag, flag_stride,
+                    dev_plan);
 }
 
 template void rng_draw_real<float>(const RngPlan &, const std::vector<RngLevelOut> &, void *, size_t, hipStream_t,
-                                   TimingHook *, double, uint32_t *, const void *);
+                                   TimingHook *, double, uint32_t *, int, const void *);
 template void rng_draw_real<double>(const RngPlan &, const std::vector<RngLevelOut> &, void *, size_t, hipStream_t,
-                                    TimingHook *, double, uint32_t *, const void *);
+                                    TimingHook *, double, uint32_t *, int, const void *);
 
 // ---- draws with a fixed workspace ------------------------------------------------
 // For callers that cannot allocate device memory: the draw's workspace (chunk
-// summaries, segment maps and starts, raw numbers, the plan) lives in this
+// states and maps, wavefront maps and starts, the plan) lives in this
 // file-scope device array, one copy per GPU, held until the process ends.
 // Its address on each device is looked up once (rng_scratch_setup, called by
 // gic_create with the device current) and only that address is passed to
@@ -1003,14 +1147,15 @@ void rng_gaussians_noalloc(int device, unsigned long seed, double *dev_out, size
   if (rng_workspace_bytes(plan) > NOALLOC_SCRATCH_BYTES)
     throw std::runtime_error("internal error: the fixed RNG workspace is too small for this draw");
   RngLevelOut out{dev_out, 0, n};
-  draw_real_list<double>(plan, &out, 1, ws, NOALLOC_SCRATCH_BYTES, st, nullptr, 1.0, nullptr, nullptr);
+  draw_real_list<double>(plan, &out, 1, ws, NOALLOC_SCRATCH_BYTES, st, nullptr, 1.0, nullptr, 0, nullptr);
 }
 
-void rng_raw(const RngPlan &plan, uint32_t *d_out, size_t n, void *, size_t, hipStream_t st) {
-  if (n > size_t(plan.nchunks) * plan.ch()) throw std::runtime_error("rng_raw: plan too small");
-  RngDev d = to_dev(plan);
-  long nc = long((n + plan.ch() - 1) / plan.ch());
-  hipLaunchKernelGGL(k_rng_raw, dim3((nc + 255) / 256), dim3(256), 0, st, d, nc, d_out, n);
+void rng_raw(const RngPlan &plan, uint32_t *d_out, size_t n, hipStream_t st) {
+  upload_tables();
+  size_t nc = (n + plan.ch() - 1) / plan.ch();
+  if (nc > size_t(plan.nseg) * 64) throw std::runtime_error("rng_raw: plan too small");
+  RngDev d = to_dev(plan, 0);
+  hipLaunchKernelGGL(k_rng_raw, dim3((nc + 255) / 256), dim3(256), 0, st, d, plan.kclog, long(nc), d_out, n);
   GIC_HIP(hipGetLastError());
 }
 
