@@ -157,8 +157,8 @@ template <typename T> void do_displacement_adjoint(gic_context *c, const T *cons
         T *u = (T *)C.adj_u.p;
         fill<T>(u, C.g.padded_reals(), T(0), c->st);
         InterpGeom ig = interp_geom(L.g, C.g);
-        if (g_pad) interp_adjoint<T>(g_pad, n, n + 2, u, ig, c->st);
-        else interp_adjoint<T>(g_src, n, n, u, ig, c->st);
+        c->adj_fold.ensure(interp_adjoint_bytes<T>(n, ig));
+        interp_adjoint<T>(g_pad ? g_pad : g_src, n, g_pad ? n + 2 : n, u, ig, (T *)c->adj_fold.p, c->st);
       }
       T *acc = (T *)L.adj_acc.p;
       if (g_pad) {

@@ -257,7 +257,7 @@ struct gic_context {
   bool seeded = false, drawn = false, power_applied = false, zeldovich_done = false;
   int lpt_order = 1;   // 1: Zel'dovich, 2: second-order LPT on top
   bool fix_power = false;   // fix_power: unit-modulus white noise after the draw
-  DevBuf work, stage, tab_a, tab_b, tab_c, lpt_win, adj_scratch;
+  DevBuf work, stage, tab_a, tab_b, tab_c, lpt_win, adj_scratch, adj_fold;
   // three padded fields of data transformed along x only (fft_c2r_xpass), so
   // that one x pass serves several displacement or second-derivative fields;
   // after the Zel'dovich pass it holds the base level's X0, X1 for 2LPT
