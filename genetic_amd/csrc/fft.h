@@ -84,13 +84,6 @@ void fft_r2c_za_adjoint(const T *src, T *d, T *acc, int n, const T *tab, int com
 template <typename T>
 void fft_c2r_from(const T *spec, T *out, int n, int pre, const T *tab, int comp, double kmin, hipStream_t st,
                   TimingHook *hook, T *dst = nullptr, double inv_k2 = 0, const FilterInline *fil = nullptr);
-// The second derivative phi_ab = c2r(k_a k_b tab[|k|^2] spec) (comp = a + 3b,
-// as FFT_PRE_KK) folded into the 2LPT source by the last pass instead of being
-// stored: epi 1: S = A phi, A += phi;  2: S += A phi;  3: S -= phi^2
-// (S, A padded real fields; scratch holds the intermediate passes).
-template <typename T>
-void fft_c2r_lpt(const T *spec, T *scratch, int n, const T *tab, int comp, double kmin, int epi, T *S, T *A,
-                 hipStream_t st, TimingHook *hook, double inv_k2 = 0);
 // The same transforms split after their first pass, so that one x pass serves
 // several outputs (c2r is linear and a factor of k_y, k_z commutes with the
 // transform along x):
@@ -100,7 +93,8 @@ void fft_c2r_lpt(const T *spec, T *scratch, int n, const T *tab, int comp, doubl
 //           mode by m(k_y, k_z) as it reads it (FFT_YZ_*; dst as for
 //           fft_c2r_from);
 //   fft_c2r_yz_lpt: the same, its last pass folding the result into the 2LPT
-//           source as fft_c2r_lpt does (out is scratch).
+//           source instead of storing it (out is scratch): epi 1: S = A phi,
+//           A += phi;  2: S += A phi;  3: S -= phi^2 (S, A padded fields).
 // With X0 = x pass of tab spec, X1 = x pass of i k_x tab spec (FFT_PRE_ZA comp 0)
 // and X2 = x pass of k_x^2 tab spec (FFT_PRE_KK comp 0): the Zel'dovich
 // components are yz(X1, ONE), yz(X0, IKY), yz(X0, IKZ) and the second
