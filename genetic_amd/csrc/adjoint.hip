@@ -62,45 +62,35 @@ template <typename T> void do_displacement_forward(gic_context *c, const T *cons
   for (size_t l = 0; l < nl; ++l)
     if (!noise[l] || !psi[3 * l] || !psi[3 * l + 1] || !psi[3 * l + 2])
       throw std::runtime_error("displacement forward: null device pointer");
-  // delta_l = sqrtP r2c(w_l), read straight from the caller's dense arrays
-  for (auto &Lp : c->levels) {
-    Level &L = *Lp;
-    alloc_field(c, L.noise, L.g);
-    build_sqrtp<T>(c, L);
-  }
+  // the noise along z and y, read straight from the caller's dense arrays;
+  // the x pass of do_zeldovich makes delta_l = sqrtP r2c(w_l) and what the
+  // displacements need of it
   for (size_t l = 0; l < nl; ++l) {
     Level &L = *c->levels[l];
-    fft_r2c_post<T>((T *)L.noise.p, L.g.n, (const T *)L.sqrtp.p, c->st, c->hook(), noise[l]);
-    L.noise_fourier = true;
-    L.dc_pending = false;
+    alloc_field(c, L.noise, L.g);
+    build_sqrtp<T>(c, L);
+    FftZFwd<T> z;
+    z.add(noise[l], (T *)L.noise.p, true);
+    fft_z_forward<T>(z, L.g.n, c->st, c->hook());
+    FftYFwd<T> y;
+    y.add((const T *)L.noise.p, nullptr, (T *)L.noise.p);
+    fft_y_forward<T>(y, L.g.n, c->st, c->hook());
     L.have_psi = L.have_psi2 = false;
   }
   c->seeded = c->drawn = c->power_applied = true;
-  c->zeldovich_done = false;
-  if (nl == 1) {
-    // one level: each component's c2r writes the caller's array directly
-    Level &L = *c->levels[0];
-    long nent = table_entries(L.g);
-    c->tab_c.ensure(nent * sizeof(T));
-    filter_table<T>(2, 0.0, L.g.kmin(), nent, (T *)c->tab_c.p, c->st, true);
-    alloc_field(c, L.psi[0], L.g);
-    for (int a = 0; a < 3; ++a)
-      fft_c2r_from<T>((const T *)L.noise.p, (T *)L.psi[0].p, L.g.n, FFT_PRE_ZA, nullptr, a, L.g.kmin(), c->st,
-                      c->hook(), psi[a], 1.0);
-  } else {
-    int order = c->lpt_order;
-    c->lpt_order = 1;
-    try {
-      do_zeldovich<T>(c);
-    } catch (...) {
-      c->lpt_order = order;
-      throw;
-    }
+  int order = c->lpt_order;
+  c->lpt_order = 1;
+  try {
+    do_zeldovich<T>(c, psi);
+  } catch (...) {
     c->lpt_order = order;
-    for (size_t l = 0; l < nl; ++l) {
-      Level &L = *c->levels[l];
-      for (int a = 0; a < 3; ++a) unpad<T, T>((const T *)L.psi[a].p, L.g.n, psi[3 * l + a], c->st);
-    }
+    throw;
+  }
+  c->lpt_order = order;
+  c->zeldovich_done = nl > 1;
+  for (size_t l = 1; l < nl; ++l) {
+    Level &L = *c->levels[l];
+    for (int a = 0; a < 3; ++a) unpad<T, T>((const T *)L.psi[a].p, L.g.n, psi[3 * l + a], c->st);
   }
   GIC_HIP(hipStreamSynchronize(c->st));
 }
@@ -112,15 +102,14 @@ template <typename T> void do_displacement_adjoint(gic_context *c, const T *cons
     if (!noise_bar[l] || !psi_bar[3 * l] || !psi_bar[3 * l + 1] || !psi_bar[3 * l + 2])
       throw std::runtime_error("displacement adjoint: null device pointer");
   size_t maxreals = 0;
-  for (auto &Lp : c->levels) {
-    Level &L = *Lp;
+  for (size_t l = 0; l < nl; ++l) {
+    Level &L = *c->levels[l];
     build_sqrtp<T>(c, L);
-    alloc_field(c, L.adj_acc, L.g);
+    if (l + 1 < nl)
+      for (auto &u : L.adj_u) alloc_field(c, u, L.g);
     maxreals = std::max(maxreals, L.g.padded_reals());
   }
-  for (size_t l = 0; l + 1 < nl; ++l) alloc_field(c, c->levels[l]->adj_u, c->levels[l]->g);
-  c->adj_scratch.ensure(maxreals * sizeof(T));
-  T *scratch = (T *)c->adj_scratch.p;
+  c->xhalf.ensure(3 * maxreals * sizeof(T));
   // per level: the Zel'dovich operator's table sqrtP F_l / k^2, and the low
   // pass towards the next finer level (for level 0 with sqrtP / k^2 folded in)
   for (size_t l = 0; l < nl; ++l) {
@@ -135,47 +124,62 @@ template <typename T> void do_displacement_adjoint(gic_context *c, const T *cons
       }
     }
   }
-  for (int a = 0; a < 3; ++a) {
-    for (size_t li = nl; li-- > 0;) {
-      Level &L = *c->levels[li];
-      int n = L.g.n;
-      const T *pb = psi_bar[3 * li + a];
-      // the level's gradient g: psibar alone on the finest level, else
-      // psibar + LP c2r r2c (I^T g_finer) held in adj_u (padded)
-      const T *g_src = pb;      // dense
-      T *g_pad = nullptr;       // padded
-      if (li + 1 < nl && li >= 1) {
-        g_pad = (T *)L.adj_u.p;
-        fft_r2c_post<T>(g_pad, n, (const T *)L.adj_lp.p, c->st, c->hook());
-        fft3d<T>(g_pad, n, +1, c->st, c->hook());
-        hipLaunchKernelGGL(k_add_dense<T>, dim3((L.g.n3() + 255) / 256), dim3(256), 0, c->st, g_pad, pb, n);
+  for (size_t li = nl; li-- > 0;) {
+    Level &L = *c->levels[li];
+    const int n = L.g.n;
+    const size_t reals = L.g.padded_reals();
+    const bool finer = li + 1 < nl;
+    // the level's gradient g: psibar alone (dense) on the finest level, on a
+    // middle one psibar + LP c2r r2c (I^T g_finer), held in adj_u (padded);
+    // on the base level the second term enters through adj_lp below
+    const bool mid = finer && li >= 1;
+    T *u[3] = {(T *)L.adj_u[0].p, (T *)L.adj_u[1].p, (T *)L.adj_u[2].p};
+    if (mid) {
+      for (int a = 0; a < 3; ++a) {
+        fft_r2c_post<T>(u[a], n, (const T *)L.adj_lp.p, c->st, c->hook());
+        fft3d<T>(u[a], n, +1, c->st, c->hook());
+        hipLaunchKernelGGL(k_add_dense<T>, dim3((L.g.n3() + 255) / 256), dim3(256), 0, c->st, u[a],
+                           psi_bar[3 * li + a], n);
         GIC_HIP(hipGetLastError());
       }
-      if (li >= 1) {
-        // push g to the coarser level through the transposed interpolation
-        Level &C = *c->levels[li - 1];
-        T *u = (T *)C.adj_u.p;
-        fill<T>(u, C.g.padded_reals(), T(0), c->st);
-        InterpGeom ig = interp_geom(L.g, C.g);
-        c->adj_fold.ensure(interp_adjoint_bytes<T>(n, ig));
-        interp_adjoint<T>(g_pad ? g_pad : g_src, n, g_pad ? n + 2 : n, u, ig, (T *)c->adj_fold.p, c->st);
-      }
-      T *acc = (T *)L.adj_acc.p;
-      if (g_pad) {
-        fft_r2c_za_adjoint<T>(nullptr, g_pad, acc, n, (const T *)L.adj_tab.p, a, L.g.kmin(), a > 0, c->st, c->hook());
-      } else {
-        fft_r2c_za_adjoint<T>(g_src, scratch, acc, n, (const T *)L.adj_tab.p, a, L.g.kmin(), a > 0, c->st, c->hook());
-        if (li == 0 && nl >= 2) {
-          // level 0 under level 1: its LP part enters through r2c(I^T g_1)
-          fft_r2c_za_adjoint<T>(nullptr, (T *)L.adj_u.p, acc, n, (const T *)L.adj_lp.p, a, L.g.kmin(), true, c->st,
-                                c->hook());
-        }
+    }
+    if (li >= 1) {
+      // push g to the coarser level through the transposed interpolation
+      Level &C = *c->levels[li - 1];
+      InterpGeom ig = interp_geom(L.g, C.g);
+      c->adj_fold.ensure(interp_adjoint_bytes<T>(n, ig));
+      for (int a = 0; a < 3; ++a) {
+        T *cu = (T *)C.adj_u[a].p;
+        fill<T>(cu, C.g.padded_reals(), T(0), c->st);
+        interp_adjoint<T>(mid ? u[a] : psi_bar[3 * li + a], n, mid ? n + 2 : n, cu, ig, (T *)c->adj_fold.p, c->st);
       }
     }
-  }
-  for (size_t l = 0; l < nl; ++l) {
-    Level &L = *c->levels[l];
-    fft_c2r_to<T>((T *)L.adj_acc.p, noise_bar[l], L.g.n, c->st, c->hook());
+    // the transposed displacement: the gradients of psi_y and psi_z meet in
+    // the y pass, those of psi_x and of both in the x pass
+    T *h[3] = {(T *)c->xhalf.p, (T *)c->xhalf.p + reals, (T *)c->xhalf.p + 2 * reals};
+    const bool low = finer && li == 0;
+    FftZFwd<T> z;
+    for (int a = 0; a < 3; ++a) z.add(mid ? u[a] : psi_bar[3 * li + a], h[a], !mid);
+    if (low)
+      for (int a = 0; a < 3; ++a) z.add(u[a], u[a], false);
+    fft_z_forward<T>(z, n, c->st, c->hook());
+    FftYFwd<T> y;
+    y.kmin = L.g.kmin();
+    y.add(h[0], nullptr, h[0]);
+    y.add(h[1], h[2], h[1]);
+    if (low) {
+      y.add(u[0], nullptr, u[0]);
+      y.add(u[1], u[2], u[1]);
+    }
+    fft_y_forward<T>(y, n, c->st, c->hook());
+    fft_x_adjoint<T>(h[0], h[1], (const T *)L.adj_tab.p, low ? u[0] : nullptr, low ? u[1] : nullptr,
+                     low ? (const T *)L.adj_lp.p : nullptr, n, L.g.kmin(), c->st, c->hook());
+    FftY<T> yb;
+    yb.add(h[0], h[0], FFT_YZ_ONE);
+    fft_y<T>(yb, n, c->st, c->hook());
+    FftZ<T> zb;
+    zb.add(h[0], nullptr, noise_bar[li], FFT_YZ_ONE);
+    fft_z<T>(zb, n, c->st, c->hook());
   }
   GIC_HIP(hipStreamSynchronize(c->st));
 }

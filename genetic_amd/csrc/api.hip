@@ -122,35 +122,26 @@ template <typename T> void do_draw(gic_context *c) {
     c->stage.ensure(gbytes + maxslots * 4);
     T *gauss = (T *)c->stage.p;
     uint32_t *owner = (uint32_t *)((char *)c->stage.p + gbytes);
-    if (!parallel) {
-      if (total) {
-        RngPlan plan;
-        rng_plan(c->seed, total, plan);
-        c->work.ensure(rng_workspace_bytes(plan));
-        std::vector<RngLevelOut> outs{{gauss, 0, total}};
-        rng_draw_real<T>(plan, outs, c->work.p, c->work.bytes, c->st, c->hook(), sigma);
-      }
-    } else {
-      int hmax = 0;
-      for (auto &L : c->levels) hmax = std::max(hmax, L->g.n / 2);
-      if (hmax > 1) {
-        RngPlan big;
-        rng_plan(c->seed, 24 * size_t(hmax - 1) * (hmax - 1), big);
-        c->work.ensure(rng_workspace_bytes(big));
-      }
-      for (size_t l = 0; l < c->levels.size(); ++l) {
-        int h = c->levels[l]->g.n / 2;
-        size_t pos = off[l];
-        for (int ks = 1; ks < h; ++ks) {
-          size_t cnt = 24 * size_t(ks) * ks;
-          RngPlan plan;
-          rng_plan(c->seed + ks, cnt, plan);
-          c->work.ensure(rng_workspace_bytes(plan));
-          std::vector<RngLevelOut> outs{{gauss + pos, 0, cnt}};
-          rng_draw_real<T>(plan, outs, c->work.p, c->work.bytes, c->st, c->hook(), sigma);
-          pos += cnt;
+    if (total) {
+      // one stream, or all shells' streams in one draw
+      std::vector<RngStream> streams;
+      if (!parallel) {
+        streams.push_back({c->seed, total, 0});
+      } else {
+        for (size_t l = 0; l < c->levels.size(); ++l) {
+          size_t pos = off[l];
+          for (int ks = 1; ks < c->levels[l]->g.n / 2; ++ks) {
+            size_t cnt = 24 * size_t(ks) * ks;
+            streams.push_back({c->seed + ks, cnt, pos});
+            pos += cnt;
+          }
         }
       }
+      RngPlan plan;
+      rng_plan(streams, plan);
+      c->work.ensure(rng_workspace_bytes(plan));
+      std::vector<RngLevelOut> outs{{gauss, 0, total}};
+      rng_draw_real<T>(plan, outs, c->work.p, c->work.bytes, c->st, c->hook(), sigma);
     }
     for (size_t l = 0; l < c->levels.size(); ++l) {
       Level &L = *c->levels[l];
@@ -249,13 +240,93 @@ void coarse_window(const LevelGeom &gf, const LevelGeom &gc, int *w0, int *wl) {
   }
 }
 
+// What a fine level takes of the base level's spectrum m (already multiplied
+// by its own factor where it has one): the low-passed displacement LP/k^2 i k m
+// scale and with delta the low-passed m itself, in the coarse window only --
+// one x pass, one y pass, then the rows.  view[0..2] receive the
+// displacements, view[3] the low-passed m; they lie in buf.
+template <typename T>
+void coarse_parts(gic_context *c, const T *m, const LevelGeom &g, double kc, double scale, bool delta, const int *w0,
+                  const int *wl, DevBuf &buf, CoarseView *view) {
+  const int n = g.n, nz = n / 2 + 1, nv = delta ? 4 : 3;
+  const size_t a_n = size_t(wl[0]) * n * nz * 2, b_n = size_t(wl[0]) * wl[1] * nz * 2;
+  const size_t o_n = size_t(wl[0]) * wl[1] * wl[2];
+  buf.ensure(((nv - 1) * a_n + nv * (b_n + o_n)) * sizeof(T));
+  T *A = (T *)buf.p, *B = A + (nv - 1) * a_n, *O = B + nv * b_n;
+  long h = n / 2, nent = 3 * h * h + 1;
+  c->tab_b.ensure(nent * sizeof(T));
+  c->tab_c.ensure(nent * sizeof(T));
+  filter_table<T>(0, kc, g.kmin(), nent, (T *)c->tab_b.p, c->st);
+  filter_table<T>(0, kc, g.kmin(), nent, (T *)c->tab_c.p, c->st, true, scale);
+  FilterInline fil;   // the same low pass over k^2, formed in the pass (FP32)
+  fil.nf = 1;
+  fil.kind[0] = 0;
+  fil.kc[0] = kc;
+  fil.scale = scale;
+  fil.over_k2 = 1;
+  FftX<T> x;
+  x.in = m;
+  x.out[1] = A;
+  x.out[2] = A + a_n;
+  if (delta) {
+    x.out[0] = A + 2 * a_n;
+    x.plain0 = true;
+  }
+  x.fil = &fil;
+  x.tab = (const T *)c->tab_c.p;
+  x.tab0 = (const T *)c->tab_b.p;
+  x.kmin = g.kmin();
+  x.win0 = w0[0];
+  x.wlen = wl[0];
+  fft_x<T>(x, n, c->st, c->hook());
+  FftY<T> y;
+  y.kmin = g.kmin();
+  y.nouter = wl[0];
+  y.win0 = w0[1];
+  y.wlen = wl[1];
+  y.add(A + a_n, B, FFT_YZ_ONE);
+  y.add(A, B + b_n, FFT_YZ_IKY, B + 2 * b_n, FFT_YZ_IKZ);
+  if (delta) y.add(A + 2 * a_n, B + 3 * b_n, FFT_YZ_ONE);
+  fft_y<T>(y, n, c->st, c->hook());
+  for (int f = 0; f < nv; ++f) {
+    fft_z_window<T>(B + f * b_n, O + f * o_n, long(wl[0]) * wl[1], w0[2], wl[2], n, c->st, c->hook());
+    view[f].p = O + f * o_n;
+    for (int a = 0; a < 3; ++a) {
+      view[f].org[a] = w0[a];
+      view[f].len[a] = wl[a];
+    }
+    view[f].sx = long(wl[1]) * wl[2];
+    view[f].sy = wl[2];
+  }
+}
+
+// out[a] (padded) and, if given, dense[a] <- the displacement of x passes X0
+// (of f m) and X1 (of i k_x f m): psi_y and psi_z share X0's y pass, psi_z's
+// factor k_z rides on its z pass.  X0 and X1 may be outputs.
+template <typename T>
+void displacement_yz(gic_context *c, const T *X0, const T *X1, T *const *out, T *const *dense, bool padded,
+                     const LevelGeom &g) {
+  FftY<T> y;
+  y.kmin = g.kmin();
+  y.add(X1, out[0], FFT_YZ_ONE);
+  y.add(X0, out[1], FFT_YZ_IKY, out[2], FFT_YZ_ONE);
+  fft_y<T>(y, g.n, c->st, c->hook());
+  FftZ<T> z;
+  z.kmin = g.kmin();
+  for (int a = 0; a < 3; ++a)
+    z.add(out[a], padded ? out[a] : nullptr, dense ? dense[a] : nullptr, a == 2 ? FFT_YZ_IKZ : FFT_YZ_ONE);
+  fft_z<T>(z, g.n, c->st, c->hook());
+}
+
 // Second-order LPT (no counterpart in the reference, which stops at
 // Zel'dovich, zeldovich.hpp:152-253).  With phi_ij = k_i k_j delta / k^2 the
 // source is S = sum_{i<j} (phi_ii phi_jj - phi_ij^2) and
 // psi2 = (3/7) i k S / k^2, i.e. D2 = -3/7 D1^2 with delta at the output
 // redshift; the velocity uses f2 = 2 f1.  Each level is built from its
 // combined overdensity; a zoom level keeps the high-pass part of its own
-// psi2 and takes the low-pass part from the level above, as for psi.
+// psi2 and takes the low-pass part from the level above, as for psi.  The
+// base level's source comes from its Zel'dovich passes, in the first field
+// of xhalf.
 template <typename T> void do_second_order(gic_context *c) {
   size_t nl = c->levels.size();
   CoarseView win_view[3];
@@ -266,222 +337,210 @@ template <typename T> void do_second_order(gic_context *c) {
     int n = g.n;
     size_t reals = g.padded_reals(), bytes = reals * sizeof(T);
     for (auto &p : L.psi2) alloc_field(c, p, g);
-    c->stage.ensure(2 * bytes);
-    T *D = (T *)c->stage.p;
-    T *S = D + reals;
-    const T *spec = (const T *)L.noise.p;
-    if (!L.noise_fourier) {
-      GIC_HIP(hipMemcpyAsync(D, L.noise.p, bytes, hipMemcpyDeviceToDevice, c->st));
-      fft3d<T>(D, n, -1, c->st, c->hook());
-      spec = D;
-    }
     long h = n / 2, nent = 3 * h * h + 1;
-    c->tab_a.ensure(nent * sizeof(T));
     c->tab_c.ensure(nent * sizeof(T));
-    filter_table<T>(2, 0.0, g.kmin(), nent, (T *)c->tab_a.p, c->st, true);
-    T *A = (T *)L.psi2[0].p, *B = (T *)L.psi2[1].p;
-    // the x passes of (1/k^2) delta, i k_x (1/k^2) delta and k_x^2 (1/k^2)
-    // delta serve all six phi_ab (their y passes multiply by the k_y, k_z
-    // factors); the base level's first two are left by the Zel'dovich pass
+    T *q[3] = {(T *)L.psi2[0].p, (T *)L.psi2[1].p, (T *)L.psi2[2].p};
     c->xhalf.ensure(3 * bytes);
-    T *X0 = (T *)c->xhalf.p, *X1 = X0 + reals, *X2 = X1 + reals;
+    T *X[3] = {(T *)c->xhalf.p, (T *)c->xhalf.p + reals, (T *)c->xhalf.p + 2 * reals};
+    T *S = X[0];
     if (c->hook()) c->hook()->begin("lpt_source", c->st);
-    if (!(l == 0 && c->xhalf_base && spec == (const T *)L.noise.p)) {
-      fft_c2r_xpass<T>(spec, X0, n, FFT_PRE_TABLE, nullptr, 0, g.kmin(), c->st, c->hook(), 1.0);
-      fft_c2r_xpass<T>(spec, X1, n, FFT_PRE_ZA, nullptr, 0, g.kmin(), c->st, c->hook(), 1.0);
+    if (l > 0) {
+      // the x passes of (1/k^2) delta, i k_x (1/k^2) delta and k_x^2 (1/k^2) delta
+      c->stage.ensure(2 * bytes);
+      T *D = (T *)c->stage.p;
+      S = D + reals;
+      FftX<T> x;
+      if (L.noise_fourier) {
+        x.in = (const T *)L.noise.p;
+      } else {
+        FftZFwd<T> zf;
+        zf.add((const T *)L.noise.p, D, false);
+        fft_z_forward<T>(zf, n, c->st, c->hook());
+        FftYFwd<T> yf;
+        yf.add(D, nullptr, D);
+        fft_y_forward<T>(yf, n, c->st, c->hook());
+        x.in = D;
+        x.forward = true;
+      }
+      for (int i = 0; i < 3; ++i) x.out[i + 1] = X[i];
+      x.inv_k2 = 1.0;
+      x.kmin = g.kmin();
+      fft_x<T>(x, n, c->st, c->hook());
+      FftY<T> y;
+      y.kmin = g.kmin();
+      y.add(X[2], q[0], FFT_YZ_ONE);
+      y.add(X[1], X[1], FFT_YZ_ONE, q[2], FFT_YZ_MIKY);
+      y.add(X[0], X[0], FFT_YZ_ONE, D, FFT_YZ_KY, q[1], FFT_YZ_KYKY);
+      fft_y<T>(y, n, c->st, c->hook());
+      fft_z_lpt<T>(X[1], D, X[0], q[0], q[1], q[2], S, false, n, g.kmin(), c->st, c->hook());
     }
-    c->xhalf_base = false;
-    fft_c2r_xpass<T>(spec, X2, n, FFT_PRE_KK, nullptr, 0, g.kmin(), c->st, c->hook(), 1.0);
-    // each phi_ab but xx is folded into S by its transform's last pass
-    auto fold = [&](const T *X, int yop, int epi) {
-      fft_c2r_yz_lpt<T>(X, B, n, yop, g.kmin(), epi, S, A, c->st, c->hook());
-    };
-    fft_c2r_yz<T>(X2, A, n, FFT_YZ_ONE, g.kmin(), c->st, c->hook());   // A = xx
-    fold(X0, FFT_YZ_KYKY, 1);   // S = xx yy, A = xx + yy
-    fold(X0, FFT_YZ_KZKZ, 2);   // S += (xx + yy) zz
-    fold(X1, FFT_YZ_MIKY, 3);   // S -= xy^2
-    fold(X1, FFT_YZ_MIKZ, 3);   // S -= xz^2
-    fold(X0, FFT_YZ_KYKZ, 3);   // S -= yz^2
     if (c->hook()) c->hook()->end("lpt_source", c->st);
-    fft3d<T>(S, n, -1, c->st, c->hook());
-    double kc = l >= 1 ? kcut_for_level(c, int(l) - 1) : 0.0;
-    filter_table<T>(l >= 1 ? 1 : 2, kc, g.kmin(), nent, (T *)c->tab_c.p, c->st, true, 3.0 / 7.0);
+    // the level whose low-pass part level 1 takes straight from the base
+    // source spectrum (a pruned c2r into the coarse window)
+    int w0[3], wl[3];
+    bool window = l == 0 && nl >= 2 && g.covers_full();
+    if (window) {
+      coarse_window(c->levels[1]->g, g, w0, wl);
+      window = wl[0] < n && wl[1] < n && wl[2] < n;
+    }
     {
-      // psi2_x from the x pass of i k_x f S, psi2_y and psi2_z from that of
-      // f S, f = the level's filter (3/7)/k^2 (unit filter on the base level,
-      // formed inside the transform)
-      const T *tab = l >= 1 ? (const T *)c->tab_c.p : nullptr;
-      double ik2 = l >= 1 ? 0.0 : 3.0 / 7.0;
-      fft_c2r_xpass<T>(S, X1, n, FFT_PRE_ZA, tab, 0, g.kmin(), c->st, c->hook(), ik2);
-      fft_c2r_yz<T>(X1, (T *)L.psi2[0].p, n, FFT_YZ_ONE, g.kmin(), c->st, c->hook());
-      fft_c2r_xpass<T>(S, X0, n, FFT_PRE_TABLE, tab, 0, g.kmin(), c->st, c->hook(), ik2);
-      fft_c2r_yz<T>(X0, (T *)L.psi2[1].p, n, FFT_YZ_IKY, g.kmin(), c->st, c->hook());
-      fft_c2r_yz<T>(X0, (T *)L.psi2[2].p, n, FFT_YZ_IKZ, g.kmin(), c->st, c->hook());
+      // S transformed, its x pass making f S and i k_x f S, f the level's
+      // filter (3/7)/k^2 (unit filter on the base level, formed in the pass)
+      FftZFwd<T> zf;
+      zf.add(S, S, false);
+      fft_z_forward<T>(zf, n, c->st, c->hook());
+      FftYFwd<T> yf;
+      yf.add(S, nullptr, S);
+      fft_y_forward<T>(yf, n, c->st, c->hook());
+      FftX<T> x;
+      x.in = S;
+      x.forward = true;
+      if (window) x.spec = S;
+      x.out[1] = X[1];
+      x.out[2] = X[2];
+      if (l >= 1) {
+        filter_table<T>(1, kcut_for_level(c, int(l) - 1), g.kmin(), nent, (T *)c->tab_c.p, c->st, true, 3.0 / 7.0);
+        x.tab = (const T *)c->tab_c.p;
+      } else {
+        x.inv_k2 = 3.0 / 7.0;
+      }
+      x.kmin = g.kmin();
+      fft_x<T>(x, n, c->st, c->hook());
+      displacement_yz<T>(c, X[1], X[2], q, nullptr, true, g);
     }
     if (l >= 1) {
       Level &C = *c->levels[l - 1];
       InterpGeom ig = interp_geom(g, C.g);
       if (l == 1 && win_ready) {
-        for (int a = 0; a < 3; ++a) interp_add<T>((T *)L.psi2[a].p, n, win_view[a], ig, c->st);
+        for (int a = 0; a < 3; ++a) interp_add<T>(q[a], n, win_view[a], ig, c->st);
       } else {
         long hc = C.g.n / 2, nc_ent = 3 * hc * hc + 1;
         c->tab_b.ensure(nc_ent * sizeof(T));
         filter_table<T>(0, kcut_for_level(c, int(l) - 1), C.g.kmin(), nc_ent, (T *)c->tab_b.p, c->st);
         for (int a = 0; a < 3; ++a) {
           CoarseView v = lowpass_full<T>(c, C.psi2[a], C.g, (const T *)c->tab_b.p);
-          interp_add<T>((T *)L.psi2[a].p, n, v, ig, c->st);
+          interp_add<T>(q[a], n, v, ig, c->st);
         }
       }
     }
-    if (l == 0 && nl >= 2 && g.covers_full()) {
-      // the low-pass part that level 1 takes from the base level, straight
-      // from the base source spectrum into the coarse window (pruned c2r)
-      const LevelGeom &gf = c->levels[1]->g;
-      int w0[3], wl[3];
-      coarse_window(gf, g, w0, wl);
-      if (wl[0] < n && wl[1] < n && wl[2] < n) {
-        int nz = n / 2 + 1;
-        size_t a_b = size_t(wl[0]) * n * nz * 2 * sizeof(T), b_b = size_t(wl[0]) * wl[1] * nz * 2 * sizeof(T);
-        size_t o_b = size_t(wl[0]) * wl[1] * wl[2] * sizeof(T);
-        c->lpt_win.ensure(a_b + b_b + 3 * o_b);
-        T *bufA = (T *)c->lpt_win.p, *bufB = (T *)((char *)c->lpt_win.p + a_b);
-        filter_table<T>(0, kcut_for_level(c, 0), g.kmin(), nent, (T *)c->tab_c.p, c->st, true, 3.0 / 7.0);
-        FilterInline fil;
-        fil.nf = 1;
-        fil.kind[0] = 0;
-        fil.kc[0] = kcut_for_level(c, 0);
-        fil.scale = 3.0 / 7.0;
-        fil.over_k2 = 1;
-        for (int a = 0; a < 3; ++a) {
-          // x: the x pass of i k_x f S; y, z: one x pass of f S, the y pass
-          // multiplying by i k_y or i k_z
-          T *out = (T *)((char *)c->lpt_win.p + a_b + b_b + a * o_b);
-          fft_c2r_window<T>(S, n, a == 0 ? FFT_PRE_ZA : FFT_PRE_TABLE, (const T *)c->tab_c.p, 0, g.kmin(), w0, wl,
-                            bufA, bufB, out, c->st, c->hook(), &fil,
-                            a == 0 ? FFT_YZ_ONE : a == 1 ? FFT_YZ_IKY : FFT_YZ_IKZ, a != 2);
-          win_view[a].p = out;
-          for (int d = 0; d < 3; ++d) {
-            win_view[a].org[d] = w0[d];
-            win_view[a].len[d] = wl[d];
-          }
-          win_view[a].sx = long(wl[1]) * wl[2];
-          win_view[a].sy = wl[2];
-        }
-        win_ready = true;
-      }
+    if (window) {
+      coarse_parts<T>(c, S, g, kcut_for_level(c, 0), 3.0 / 7.0, false, w0, wl, c->lpt_win, win_view);
+      win_ready = true;
     }
     L.have_psi2 = true;
   }
 }
 
-template <typename T> void do_zeldovich(gic_context *c) {
+// The displacements of level l from its spectrum (L.noise), or with forward
+// from noise transformed along z and y there, whose spectrum times sqrt P is
+// left in its place.  A zoom level carries its high-pass filter (the cut of
+// the level above).  The base level of a second-order run also gets its
+// source, into the first field of xhalf, from the same y passes.
+template <typename T> void level_displacements(gic_context *c, size_t l, bool forward, T *const *dense) {
+  Level &L = *c->levels[l];
+  const LevelGeom &g = L.g;
+  const bool lpt = l == 0 && c->lpt_order == 2;
+  const bool padded = !(dense && c->levels.size() == 1);   // a lone level's go to the caller only
+  size_t reals = g.padded_reals();
+  if (padded)
+    for (auto &p : L.psi) alloc_field(c, p, g);
+  c->xhalf.ensure(3 * reals * sizeof(T));
+  T *X0 = (T *)c->xhalf.p, *X1 = X0 + reals, *X2 = X1 + reals;
+  T *psi[3] = {padded ? (T *)L.psi[0].p : X1, padded ? (T *)L.psi[1].p : X0, padded ? (T *)L.psi[2].p : X2};
+  FftX<T> x;
+  x.in = (const T *)L.noise.p;
+  if (forward) {
+    x.forward = true;
+    x.spec = (T *)L.noise.p;
+    x.post = (const T *)L.sqrtp.p;
+  }
+  x.out[1] = X0;
+  x.out[2] = X1;
+  if (lpt) x.out[3] = X2;
+  if (l >= 1) {
+    long h = g.n / 2, nent = 3 * h * h + 1;
+    c->tab_c.ensure(nent * sizeof(T));
+    filter_table<T>(1, kcut_for_level(c, int(l) - 1), g.kmin(), nent, (T *)c->tab_c.p, c->st, true);
+    x.tab = (const T *)c->tab_c.p;
+  } else {
+    x.inv_k2 = 1.0;
+  }
+  x.kmin = g.kmin();
+  fft_x<T>(x, g.n, c->st, c->hook());
+  if (!lpt) {
+    displacement_yz<T>(c, X0, X1, psi, dense, padded, g);
+    return;
+  }
+  for (auto &p : L.psi2) alloc_field(c, p, g);
+  T *q[3] = {(T *)L.psi2[0].p, (T *)L.psi2[1].p, (T *)L.psi2[2].p};
+  FftY<T> y;
+  y.kmin = g.kmin();
+  y.add(X2, q[0], FFT_YZ_ONE);
+  y.add(X1, psi[0], FFT_YZ_ONE, q[2], FFT_YZ_MIKY);
+  y.add(X0, psi[2], FFT_YZ_ONE, psi[1], FFT_YZ_KY, q[1], FFT_YZ_KYKY);
+  fft_y<T>(y, g.n, c->st, c->hook());
+  fft_z_lpt<T>(psi[0], psi[1], psi[2], q[0], q[1], q[2], X0, true, g.n, g.kmin(), c->st, c->hook());
+}
+
+// io: the differentiable forward map, whose noise has been transformed along z
+// and y into the levels' fields; the displacements also go to its arrays
+template <typename T> void do_zeldovich(gic_context *c, T *const *dense) {
   if (!c->power_applied) do_apply_ps<T>(c);
   Phase ph(c, "phase:zeldovich");
   size_t nl = c->levels.size();
-  // Zel'dovich per level, formed inside the first inverse pass from the
-  // overdensity spectrum; zoom levels carry their high-pass filter (the cut
-  // of the level above) on delta and psi.  The levels are independent here;
-  // the base level goes last so that its x passes stay in xhalf for 2LPT.
-  c->xhalf_base = false;
+  // the levels are independent here; the base level goes last so that its
+  // second-order source stays in xhalf
   for (size_t li = nl; li-- > 0;) {
     size_t l = li;
     Level &L = *c->levels[l];
-    ensure_noise_fourier<T>(c, L);
-    for (auto &p : L.psi) alloc_field(c, p, L.g);
-    long h = L.g.n / 2, nent = 3 * h * h + 1;
-    c->tab_a.ensure(nent * sizeof(T));
-    c->tab_c.ensure(nent * sizeof(T));
-    double kc = l >= 1 ? kcut_for_level(c, l - 1) : 0.0;
-    filter_table<T>(l >= 1 ? 1 : 2, kc, L.g.kmin(), nent, (T *)c->tab_c.p, c->st, true);
-    {
-      // psi_x from the x pass of i k_x f delta; psi_y and psi_z share the x
-      // pass of f delta, their y passes multiplying by i k_y and i k_z
-      // (f: the high-pass filter over k^2 on a zoom level, 1/k^2 formed
-      // inside the transform on the base level)
-      size_t reals = L.g.padded_reals();
-      c->xhalf.ensure(3 * reals * sizeof(T));
-      T *X0 = (T *)c->xhalf.p, *X1 = X0 + reals;
-      const T *tab = l >= 1 ? (const T *)c->tab_c.p : nullptr;
-      double ik2 = l >= 1 ? 0.0 : 1.0;
-      const T *spec = (const T *)L.noise.p;
-      int n = L.g.n;
-      fft_c2r_xpass<T>(spec, X1, n, FFT_PRE_ZA, tab, 0, L.g.kmin(), c->st, c->hook(), ik2);
-      fft_c2r_yz<T>(X1, (T *)L.psi[0].p, n, FFT_YZ_ONE, L.g.kmin(), c->st, c->hook());
-      fft_c2r_xpass<T>(spec, X0, n, FFT_PRE_TABLE, tab, 0, L.g.kmin(), c->st, c->hook(), ik2);
-      fft_c2r_yz<T>(X0, (T *)L.psi[1].p, n, FFT_YZ_IKY, L.g.kmin(), c->st, c->hook());
-      fft_c2r_yz<T>(X0, (T *)L.psi[2].p, n, FFT_YZ_IKZ, L.g.kmin(), c->st, c->hook());
-      // the base level's X0 (1/k^2 delta) and X1 (i k_x / k^2 delta) are the
-      // first two x passes of the second derivatives
-      c->xhalf_base = l == 0 && c->lpt_order == 2;
+    if (!dense) ensure_noise_fourier<T>(c, L);
+    level_displacements<T>(c, l, dense != nullptr, dense && l == 0 ? dense : nullptr);
+    if (dense) {
+      L.noise_fourier = true;
+      L.dc_pending = false;
     }
     if (l >= 1) {
-      filter_table<T>(1, kc, L.g.kmin(), nent, (T *)c->tab_a.p, c->st);
+      long h = L.g.n / 2, nent = 3 * h * h + 1;
+      c->tab_a.ensure(nent * sizeof(T));
+      filter_table<T>(1, kcut_for_level(c, int(l) - 1), L.g.kmin(), nent, (T *)c->tab_a.p, c->st);
       mul_table<T>((T *)L.noise.p, L.g.n, (const T *)c->tab_a.p, c->st);
       to_real<T>(c, L.noise, L.g.n, L.noise_fourier);
     }
     L.psi_fourier = false;
-    L.have_psi = true;
+    L.have_psi = !dense || nl > 1;
   }
   // fine <- HP(fine) + interpolate(LP(coarse)), coarse already combined
   for (size_t l = 1; l < nl; ++l) {
     Level &F = *c->levels[l];
     Level &C = *c->levels[l - 1];
-    long h = C.g.n / 2, nent = 3 * h * h + 1;
-    double kc = kcut_for_level(c, l - 1);
-    c->tab_b.ensure(nent * sizeof(T));
-    c->tab_c.ensure(nent * sizeof(T));
-    filter_table<T>(0, kc, C.g.kmin(), nent, (T *)c->tab_b.p, c->st);
-    filter_table<T>(0, kc, C.g.kmin(), nent, (T *)c->tab_c.p, c->st, true);
-    const T *lp = (const T *)c->tab_b.p;
-    const T *lp_k2 = (const T *)c->tab_c.p;
+    double kc = kcut_for_level(c, int(l) - 1);
     InterpGeom ig = interp_geom(F.g, C.g);
     int w0[3], wl[3];
     coarse_window(F.g, C.g, w0, wl);
     bool pruned = l == 1 && C.noise_fourier && C.g.covers_full() && wl[0] < C.g.n && wl[1] < C.g.n && wl[2] < C.g.n;
-    DevBuf *targets[4] = {&F.noise, &F.psi[0], &F.psi[1], &F.psi[2]};
-    for (int f = 0; f < 4; ++f) {
-      CoarseView v;
-      if (pruned) {
-        // the base level's delta spectrum is intact: low-pass it (and form
-        // psi from it) straight into the coarse window only
-        int nz = C.g.n / 2 + 1;
-        size_t a_bytes = size_t(wl[0]) * C.g.n * nz * 2 * sizeof(T);
-        size_t b_bytes = size_t(wl[0]) * wl[1] * nz * 2 * sizeof(T);
-        size_t o_bytes = size_t(wl[0]) * wl[1] * wl[2] * sizeof(T);
-        c->stage.ensure(a_bytes + b_bytes + o_bytes);
-        T *bufA = (T *)c->stage.p;
-        T *bufB = (T *)((char *)c->stage.p + a_bytes);
-        T *out = (T *)((char *)c->stage.p + a_bytes + b_bytes);
-        FilterInline fil;   // the same low pass (over k^2 for psi), formed in the pass
-        fil.nf = 1;
-        fil.kind[0] = 0;
-        fil.kc[0] = kc;
-        fil.over_k2 = f == 0 ? 0 : 1;
-        // delta: the low pass; psi_x: the x pass of i k_x LP/k^2 delta;
-        // psi_y, psi_z: one x pass of LP/k^2 delta, the y pass multiplying
-        // by i k_y or i k_z
-        fft_c2r_window<T>((const T *)C.noise.p, C.g.n, f == 1 ? FFT_PRE_ZA : FFT_PRE_TABLE, f == 0 ? lp : lp_k2, 0,
-                          C.g.kmin(), w0, wl, bufA, bufB, out, c->st, c->hook(), &fil,
-                          f <= 1 ? FFT_YZ_ONE : f == 2 ? FFT_YZ_IKY : FFT_YZ_IKZ, f != 3);
-        v.p = out;
-        for (int a = 0; a < 3; ++a) {
-          v.org[a] = w0[a];
-          v.len[a] = wl[a];
-        }
-        v.sx = long(wl[1]) * wl[2];
-        v.sy = wl[2];
-      } else {
-        const DevBuf &src = f == 0 ? C.noise : C.psi[f - 1];
-        if (f == 0) to_real<T>(c, C.noise, C.g.n, C.noise_fourier);
-        v = lowpass_full<T>(c, src, C.g, lp);
+    CoarseView view[4];
+    const T *lp = nullptr;
+    if (pruned) {
+      // the base level's delta spectrum is intact: low-pass it (and form
+      // psi from it) straight into the coarse window only
+      coarse_parts<T>(c, (const T *)C.noise.p, C.g, kc, 1.0, true, w0, wl, c->stage, view);
+    } else {
+      long h = C.g.n / 2, nent = 3 * h * h + 1;
+      c->tab_b.ensure(nent * sizeof(T));
+      filter_table<T>(0, kc, C.g.kmin(), nent, (T *)c->tab_b.p, c->st);
+      lp = (const T *)c->tab_b.p;
+    }
+    to_real<T>(c, F.noise, F.g.n, F.noise_fourier);
+    for (int f = 0; f < 4; ++f) {   // psi, then delta
+      DevBuf &target = f == 3 ? F.noise : F.psi[f];
+      if (!pruned) {
+        if (f == 3) to_real<T>(c, C.noise, C.g.n, C.noise_fourier);
+        view[f] = lowpass_full<T>(c, f == 3 ? C.noise : C.psi[f], C.g, lp);
       }
-      if (f == 0) to_real<T>(c, F.noise, F.g.n, F.noise_fourier);
-      {
-        // the fine field read and written, the coarse window read once
-        double coarse = double(v.len[0]) * v.len[1] * v.len[2];
-        Timed t(c, "interp_add", (2.0 * F.g.n3() + coarse) * sizeof(T));
-        interp_add<T>((T *)targets[f]->p, F.g.n, v, ig, c->st);
-      }
+      // the fine field read and written, the coarse window read once
+      double coarse = double(view[f].len[0]) * view[f].len[1] * view[f].len[2];
+      Timed t(c, "interp_add", (2.0 * F.g.n3() + coarse) * sizeof(T));
+      interp_add<T>((T *)target.p, F.g.n, view[f], ig, c->st);
     }
   }
   if (c->lpt_order == 2) {
@@ -691,8 +750,8 @@ template void do_draw<float>(gic_context *);
 template void do_draw<double>(gic_context *);
 template void ensure_noise_fourier<float>(gic_context *, Level &);
 template void ensure_noise_fourier<double>(gic_context *, Level &);
-template void do_zeldovich<float>(gic_context *);
-template void do_zeldovich<double>(gic_context *);
+template void do_zeldovich<float>(gic_context *, float *const *);
+template void do_zeldovich<double>(gic_context *, double *const *);
 
 template <typename T> void do_import_level(gic_context *c, int level, const double *host) {
   if (!c->drawn) do_draw<T>(c);
@@ -989,7 +1048,7 @@ int gic_apply_power_spectrum(gic_context *c) {
 
 int gic_zeldovich(gic_context *c) {
   return guarded(c, [&] {
-    DISPATCH(c, do_zeldovich, c);
+    DISPATCH(c, do_zeldovich, c, nullptr);
     GIC_HIP(hipStreamSynchronize(c->st));
   });
 }

@@ -211,8 +211,7 @@ struct Level {
   bool psi_fourier = false;
   bool have_psi = false;
   bool have_psi2 = false;
-  DevBuf adj_acc;          // adjoint: the noise gradient's spectrum
-  DevBuf adj_u;            // adjoint: gradient arriving from the finer level
+  DevBuf adj_u[3];         // adjoint: gradient arriving from the finer level, per component
   DevBuf adj_tab, adj_lp;  // adjoint: |k|^2 tables of the level's operators
 };
 
@@ -257,12 +256,11 @@ struct gic_context {
   bool seeded = false, drawn = false, power_applied = false, zeldovich_done = false;
   int lpt_order = 1;   // 1: Zel'dovich, 2: second-order LPT on top
   bool fix_power = false;   // fix_power: unit-modulus white noise after the draw
-  DevBuf work, stage, tab_a, tab_b, tab_c, lpt_win, adj_scratch, adj_fold;
-  // three padded fields of data transformed along x only (fft_c2r_xpass), so
-  // that one x pass serves several displacement or second-derivative fields;
-  // after the Zel'dovich pass it holds the base level's X0, X1 for 2LPT
+  DevBuf work, stage, tab_a, tab_b, tab_c, lpt_win, adj_fold;
+  // three padded fields of data transformed along x only (fft_x), so that one
+  // x pass serves several displacement or second-derivative fields; after the
+  // Zel'dovich pass of a second-order run the first holds the base level's source
   DevBuf xhalf;
-  bool xhalf_base = false;
   std::unique_ptr<EventTimer> timer;
   TimingHook *hook() { return timer.get(); }
   size_t tsize() const { return prec == 32 ? 4 : 8; }
@@ -321,7 +319,9 @@ template <typename T> void build_sqrtp(gic_context *c, Level &L);
 template <typename T> void build_sqrtp_dm(gic_context *c, Level &L);
 template <typename T> void do_draw(gic_context *c);
 template <typename T> void ensure_noise_fourier(gic_context *c, Level &L);
-template <typename T> void do_zeldovich(gic_context *c);
+// dense (optional): 3 arrays per level that also receive the base level's
+// displacements; the levels' fields then hold noise transformed along z and y
+template <typename T> void do_zeldovich(gic_context *c, T *const *dense);
 
 // ---- displacement map and its transpose (adjoint.hip) ----------------------------------
 // noise[l]: dense n_l^3 white noise; psi[3l+a]: dense displacement components

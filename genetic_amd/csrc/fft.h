@@ -108,7 +108,10 @@ enum {
   FFT_YZ_MIKZ = 4,   // -i k_z (0 at k_z = +Nyquist)
   FFT_YZ_KYKY = 5,   // k_y^2
   FFT_YZ_KYKZ = 6,   // k_y k_z (0 at either +Nyquist)
-  FFT_YZ_KZKZ = 7    // k_z^2
+  FFT_YZ_KZKZ = 7,   // k_z^2
+  FFT_YZ_I = 8,      // i
+  FFT_YZ_KZ = 9,     // k_z (0 at k_z = +Nyquist)
+  FFT_YZ_KY = 10     // k_y (0 at k_y = +Nyquist)
 };
 template <typename T>
 void fft_c2r_xpass(const T *spec, T *half, int n, int pre, const T *tab, int comp, double kmin, hipStream_t st,
@@ -119,6 +122,114 @@ void fft_c2r_yz(const T *half, T *out, int n, int yop, double kmin, hipStream_t 
 template <typename T>
 void fft_c2r_yz_lpt(const T *half, T *scratch, int n, int yop, double kmin, int epi, T *S, T *A, hipStream_t st,
                     TimingHook *hook);
+// ---- fused passes (fft_fused.h) ----------------------------------------------------
+// Fields are padded (n * n * (n + 2) values of T); nb of them form a batch,
+// *_bs values apart.
+
+// One pass along x over a spectrum, or (forward) over fields transformed
+// along z and y, which are transformed along x first, scaled by n^-1.5 and
+// post[|k|^2] (if given) and stored as the spectrum spec (if given).  Of the
+// spectrum m it makes the inverse x transforms
+//   out[0]: m (times the filter alone with plain0)   out[1]: f m
+//   out[2]: i k_x f m (0 at +Nyquist)                  out[3]: k_x^2 f m
+// (those not null) with f given as for fft_c2r_from: tab, fil (FP32) or
+// inv_k2.  plain0: fil holds a filter over k^2 and tab0 the filter's table.
+// With wlen > 0 the outputs keep the points [win0, win0 + wlen) mod n, as
+// wlen planes.
+constexpr int FFT_JOBS = 6;
+template <typename T> struct FftX {
+  const T *in = nullptr;
+  bool forward = false;
+  T *spec = nullptr, *out[4] = {nullptr, nullptr, nullptr, nullptr};
+  long in_bs = 0, spec_bs = 0, out_bs = 0;
+  int nb = 1;
+  const T *post = nullptr, *tab = nullptr, *tab0 = nullptr;
+  const FilterInline *fil = nullptr;
+  bool plain0 = false;
+  double inv_k2 = 0, kmin = 0;
+  int win0 = 0, wlen = 0;
+};
+template <typename T> void fft_x(const FftX<T> &x, int n, hipStream_t st, TimingHook *hook);
+
+// Inverse y passes: each job's input (of nouter planes, 0: n) times factors
+// FFT_YZ_*, up to three outputs (the first null one ends them).  With
+// wlen > 0 the outputs keep the points [win0, win0 + wlen) mod n of each
+// plane.  An output may be its job's input.
+template <typename T> struct FftY {
+  struct Job {
+    const T *in;
+    T *out[3];
+    int op[3];
+  } job[FFT_JOBS] = {};
+  int njob = 0, nb = 1, nouter = 0, win0 = 0, wlen = 0;
+  long in_bs = 0, out_bs = 0;
+  double kmin = 0;
+  void add(const T *in, T *o0, int p0, T *o1 = nullptr, int p1 = 0, T *o2 = nullptr, int p2 = 0) {
+    job[njob++] = Job{in, {o0, o1, o2}, {p0, p1, p2}};
+  }
+};
+template <typename T> void fft_y(const FftY<T> &y, int n, hipStream_t st, TimingHook *hook);
+
+// c2r along z, scaled by n^-1.5: each job's complex rows times a factor of
+// k_z (FFT_YZ_ONE, IKZ, MIKZ, KZ, KZKZ, I) to a padded field, a dense array or both
+template <typename T> struct FftZ {
+  struct Job {
+    const T *in;
+    T *out, *dense;
+    int op;
+  } job[FFT_JOBS] = {};
+  int njob = 0, nb = 1;
+  long in_bs = 0, out_bs = 0, dense_bs = 0;
+  double kmin = 0;
+  void add(const T *in, T *out, T *dense, int op) { job[njob++] = Job{in, out, dense, op}; }
+};
+template <typename T> void fft_z(const FftZ<T> &z, int n, hipStream_t st, TimingHook *hook);
+
+// c2r along z of nrows complex rows into the points [z0, z0 + wz) mod n of each
+template <typename T>
+void fft_z_window(const T *in, T *out, long nrows, int z0, int wz, int n, hipStream_t st, TimingHook *hook);
+
+// r2c along z of each job's padded (dense false) or dense field
+template <typename T> struct FftZFwd {
+  struct Job {
+    const T *src;
+    T *out;
+    bool dense;
+  } job[FFT_JOBS] = {};
+  int njob = 0, nb = 1;
+  long src_bs = 0, out_bs = 0;
+  void add(const T *src, T *out, bool dense) { job[njob++] = Job{src, out, dense}; }
+};
+template <typename T> void fft_z_forward(const FftZFwd<T> &z, int n, hipStream_t st, TimingHook *hook);
+
+// forward y passes: out = Y in, or with a second input -i k_y Y in - i k_z Y in2
+template <typename T> struct FftYFwd {
+  struct Job {
+    const T *in, *in2;
+    T *out;
+  } job[FFT_JOBS] = {};
+  int njob = 0, nb = 1;
+  long bs = 0;
+  double kmin = 0;
+  void add(const T *in, const T *in2, T *out) { job[njob++] = Job{in, in2, out}; }
+};
+template <typename T> void fft_y_forward(const FftYFwd<T> &y, int n, hipStream_t st, TimingHook *hook);
+
+// h1 <- inverse x transform of tab[|k|^2] n^-1.5 (-i k_x X h1 + X h0), plus the
+// same of g1, g0 with gtab if given (X the forward x transform)
+template <typename T>
+void fft_x_adjoint(T *h1, const T *h0, const T *tab, const T *g1, const T *g0, const T *gtab, int n, double kmin,
+                   hipStream_t st, TimingHook *hook);
+
+// The z passes of the second-order source S = xx yy + (xx + yy) zz - xy^2 -
+// xz^2 - yz^2, and with psi of the displacements over px, py, pz, from the
+// fields transformed along x and y of X0 = x pass of f m, X1 of i k_x f m, X2
+// of k_x^2 f m: px = y(X1), py = y(k_y X0), pz = y(X0), xx = y(X2),
+// yy = y(k_y^2 X0), xy = y(-i k_y X1)
+template <typename T>
+void fft_z_lpt(T *px, T *py, T *pz, const T *xx, const T *yy, const T *xy, T *S, bool psi, int n, double kmin,
+               hipStream_t st, TimingHook *hook);
+
 // Spectrum (r2c, N^-1.5) of a field that is zero outside the real-space window
 // [w0, w0+wl) (per axis, wrapping mod n), given as the dense window win
 // (wl[0]*wl[1]*wl[2] reals, z fastest): pruned z and y passes and a full x

@@ -5,7 +5,7 @@
 #include <cmath>
 #include <string>
 #ifndef GIC_FFT_SPLIT
-#include "fft_passes.h"
+#include "fft_fused.h"
 #endif
 
 namespace gic {
@@ -97,7 +97,55 @@ void fft_c2r_window(const T *spec, int n, int pre, const T *tab, int comp, doubl
   api<T>(n).c2r_window(spec, pre, tab, comp, T(kmin), w0, wl, bufA, bufB, out, st, hook, fil, yop, xpass);
 }
 
+template <typename T> void fft_x(const FftX<T> &x, int n, hipStream_t st, TimingHook *hook) {
+  if (x.wlen < 0 || x.wlen > n || x.win0 < 0 || x.win0 >= n) throw std::runtime_error("fft_x: bad window");
+  api<T>(n).x(x, st, hook);
+}
+template <typename T> void fft_y(const FftY<T> &y, int n, hipStream_t st, TimingHook *hook) {
+  if (y.njob < 1 || y.njob > FFT_JOBS || y.nouter < 0 || y.nouter > n || y.wlen < 0 || y.wlen > n || y.win0 < 0 ||
+      y.win0 >= n)
+    throw std::runtime_error("fft_y: bad jobs or window");
+  api<T>(n).y(y, st, hook);
+}
+template <typename T> void fft_z(const FftZ<T> &z, int n, hipStream_t st, TimingHook *hook) {
+  if (z.njob < 1 || z.njob > FFT_JOBS) throw std::runtime_error("fft_z: bad jobs");
+  api<T>(n).z(z, st, hook);
+}
+template <typename T>
+void fft_z_window(const T *in, T *out, long nrows, int z0, int wz, int n, hipStream_t st, TimingHook *hook) {
+  if (nrows < 1 || wz < 1 || wz > n || z0 < 0 || z0 >= n) throw std::runtime_error("fft_z_window: bad window");
+  api<T>(n).z_window(in, out, nrows, z0, wz, st, hook);
+}
+template <typename T> void fft_z_forward(const FftZFwd<T> &z, int n, hipStream_t st, TimingHook *hook) {
+  if (z.njob < 1 || z.njob > FFT_JOBS) throw std::runtime_error("fft_z_forward: bad jobs");
+  api<T>(n).z_forward(z, st, hook);
+}
+template <typename T> void fft_y_forward(const FftYFwd<T> &y, int n, hipStream_t st, TimingHook *hook) {
+  if (y.njob < 1 || y.njob > FFT_JOBS) throw std::runtime_error("fft_y_forward: bad jobs");
+  api<T>(n).y_forward(y, st, hook);
+}
+template <typename T>
+void fft_x_adjoint(T *h1, const T *h0, const T *tab, const T *g1, const T *g0, const T *gtab, int n, double kmin,
+                   hipStream_t st, TimingHook *hook) {
+  api<T>(n).x_adjoint(h1, h0, tab, g1, g0, gtab, kmin, st, hook);
+}
+template <typename T>
+void fft_z_lpt(T *px, T *py, T *pz, const T *xx, const T *yy, const T *xy, T *S, bool psi, int n, double kmin,
+               hipStream_t st, TimingHook *hook) {
+  api<T>(n).z_lpt(px, py, pz, xx, yy, xy, S, psi, kmin, st, hook);
+}
+
 #define GIC_FFT_INST(T)                                                                                     \
+  template void fft_x<T>(const FftX<T> &, int, hipStream_t, TimingHook *);                                  \
+  template void fft_y<T>(const FftY<T> &, int, hipStream_t, TimingHook *);                                  \
+  template void fft_z<T>(const FftZ<T> &, int, hipStream_t, TimingHook *);                                  \
+  template void fft_z_window<T>(const T *, T *, long, int, int, int, hipStream_t, TimingHook *);             \
+  template void fft_z_forward<T>(const FftZFwd<T> &, int, hipStream_t, TimingHook *);                       \
+  template void fft_y_forward<T>(const FftYFwd<T> &, int, hipStream_t, TimingHook *);                       \
+  template void fft_x_adjoint<T>(T *, const T *, const T *, const T *, const T *, const T *, int, double,    \
+                                 hipStream_t, TimingHook *);                                                 \
+  template void fft_z_lpt<T>(T *, T *, T *, const T *, const T *, const T *, T *, bool, int, double,         \
+                             hipStream_t, TimingHook *);                                                     \
   template void fft_r2c_post<T>(T *, int, const T *, hipStream_t, TimingHook *, const T *);                 \
   template void fft_c2r_to<T>(T *, T *, int, hipStream_t, TimingHook *);                                    \
   template void fft_r2c_batch<T>(T *, int, int, const T *, hipStream_t, TimingHook *);                      \

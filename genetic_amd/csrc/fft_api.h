@@ -26,6 +26,17 @@ template <typename T> struct FftApi {
                      T *bufB, T *out, hipStream_t st, TimingHook *hook, const FilterInline *fil, int yop, bool xpass);
   void (*r2c_window)(const T *win, const int *w0, const int *wl, T *bufB, T *bufA, T *spec, const T *post, bool accum,
                      hipStream_t st, TimingHook *hook, const T *aux, const FilterInline *fil, double kmin);
+  void (*z_window)(const T *in, T *out, long nrows, int z0, int wz, hipStream_t st, TimingHook *hook);
+  // fused passes
+  void (*x)(const FftX<T> &q, hipStream_t st, TimingHook *hook);
+  void (*y)(const FftY<T> &q, hipStream_t st, TimingHook *hook);
+  void (*y_forward)(const FftYFwd<T> &q, hipStream_t st, TimingHook *hook);
+  void (*x_adjoint)(T *h1, const T *h0, const T *tab, const T *g1, const T *g0, const T *gtab, double kmin,
+                    hipStream_t st, TimingHook *hook);
+  void (*z)(const FftZ<T> &q, hipStream_t st, TimingHook *hook);
+  void (*z_forward)(const FftZFwd<T> &q, hipStream_t st, TimingHook *hook);
+  void (*z_lpt)(T *px, T *py, T *pz, const T *xx, const T *yy, const T *xy, T *S, bool psi, double kmin,
+                hipStream_t st, TimingHook *hook);
 };
 
 template <typename T, int N> const FftApi<T> &fft_api();

@@ -1,0 +1,873 @@
+// Fused passes of the 3D transforms: one launch transforms several fields, or
+// makes several fields of one, so that a field is read once for all that is
+// made of it.  The displacement map, its transpose, the second-order source
+// and the batches are built of these; fft_passes.h has the plain passes.
+//
+// A strided tile (C adjacent kz columns of one line direction) is held in
+// registers, E points a thread; LDS only exchanges points between the stages
+// of a transform.  So a tile's spectrum stays in registers while one inverse
+// transform after the other is made of it.
+#pragma once
+#include "fft_passes.h"
+
+namespace gic {
+
+// Radices of a line and points per thread.  FP32 lines of 128 points and
+// more take 16 points a thread where the radices allow: one exchange fewer
+// at 256 and 1024; FP64 takes 8 (16 would leave two wavefronts per SIMD).
+template <typename T, int L> struct LinePlan;
+#define GIC_LINE_PLAN(T, L, e, ...)                      \
+  template <> struct LinePlan<T, L> {                    \
+    static constexpr int E = e;                          \
+    static constexpr int R[] = {__VA_ARGS__};            \
+    static constexpr int NS = sizeof(R) / sizeof(R[0]);  \
+  };
+GIC_LINE_PLAN(float, 4, 4, 4)
+GIC_LINE_PLAN(float, 8, 8, 8)
+GIC_LINE_PLAN(float, 16, 16, 16)
+GIC_LINE_PLAN(float, 32, 8, 4, 8)
+GIC_LINE_PLAN(float, 64, 8, 8, 8)
+GIC_LINE_PLAN(float, 128, 16, 16, 8)
+GIC_LINE_PLAN(float, 256, 16, 16, 16)
+GIC_LINE_PLAN(float, 512, 8, 8, 8, 8)
+GIC_LINE_PLAN(float, 1024, 16, 16, 8, 8)
+GIC_LINE_PLAN(double, 4, 4, 4)
+GIC_LINE_PLAN(double, 8, 8, 8)
+GIC_LINE_PLAN(double, 16, 8, 2, 8)
+GIC_LINE_PLAN(double, 32, 8, 4, 8)
+GIC_LINE_PLAN(double, 64, 8, 8, 8)
+GIC_LINE_PLAN(double, 128, 8, 2, 8, 8)
+GIC_LINE_PLAN(double, 256, 8, 4, 8, 8)
+GIC_LINE_PLAN(double, 512, 8, 8, 8, 8)
+GIC_LINE_PLAN(double, 1024, 8, 2, 8, 8, 8)
+#undef GIC_LINE_PLAN
+
+// Columns of a tile: 128-byte segments where a tile and its twiddles leave
+// two blocks per CU, 64-byte ones for the x lines of 1024 points (and FP64).
+template <typename T, int L> struct FusedCols {
+  static constexpr int x = sizeof(T) == 4 ? (L == 1024 ? 8 : 16) : (L == 1024 ? 4 : 8);
+  static constexpr int y = sizeof(T) == 4 ? 16 : (L == 1024 ? 4 : 8);
+};
+
+// One line transform of the tile in registers.  REV runs the radices in
+// reverse order, so that an inverse transform starts from the points where a
+// forward one ended.  A thread holds line tid % C; its element e is the point
+// i0 + at<R>(e), i0 = tid / C, before the first stage and after the last (R
+// that stage's radix): one offset a thread and constants for the rest, so
+// that addresses take one register.  The caller makes sure that LDS is free.
+template <typename T, int L, int C, int DIR, bool REV> struct LineFft {
+  using P = LinePlan<T, L>;
+  static constexpr int E = P::E, NS = P::NS, TH = C * L / E;
+  static constexpr int radix(int s) { return P::R[REV ? NS - 1 - s : s]; }
+  static constexpr int first = radix(0), last = radix(NS - 1);
+  static constexpr int pbefore(int s) {
+    int p = 1;
+    for (int i = 0; i < s; ++i) p *= radix(i);
+    return p;
+  }
+  template <int R> __host__ __device__ static constexpr int at(int e) { return (e / R) * (L / E) + (e % R) * (L / R); }
+  template <int S>
+  __device__ __forceinline__ static void stages(cx<T> (&v)[E], cx<T> *lds, const cx<T> *tw, int i0, int line) {
+    constexpr int R = radix(S), p = pbefore(S), PER = E / R;
+#pragma unroll
+    for (int b = 0; b < PER; ++b) {
+      const int i = i0 + b * (L / E), k = i % p;
+      if constexpr (p > 1) {
+#pragma unroll
+        for (int r = 1; r < R; ++r) {
+          cx<T> w = tw[r * k * (L / (p * R))];
+          if (DIR > 0) w.y = -w.y;
+          v[b * R + r] = cmul(v[b * R + r], w);
+        }
+      }
+      Dft<R, DIR, T>::run(v + b * R);
+    }
+    if constexpr (S < NS - 1) {
+      if constexpr (S > 0) __syncthreads();   // the stage before has read
+#pragma unroll
+      for (int b = 0; b < PER; ++b) {
+        const int i = i0 + b * (L / E), k = i % p, j = (i - k) * R + k;
+        cx<T> *o = lds + j * C + line;
+#pragma unroll
+        for (int s = 0; s < R; ++s) o[s * p * C] = v[b * R + s];
+      }
+      __syncthreads();
+      constexpr int R2 = radix(S + 1);
+      const cx<T> *o = lds + i0 * C + line;
+#pragma unroll
+      for (int e = 0; e < E; ++e) v[e] = o[at<R2>(e) * C];
+      stages<S + 1>(v, lds, tw, i0, line);
+    }
+  }
+  __device__ __forceinline__ static void run(cx<T> (&v)[E], cx<T> *lds, const cx<T> *tw) {
+    stages<0>(v, lds, tw, fresh(int(threadIdx.x)) / C, fresh(int(threadIdx.x)) % C);
+  }
+  // a value the compiler takes as new: indexes formed from it are formed
+  // where they are used, not held in registers through every stage
+  __device__ __forceinline__ static int fresh(int x) {
+    asm volatile("" : "+v"(x));
+    return x;
+  }
+  // element e from / to base + (i0 + at<R>(e)) ls + line; base and ls are the
+  // same for the whole block, the thread's part fits 32 bits of bytes
+  __device__ __forceinline__ static uint32_t offset(long ls) {
+    const int t = fresh(int(threadIdx.x));
+    return uint32_t((t / C) * uint32_t(ls) + t % C) * uint32_t(sizeof(cx<T>));
+  }
+  template <int R> __device__ __forceinline__ static void load(cx<T> (&v)[E], const cx<T> *base, long ls, int nc) {
+    const uint32_t off = offset(ls);
+    if (int(threadIdx.x) % C < nc) {
+#pragma unroll
+      for (int e = 0; e < E; ++e)
+        v[e] = *reinterpret_cast<const cx<T> *>(reinterpret_cast<const char *>(base + at<R>(e) * ls) + off);
+    } else {
+#pragma unroll
+      for (int e = 0; e < E; ++e) v[e] = cx<T>{0, 0};
+    }
+  }
+  template <int R>
+  __device__ __forceinline__ static void store(const cx<T> (&v)[E], cx<T> *base, long ls, int nc, int win0, int wlen) {
+    if (int(threadIdx.x) % C >= nc) return;
+    if (wlen < L) {
+      const int i0 = fresh(int(threadIdx.x)) / C, line = int(threadIdx.x) % C;
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        int o = i0 + at<R>(e) - win0;
+        if (o < 0) o += L;
+        if (o < wlen) base[o * ls + line] = v[e];
+      }
+      return;
+    }
+    const uint32_t off = offset(ls);
+#pragma unroll
+    for (int e = 0; e < E; ++e) *reinterpret_cast<cx<T> *>(reinterpret_cast<char *>(base + at<R>(e) * ls) + off) = v[e];
+  }
+};
+
+// ---- x passes ---------------------------------------------------------------------
+// What an x pass makes of a spectrum m(k): the inverse x transforms of
+//   out[0]: m (f0 m with the filter given as plain0)   out[1]: f m
+//   out[2]: i k_x f m (0 at +Nyquist)                    out[3]: k_x^2 f m
+// f is the |k|^2 factor of kfactor (a table, a filter product or inv_k2 /
+// k^2).  With FWD the input is a field already transformed along z and y: it
+// is transformed along x first, scaled by norm and post[|k|^2], and stored as
+// the spectrum spec (if given).  Outputs keep the points [win0, win0 + wlen).
+template <typename T> struct XArgs {
+  const cx<T> *in;
+  cx<T> *spec, *out[4];
+  long in_bs, spec_bs, out_bs;   // from one field of a batch (blockIdx.y) to the next
+  const T *post;
+  T norm, kmin;
+  PreArgs<T> f;
+  const T *tab0;   // the filter of out[0] where f divides it by k^2 (FP64)
+  int plain0;
+  int nkzb, win0, wlen;
+};
+
+template <typename T, int L, int C, bool FWD>
+__global__ __launch_bounds__((LineFft<T, L, C, 1, true>::TH), 2) void k_fft_x_fused(XArgs<T> a,
+                                                                                   const cx<T> *__restrict__ tw) {
+  using Fw = LineFft<T, L, C, -1, false>;
+  using Bw = LineFft<T, L, C, 1, true>;
+  constexpr int E = Bw::E, NZ = L / 2 + 1, R = Bw::first;   // the spectrum's points: at<R>
+  constexpr long LS = long(L) * NZ;                          // from one x to the next
+  extern __shared__ char smem_raw[];
+  cx<T> *lds = reinterpret_cast<cx<T> *>(smem_raw), *ltw = lds + C * L;
+  for (int i = int(threadIdx.x); i < L; i += Bw::TH) ltw[i] = tw[i];
+  const int tile = xcd_tile(blockIdx.x, gridDim.x), outer = tile / a.nkzb, col0 = (tile - outer * a.nkzb) * C;
+  const int nc = min(C, NZ - col0), ky = signed_k(outer, L), ky2 = ky * ky;
+  const long base = long(outer) * NZ + col0;
+  const cx<T> *in = a.in + long(blockIdx.y) * a.in_bs + base;
+  cx<T> v[E];
+  if constexpr (FWD) {
+    Fw::template load<Fw::first>(v, in, LS, nc);
+    __syncthreads();   // the twiddles
+    Fw::run(v, lds, ltw);
+  } else {
+    Bw::template load<R>(v, in, LS, nc);
+  }
+  // |k|^2 of element e; past the last column any entry of the table
+  auto ksq_at = [&](int i0, int kz, int e) {
+    const int kx = signed_k(i0 + Bw::template at<R>(e), L);
+    return kx * kx + ky2 + kz * kz;
+  };
+  auto own = [&](int &i0, int &kz) {
+    const int t = Bw::fresh(int(threadIdx.x));
+    i0 = t / C;
+    kz = min(col0 + t % C, NZ - 1);
+  };
+  if constexpr (FWD) {
+    int i0, kz;
+    own(i0, kz);
+    if (a.post) {
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const T s = a.norm * a.post[ksq_at(i0, kz, e)];
+        v[e] = cx<T>{v[e].x * s, v[e].y * s};
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < E; ++e) v[e] = cx<T>{v[e].x * a.norm, v[e].y * a.norm};
+    }
+  }
+  if (a.spec) Bw::template store<R>(v, a.spec + long(blockIdx.y) * a.spec_bs + base, LS, nc, 0, L);
+  const PreArgs<T> fa = a.f;
+  T f[E];
+#pragma unroll 1
+  for (int s = 0; s < 4; ++s) {
+    cx<T> *out = a.out[s];
+    const bool more = s == 0 && (a.out[1] || a.out[2] || a.out[3]);
+    cx<T> t[E];
+    int i0, kz;
+    own(i0, kz);
+    if (s == 0) {
+      if (out) {
+        if (a.plain0) {
+#pragma unroll
+          for (int e = 0; e < E; ++e) {
+            T g;
+            if constexpr (sizeof(T) == 4) {
+              FilterF F = fa.ff;
+              F.over_k2 = 0;
+              g = filter_fast_f(F, ksq_at(i0, kz, e));
+            } else {
+              g = a.tab0[ksq_at(i0, kz, e)];
+            }
+            t[e] = cx<T>{v[e].x * g, v[e].y * g};
+          }
+        } else {
+#pragma unroll
+          for (int e = 0; e < E; ++e) t[e] = v[e];
+        }
+      }
+      if (more) {
+        bool done = false;
+        if constexpr (sizeof(T) == 4) {
+          if (fa.ff.nf >= 0) {
+            // one factor at a time across four elements (see filter_fast_f_n)
+#pragma unroll
+            for (int c0 = 0; c0 < E; c0 += 4) {
+              const int k4[4] = {ksq_at(i0, kz, c0), ksq_at(i0, kz, c0 + 1), ksq_at(i0, kz, c0 + 2),
+                                 ksq_at(i0, kz, c0 + 3)};
+              float f4[4];
+              filter_fast_f_n<4>(fa.ff, k4, f4);
+#pragma unroll
+              for (int j = 0; j < 4; ++j) f[c0 + j] = f4[j];
+            }
+            done = true;
+          }
+        }
+        if (!done) {
+#pragma unroll
+          for (int e = 0; e < E; ++e) f[e] = kfactor<T>(fa, ksq_at(i0, kz, e));
+        }
+      }
+    }
+    if (!out) continue;
+    if (s > 0) {
+      const T kmin = a.kmin;
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const int kx = signed_k(i0 + Bw::template at<R>(e), L);
+        const T k = T(kx) * kmin;
+        T g = f[e];
+        if (s == 2) g = kx == L / 2 ? T(0) : g * k;
+        if (s == 3) g = g * (k * k);
+        t[e] = s == 2 ? cx<T>{-v[e].y * g, v[e].x * g} : cx<T>{v[e].x * g, v[e].y * g};
+      }
+    }
+    __syncthreads();   // the twiddles; that the transform before has read LDS
+    Bw::run(t, lds, ltw);
+    Bw::template store<Bw::last>(t, out + long(blockIdx.y) * a.out_bs + base, LS, nc, a.win0, a.wlen);
+  }
+}
+
+// The transpose of a displacement map's x passes: from h1 and h0, transformed
+// along z and y, the inverse x transform of
+//   tab[|k|^2] norm ( -i k_x X h1 + X h0 ),   X the forward x transform,
+// (0 for the first term at +Nyquist), plus the same of a second pair with a
+// table of its own, if given.  Written over h1.
+template <typename T> struct XAdjArgs {
+  cx<T> *h1;
+  const cx<T> *h0, *g1, *g0;
+  const T *tab, *gtab;
+  T norm, kmin;
+  int nkzb;
+};
+template <typename T, int L, int C>
+__global__ __launch_bounds__((LineFft<T, L, C, 1, true>::TH), 2) void k_fft_x_adjoint(XAdjArgs<T> a,
+                                                                                     const cx<T> *__restrict__ tw) {
+  using Fw = LineFft<T, L, C, -1, false>;
+  using Bw = LineFft<T, L, C, 1, true>;
+  constexpr int E = Bw::E, NZ = L / 2 + 1, R = Bw::first;
+  constexpr long LS = long(L) * NZ;
+  extern __shared__ char smem_raw[];
+  cx<T> *lds = reinterpret_cast<cx<T> *>(smem_raw), *ltw = lds + C * L;
+  for (int i = int(threadIdx.x); i < L; i += Bw::TH) ltw[i] = tw[i];
+  const int tile = xcd_tile(blockIdx.x, gridDim.x), outer = tile / a.nkzb, col0 = (tile - outer * a.nkzb) * C;
+  const int nc = min(C, NZ - col0), ky = signed_k(outer, L), ky2 = ky * ky;
+  const long base = long(outer) * NZ + col0;
+  cx<T> v[E], acc[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) acc[e] = cx<T>{0, 0};
+#pragma unroll 1
+  for (int s = 0; s < 4; ++s) {
+    const cx<T> *h = s == 0 ? a.h1 : s == 1 ? a.h0 : s == 2 ? a.g1 : a.g0;
+    const T *tab = s < 2 ? a.tab : a.gtab;
+    if (!h) continue;
+    Fw::template load<Fw::first>(v, h + base, LS, nc);
+    __syncthreads();   // LDS is free, the twiddles are there
+    Fw::run(v, lds, ltw);
+    const int t = Bw::fresh(int(threadIdx.x)), i0 = t / C, kz = min(col0 + t % C, NZ - 1);
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int kx = signed_k(i0 + Bw::template at<R>(e), L);
+      const T f = a.norm * tab[kx * kx + ky2 + kz * kz];
+      if (s & 1) {
+        acc[e].x += f * v[e].x;
+        acc[e].y += f * v[e].y;
+      } else {
+        const T g = kx == L / 2 ? T(0) : f * (T(kx) * a.kmin);
+        acc[e].x += g * v[e].y;
+        acc[e].y -= g * v[e].x;
+      }
+    }
+  }
+  __syncthreads();
+  Bw::run(acc, lds, ltw);
+  Bw::template store<Bw::last>(acc, a.h1 + base, LS, nc, 0, L);
+}
+
+// ---- y passes ---------------------------------------------------------------------
+// Inverse: job j (blockIdx.y) transforms its input times FFT_YZ_* factors of
+// (k_y, k_z), up to three fields from one read; outputs keep the points
+// [win0, win0 + wlen).  An output may be the input's own memory.
+constexpr int FUSED_JOBS = 6;
+template <typename T> struct YArgs {
+  struct Job {
+    const cx<T> *in;
+    cx<T> *out[3];
+    int op[3];
+  } job[FUSED_JOBS];
+  long in_bs, out_bs;   // batch (blockIdx.z)
+  long in_os, out_os;   // from one outer line to the next
+  int nkzb, win0, wlen;
+  T kmin;
+};
+// FFT_YZ_* as i^rot k_y^py k_z^pz, the first powers 0 at +Nyquist
+struct YzOp {
+  int rot, py, pz;
+};
+__device__ __forceinline__ YzOp yz_op(int op) {
+  YzOp r{0, 0, 0};
+  switch (op) {
+    case FFT_YZ_IKY: return {1, 1, 0};
+    case FFT_YZ_IKZ: return {1, 0, 1};
+    case FFT_YZ_MIKY: return {3, 1, 0};
+    case FFT_YZ_MIKZ: return {3, 0, 1};
+    case FFT_YZ_KYKY: return {0, 2, 0};
+    case FFT_YZ_KYKZ: return {0, 1, 1};
+    case FFT_YZ_KZKZ: return {0, 0, 2};
+    case FFT_YZ_I: return {1, 0, 0};
+    case FFT_YZ_KZ: return {0, 0, 1};
+    case FFT_YZ_KY: return {0, 1, 0};
+  }
+  return r;
+}
+template <typename T> __device__ __forceinline__ T k_power(int p, int k, int nyq, T kmin) {
+  const T f = T(k) * kmin;
+  return p == 0 ? T(1) : p == 2 ? f * f : k == nyq ? T(0) : f;
+}
+template <typename T> __device__ __forceinline__ cx<T> rot_mul(int rot, cx<T> v, T f) {
+  if (rot == 0) return cx<T>{v.x * f, v.y * f};
+  if (rot == 3) f = -f;
+  return cx<T>{-v.y * f, v.x * f};
+}
+
+template <typename T, int L, int C>
+__global__ __launch_bounds__((LineFft<T, L, C, 1, false>::TH), (LineFft<T, L, C, 1, false>::TH > 512 ? 1 : 2)) void
+k_fft_y_fused(YArgs<T> a, const cx<T> *__restrict__ tw) {
+  using Bw = LineFft<T, L, C, 1, false>;
+  constexpr int E = Bw::E, NZ = L / 2 + 1, R = Bw::first;
+  extern __shared__ char smem_raw[];
+  cx<T> *lds = reinterpret_cast<cx<T> *>(smem_raw), *ltw = lds + C * L;
+  for (int i = int(threadIdx.x); i < L; i += Bw::TH) ltw[i] = tw[i];
+  const auto &job = a.job[blockIdx.y];
+  const int tile = xcd_tile(blockIdx.x, gridDim.x), outer = tile / a.nkzb, col0 = (tile - outer * a.nkzb) * C;
+  const int nc = min(C, NZ - col0);
+  cx<T> v[E];
+  Bw::template load<R>(v, job.in + long(blockIdx.z) * a.in_bs + outer * a.in_os + col0, NZ, nc);
+#pragma unroll 1
+  for (int s = 0; s < 3; ++s) {
+    cx<T> *out = job.out[s];
+    if (!out) break;
+    const YzOp op = yz_op(job.op[s]);
+    const int t0 = Bw::fresh(int(threadIdx.x)), i0 = t0 / C;
+    const T gz = k_power<T>(op.pz, col0 + t0 % C, L / 2, a.kmin), kmin = a.kmin;
+    cx<T> t[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e)
+      t[e] = rot_mul<T>(op.rot, v[e], gz * k_power<T>(op.py, signed_k(i0 + Bw::template at<R>(e), L), L / 2, kmin));
+    __syncthreads();   // the twiddles; later, that LDS has been read
+    Bw::run(t, lds, ltw);
+    Bw::template store<Bw::last>(t, out + long(blockIdx.z) * a.out_bs + outer * a.out_os + col0, NZ, nc, a.win0,
+                                 a.wlen);
+  }
+}
+
+// Forward: out = Y in (op[0] one), or with a second input
+// out = -i k_y Y in - i k_z Y in2 (0 at +Nyquist): the y passes of the
+// transpose of psi_y and psi_z, whose x passes they share.
+template <typename T> struct YFwdArgs {
+  struct Job {
+    const cx<T> *in, *in2;
+    cx<T> *out;
+  } job[FUSED_JOBS];
+  long bs;
+  int nkzb;
+  T kmin;
+};
+template <typename T, int L, int C>
+__global__ __launch_bounds__((LineFft<T, L, C, 1, false>::TH), (LineFft<T, L, C, 1, false>::TH > 512 ? 1 : 2)) void
+k_fft_y_forward(YFwdArgs<T> a, const cx<T> *__restrict__ tw) {
+  using Fw = LineFft<T, L, C, -1, false>;
+  constexpr int E = Fw::E, NZ = L / 2 + 1, R = Fw::last;
+  extern __shared__ char smem_raw[];
+  cx<T> *lds = reinterpret_cast<cx<T> *>(smem_raw), *ltw = lds + C * L;
+  for (int i = int(threadIdx.x); i < L; i += Fw::TH) ltw[i] = tw[i];
+  const auto &job = a.job[blockIdx.y];
+  const int tile = xcd_tile(blockIdx.x, gridDim.x), outer = tile / a.nkzb, col0 = (tile - outer * a.nkzb) * C;
+  const int nc = min(C, NZ - col0);
+  const long at = long(blockIdx.z) * a.bs + long(outer) * L * NZ + col0;
+  cx<T> v[E];
+  Fw::template load<Fw::first>(v, job.in + at, NZ, nc);
+  __syncthreads();
+  Fw::run(v, lds, ltw);
+  if (job.in2) {
+    cx<T> r[E];
+    {
+      const int i0 = Fw::fresh(int(threadIdx.x)) / C;
+#pragma unroll
+      for (int e = 0; e < E; ++e)
+        r[e] = rot_mul<T>(3, v[e], k_power<T>(1, signed_k(i0 + Fw::template at<R>(e), L), L / 2, a.kmin));
+    }
+    Fw::template load<Fw::first>(v, job.in2 + at, NZ, nc);
+    __syncthreads();
+    Fw::run(v, lds, ltw);
+    const T gz = k_power<T>(1, col0 + Fw::fresh(int(threadIdx.x)) % C, L / 2, a.kmin);
+#pragma unroll
+    for (int e = 0; e < E; ++e) v[e] = cadd(r[e], rot_mul<T>(3, v[e], gz));
+  }
+  Fw::template store<R>(v, job.out + at, NZ, nc, 0, L);
+}
+
+// ---- z passes ---------------------------------------------------------------------
+// c2r of several fields (blockIdx.y) of a batch (blockIdx.z): complex rows
+// times a factor of k_z (FFT_YZ_ONE, IKZ, MIKZ, KZ, KZKZ or I), the real rows
+// to the padded field out (may be the input), a dense array, or both.
+template <typename T> struct ZArgs {
+  struct Job {
+    const T *in;
+    T *out, *dense;
+    int op;
+  } job[FUSED_JOBS];
+  long in_bs, out_bs, dense_bs;   // reals
+  T scale, kmin;
+};
+
+// the packed complex row of a c2r's half-length transform into LDS
+template <typename T, int N, int ROWS, int THREADS, class In>
+__device__ __forceinline__ void z_c2r_pack(cx<T> *lds, const cx<T> *__restrict__ twN, In in, int tid) {
+  constexpr int M = N / 2, H = M / 2 + 1;
+  for (int q = tid; q < ROWS * H; q += THREADS) {
+    int line = q / H, k = q - line * H;
+    cx<T> xk = in(line, k), xm = in(line, M - k);
+    if (k == 0) {   // c2r ignores the imaginary parts of the kz=0 and kz=N/2 entries
+      xk.y = 0;
+      xm.y = 0;
+    }
+    cx<T> Ev{xk.x + xm.x, xk.y - xm.y};
+    cx<T> D{xk.x - xm.x, xk.y + xm.y};
+    cx<T> w = twN[k];
+    w.y = -w.y;
+    cx<T> O = cmul(D, w);
+    lds[ZRow<M>::idx(line, k)] = cx<T>{Ev.x - O.y, Ev.y + O.x};
+    if (k != 0 && M - k != k) lds[ZRow<M>::idx(line, M - k)] = cx<T>{Ev.x + O.y, -Ev.y + O.x};
+  }
+}
+
+template <typename T, int N, int ROWS, int THREADS>
+__global__ __launch_bounds__(THREADS) void k_fft_z_c2r_fused(ZArgs<T> a, const cx<T> *__restrict__ twN) {
+  constexpr int M = N / 2;
+  extern __shared__ char smem_raw[];
+  cx<T> *lds = reinterpret_cast<cx<T> *>(smem_raw), *ltw = lds + ROWS * ZRow<M>::len;
+  for (int i = int(threadIdx.x); i < M; i += THREADS) ltw[i] = twN[2 * i];
+  const auto &job = a.job[blockIdx.y];
+  const long row0 = long(blockIdx.x) * ROWS;
+  const cx<T> *rows = reinterpret_cast<const cx<T> *>(job.in + long(blockIdx.z) * a.in_bs) + row0 * (M + 1);
+  const YzOp op = yz_op(job.op);
+  z_c2r_pack<T, N, ROWS, THREADS>(lds, twN, [&](int line, int k) {
+    return rot_mul<T>(op.rot, rows[long(line) * (M + 1) + k], k_power<T>(op.pz, k, M, a.kmin));
+  }, int(threadIdx.x));
+  __syncthreads();
+  cx<T> *out = job.out ? reinterpret_cast<cx<T> *>(job.out + long(blockIdx.z) * a.out_bs) + row0 * (M + 1) : nullptr;
+  cx<T> *dense = job.dense ? reinterpret_cast<cx<T> *>(job.dense + long(blockIdx.z) * a.dense_bs) + row0 * M : nullptr;
+  auto lidx = [](int line, int pt) { return ZRow<M>::idx(line, pt); };
+  auto lld = [&](int line, int pt) -> cx<T> { return lds[lidx(line, pt)]; };
+  auto gst = [&](int line, int pt, cx<T> v) {
+    cx<T> r{v.x * a.scale, v.y * a.scale};
+    if (out) out[long(line) * (M + 1) + pt] = r;
+    if (dense) dense[long(line) * M + pt] = r;
+  };
+  run_stages<T, M, ROWS, THREADS, +1, false, true, false, 0, false>(lds, ltw, 1, lld, gst, lidx);
+}
+
+// r2c of several fields: real rows from a padded field or a dense array (row
+// stride srs reals) to padded complex rows (may be the input).
+template <typename T> struct ZFwdArgs {
+  struct Job {
+    const T *src;
+    T *out;
+    long srs;
+  } job[FUSED_JOBS];
+  long src_bs, out_bs;
+};
+template <typename T, int N, int ROWS, int THREADS>
+__global__ __launch_bounds__(THREADS) void k_fft_z_r2c_fused(ZFwdArgs<T> a, const cx<T> *__restrict__ twN) {
+  constexpr int M = N / 2, H = M / 2 + 1;
+  extern __shared__ char smem_raw[];
+  cx<T> *lds = reinterpret_cast<cx<T> *>(smem_raw), *ltw = lds + ROWS * ZRow<M>::len;
+  for (int i = int(threadIdx.x); i < M; i += THREADS) ltw[i] = twN[2 * i];
+  const auto &job = a.job[blockIdx.y];
+  const long row0 = long(blockIdx.x) * ROWS, srs = job.srs / 2;
+  const cx<T> *src = reinterpret_cast<const cx<T> *>(job.src + long(blockIdx.z) * a.src_bs) + row0 * srs;
+  cx<T> *rows = reinterpret_cast<cx<T> *>(job.out + long(blockIdx.z) * a.out_bs) + row0 * (M + 1);
+  auto gld = [&](int line, int pt) -> cx<T> { return src[long(line) * srs + pt]; };
+  auto lidx = [](int line, int pt) { return ZRow<M>::idx(line, pt); };
+  auto lst = [&](int line, int pt, cx<T> v) { lds[lidx(line, pt)] = v; };
+  run_stages<T, M, ROWS, THREADS, -1, false, false, true, 0, false>(lds, ltw, 1, gld, lst, lidx);
+  __syncthreads();
+  for (int q = threadIdx.x; q < ROWS * H; q += THREADS) {
+    int line = q / H, k = q - line * H;
+    cx<T> zk = lds[lidx(line, k % M)], zm = lds[lidx(line, (M - k) % M)];
+    cx<T> F{(zk.x + zm.x) * T(0.5), (zk.y - zm.y) * T(0.5)};
+    cx<T> D{(zk.x - zm.x) * T(0.5), (zk.y + zm.y) * T(0.5)};
+    cx<T> wg = cmul(twN[k], cx<T>{D.y, -D.x});
+    cx<T> *o = rows + long(line) * (M + 1);
+    o[k] = cx<T>{F.x + wg.x, F.y + wg.y};
+    if (M - k != k) o[M - k] = cx<T>{F.x - wg.x, -(F.y - wg.y)};
+  }
+}
+
+// The stages of a row transform from LDS into registers: element b R + s of v
+// is point i + s M / R of butterfly q = tid + b THREADS = line (M / R) + i, R
+// the last stage's radix.  (A thread past the last butterfly repeats it.)
+template <typename T, int M, int ROWS, int THREADS, int S, int NV>
+__device__ __forceinline__ void rows_to_regs(cx<T> *lds, const cx<T> *ltw, cx<T> (&v)[NV], int tid) {
+  using P = RadixPlan<M, false>;
+  constexpr int R = P::radix(S), p = P::pbefore(S), NB = ROWS * (M / R), PER = (NB + THREADS - 1) / THREADS;
+  auto butterfly = [&](int b, cx<T> *x, int &line, int &i) {
+    const int q = min(tid + b * THREADS, NB - 1);
+    line = q / (M / R);
+    i = q % (M / R);
+    const int k = i % p;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      x[r] = lds[ZRow<M>::idx(line, i + r * (M / R))];
+      if (p > 1 && r > 0) {
+        cx<T> w = ltw[r * k * (M / (p * R))];
+        w.y = -w.y;
+        x[r] = cmul(x[r], w);
+      }
+    }
+    Dft<R, +1, T>::run(x);
+  };
+  if constexpr (S < P::nstages - 1) {
+    cx<T> x[PER][R];
+    int line[PER], i[PER];
+#pragma unroll
+    for (int b = 0; b < PER; ++b) butterfly(b, x[b], line[b], i[b]);
+    __syncthreads();
+#pragma unroll
+    for (int b = 0; b < PER; ++b) {
+      const int k = i[b] % p, j = (i[b] - k) * R + k;
+      if (NB % THREADS == 0 || tid + b * THREADS < NB) {
+#pragma unroll
+        for (int s = 0; s < R; ++s) lds[ZRow<M>::idx(line[b], j + s * p)] = x[b][s];
+      }
+    }
+    __syncthreads();
+    rows_to_regs<T, M, ROWS, THREADS, S + 1>(lds, ltw, v, tid);
+  } else {
+    static_assert(NV == PER * R, "one register per element");
+    int line, i;
+#pragma unroll
+    for (int b = 0; b < PER; ++b) butterfly(b, v + b * R, line, i);
+  }
+}
+
+// The second-order source and the first-order displacements of one level
+// from six fields transformed along x and y:
+//   px: of i k_x f m   py: of k_y f m times X0   pz: of f m   (X0, X1 of the x pass)
+//   xx: of k_x^2 f m   yy: of k_y^2 f m           xy: of k_x k_y f m
+// psi_x = Z px, psi_y = Z i py, psi_z = Z i k_z pz, phi_xz = Z (-i k_z) px,
+// phi_yz = Z k_z py, phi_zz = Z k_z^2 pz, and
+//   S = xx yy + (xx + yy) zz - xy^2 - xz^2 - yz^2
+// so that each of the six is read once for the nine transforms made of it.
+// With PSI the displacements go over px, py, pz; S to a padded field.
+template <typename T> struct ZLptArgs {
+  T *px, *py, *pz;
+  const T *xx, *yy, *xy;
+  T *S;
+  T scale, kmin;
+};
+template <typename T, int N, int ROWS, int THREADS, bool PSI>
+__global__ __launch_bounds__(THREADS, (sizeof(T) == 4 ? 4 : 2)) void k_fft_z_lpt(ZLptArgs<T> a, const cx<T> *__restrict__ twN) {
+  constexpr int M = N / 2;
+  using P = RadixPlan<M, false>;
+  constexpr int RL = P::radix(P::nstages - 1);   // the last stage's radix
+  constexpr int NB = ROWS * (M / RL), PER = (NB + THREADS - 1) / THREADS;
+  extern __shared__ char smem_raw[];
+  cx<T> *lds = reinterpret_cast<cx<T> *>(smem_raw), *ltw = lds + ROWS * ZRow<M>::len;
+  for (int i = int(threadIdx.x); i < M; i += THREADS) ltw[i] = twN[2 * i];
+  const long row0 = long(blockIdx.x) * ROWS;
+  cx<T> S[PER * RL], A[PER * RL];
+  // one piece of code for the nine transforms; indexes formed anew in each
+  // (they would fill the registers that S and A need)
+#pragma unroll 1
+  for (int s = 0; s < (PSI ? 9 : 6); ++s) {
+    // xx, yy, zz, xy, xz, yz, then the displacements, each over its own rows,
+    // whose last reading this is
+    T *own = s == 6 ? a.px : s == 7 ? a.py : a.pz;
+    const T *src = s == 0 ? a.xx : s == 1 ? a.yy : s == 2 ? a.pz : s == 3 ? a.xy : s == 4 ? a.px : s == 5 ? a.py : own;
+    const YzOp f = s == 2 ? YzOp{0, 0, 2} : s == 4 ? YzOp{3, 0, 1} : s == 5 ? YzOp{0, 0, 1} : s == 7 ? YzOp{1, 0, 0}
+                   : s == 8 ? YzOp{1, 0, 1} : YzOp{0, 0, 0};
+    const cx<T> *rows = reinterpret_cast<const cx<T> *>(src) + row0 * (M + 1);
+    int tid = int(threadIdx.x);
+    asm volatile("" : "+v"(tid));
+    __syncthreads();   // LDS is free, the twiddles are there
+    z_c2r_pack<T, N, ROWS, THREADS>(lds, twN, [&](int line, int k) {
+      return rot_mul<T>(f.rot, rows[long(line) * (M + 1) + k], k_power<T>(f.pz, k, M, a.kmin));
+    }, tid);
+    __syncthreads();
+    cx<T> v[PER * RL];
+    rows_to_regs<T, M, ROWS, THREADS, 0>(lds, ltw, v, tid);
+#pragma unroll
+    for (int e = 0; e < PER * RL; ++e) {
+      const cx<T> x{v[e].x * a.scale, v[e].y * a.scale};
+      if (s == 0) {
+        A[e] = x;
+      } else if (s == 1) {
+        S[e] = cx<T>{A[e].x * x.x, A[e].y * x.y};
+        A[e] = cadd(A[e], x);
+      } else if (s == 2) {
+        S[e] = cx<T>{S[e].x + A[e].x * x.x, S[e].y + A[e].y * x.y};
+      } else if (s < 6) {
+        S[e] = cx<T>{S[e].x - x.x * x.x, S[e].y - x.y * x.y};
+      } else {
+        A[e] = x;
+      }
+    }
+    if (s >= 5) {
+      T *dst = s == 5 ? a.S : own;
+      cx<T> *o = reinterpret_cast<cx<T> *>(dst) + row0 * (M + 1);
+#pragma unroll
+      for (int b = 0; b < PER; ++b) {
+        const int q = tid + b * THREADS, line = q / (M / RL), i = q % (M / RL);
+        if (NB % THREADS == 0 || q < NB) {
+#pragma unroll
+          for (int r = 0; r < RL; ++r) {
+            // both read, then chosen: chosen by address they would live in memory
+            const cx<T> vs = S[b * RL + r], va = A[b * RL + r];
+            o[long(line) * (M + 1) + i + r * (M / RL)] = cx<T>{s == 5 ? vs.x : va.x, s == 5 ? vs.y : va.y};
+          }
+        }
+      }
+    }
+  }
+}
+
+// ---- launches ---------------------------------------------------------------------
+template <typename T, int N> struct FftFused {
+  using F = FftN<T, N>;
+  static constexpr int NZ = N / 2 + 1, M = N / 2, ROWS = F::ROWS, ZTH = F::THREADS;
+  static constexpr int CX = FusedCols<T, N>::x, CY = FusedCols<T, N>::y;
+  static constexpr double FIELD = double(N) * N * NZ * sizeof(cx<T>);   // bytes of a spectrum
+  static cx<T> *c(T *p) { return reinterpret_cast<cx<T> *>(p); }
+  static const cx<T> *c(const T *p) { return reinterpret_cast<const cx<T> *>(p); }
+  template <class K, class... A>
+  static void launch(K kern, dim3 grid, int threads, size_t shm, const char *name, double bytes, hipStream_t st,
+                     TimingHook *hook, const A &...args) {
+    if (shm > 65536)
+      GIC_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm));
+    std::string tag;
+    if (hook) {
+      tag = std::string(name) + "." + std::to_string(N);
+      hook->begin(tag.c_str(), st);
+      hook->bytes(tag.c_str(), bytes);
+    }
+    hipLaunchKernelGGL(kern, grid, dim3(threads), shm, st, args..., twtable<T>().get(N));
+    GIC_HIP(hipGetLastError());
+    if (hook) hook->end(tag.c_str(), st);
+  }
+  static size_t tile_lds(int cols) { return sizeof(cx<T>) * (cols + 1) * N; }
+  static size_t row_lds(int rows = ROWS) { return sizeof(cx<T>) * (rows * ZRow<M>::len + M); }
+  // rows per block of the 2LPT z pass: 8 (FP32) or 4 points a thread, of which
+  // three sets are held
+  static constexpr int LROWS0 = ZTH * (sizeof(T) == 4 ? 8 : 4) / M;
+  static constexpr int LROWS = LROWS0 > N * N ? N * N : LROWS0;
+
+  static void x(const FftX<T> &q, hipStream_t st, TimingHook *hook) {
+    XArgs<T> a{};
+    a.in = c(q.in);
+    a.spec = c(q.spec);
+    for (int i = 0; i < 4; ++i) a.out[i] = c(q.out[i]);
+    a.in_bs = q.in_bs / 2;
+    a.spec_bs = q.spec_bs / 2;
+    a.out_bs = q.out_bs / 2;
+    a.post = q.post;
+    a.norm = F::norm();
+    a.kmin = T(q.kmin);
+    StridedArgs<T> s{};   // the factor's parameters, as the plain passes prepare them
+    s.tab = q.tab;
+    s.kmin_d = q.kmin;
+    s.inv_k2 = q.inv_k2;
+    if (q.fil) s.fil = *q.fil;
+    F::prepare_factor(s);
+    a.f = PreArgs<T>{s.tab, 0, NZ, N, T(q.kmin), s.inv_k2, s.kmin_d, s.ff, s.inv_k2_f};
+    a.tab0 = q.tab0;
+    a.plain0 = q.plain0 ? 1 : 0;
+    if ((q.out[1] || q.out[2] || q.out[3]) && !q.tab && q.inv_k2 == 0 && s.ff.nf < 0)
+      throw std::runtime_error("fft_x: outputs without a factor");
+    if (q.plain0 && (!q.fil || !q.tab0)) throw std::runtime_error("fft_x: plain0 without its filter");
+    a.nkzb = (NZ + CX - 1) / CX;
+    a.win0 = q.wlen > 0 ? q.win0 : 0;
+    a.wlen = q.wlen > 0 ? q.wlen : N;
+    int outs = 0;
+    for (auto *o : q.out) outs += o ? 1 : 0;
+    double bytes = q.nb * FIELD * (1.0 + (q.spec ? 1.0 : 0.0) + outs * double(a.wlen) / N);
+    constexpr int TH = LineFft<T, N, CX, 1, true>::TH;
+    dim3 grid(N * a.nkzb, q.nb);
+    if (q.forward)
+      launch(k_fft_x_fused<T, N, CX, true>, grid, TH, tile_lds(CX), "fft_x_fwd_inv", bytes, st, hook, a);
+    else
+      launch(k_fft_x_fused<T, N, CX, false>, grid, TH, tile_lds(CX), q.wlen > 0 ? "fft_x_multi_win" : "fft_x_multi",
+             bytes, st, hook, a);
+  }
+  static void y(const FftY<T> &q, hipStream_t st, TimingHook *hook) {
+    YArgs<T> a{};
+    double fields = 0;
+    a.win0 = q.wlen > 0 ? q.win0 : 0;
+    a.wlen = q.wlen > 0 ? q.wlen : N;
+    for (int j = 0; j < q.njob; ++j) {
+      a.job[j].in = c(q.job[j].in);
+      fields += 1;
+      for (int i = 0; i < 3; ++i) {
+        a.job[j].out[i] = c(q.job[j].out[i]);
+        a.job[j].op[i] = q.job[j].op[i];
+        if (q.job[j].out[i]) fields += double(a.wlen) / N;
+      }
+    }
+    const int nouter = q.nouter > 0 ? q.nouter : N;
+    a.in_bs = q.in_bs / 2;
+    a.out_bs = q.out_bs / 2;
+    a.in_os = long(N) * NZ;
+    a.out_os = long(a.wlen) * NZ;
+    a.nkzb = (NZ + CY - 1) / CY;
+    a.kmin = T(q.kmin);
+    constexpr int TH = LineFft<T, N, CY, 1, false>::TH;
+    launch(k_fft_y_fused<T, N, CY>, dim3(nouter * a.nkzb, q.njob, q.nb), TH, tile_lds(CY),
+           q.wlen > 0 ? "fft_y_multi_win" : "fft_y_multi", q.nb * FIELD * fields * nouter / N, st, hook, a);
+  }
+  static void y_forward(const FftYFwd<T> &q, hipStream_t st, TimingHook *hook) {
+    YFwdArgs<T> a{};
+    double fields = 0;
+    for (int j = 0; j < q.njob; ++j) {
+      a.job[j].in = c(q.job[j].in);
+      a.job[j].in2 = c(q.job[j].in2);
+      a.job[j].out = c(q.job[j].out);
+      fields += q.job[j].in2 ? 3 : 2;
+    }
+    a.bs = q.bs / 2;
+    a.nkzb = (NZ + CY - 1) / CY;
+    a.kmin = T(q.kmin);
+    constexpr int TH = LineFft<T, N, CY, 1, false>::TH;
+    launch(k_fft_y_forward<T, N, CY>, dim3(N * a.nkzb, q.njob, q.nb), TH, tile_lds(CY), "fft_y_fwd_multi",
+           q.nb * FIELD * fields, st, hook, a);
+  }
+  static void x_adjoint(T *h1, const T *h0, const T *tab, const T *g1, const T *g0, const T *gtab, double kmin,
+                        hipStream_t st, TimingHook *hook) {
+    XAdjArgs<T> a{c(h1), c(h0), c(g1), c(g0), tab, gtab, F::norm(), T(kmin), (NZ + CX - 1) / CX};
+    constexpr int TH = LineFft<T, N, CX, 1, true>::TH;
+    launch(k_fft_x_adjoint<T, N, CX>, dim3(N * a.nkzb), TH, tile_lds(CX), "fft_x_adjoint", FIELD * (g1 ? 5 : 3), st,
+           hook, a);
+  }
+  static void z(const FftZ<T> &q, hipStream_t st, TimingHook *hook) {
+    ZArgs<T> a{};
+    double fields = 0;
+    for (int j = 0; j < q.njob; ++j) {
+      a.job[j] = {q.job[j].in, q.job[j].out, q.job[j].dense, q.job[j].op};
+      fields += 1 + (q.job[j].out ? 1 : 0) + (q.job[j].dense ? 1 : 0);
+    }
+    a.in_bs = q.in_bs;
+    a.out_bs = q.out_bs;
+    a.dense_bs = q.dense_bs;
+    a.scale = F::norm();
+    a.kmin = T(q.kmin);
+    launch(k_fft_z_c2r_fused<T, N, ROWS, ZTH>, dim3(N * N / ROWS, q.njob, q.nb), ZTH, row_lds(), "fft_z_c2r_multi",
+           q.nb * FIELD * fields, st, hook, a);
+  }
+  static void z_forward(const FftZFwd<T> &q, hipStream_t st, TimingHook *hook) {
+    ZFwdArgs<T> a{};
+    for (int j = 0; j < q.njob; ++j) a.job[j] = {q.job[j].src, q.job[j].out, q.job[j].dense ? long(N) : long(N + 2)};
+    a.src_bs = q.src_bs;
+    a.out_bs = q.out_bs;
+    launch(k_fft_z_r2c_fused<T, N, ROWS, ZTH>, dim3(N * N / ROWS, q.njob, q.nb), ZTH, row_lds(), "fft_z_r2c_multi",
+           q.nb * FIELD * 2 * q.njob, st, hook, a);
+  }
+  static void z_lpt(T *px, T *py, T *pz, const T *xx, const T *yy, const T *xy, T *S, bool psi, double kmin,
+                    hipStream_t st, TimingHook *hook) {
+    ZLptArgs<T> a{px, py, pz, xx, yy, xy, S, F::norm(), T(kmin)};
+    dim3 grid(N * N / LROWS);
+    if (psi)
+      launch(k_fft_z_lpt<T, N, LROWS, ZTH, true>, grid, ZTH, row_lds(LROWS), "fft_z_lpt", FIELD * 10, st, hook, a);
+    else
+      launch(k_fft_z_lpt<T, N, LROWS, ZTH, false>, grid, ZTH, row_lds(LROWS), "fft_z_lpt", FIELD * 7, st, hook, a);
+  }
+};
+
+template <typename T, int N> FftApi<T> fft_api_of() {
+  using F = FftN<T, N>;
+  using G = FftFused<T, N>;
+  FftApi<T> a;
+  a.rows = F::ROWS;
+  a.prepare = [] { twtable<T>().get(N); };
+  a.r2c = F::r2c;
+  a.r2c_batch = F::r2c_batch;
+  a.r2c_boxes = F::r2c_boxes;
+  a.c2r = F::c2r;
+  a.r2c_za_adjoint = F::r2c_za_adjoint;
+  a.c2r_from = F::c2r_from;
+  a.xpass_from = F::xpass_from;
+  a.yz_from = F::yz_from;
+  a.yz_from_epi = F::yz_from_epi;
+  a.c2r_window = F::c2r_window;
+  a.r2c_window = F::r2c_window;
+  a.z_window = F::z_window;
+  a.x = G::x;
+  a.y = G::y;
+  a.y_forward = G::y_forward;
+  a.x_adjoint = G::x_adjoint;
+  a.z = G::z;
+  a.z_forward = G::z_forward;
+  a.z_lpt = G::z_lpt;
+  return a;
+}
+#ifndef GIC_FFT_SPLIT
+template <typename T, int N> const FftApi<T> &fft_api() {
+  static const FftApi<T> a = fft_api_of<T, N>();
+  return a;
+}
+#endif
+
+}  // namespace gic

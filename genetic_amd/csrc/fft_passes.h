@@ -950,12 +950,8 @@ template <typename T, int N> struct FftN {
   static constexpr int ROWS = ROWS0 > N * N ? N * N : ROWS0;
 
   static constexpr int STHREADS = strided_threads<T, N>();
-  template <int DIR, int PRE, int POST, int PASS = 0>
-  static void strided(const StridedArgs<T> &a0, int nouter, hipStream_t st, TimingHook *hook, const char *name) {
-    constexpr bool YP = PASS == 1 || PASS == 3 || PASS == 5;
-    constexpr int CP = YP ? YShape<T, N>::cols : C;
-    constexpr int TP = YP ? YShape<T, N>::threads : STHREADS;
-    StridedArgs<T> a = a0;
+  // FP32: the factor's filter and 1/k^2 in single precision
+  static void prepare_factor(StridedArgs<T> &a) {
     a.ff.nf = -1;
     if (sizeof(T) == 4) {
       if (a.fil.nf >= 0) {
@@ -974,6 +970,14 @@ template <typename T, int N> struct FftN {
       }
       a.inv_k2_f = a.kmin_d > 0 ? float(a.inv_k2 / (a.kmin_d * a.kmin_d)) : 0.f;
     }
+  }
+  template <int DIR, int PRE, int POST, int PASS = 0>
+  static void strided(const StridedArgs<T> &a0, int nouter, hipStream_t st, TimingHook *hook, const char *name) {
+    constexpr bool YP = PASS == 1 || PASS == 3 || PASS == 5;
+    constexpr int CP = YP ? YShape<T, N>::cols : C;
+    constexpr int TP = YP ? YShape<T, N>::threads : STHREADS;
+    StridedArgs<T> a = a0;
+    prepare_factor(a);
     a.ncol = NZ;
     a.nkzb = (NZ + CP - 1) / CP;
     a.n = N;
@@ -1299,8 +1303,10 @@ template <typename T, int N> struct FftN {
     if (yop < FFT_YZ_ONE || yop > FFT_YZ_KZKZ) throw std::runtime_error("c2r_window: bad y factor");
     if (yop == FFT_YZ_ONE) strided<+1, PRE_NONE, POST_NONE, 3>(ay, wl[0], st, hook, "fft_y_win");
     else strided<+1, PRE_YZ, POST_NONE, 3>(ay, wl[0], st, hook, "fft_y_op_win");
-    // z pass: rows (x_local, y_local), keep z in window
-    long nrows = long(wl[0]) * wl[1];
+    z_window(bufB, out, long(wl[0]) * wl[1], w0[2], wl[2], st, hook);
+  }
+  // c2r of nrows complex rows, z in [z0, z0 + wz) (mod N) of each kept
+  static void z_window(const T *in, T *out, long nrows, int z0, int wz, hipStream_t st, TimingHook *hook) {
     int nblk = int((nrows + ROWS - 1) / ROWS);
     size_t shm = sizeof(cx<T>) * (ROWS * ZRow<M>::len + M);   // rows, then the M-point twiddles
     const cx<T> *tw = twtable<T>().get(N);
@@ -1309,9 +1315,9 @@ template <typename T, int N> struct FftN {
     std::string tag = "fft_z_c2r_win." + std::to_string(N);
     if (hook) {
       hook->begin(tag.c_str(), st);
-      hook->bytes(tag.c_str(), double(nrows) * ((N + 2) + wl[2]) * sizeof(T));
+      hook->bytes(tag.c_str(), double(nrows) * ((N + 2) + wz) * sizeof(T));
     }
-    hipLaunchKernelGGL(kern, dim3(nblk), dim3(THREADS), shm, st, bufB, out, nrows, w0[2], wl[2], norm(), tw);
+    hipLaunchKernelGGL(kern, dim3(nblk), dim3(THREADS), shm, st, in, out, nrows, z0, wz, norm(), tw);
     GIC_HIP(hipGetLastError());
     if (hook) hook->end(tag.c_str(), st);
   }
@@ -1374,30 +1380,5 @@ template <typename T, int N> struct FftN {
     else strided<-1, PRE_NONE, POST_NONE, 4>(ax, N, st, hook, "fft_x_fwd_win");
   }
 };
-
-template <typename T, int N> FftApi<T> fft_api_of() {
-  using F = FftN<T, N>;
-  FftApi<T> a;
-  a.rows = F::ROWS;
-  a.prepare = [] { twtable<T>().get(N); };
-  a.r2c = F::r2c;
-  a.r2c_batch = F::r2c_batch;
-  a.r2c_boxes = F::r2c_boxes;
-  a.c2r = F::c2r;
-  a.r2c_za_adjoint = F::r2c_za_adjoint;
-  a.c2r_from = F::c2r_from;
-  a.xpass_from = F::xpass_from;
-  a.yz_from = F::yz_from;
-  a.yz_from_epi = F::yz_from_epi;
-  a.c2r_window = F::c2r_window;
-  a.r2c_window = F::r2c_window;
-  return a;
-}
-#ifndef GIC_FFT_SPLIT
-template <typename T, int N> const FftApi<T> &fft_api() {
-  static const FftApi<T> a = fft_api_of<T, N>();
-  return a;
-}
-#endif
 
 }  // namespace gic

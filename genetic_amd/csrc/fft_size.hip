@@ -1,6 +1,6 @@
 // The passes of one precision and size (GIC_FFT_T, GIC_FFT_N), a unit of its
 // own so that the sizes compile side by side.
-#include "fft_passes.h"
+#include "fft_fused.h"
 
 namespace gic {
 
