@@ -6,7 +6,7 @@
 // function (field.hpp:394-412) and the Zel'dovich displacement
 // (zeldovich.hpp:152-253).  Here many seeds, each with its own set of top-hat
 // overdensity constraints, run as one sequence of device work with no host
-// synchronisation inside, which is recorded into one HIP graph per batch:
+// synchronisation inside; every launch works on several realisations:
 //   w      = draw(seed)                          (the stream of gic_draw)
 //   c_i    = sqrtP_dm r2c(1_{S_i})               (the realisation's constraints in one batched r2c)
 //   G_ij   = <c_i, c_j>,  d_i = <c_i, w>         (FP64 sums, one pass over all vectors)
@@ -148,6 +148,8 @@ template <typename T>
 __global__ __launch_bounds__(GRAM_THREADS) void k_batch_gram(const cx<T> *__restrict__ cov, long fs,
                                                              const cx<T> *__restrict__ w, int nm, int n,
                                                              double *__restrict__ part) {
+  cov += size_t(blockIdx.y) * nm * fs;
+  w += size_t(blockIdx.y) * fs;
   constexpr int K = sizeof(T) == 4 ? 128 : 64;
   constexpr int S = K + 1;   // LDS row stride: rows of different vectors start in different banks
   __shared__ cx<T> sv[GRAM_VMAX * S];
@@ -220,6 +222,7 @@ __global__ __launch_bounds__(GRAM_THREADS) void k_batch_gram(const cx<T> *__rest
     }
     __syncthreads();
   }
+  part += size_t(blockIdx.y) * gridDim.x * nw * 16;
   for (int e = t; e < nw * 16; e += GRAM_THREADS) part[size_t(blockIdx.x) * nw * 16 + e] = red[e];
 }
 
@@ -234,6 +237,8 @@ __global__ __launch_bounds__(256) void k_batch_reduce(const double *__restrict__
                                                       double *__restrict__ sums) {
   __shared__ double sh[256];
   int p = blockIdx.x;
+  part += size_t(blockIdx.y) * nblk * np;
+  sums += size_t(blockIdx.y) * np;
   double s = 0;
   for (int b = threadIdx.x; b < nblk; b += 256) s += part[size_t(b) * np + p];
   sh[threadIdx.x] = s;
@@ -252,9 +257,14 @@ __global__ __launch_bounds__(256) void k_batch_reduce(const double *__restrict__
 // the constraints are not linearly independent (the RNG coverage check uses
 // 1); either leaves the coefficients at 0.
 __global__ __launch_bounds__(64) void k_batch_solve(const double *__restrict__ sums, const uint32_t *__restrict__ cnt,
-                                                    const double *__restrict__ cons, int nm,
+                                                    const double *__restrict__ cons, int nm, int np,
                                                     double *__restrict__ coef, uint32_t *__restrict__ flag) {
   __shared__ double Ls[MAXCONS * MAXCONS];
+  sums += size_t(blockIdx.x) * np;
+  cnt += size_t(blockIdx.x) * nm;
+  cons += size_t(blockIdx.x) * nm * 5;
+  coef += size_t(blockIdx.x) * nm;
+  flag += blockIdx.x;
   const int i = threadIdx.x;
   const bool row = i < nm;
   const uint32_t ni = row ? cnt[i] : 1u;
@@ -319,6 +329,9 @@ __global__ __launch_bounds__(256) void k_batch_update(cx<T> *__restrict__ w, con
                                                       int nm, const double *__restrict__ coef,
                                                       const T *__restrict__ sqrtp, int n) {
   __shared__ T s[MAXCONS];
+  w += size_t(blockIdx.y) * fs;
+  cov += size_t(blockIdx.y) * nm * fs;
+  coef += size_t(blockIdx.y) * nm;
   if (threadIdx.x < nm) s[threadIdx.x] = T(coef[threadIdx.x]);
   __syncthreads();
   size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -340,43 +353,35 @@ __global__ __launch_bounds__(256) void k_batch_update(cx<T> *__restrict__ w, con
   w[i] = cx<T>{v.x * f, v.y * f};
 }
 
+// Re(w_0) = 0 of each spectrum (randomfieldgenerator.hpp:194-195)
+template <typename T> __global__ void k_batch_dc(cx<T> *__restrict__ w, long fs, int nb) {
+  int g = threadIdx.x;
+  if (g < nb) w[size_t(g) * fs].x = T(0);
+}
+
 }  // namespace
 
-// Buffers of one chain of realisations; chains run concurrently on their own
-// streams, each realisation of a chain after the previous one.
-struct BatchLane {
-  hipStream_t st = nullptr;
-  hipEvent_t done = nullptr;
-  DevBuf w, cov, scratch, ws, part, sums, cnt, coef;
+// Device memory of a batch's groups, kept for the next call
+struct BatchState {
+  DevBuf cons, flags, win, plans, rng_ws;
+  DevBuf w, cov, x, part, sums, cnt, coef;
   DevBuf rows, zbuf, ybuf;   // covectors from the constraints' boxes
 };
 
-struct BatchState {
-  std::vector<std::unique_ptr<BatchLane>> lanes;   // lanes never move once made
-  hipEvent_t fork = nullptr;
-  DevBuf cons, flags, win, plans;
-  hipGraphExec_t exec = nullptr;   // the last recorded batch, replayed while its shape and buffers stay
-  std::vector<uint64_t> key;
-  ~BatchState() {
-    if (exec) (void)hipGraphExecDestroy(exec);
-    for (auto &l : lanes) {
-      if (l->done) (void)hipEventDestroy(l->done);
-      if (l->st) (void)hipStreamDestroy(l->st);
-    }
-    if (fork) (void)hipEventDestroy(fork);
-  }
-};
+// Realisations per launch: up to GROUP_MAX, while a group's covectors take no
+// more than GROUP_BYTES; at least the concurrency the caller asks for.
+constexpr int GROUP_MAX = 16;
+constexpr double GROUP_BYTES = 192e6;
 
 template <typename T>
 void do_batch(gic_context *c, int nreal, const uint64_t *seeds, int ncons, const double *cons, T *out, int nlanes,
-              bool graph, double *ms) {
+              bool, double *ms) {
   if (c->levels.size() != 1) throw std::runtime_error("batched realisations need exactly one grid level");
   if (!c->have_camb) throw std::runtime_error("No power spectrum has been set (use the camb command)");
   if (nreal < 1 || !seeds || !out) throw std::runtime_error("batch: no realisations, seeds or output");
   if (ncons < 1 || ncons > MAXCONS || !cons)
     throw std::runtime_error("batch: between 1 and " + std::to_string(MAXCONS) + " constraints per realisation");
   if (nlanes < 1 || nlanes > 16) throw std::runtime_error("batch: 1 to 16 concurrent chains");
-  nlanes = std::min(nlanes, nreal);
   for (int i = 0; i < nreal * ncons; ++i)
     if (!(cons[5 * i + 3] > 0) || !std::isfinite(cons[5 * i + 4]))
       throw std::runtime_error("batch: each constraint needs a positive radius and a finite target");
@@ -389,23 +394,23 @@ void do_batch(gic_context *c, int nreal, const uint64_t *seeds, int ncons, const
   const int ntile = (ncons + 1 + 3) / 4;
   const int np = ntile * (ntile + 1) / 2 * 16;   // tile sums of the Gram kernel
 
-  // everything a recorded graph needs exists before the first launch
-  fft_prepare<T>(n);
-  rng_prepare();
+  hipEvent_t t0 = nullptr, t1 = nullptr;
+  if (ms) {
+    GIC_HIP(hipEventCreate(&t0));
+    GIC_HIP(hipEventCreate(&t1));
+    GIC_HIP(hipEventRecord(t0, c->st));
+  }
   build_sqrtp<T>(c, L);
   build_sqrtp_dm<T>(c, L);
   if (!c->batch) c->batch = std::make_shared<BatchState>();
   BatchState &B = *c->batch;
-  RngPlan plan0;
-  rng_plan(seeds[0], n3, plan0);
-  size_t wsb = rng_workspace_bytes(plan0);
-  while (int(B.lanes.size()) < nlanes) {
-    B.lanes.push_back(std::make_unique<BatchLane>());
-    BatchLane &ln = *B.lanes.back();
-    GIC_HIP(hipStreamCreateWithFlags(&ln.st, hipStreamNonBlocking));
-    GIC_HIP(hipEventCreateWithFlags(&ln.done, hipEventDisableTiming));
-  }
-  if (!B.fork) GIC_HIP(hipEventCreateWithFlags(&B.fork, hipEventDisableTiming));
+  // one draw of every realisation's stream: each goes, dense, into the first
+  // of its output arrays, which its transform reads
+  std::vector<RngStream> streams;
+  for (int r = 0; r < nreal; ++r) streams.push_back({(unsigned long)seeds[r], n3, size_t(r) * 4 * n3});
+  RngPlan plan;
+  rng_plan(streams, plan);
+  B.rng_ws.ensure(rng_workspace_bytes(plan));
   // boxes around the spheres: x, y windows of wl cells from
   // floor((c - o - R)/dx - 1/2) (mod n), which hold every selected cell
   int wl = 0;
@@ -415,184 +420,142 @@ void do_batch(gic_context *c, int nreal, const uint64_t *seeds, int ncons, const
   }
   // (the row kernel indexes rows x n values in 32 bits)
   const bool boxes = wl < n && (double(ncons) * wl * wl + 1024.0) * n < 2e9;
+  int group = std::max(nlanes, std::min(GROUP_MAX, int(GROUP_BYTES / (double(ncons) * fs_reals * sizeof(T)))));
+  group = std::min(group, nreal);
+  if (boxes) group = std::min(group, int(2e9 / ((double(ncons) * wl * wl + 1024.0) * n)));
   const int rows_mult = fft_box_rows_multiple<T>(n);
-  const long nrows = boxes ? (long(ncons) * wl * wl + rows_mult - 1) / rows_mult * rows_mult : 0;
+  auto nrows_of = [&](int k) { return boxes ? (long(k) * ncons * wl * wl + rows_mult - 1) / rows_mult * rows_mult : 0; };
+  // the boxes' x origins of every constraint, then the y origins
   std::vector<int> win(boxes ? size_t(nreal) * ncons * 2 : 0);
   if (boxes) {
     const double org[2] = {g.ox, g.oy};
-    for (int q = 0; q < nreal * ncons; ++q)
-      for (int a = 0; a < 2; ++a) {
+    for (int a = 0; a < 2; ++a)
+      for (int q = 0; q < nreal * ncons; ++q) {
         long w0 = long(std::floor((cons[5 * q + a] - org[a] - cons[5 * q + 3]) / g.dx - 0.5));
         w0 %= n;
         if (w0 < 0) w0 += n;
-        win[size_t(q) * 2 + a] = int(w0);
+        win[size_t(a) * nreal * ncons + q] = int(w0);
       }
+    B.rows.ensure(size_t(nrows_of(group)) * n * sizeof(T));
+    B.zbuf.ensure(size_t(nrows_of(group)) * (n + 2) * sizeof(T));
+    B.ybuf.ensure(size_t(group) * ncons * wl * n * (n + 2) * sizeof(T));
   }
-  for (int k = 0; k < nlanes; ++k) {
-    BatchLane &ln = *B.lanes[k];
-    if (boxes) {
-      ln.rows.ensure(size_t(nrows) * n * sizeof(T));
-      ln.zbuf.ensure(size_t(nrows) * (n + 2) * sizeof(T));
-      ln.ybuf.ensure(size_t(ncons) * wl * n * (n + 2) * sizeof(T));
-    }
-    ln.w.ensure(fs_reals * sizeof(T));
-    ln.cov.ensure(size_t(ncons) * fs_reals * sizeof(T));
-    ln.scratch.ensure(fs_reals * sizeof(T));
-    ln.ws.ensure(wsb);
-    ln.part.ensure(size_t(GRAM_BLOCKS) * np * sizeof(double));
-    ln.sums.ensure(size_t(np) * sizeof(double));
-    ln.cnt.ensure(size_t(ncons) * sizeof(uint32_t));
-    ln.coef.ensure(size_t(ncons) * sizeof(double));
-  }
+  B.w.ensure(size_t(group) * fs_reals * sizeof(T));
+  B.cov.ensure(size_t(group) * ncons * fs_reals * sizeof(T));
+  B.x.ensure(size_t(group) * 4 * fs_reals * sizeof(T));
+  B.part.ensure(size_t(group) * GRAM_BLOCKS * np * sizeof(double));
+  B.sums.ensure(size_t(group) * np * sizeof(double));
+  B.cnt.ensure(size_t(group) * ncons * sizeof(uint32_t));
+  B.coef.ensure(size_t(group) * ncons * sizeof(double));
   B.cons.ensure(size_t(nreal) * ncons * 5 * sizeof(double));
   B.flags.ensure(size_t(nreal) * sizeof(uint32_t));
   GIC_HIP(hipMemcpyAsync(B.cons.p, cons, size_t(nreal) * ncons * 5 * sizeof(double), hipMemcpyHostToDevice, c->st));
   if (boxes) {
-    // per realisation: the x origins of its boxes, then the y origins
-    std::vector<int> wxy(size_t(nreal) * ncons * 2);
-    for (int r = 0; r < nreal; ++r)
-      for (int f = 0; f < ncons; ++f) {
-        wxy[(size_t(r) * 2 + 0) * ncons + f] = win[(size_t(r) * ncons + f) * 2 + 0];
-        wxy[(size_t(r) * 2 + 1) * ncons + f] = win[(size_t(r) * ncons + f) * 2 + 1];
-      }
-    B.win.ensure(wxy.size() * sizeof(int));
-    GIC_HIP(hipMemcpy(B.win.p, wxy.data(), wxy.size() * sizeof(int), hipMemcpyHostToDevice));
+    B.win.ensure(win.size() * sizeof(int));
+    GIC_HIP(hipMemcpyAsync(B.win.p, win.data(), win.size() * sizeof(int), hipMemcpyHostToDevice, c->st));
   }
   fill<uint32_t>((uint32_t *)B.flags.p, size_t(nreal), 0u, c->st);
-  // every realisation's RNG plan in device memory: the recorded work holds
-  // no seed, so one instantiated graph serves every batch of this shape
-  std::vector<RngPlan> plans(nreal);
-  const size_t pb = (rng_dev_bytes(plan0) + 255) / 256 * 256;
-  std::vector<char> hplans(size_t(nreal) * pb, 0);
-  for (int r = 0; r < nreal; ++r) {
-    rng_plan(seeds[r], n3, plans[r]);
-    rng_dev_pack(plans[r], hplans.data() + size_t(r) * pb);
-  }
-  B.plans.ensure(hplans.size());
-  GIC_HIP(hipMemcpy(B.plans.p, hplans.data(), hplans.size(), hipMemcpyHostToDevice));
-  GIC_HIP(hipStreamSynchronize(c->st));
-  std::vector<uint64_t> key;
-  {
-    auto u = [&](double v) {
-      uint64_t b;
-      memcpy(&b, &v, 8);
-      key.push_back(b);
-    };
-    auto q = [&](const void *ptr) { key.push_back(uint64_t(uintptr_t(ptr))); };
-    for (long v : {long(sizeof(T)), long(n), long(nreal), long(ncons), long(nlanes), long(boxes), long(wl), nrows,
-                   long(np), plans[0].nseg, long(plans[0].kclog)})
-      key.push_back(uint64_t(v));
-    for (double v : {g.dx, g.ox, g.oy, g.oz, g.periodic, g.kmin()}) u(v);
-    for (const void *ptr : std::initializer_list<const void *>{out, B.cons.p, B.flags.p, B.win.p, B.plans.p, L.sqrtp.p,
-                                                               L.sqrtp_dm.p})
-      q(ptr);
-    for (int k = 0; k < nlanes; ++k) {
-      BatchLane &ln = *B.lanes[k];
-      for (const void *ptr : std::initializer_list<const void *>{ln.st, ln.w.p, ln.cov.p, ln.scratch.p, ln.ws.p,
-                                                                 ln.part.p, ln.sums.p, ln.cnt.p, ln.coef.p, ln.rows.p,
-                                                                 ln.zbuf.p, ln.ybuf.p})
-        q(ptr);
-      key.push_back(uint64_t(ln.ws.bytes));
-    }
-  }
+  std::vector<char> hplan(rng_dev_bytes(plan), 0);
+  rng_dev_pack(plan, hplan.data());
+  B.plans.ensure(hplan.size());
+  GIC_HIP(hipMemcpyAsync(B.plans.p, hplan.data(), hplan.size(), hipMemcpyHostToDevice, c->st));
 
-  hipEvent_t t0 = nullptr, t1 = nullptr;
-  if (ms) {
-    GIC_HIP(hipEventCreate(&t0));
-    GIC_HIP(hipEventCreate(&t1));
-    GIC_HIP(hipEventRecord(t0, c->st));
-  }
-  auto record = [&]() {
-    GIC_HIP(hipEventRecord(B.fork, c->st));
-    for (int k = 0; k < nlanes; ++k) GIC_HIP(hipStreamWaitEvent(B.lanes[k]->st, B.fork, 0));
-    const double *dcons = (const double *)B.cons.p;
-    uint32_t *dflags = (uint32_t *)B.flags.p;
-    for (int r = 0; r < nreal; ++r) {
-      BatchLane &ln = *B.lanes[r % nlanes];
-      hipStream_t st = ln.st;
-      T *w = (T *)ln.w.p;
-      T *cv = (T *)ln.cov.p;
-      const double *rc = dcons + size_t(r) * ncons * 5;
-      // the white noise, then its spectrum with Re(w_0) = 0 (randomfieldgenerator.hpp:194-195)
-      std::vector<RngLevelOut> outs{{ln.w.p, n, n3}};
-      rng_draw_real<T>(plans[r], outs, ln.ws.p, ln.ws.bytes, st, nullptr, 1.0, dflags + r, 0,
-                       (const char *)B.plans.p + size_t(r) * pb);
-      fft_r2c_post<T>(w, n, nullptr, st, nullptr);
-      fill<T>(w, 1, T(0), st);
-      // the constraints' covectors in white-noise space
-      fill<uint32_t>((uint32_t *)ln.cnt.p, size_t(ncons), 0u, st);
-      if (boxes) {
-        const int *wx = (const int *)B.win.p + size_t(r) * 2 * ncons, *wy = wx + ncons;
-        unsigned ne = unsigned(nrows) * unsigned(n);
-        hipLaunchKernelGGL(k_batch_box_rows<T>, dim3((ne + 255) / 256), dim3(256), 0, st, (T *)ln.rows.p,
-                           unsigned(nrows), ncons, wl, n, g.dx, g.ox, g.oy, g.oz, g.periodic, rc, wx, wy,
-                           (uint32_t *)ln.cnt.p);
-        GIC_HIP(hipGetLastError());
-        fft_r2c_boxes<T>((const T *)ln.rows.p, n, nrows, ncons, wl, wx, wy, (T *)ln.zbuf.p, (T *)ln.ybuf.p, cv, fs,
-                         (const T *)L.sqrtp_dm.p, st, nullptr);
-      } else {
-        hipLaunchKernelGGL(k_batch_tophat<T>, dim3(unsigned((fs_reals + 255) / 256), ncons), dim3(256), 0, st, cv,
-                           fs_reals, n, g.dx, g.ox, g.oy, g.oz, g.periodic, rc, (uint32_t *)ln.cnt.p);
-        GIC_HIP(hipGetLastError());
-        fft_r2c_batch<T>(cv, n, ncons, (const T *)L.sqrtp_dm.p, st, nullptr);
-      }
-      // Gram matrix and current values, FP64 solve, update with the transfer function
-      hipLaunchKernelGGL(k_batch_gram<T>, dim3(GRAM_BLOCKS), dim3(GRAM_THREADS), 0, st,
-                         reinterpret_cast<const cx<T> *>(cv), fs, reinterpret_cast<const cx<T> *>(w), ncons, n,
-                         (double *)ln.part.p);
+  hipStream_t st = c->st;
+  TimingHook *hook = c->hook();
+  const double *dcons = (const double *)B.cons.p;
+  uint32_t *dflags = (uint32_t *)B.flags.p;
+  rng_draw_real<T>(plan, {{out, 0, size_t(nreal) * 4 * n3}}, B.rng_ws.p, B.rng_ws.bytes, st, hook, 1.0, dflags, 1,
+                   B.plans.p);
+  for (int r0 = 0; r0 < nreal; r0 += group) {
+    const int nb = std::min(group, nreal - r0), nc = nb * ncons;
+    T *w = (T *)B.w.p, *cv = (T *)B.cov.p, *o = out + size_t(r0) * 4 * n3;
+    const double *rc = dcons + size_t(r0) * ncons * 5;
+    // the white noise's spectra
+    FftZFwd<T> zf;
+    zf.add(o, w, true);
+    zf.nb = nb;
+    zf.src_bs = long(4 * n3);
+    zf.out_bs = fs_reals;
+    fft_z_forward<T>(zf, n, st, hook);
+    FftYFwd<T> yf;
+    yf.add(w, nullptr, w);
+    yf.nb = nb;
+    yf.bs = fs_reals;
+    fft_y_forward<T>(yf, n, st, hook);
+    FftX<T> xf;
+    xf.in = xf.spec = w;
+    xf.forward = true;
+    xf.nb = nb;
+    xf.in_bs = xf.spec_bs = fs_reals;
+    xf.kmin = g.kmin();
+    fft_x<T>(xf, n, st, hook);
+    hipLaunchKernelGGL(k_batch_dc<T>, dim3(1), dim3(64), 0, st, reinterpret_cast<cx<T> *>(w), fs, nb);
+    GIC_HIP(hipGetLastError());
+    // the constraints' covectors in white-noise space
+    fill<uint32_t>((uint32_t *)B.cnt.p, size_t(nc), 0u, st);
+    if (boxes) {
+      const int *wx = (const int *)B.win.p + size_t(r0) * ncons, *wy = wx + size_t(nreal) * ncons;
+      const long nrows = nrows_of(nb);
+      unsigned ne = unsigned(nrows) * unsigned(n);
+      hipLaunchKernelGGL(k_batch_box_rows<T>, dim3((ne + 255) / 256), dim3(256), 0, st, (T *)B.rows.p, unsigned(nrows),
+                         nc, wl, n, g.dx, g.ox, g.oy, g.oz, g.periodic, rc, wx, wy, (uint32_t *)B.cnt.p);
       GIC_HIP(hipGetLastError());
-      hipLaunchKernelGGL(k_batch_reduce, dim3(np), dim3(256), 0, st, (const double *)ln.part.p, GRAM_BLOCKS, np,
-                         (double *)ln.sums.p);
+      fft_r2c_boxes<T>((const T *)B.rows.p, n, nrows, nc, wl, wx, wy, (T *)B.zbuf.p, (T *)B.ybuf.p, cv, fs,
+                       (const T *)L.sqrtp_dm.p, st, hook);
+    } else {
+      hipLaunchKernelGGL(k_batch_tophat<T>, dim3(unsigned((fs_reals + 255) / 256), nc), dim3(256), 0, st, cv, fs_reals,
+                         n, g.dx, g.ox, g.oy, g.oz, g.periodic, rc, (uint32_t *)B.cnt.p);
       GIC_HIP(hipGetLastError());
-      hipLaunchKernelGGL(k_batch_solve, dim3(1), dim3(64), 0, st, (const double *)ln.sums.p,
-                         (const uint32_t *)ln.cnt.p, rc, ncons, (double *)ln.coef.p, dflags + r);
-      GIC_HIP(hipGetLastError());
-      hipLaunchKernelGGL(k_batch_update<T>, dim3(unsigned((fs + 255) / 256)), dim3(256), 0, st,
-                         reinterpret_cast<cx<T> *>(w), reinterpret_cast<const cx<T> *>(cv), fs, ncons,
-                         (const double *)ln.coef.p, (const T *)L.sqrtp.p, n);
-      GIC_HIP(hipGetLastError());
-      // delta and the Zel'dovich displacements, dense, into the caller's slots
-      T *o = out + size_t(r) * 4 * n3;
-      fft_c2r_from<T>(w, (T *)ln.scratch.p, n, FFT_PRE_NONE, nullptr, 0, g.kmin(), st, nullptr, o);
-      for (int a = 0; a < 3; ++a)
-        fft_c2r_from<T>(w, (T *)ln.scratch.p, n, FFT_PRE_ZA, nullptr, a, g.kmin(), st, nullptr, o + (a + 1) * n3,
-                        1.0);
+      fft_r2c_batch<T>(cv, n, nc, (const T *)L.sqrtp_dm.p, st, hook);
     }
-    for (int k = 0; k < nlanes; ++k) {
-      GIC_HIP(hipEventRecord(B.lanes[k]->done, B.lanes[k]->st));
-      GIC_HIP(hipStreamWaitEvent(c->st, B.lanes[k]->done, 0));
-    }
-  };
-  if (!graph) {
-    record();
-  } else {
-    if (B.exec && B.key != key) {
-      GIC_HIP(hipGraphExecDestroy(B.exec));
-      B.exec = nullptr;
-    }
-    if (!B.exec) {
-      hipGraph_t gr = nullptr;
-      GIC_HIP(hipStreamBeginCapture(c->st, hipStreamCaptureModeThreadLocal));
-      try {
-        record();
-      } catch (...) {
-        hipGraph_t junk = nullptr;
-        (void)hipStreamEndCapture(c->st, &junk);
-        if (junk) (void)hipGraphDestroy(junk);
-        throw;
-      }
-      GIC_HIP(hipStreamEndCapture(c->st, &gr));
-      hipError_t e = hipGraphInstantiate(&B.exec, gr, nullptr, nullptr, 0);
-      (void)hipGraphDestroy(gr);
-      if (e != hipSuccess) {
-        B.exec = nullptr;
-        GIC_HIP(e);
-      }
-      B.key = key;
-    }
-    GIC_HIP(hipGraphLaunch(B.exec, c->st));
+    // Gram matrices and current values, FP64 solves, update with the transfer function
+    hipLaunchKernelGGL(k_batch_gram<T>, dim3(GRAM_BLOCKS, nb), dim3(GRAM_THREADS), 0, st,
+                       reinterpret_cast<const cx<T> *>(cv), fs, reinterpret_cast<const cx<T> *>(w), ncons, n,
+                       (double *)B.part.p);
+    GIC_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_batch_reduce, dim3(np, nb), dim3(256), 0, st, (const double *)B.part.p, GRAM_BLOCKS, np,
+                       (double *)B.sums.p);
+    GIC_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_batch_solve, dim3(nb), dim3(64), 0, st, (const double *)B.sums.p, (const uint32_t *)B.cnt.p,
+                       rc, ncons, np, (double *)B.coef.p, dflags + r0);
+    GIC_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_batch_update<T>, dim3(unsigned((fs + 255) / 256), nb), dim3(256), 0, st,
+                       reinterpret_cast<cx<T> *>(w), reinterpret_cast<const cx<T> *>(cv), fs, ncons,
+                       (const double *)B.coef.p, (const T *)L.sqrtp.p, n);
+    GIC_HIP(hipGetLastError());
+    // delta and the Zel'dovich displacements, dense, into the caller's arrays
+    T *X = (T *)B.x.p;   // per realisation: of delta, delta/k^2 and i k_x delta/k^2, and one more
+    FftX<T> x;
+    x.in = w;
+    x.in_bs = fs_reals;
+    for (int i = 0; i < 3; ++i) x.out[i] = X + i * fs_reals;
+    x.out_bs = 4 * fs_reals;
+    x.nb = nb;
+    x.inv_k2 = 1.0;
+    x.kmin = g.kmin();
+    fft_x<T>(x, n, st, hook);
+    FftY<T> y;
+    y.nb = nb;
+    y.in_bs = y.out_bs = 4 * fs_reals;
+    y.kmin = g.kmin();
+    y.add(X, X, FFT_YZ_ONE);
+    y.add(X + 2 * fs_reals, X + 2 * fs_reals, FFT_YZ_ONE);
+    y.add(X + fs_reals, X + fs_reals, FFT_YZ_IKY, X + 3 * fs_reals, FFT_YZ_ONE);
+    fft_y<T>(y, n, st, hook);
+    FftZ<T> z;
+    z.nb = nb;
+    z.in_bs = 4 * fs_reals;
+    z.dense_bs = long(4 * n3);
+    z.kmin = g.kmin();
+    z.add(X, nullptr, o, FFT_YZ_ONE);
+    z.add(X + 2 * fs_reals, nullptr, o + n3, FFT_YZ_ONE);
+    z.add(X + fs_reals, nullptr, o + 2 * n3, FFT_YZ_ONE);
+    z.add(X + 3 * fs_reals, nullptr, o + 3 * n3, FFT_YZ_IKZ);
+    fft_z<T>(z, n, st, hook);
   }
   if (ms) GIC_HIP(hipEventRecord(t1, c->st));
+  std::vector<uint32_t> fl(nreal);
+  GIC_HIP(hipMemcpyAsync(fl.data(), B.flags.p, size_t(nreal) * sizeof(uint32_t), hipMemcpyDeviceToHost, c->st));
   GIC_HIP(hipStreamSynchronize(c->st));
   if (ms) {
     float e = 0;
@@ -601,8 +564,6 @@ void do_batch(gic_context *c, int nreal, const uint64_t *seeds, int ncons, const
     (void)hipEventDestroy(t0);
     (void)hipEventDestroy(t1);
   }
-  std::vector<uint32_t> fl(nreal);
-  GIC_HIP(hipMemcpy(fl.data(), B.flags.p, size_t(nreal) * sizeof(uint32_t), hipMemcpyDeviceToHost));
   for (int r = 0; r < nreal; ++r) {
     if (fl[r] & 1u) throw std::runtime_error("internal error: RNG plan produced too few Gaussians");
     if (fl[r] & 2u)
