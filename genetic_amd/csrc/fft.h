@@ -135,7 +135,9 @@ void fft_c2r_yz_lpt(const T *half, T *scratch, int n, int yop, double kmin, int 
 // (those not null) with f given as for fft_c2r_from: tab, fil (FP32) or
 // inv_k2.  plain0: fil holds a filter over k^2 and tab0 the filter's table.
 // With wlen > 0 the outputs keep the points [win0, win0 + wlen) mod n, as
-// wlen planes.
+// wlen planes; with iwlen > 0 (forward) the input is the iwlen planes from
+// iwin0 on of fields that are 0 elsewhere.  Outputs may be the input where
+// their windows are the same.
 constexpr int FFT_JOBS = 6;
 template <typename T> struct FftX {
   const T *in = nullptr;
@@ -147,7 +149,7 @@ template <typename T> struct FftX {
   const FilterInline *fil = nullptr;
   bool plain0 = false;
   double inv_k2 = 0, kmin = 0;
-  int win0 = 0, wlen = 0;
+  int win0 = 0, wlen = 0, iwin0 = 0, iwlen = 0;
 };
 template <typename T> void fft_x(const FftX<T> &x, int n, hipStream_t st, TimingHook *hook);
 
@@ -170,7 +172,7 @@ template <typename T> struct FftY {
 };
 template <typename T> void fft_y(const FftY<T> &y, int n, hipStream_t st, TimingHook *hook);
 
-// c2r along z, scaled by n^-1.5: each job's complex rows times a factor of
+// c2r along z, scaled by scale n^-1.5: each job's complex rows times a factor of
 // k_z (FFT_YZ_ONE, IKZ, MIKZ, KZ, KZKZ, I) to a padded field, a dense array or both
 template <typename T> struct FftZ {
   struct Job {
@@ -180,7 +182,7 @@ template <typename T> struct FftZ {
   } job[FFT_JOBS] = {};
   int njob = 0, nb = 1;
   long in_bs = 0, out_bs = 0, dense_bs = 0;
-  double kmin = 0;
+  double kmin = 0, scale = 1;
   void add(const T *in, T *out, T *dense, int op) { job[njob++] = Job{in, out, dense, op}; }
 };
 template <typename T> void fft_z(const FftZ<T> &z, int n, hipStream_t st, TimingHook *hook);
@@ -242,6 +244,10 @@ template <typename T>
 void fft_r2c_window(const T *win, int n, const int *w0, const int *wl, T *bufB, T *bufA, T *spec, const T *post,
                     bool accumulate, hipStream_t st, TimingHook *hook, const T *aux = nullptr,
                     const FilterInline *fil = nullptr, double kmin = 0);
+// its z and y passes alone: bufA <- the window's planes transformed along z and y
+template <typename T>
+void fft_r2c_window_zy(const T *win, int n, const int *w0, const int *wl, T *bufB, T *bufA, hipStream_t st,
+                       TimingHook *hook);
 // Only the real-space window [w0, w0+wl) (per axis, wrapping mod n) of
 // c2r(op(spec)), via pruned passes: bufA holds wl[0]*n*(n/2+1) complex,
 // bufB wl[0]*wl[1]*(n/2+1) complex, out wl[0]*wl[1]*wl[2] reals.  yop

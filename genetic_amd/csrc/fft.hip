@@ -80,6 +80,13 @@ void fft_c2r_yz_lpt(const T *half, T *scratch, int n, int yop, double kmin, int 
   api<T>(n).yz_from_epi(half, scratch, yop, kmin, epi, S, A, st, hook);
 }
 template <typename T>
+void fft_r2c_window_zy(const T *win, int n, const int *w0, const int *wl, T *bufB, T *bufA, hipStream_t st,
+                       TimingHook *hook) {
+  for (int a = 0; a < 3; ++a)
+    if (wl[a] < 1 || wl[a] > n || w0[a] < 0 || w0[a] >= n) throw std::runtime_error("fft_r2c_window: bad window");
+  api<T>(n).r2c_window_zy(win, w0, wl, bufB, bufA, st, hook);
+}
+template <typename T>
 void fft_r2c_window(const T *win, int n, const int *w0, const int *wl, T *bufB, T *bufA, T *spec, const T *post,
                     bool accumulate, hipStream_t st, TimingHook *hook, const T *aux, const FilterInline *fil,
                     double kmin) {
@@ -161,6 +168,7 @@ void fft_z_lpt(T *px, T *py, T *pz, const T *xx, const T *yy, const T *xy, T *S,
                                  double);                                                                    \
   template void fft_c2r_yz<T>(const T *, T *, int, int, double, hipStream_t, TimingHook *, T *);              \
   template void fft_c2r_yz_lpt<T>(const T *, T *, int, int, double, int, T *, T *, hipStream_t, TimingHook *); \
+  template void fft_r2c_window_zy<T>(const T *, int, const int *, const int *, T *, T *, hipStream_t, TimingHook *); \
   template void fft_r2c_window<T>(const T *, int, const int *, const int *, T *, T *, T *, const T *, bool,      \
                                   hipStream_t, TimingHook *, const T *, const FilterInline *, double);         \
   template void fft_c2r_window<T>(const T *, int, int, const T *, int, double, const int *, const int *, T *, T *, \

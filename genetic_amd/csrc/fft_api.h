@@ -26,6 +26,7 @@ template <typename T> struct FftApi {
                      T *bufB, T *out, hipStream_t st, TimingHook *hook, const FilterInline *fil, int yop, bool xpass);
   void (*r2c_window)(const T *win, const int *w0, const int *wl, T *bufB, T *bufA, T *spec, const T *post, bool accum,
                      hipStream_t st, TimingHook *hook, const T *aux, const FilterInline *fil, double kmin);
+  void (*r2c_window_zy)(const T *win, const int *w0, const int *wl, T *bufB, T *bufA, hipStream_t st, TimingHook *hook);
   void (*z_window)(const T *in, T *out, long nrows, int z0, int wz, hipStream_t st, TimingHook *hook);
   // fused passes
   void (*x)(const FftX<T> &q, hipStream_t st, TimingHook *hook);

@@ -128,6 +128,18 @@ template <typename T, int L, int C, int DIR, bool REV> struct LineFft {
       for (int e = 0; e < E; ++e) v[e] = cx<T>{0, 0};
     }
   }
+  // the same of an input that holds only the points [win0, win0 + wlen)
+  template <int R>
+  __device__ __forceinline__ static void load_window(cx<T> (&v)[E], const cx<T> *base, long ls, int nc, int win0,
+                                                     int wlen) {
+    const int i0 = fresh(int(threadIdx.x)) / C, line = int(threadIdx.x) % C;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      int o = i0 + at<R>(e) - win0;
+      if (o < 0) o += L;
+      v[e] = line < nc && o < wlen ? base[o * ls + line] : cx<T>{0, 0};
+    }
+  }
   template <int R>
   __device__ __forceinline__ static void store(const cx<T> (&v)[E], cx<T> *base, long ls, int nc, int win0, int wlen) {
     if (int(threadIdx.x) % C >= nc) return;
@@ -154,7 +166,8 @@ template <typename T, int L, int C, int DIR, bool REV> struct LineFft {
 // f is the |k|^2 factor of kfactor (a table, a filter product or inv_k2 /
 // k^2).  With FWD the input is a field already transformed along z and y: it
 // is transformed along x first, scaled by norm and post[|k|^2], and stored as
-// the spectrum spec (if given).  Outputs keep the points [win0, win0 + wlen).
+// the spectrum spec (if given).  Outputs keep the points [win0, win0 + wlen);
+// a FWD input holds the points [iwin0, iwin0 + iwlen) and is 0 elsewhere.
 template <typename T> struct XArgs {
   const cx<T> *in;
   cx<T> *spec, *out[4];
@@ -164,7 +177,7 @@ template <typename T> struct XArgs {
   PreArgs<T> f;
   const T *tab0;   // the filter of out[0] where f divides it by k^2 (FP64)
   int plain0;
-  int nkzb, win0, wlen;
+  int nkzb, win0, wlen, iwin0, iwlen;
 };
 
 template <typename T, int L, int C, bool FWD>
@@ -183,7 +196,8 @@ __global__ __launch_bounds__((LineFft<T, L, C, 1, true>::TH), 2) void k_fft_x_fu
   const cx<T> *in = a.in + long(blockIdx.y) * a.in_bs + base;
   cx<T> v[E];
   if constexpr (FWD) {
-    Fw::template load<Fw::first>(v, in, LS, nc);
+    if (a.iwlen < L) Fw::template load_window<Fw::first>(v, in, LS, nc, a.iwin0, a.iwlen);
+    else Fw::template load<Fw::first>(v, in, LS, nc);
     __syncthreads();   // the twiddles
     Fw::run(v, lds, ltw);
   } else {
@@ -746,9 +760,11 @@ template <typename T, int N> struct FftFused {
     a.nkzb = (NZ + CX - 1) / CX;
     a.win0 = q.wlen > 0 ? q.win0 : 0;
     a.wlen = q.wlen > 0 ? q.wlen : N;
+    a.iwin0 = q.iwlen > 0 ? q.iwin0 : 0;
+    a.iwlen = q.iwlen > 0 ? q.iwlen : N;
     int outs = 0;
     for (auto *o : q.out) outs += o ? 1 : 0;
-    double bytes = q.nb * FIELD * (1.0 + (q.spec ? 1.0 : 0.0) + outs * double(a.wlen) / N);
+    double bytes = q.nb * FIELD * (double(a.iwlen) / N + (q.spec ? 1.0 : 0.0) + outs * double(a.wlen) / N);
     constexpr int TH = LineFft<T, N, CX, 1, true>::TH;
     dim3 grid(N * a.nkzb, q.nb);
     if (q.forward)
@@ -815,7 +831,7 @@ template <typename T, int N> struct FftFused {
     a.in_bs = q.in_bs;
     a.out_bs = q.out_bs;
     a.dense_bs = q.dense_bs;
-    a.scale = F::norm();
+    a.scale = F::norm() * T(q.scale);
     a.kmin = T(q.kmin);
     launch(k_fft_z_c2r_fused<T, N, ROWS, ZTH>, dim3(N * N / ROWS, q.njob, q.nb), ZTH, row_lds(), "fft_z_c2r_multi",
            q.nb * FIELD * fields, st, hook, a);
@@ -856,6 +872,7 @@ template <typename T, int N> FftApi<T> fft_api_of() {
   a.yz_from_epi = F::yz_from_epi;
   a.c2r_window = F::c2r_window;
   a.r2c_window = F::r2c_window;
+  a.r2c_window_zy = F::r2c_window_zy;
   a.z_window = F::z_window;
   a.x = G::x;
   a.y = G::y;

@@ -1321,14 +1321,9 @@ template <typename T, int N> struct FftN {
     GIC_HIP(hipGetLastError());
     if (hook) hook->end(tag.c_str(), st);
   }
-  // spectrum of a field that is zero outside the real-space window
-  // [w0, w0+wl) (per axis, mod N), given as the dense window `win`
-  // (wl[0]*wl[1]*wl[2] reals): pruned z and y passes, a full x pass whose
-  // output is scaled by post[|k|^2] (if given) and stored or added into spec.
-  // bufB holds wl[0]*wl[1] padded rows, bufA wl[0]*N*(N/2+1) complex.
-  static void r2c_window(const T *win, const int *w0, const int *wl, T *bufB, T *bufA, T *spec, const T *post,
-                         bool accum, hipStream_t st, TimingHook *hook, const T *aux = nullptr, const FilterInline *fil = nullptr,
-                         double kmin = 0) {
+  // the z and y passes of r2c_window: bufA <- wl[0] planes
+  static void r2c_window_zy(const T *win, const int *w0, const int *wl, T *bufB, T *bufA, hipStream_t st,
+                            TimingHook *hook) {
     long nrows = long(wl[0]) * wl[1];
     int nblk = int((nrows + ROWS - 1) / ROWS);
     size_t shm = sizeof(cx<T>) * (ROWS * ZRow<M>::len + M);   // rows, then the M-point twiddles
@@ -1357,6 +1352,16 @@ template <typename T, int N> struct FftN {
     ay.in_wlen = wl[1];
     ay.scale = T(1);
     strided<-1, PRE_NONE, POST_NONE, 5>(ay, wl[0], st, hook, "fft_y_fwd_win");
+  }
+  // spectrum of a field that is zero outside the real-space window
+  // [w0, w0+wl) (per axis, mod N), given as the dense window `win`
+  // (wl[0]*wl[1]*wl[2] reals): pruned z and y passes, a full x pass whose
+  // output is scaled by post[|k|^2] (if given) and stored or added into spec.
+  // bufB holds wl[0]*wl[1] padded rows, bufA wl[0]*N*(N/2+1) complex.
+  static void r2c_window(const T *win, const int *w0, const int *wl, T *bufB, T *bufA, T *spec, const T *post,
+                         bool accum, hipStream_t st, TimingHook *hook, const T *aux = nullptr, const FilterInline *fil = nullptr,
+                         double kmin = 0) {
+    r2c_window_zy(win, w0, wl, bufB, bufA, st, hook);
     // x pass: tiles (ky, kz block), lines over kx from the wl[0] window planes
     StridedArgs<T> ax{};
     ax.in = reinterpret_cast<const cx<T> *>(bufA);

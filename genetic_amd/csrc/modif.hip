@@ -535,6 +535,46 @@ __global__ void k_flag_center(T *__restrict__ f, int n, const uint64_t *__restri
   f[p] = v / T(m);
 }
 
+// The same on a box of the level, all of its cells read in order: mask is 1
+// at the flagged ones.
+__global__ void k_box_mask(const uint64_t *__restrict__ idx, size_t m, int n, int x0, int y0, int z0, int by, int bz,
+                           uint8_t *__restrict__ mask) {
+  size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= m) return;
+  const uint64_t c = idx[i], r = c / uint64_t(n);
+  int x = int(r / uint64_t(n)) - x0, y = int(r % uint64_t(n)) - y0, z = int(c % uint64_t(n)) - z0;
+  x += x < 0 ? n : 0;
+  y += y < 0 ? n : 0;
+  z += z < 0 ? n : 0;
+  mask[(size_t(x) * by + y) * bz + z] = 1;
+}
+template <typename T>
+__global__ void k_box_keep(T *__restrict__ f, const uint8_t *__restrict__ mask, size_t n, T *__restrict__ copy) {
+  size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const T v = mask[i] ? f[i] : T(0);
+  f[i] = v;
+  if (copy) copy[i] = v;
+}
+template <typename T>
+__global__ __launch_bounds__(RED_THREADS) void k_box_sum(const T *__restrict__ f, const uint8_t *__restrict__ mask,
+                                                         size_t n, double *__restrict__ part) {
+  double acc = 0;
+  for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += size_t(gridDim.x) * blockDim.x)
+    if (mask[i]) acc += double(f[i]);
+  double s = block_sum(acc);
+  if (threadIdx.x == 0) part[blockIdx.x] = s;
+}
+template <typename T>
+__global__ void k_box_center(T *__restrict__ f, const uint8_t *__restrict__ mask, size_t n, size_t m,
+                             const double *__restrict__ sum) {
+  size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const T mean = T(*sum) / T(m);
+  const T v = f[i] - mean;
+  f[i] = mask[i] ? v / T(m) : T(0);
+}
+
 // fine -> coarse: the mean of the contained fine subcells of each coarse
 // cell whose first or last subcell lies in the fine grid (SubSampleEvaluator
 // over a SectionOfGrid of the fine grid)
@@ -1568,28 +1608,158 @@ template <typename T> MLF<T> linear_covector(gic_context *c, const std::string &
   return m;
 }
 
+// The variance operator W H C W H W of one level (W keeps the flagged cells,
+// H the high pass, C subtracts the mean and divides by the number of cells)
+// acts on flagged cells only: all that it needs are the values on the box
+// around them, and H from box to box, through transforms whose z and y
+// passes and both ends of whose x pass are cut to the box.
+template <typename T> struct VarianceBox {
+  gic_context *c;
+  size_t l;
+  Box3 B;
+  size_t nb = 0;
+  DevList cells;
+  PBuf mask, box, a, b;
+
+  // false where the cells span more than half the level along x: there the
+  // cut passes' scratch would exceed a field's (256^3 FP32, 14000 cells, value
+  // and gradient: a box of 31 cells a side 0.50 ms, of 128 0.51 ms, of 129 and
+  // more 1.30 ms with full transforms)
+  bool make(gic_context *cc, size_t level, const std::vector<uint64_t> &idx) {
+    c = cc;
+    l = level;
+    const LevelGeom &g = c->levels[l]->g;
+    const uint64_t n = uint64_t(g.n), n3 = g.n3();
+    if (idx.empty()) return false;
+    std::vector<uint8_t> member(3 * n, 0);
+    uint8_t *mx = member.data(), *my = mx + n, *mz = my + n;
+    const bool pow2 = (n & (n - 1)) == 0;
+    const int sh = __builtin_ctzll(n);
+    for (uint64_t i : idx) {
+      if (i >= n3) return false;
+      const uint64_t r = pow2 ? i >> sh : i / n, x = pow2 ? r >> sh : r / n;
+      mx[x] = my[r - x * n] = mz[i - r * n] = 1;
+    }
+    for (int d = 0; d < 3; ++d) {
+      // all but the longest cyclic run of indices without a flagged cell
+      const uint8_t *u = member.data() + d * n;
+      int best = 0, end = 0, run = 0;
+      for (int i = 0; i < 2 * int(n); ++i) {
+        run = u[i % int(n)] ? 0 : run + 1;
+        if (run > best && run < int(n)) {
+          best = run;
+          end = i + 1;
+        }
+      }
+      B.b0[d] = end % int(n);
+      B.bl[d] = int(n) - best;
+    }
+    if (B.bl[0] > int(n) / 2) return false;
+    nb = box_cells(B);
+    upload_list(c, idx, cells);
+    mask = PBuf(c->mod->pool, nb);
+    fill<uint8_t>((uint8_t *)mask.p, nb, 0, c->st);
+    hipLaunchKernelGGL(k_box_mask, dim3(blocks(cells.n)), dim3(256), 0, c->st, (const uint64_t *)cells.idx.p, cells.n,
+                       g.n, B.b0[0], B.b0[1], B.b0[2], B.bl[1], B.bl[2], (uint8_t *)mask.p);
+    GIC_HIP(hipGetLastError());
+    box = PBuf(c->mod->pool, nb * sizeof(T));
+    BoxBufs<T> bb(c, g.n, B);
+    a = std::move(bb.a);
+    b = std::move(bb.b);
+    return true;
+  }
+  T *v() { return (T *)box.p; }
+  T *A() { return (T *)a.p; }
+  // W; the kept values also to copy, if given
+  void window(T *copy = nullptr) {
+    hipLaunchKernelGGL(k_box_keep<T>, dim3(blocks(nb)), dim3(256), 0, c->st, v(), (const uint8_t *)mask.p, nb, copy);
+    GIC_HIP(hipGetLastError());
+  }
+  // the box of planes A (transformed along x already), to v()
+  void from_planes() {
+    const int n = c->levels[l]->g.n;
+    FftY<T> y;
+    y.nouter = B.bl[0];
+    y.win0 = B.b0[1];
+    y.wlen = B.bl[1];
+    y.add(A(), (T *)b.p, FFT_YZ_ONE);
+    fft_y<T>(y, n, c->st, c->hook());
+    fft_z_window<T>((const T *)b.p, v(), long(B.bl[0]) * B.bl[1], B.b0[2], B.bl[2], n, c->st, c->hook());
+  }
+  void to_planes() { fft_r2c_window_zy<T>(v(), c->levels[l]->g.n, B.b0, B.bl, (T *)b.p, A(), c->st, c->hook()); }
+  void high_pass(const T *tab) {
+    to_planes();
+    FftX<T> x;
+    x.in = A();
+    x.forward = true;
+    x.post = tab;
+    x.out[0] = A();
+    x.win0 = x.iwin0 = B.b0[0];
+    x.wlen = x.iwlen = B.bl[0];
+    fft_x<T>(x, c->levels[l]->g.n, c->st, c->hook());
+    from_planes();
+  }
+  void center() {
+    ensure_red(c);
+    const int nblk = std::min(RED_BLOCKS, blocks(nb));
+    hipLaunchKernelGGL(k_box_sum<T>, dim3(nblk), dim3(RED_THREADS), 0, c->st, (const T *)v(),
+                       (const uint8_t *)mask.p, nb, (double *)c->mod->part.p);
+    hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(RED_THREADS), 0, c->st, (const double *)c->mod->part.p, nblk,
+                       (double *)c->mod->scalar.p);
+    hipLaunchKernelGGL(k_box_center<T>, dim3(blocks(nb)), dim3(256), 0, c->st, v(), (const uint8_t *)mask.p, nb,
+                       cells.n, (const double *)c->mod->scalar.p);
+    GIC_HIP(hipGetLastError());
+  }
+  void apply(const FilterSpec &hp, T *first = nullptr) {
+    const T *tab = spec_table<T>(c, c->levels[l]->g, hp);
+    window(first);
+    high_pass(tab);
+    center();   // masks too
+    high_pass(tab);
+    window();
+  }
+};
+
+FilterSpec variance_high_pass(double scale) {
+  FilterSpec hp;
+  hp.na = 1;
+  hp.ka[0] = 2;
+  hp.ca[0] = 2 * M_PI / scale;
+  return hp;
+}
+
 // FilteredVarianceModification::pushMultiLevelFieldThroughMatrix
 template <typename T> MLF<T> push_variance(MLF<T> &field, const std::vector<std::vector<uint64_t>> &flags,
                                            double scale) {
   gic_context *c = field.c;
   MLF<T> f = field.clone();
   transfer_to_dm(f);
-  FilterSpec hp;
-  hp.na = 1;
-  hp.ka[0] = 2;
-  hp.ca[0] = 2 * M_PI / scale;
+  const FilterSpec hp = variance_high_pass(scale);
   for (size_t l = 0; l < f.nl(); ++l) {
     const LevelGeom &g = f.g(l);
     size_t n3 = g.n3();
     static const std::vector<uint64_t> none;
     const std::vector<uint64_t> &cells = l < flags.size() ? flags[l] : none;
+    if (cells.empty()) {   // nothing of this level is kept
+      f.zero(l);
+      f.fourier[l] = true;
+      continue;
+    }
+    VarianceBox<T> V;
+    if (V.make(c, l, cells)) {
+      fft_c2r_window<T>(f.p(l), g.n, FFT_PRE_NONE, nullptr, 0, g.kmin(), V.B.b0, V.B.bl, V.A(), (T *)V.b.p, V.v(),
+                        c->st, c->hook());
+      V.apply(hp);
+      fft_r2c_window<T>(V.v(), g.n, V.B.b0, V.B.bl, (T *)V.b.p, V.A(), f.p(l), nullptr, false, c->st, c->hook());
+      GIC_HIP(hipStreamSynchronize(c->st));   // the cell list is released here
+      continue;
+    }
     PBuf mask(c->mod->pool, n3);
     fill<uint8_t>((uint8_t *)mask.p, n3, 0, c->st);
     DevList dl;
     upload_list(c, cells, dl);
-    if (dl.n)
-      hipLaunchKernelGGL(k_mask_set, dim3(blocks(dl.n)), dim3(256), 0, c->st, (uint8_t *)mask.p,
-                         (const uint64_t *)dl.idx.p, dl.n);
+    hipLaunchKernelGGL(k_mask_set, dim3(blocks(dl.n)), dim3(256), 0, c->st, (uint8_t *)mask.p,
+                       (const uint64_t *)dl.idx.p, dl.n);
     auto window = [&]() {
       f.toR(l);
       hipLaunchKernelGGL(k_mask_keep<T>, dim3(blocks(n3)), dim3(256), 0, c->st, f.p(l), g.n, (const uint8_t *)mask.p);
@@ -1597,16 +1767,14 @@ template <typename T> MLF<T> push_variance(MLF<T> &field, const std::vector<std:
     window();
     apply_spec(f, l, hp);
     window();
-    if (dl.n) {
-      c->mod->part.ensure(RED_BLOCKS * sizeof(double));
-      c->mod->scalar.ensure(sizeof(double) * 8);
-      hipLaunchKernelGGL(k_flag_sum<T>, dim3(RED_BLOCKS), dim3(RED_THREADS), 0, c->st, (const T *)f.p(l), g.n,
-                         (const uint64_t *)dl.idx.p, dl.n, (double *)c->mod->part.p);
-      hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(RED_THREADS), 0, c->st, (const double *)c->mod->part.p,
-                         RED_BLOCKS, (double *)c->mod->scalar.p);
-      hipLaunchKernelGGL(k_flag_center<T>, dim3(blocks(dl.n)), dim3(256), 0, c->st, f.p(l), g.n,
-                         (const uint64_t *)dl.idx.p, dl.n, (const double *)c->mod->scalar.p);
-    }
+    c->mod->part.ensure(RED_BLOCKS * sizeof(double));
+    c->mod->scalar.ensure(sizeof(double) * 8);
+    hipLaunchKernelGGL(k_flag_sum<T>, dim3(RED_BLOCKS), dim3(RED_THREADS), 0, c->st, (const T *)f.p(l), g.n,
+                       (const uint64_t *)dl.idx.p, dl.n, (double *)c->mod->part.p);
+    hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(RED_THREADS), 0, c->st, (const double *)c->mod->part.p,
+                       RED_BLOCKS, (double *)c->mod->scalar.p);
+    hipLaunchKernelGGL(k_flag_center<T>, dim3(blocks(dl.n)), dim3(256), 0, c->st, f.p(l), g.n,
+                       (const uint64_t *)dl.idx.p, dl.n, (const double *)c->mod->scalar.p);
     apply_spec(f, l, hp);
     window();
     GIC_HIP(hipStreamSynchronize(c->st));   // the cell list is released here
@@ -2026,6 +2194,61 @@ template <typename T> double mod_variance_gradient(gic_context *c, const T *cons
   c->power_applied = c->zeldovich_done = false;   // the operator acts on white noise
   double v = 0;
   try {
+    VarianceBox<T> V;
+    if (c->levels.size() == 1 && noise[0] && V.make(c, 0, c->flags[0])) {
+      // One level, without a level filter: Q = T W H C W H W T, T = sqrt P_dm,
+      // and with u = W T w and g = W H C W H u, V = <g, u> on the box.  The
+      // full field passes only along x, y and z to the box and back.
+      Level &L = *c->levels[0];
+      const int n = L.g.n;
+      build_sqrtp_dm<T>(c, L);
+      const T *tr = (const T *)L.sqrtp_dm.p;
+      PBuf full(c->mod->pool, L.g.padded_reals() * sizeof(T)), first(c->mod->pool, V.nb * sizeof(T));
+      T *h = (T *)full.p;
+      FftZFwd<T> z;
+      z.add(noise[0], h, true);
+      fft_z_forward<T>(z, n, c->st, c->hook());
+      FftYFwd<T> y;
+      y.add(h, nullptr, h);
+      fft_y_forward<T>(y, n, c->st, c->hook());
+      FftX<T> x;
+      x.in = h;
+      x.forward = true;
+      x.post = tr;
+      x.out[0] = V.A();
+      x.win0 = V.B.b0[0];
+      x.wlen = V.B.bl[0];
+      fft_x<T>(x, n, c->st, c->hook());
+      V.from_planes();
+      V.apply(variance_high_pass(c->variance_scale), (T *)first.p);
+      ensure_red(c);
+      const int nblk = std::min(RED_BLOCKS, blocks(V.nb));
+      hipLaunchKernelGGL(k_dot_partial<T>, dim3(nblk), dim3(RED_THREADS), 0, c->st, (const T *)V.v(),
+                         (const T *)first.p, V.nb, (double *)c->mod->part.p);
+      if (grad) {
+        if (!grad[0]) throw std::runtime_error("variance gradient: null device pointer");
+        V.to_planes();
+        FftX<T> xb;
+        xb.in = V.A();
+        xb.forward = true;
+        xb.iwin0 = V.B.b0[0];
+        xb.iwlen = V.B.bl[0];
+        xb.post = tr;
+        xb.out[0] = h;
+        fft_x<T>(xb, n, c->st, c->hook());
+        FftY<T> yb;
+        yb.add(h, h, FFT_YZ_ONE);
+        fft_y<T>(yb, n, c->st, c->hook());
+        FftZ<T> zb;
+        zb.scale = 2;
+        zb.add(h, nullptr, grad[0], FFT_YZ_ONE);
+        fft_z<T>(zb, n, c->st, c->hook());
+      }
+      v = finish_reduction(c, 0, nblk);   // returns synchronised
+      c->power_applied = pa;
+      c->zeldovich_done = zd;
+      return v;
+    }
     MLF<T> f(c);
     for (size_t l = 0; l < f.nl(); ++l) {
       if (!noise[l]) throw std::runtime_error("variance gradient: null device pointer");
