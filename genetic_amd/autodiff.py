@@ -66,6 +66,27 @@ def displacement(gen, *noise):
     return [tuple(psi[3 * l:3 * l + 3]) for l in range(len(noise))]
 
 
+class MaskedSquares(torch.autograd.Function):
+    """sum over the cells of a bool mask of |psi(w)|^2 on one level, a float64
+    scalar.  Only the displacements of the mask's box are formed."""
+
+    @staticmethod
+    def forward(ctx, gen, noise, mask):
+        noise, mask = noise.contiguous(), mask.contiguous()
+        _check_levels(gen, (noise,), "displacement")
+        grad = torch.empty_like(noise) if ctx.needs_input_grad[1] else None
+        torch.cuda.current_stream().synchronize()
+        v = gen.masked_displacement(noise.data_ptr(), mask.data_ptr(), None if grad is None else grad.data_ptr())
+        if grad is not None:
+            ctx.save_for_backward(grad)
+        return torch.tensor(v, dtype=torch.float64, device=noise.device)
+
+    @staticmethod
+    def backward(ctx, grad_v):
+        grad, = ctx.saved_tensors
+        return None, grad * grad_v.to(grad.dtype), None
+
+
 class FilteredVariance(torch.autograd.Function):
     """V(w): the filtered variance of the flagged cells (calculate variance at
     the context's filtering_scale) as a float64 scalar; d V / d w = 2 Q w."""
@@ -74,10 +95,11 @@ class FilteredVariance(torch.autograd.Function):
     def forward(ctx, gen, *noise):
         noise = [t.contiguous() for t in noise]
         _check_levels(gen, noise, "variance")
-        grads = [torch.empty_like(t) for t in noise]
+        grads = [torch.empty_like(t) for t in noise] if any(ctx.needs_input_grad[1:]) else None
         torch.cuda.current_stream().synchronize()
-        v = gen.variance_gradient([t.data_ptr() for t in noise], [g.data_ptr() for g in grads])
-        ctx.save_for_backward(*grads)
+        v = gen.variance_gradient([t.data_ptr() for t in noise], grads and [g.data_ptr() for g in grads])
+        if grads:
+            ctx.save_for_backward(*grads)
         return torch.tensor(v, dtype=torch.float64, device=noise[0].device)
 
     @staticmethod
@@ -93,8 +115,11 @@ def filtered_variance(gen, *noise):
 def sphere_loss(gen, noise, mask, v_target):
     """The differentiation workload's scalar loss on one level:
     sum over the masked cells of |psi|^2 plus (V - v_target)^2, in float64."""
-    (px, py, pz), = displacement(gen, noise)
-    m = mask.to(px.dtype)
-    l1 = ((px * m) ** 2 + (py * m) ** 2 + (pz * m) ** 2).double().sum()
+    if mask.dtype == torch.bool and mask.shape == noise.shape and mask.device == noise.device and len(gen.sizes) == 1:
+        l1 = MaskedSquares.apply(gen, noise, mask)
+    else:   # weights, or a mask to be broadcast
+        (px, py, pz), = displacement(gen, noise)
+        m = mask.to(px.dtype)
+        l1 = ((px * m) ** 2 + (py * m) ** 2 + (pz * m) ** 2).double().sum()
     v = filtered_variance(gen, noise)
     return l1 + (v - v_target) ** 2

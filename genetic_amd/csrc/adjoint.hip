@@ -33,6 +33,62 @@ template <typename T> __global__ void k_add_dense(T *__restrict__ g, const T *__
   g[row * (n + 2) + z] += src[i];
 }
 
+// per axis, the indices with a cell of the mask; words of W cells (4 where
+// rows are aligned to them: 16.8 MB of 256^3 cells in 8.5 us, by single bytes 20)
+template <typename W> __global__ void k_mask_axes(const W *__restrict__ mask, int n, uint8_t *__restrict__ used) {
+  // one row of cells (fixed x, y) a wavefront
+  const int row = int(blockIdx.x) * (blockDim.x / 64) + int(threadIdx.x) / 64, lane = int(threadIdx.x) % 64;
+  if (row >= n * n) return;
+  const int nw = n / int(sizeof(W));
+  const W *m = mask + size_t(row) * nw;
+  bool any = false;
+  for (int w = lane; w < nw; w += 64) {
+    const W v = m[w];
+    if (v == 0) continue;
+    any = true;
+    for (int b = 0; b < int(sizeof(W)); ++b)
+      if ((v >> (8 * b)) & 0xff) used[2 * n + w * int(sizeof(W)) + b] = 1;
+  }
+  if (any) {
+    used[row / n] = 1;
+    used[n + row % n] = 1;
+  }
+}
+
+// v (nc components of a box of cells) times the mask's cells there, and the
+// sums of squares of each block
+constexpr int MASK_BLOCKS = 512;
+template <typename T>
+__global__ __launch_bounds__(256) void k_mask_square(T *__restrict__ v, const uint8_t *__restrict__ mask, int n, int x0,
+                                                     int y0, int z0, int wx, int wy, int wz,
+                                                     double *__restrict__ part) {
+  const unsigned nb = unsigned(wx) * wy * wz;
+  double acc = 0;
+  for (unsigned i = blockIdx.x * 256u + threadIdx.x; i < nb; i += gridDim.x * 256u) {
+    const unsigned r = i / unsigned(wz);
+    int z = int(i - r * wz) + z0, x = int(r / unsigned(wy)), y = int(r - unsigned(x) * wy) + y0;
+    x += x0;
+    x -= x >= n ? n : 0;
+    y -= y >= n ? n : 0;
+    z -= z >= n ? n : 0;
+    const T m = mask[(size_t(x) * n + y) * n + z] ? T(1) : T(0);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const T q = v[size_t(c) * nb + i] * m;
+      v[size_t(c) * nb + i] = q;
+      acc += double(q) * double(q);
+    }
+  }
+  __shared__ double red[256];
+  red[threadIdx.x] = acc;
+  __syncthreads();
+  for (int s = 128; s > 0; s >>= 1) {
+    if (int(threadIdx.x) < s) red[threadIdx.x] += red[threadIdx.x + s];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) part[blockIdx.x] = red[0];
+}
+
 long table_entries(const LevelGeom &g) {
   long h = g.n / 2;
   return 3 * h * h + 1;
@@ -54,6 +110,19 @@ void check_ready(gic_context *c) {
   if (!c->have_camb) throw std::runtime_error("No power spectrum has been set (use the camb command)");
 }
 
+// L.noise <- the dense white noise transformed along z and y
+template <typename T> void load_noise_zy(gic_context *c, Level &L, const T *noise) {
+  alloc_field(c, L.noise, L.g);
+  build_sqrtp<T>(c, L);
+  FftZFwd<T> z;
+  z.add(noise, (T *)L.noise.p, true);
+  fft_z_forward<T>(z, L.g.n, c->st, c->hook());
+  FftYFwd<T> y;
+  y.add((const T *)L.noise.p, nullptr, (T *)L.noise.p);
+  fft_y_forward<T>(y, L.g.n, c->st, c->hook());
+  L.have_psi = L.have_psi2 = false;
+}
+
 }  // namespace
 
 template <typename T> void do_displacement_forward(gic_context *c, const T *const *noise, T *const *psi) {
@@ -65,18 +134,7 @@ template <typename T> void do_displacement_forward(gic_context *c, const T *cons
   // the noise along z and y, read straight from the caller's dense arrays;
   // the x pass of do_zeldovich makes delta_l = sqrtP r2c(w_l) and what the
   // displacements need of it
-  for (size_t l = 0; l < nl; ++l) {
-    Level &L = *c->levels[l];
-    alloc_field(c, L.noise, L.g);
-    build_sqrtp<T>(c, L);
-    FftZFwd<T> z;
-    z.add(noise[l], (T *)L.noise.p, true);
-    fft_z_forward<T>(z, L.g.n, c->st, c->hook());
-    FftYFwd<T> y;
-    y.add((const T *)L.noise.p, nullptr, (T *)L.noise.p);
-    fft_y_forward<T>(y, L.g.n, c->st, c->hook());
-    L.have_psi = L.have_psi2 = false;
-  }
+  for (size_t l = 0; l < nl; ++l) load_noise_zy<T>(c, *c->levels[l], noise[l]);
   c->seeded = c->drawn = c->power_applied = true;
   int order = c->lpt_order;
   c->lpt_order = 1;
@@ -172,8 +230,18 @@ template <typename T> void do_displacement_adjoint(gic_context *c, const T *cons
       y.add(u[1], u[2], u[1]);
     }
     fft_y_forward<T>(y, n, c->st, c->hook());
-    fft_x_adjoint<T>(h[0], h[1], (const T *)L.adj_tab.p, low ? u[0] : nullptr, low ? u[1] : nullptr,
-                     low ? (const T *)L.adj_lp.p : nullptr, n, L.g.kmin(), c->st, c->hook());
+    FftXAdj<T> x;
+    x.out = h[0];
+    x.h1 = h[0];
+    x.h0 = h[1];
+    x.tab = (const T *)L.adj_tab.p;
+    if (low) {
+      x.g1 = u[0];
+      x.g0 = u[1];
+      x.gtab = (const T *)L.adj_lp.p;
+    }
+    x.kmin = L.g.kmin();
+    fft_x_adjoint<T>(x, n, c->st, c->hook());
     FftY<T> yb;
     yb.add(h[0], h[0], FFT_YZ_ONE);
     fft_y<T>(yb, n, c->st, c->hook());
@@ -184,6 +252,114 @@ template <typename T> void do_displacement_adjoint(gic_context *c, const T *cons
   GIC_HIP(hipStreamSynchronize(c->st));
 }
 
+// The sum of |psi|^2 over the cells of a mask, and its gradient 2 Psi^T m Psi w:
+// displacements are needed at the mask's cells only, so the passes after the
+// forward ones are cut to the box around them (a box that spans the level
+// takes them whole).  256^3 FP32, a sphere of 31 cells, value and gradient:
+// 0.33 ms of kernels, against 0.75 for the full displacements and their
+// transpose and 0.75 for the products and sums of full fields between them.
+template <typename T>
+double do_masked_displacement(gic_context *c, const T *noise, const uint8_t *mask, T *grad) {
+  check_ready(c);
+  if (c->levels.size() != 1) throw std::runtime_error("masked displacement: one level expected");
+  if (!noise || !mask) throw std::runtime_error("masked displacement: null device pointer");
+  Level &L = *c->levels[0];
+  const int n = L.g.n;
+  const size_t nz = size_t(n / 2 + 1);
+  int w0[3], wl[3];
+  {
+    std::vector<uint8_t> used(3 * size_t(n));
+    c->stage.ensure(used.size());
+    fill<uint8_t>((uint8_t *)c->stage.p, used.size(), 0, c->st);
+    if (n % 4 == 0 && reinterpret_cast<uintptr_t>(mask) % 4 == 0)
+      hipLaunchKernelGGL(k_mask_axes<uint32_t>, dim3((n * n + 3) / 4), dim3(256), 0, c->st,
+                         reinterpret_cast<const uint32_t *>(mask), n, (uint8_t *)c->stage.p);
+    else
+      hipLaunchKernelGGL(k_mask_axes<uint8_t>, dim3((n * n + 3) / 4), dim3(256), 0, c->st, mask, n,
+                         (uint8_t *)c->stage.p);
+    GIC_HIP(hipGetLastError());
+    GIC_HIP(hipMemcpyAsync(used.data(), c->stage.p, used.size(), hipMemcpyDeviceToHost, c->st));
+    GIC_HIP(hipStreamSynchronize(c->st));
+    for (int d = 0; d < 3; ++d) {
+      cyclic_hull(used.data() + size_t(d) * n, n, w0[d], wl[d]);
+      if (wl[d] == 0) wl[d] = 1;   // an empty mask: one cell, of weight 0
+    }
+  }
+  load_noise_zy<T>(c, L, noise);
+  c->seeded = c->drawn = c->power_applied = true;
+  c->zeldovich_done = false;
+  // planes: f m and i k_x f m of the box's x; rows: of its x and y; the box
+  const size_t planes = size_t(wl[0]) * n * nz * 2, rows = size_t(wl[0]) * wl[1] * nz * 2;
+  const size_t nb = size_t(wl[0]) * wl[1] * wl[2];
+  c->stage.ensure(MASK_BLOCKS * sizeof(double) + (2 * planes + 3 * rows + 3 * nb) * sizeof(T));
+  double *part = (double *)c->stage.p;
+  T *A = (T *)(part + MASK_BLOCKS), *B = A + 2 * planes, *O = B + 3 * rows;
+  FftX<T> x;
+  x.in = x.spec = (T *)L.noise.p;
+  x.forward = true;
+  x.post = (const T *)L.sqrtp.p;
+  x.out[1] = A;
+  x.out[2] = A + planes;
+  x.inv_k2 = 1.0;
+  x.kmin = L.g.kmin();
+  x.win0 = w0[0];
+  x.wlen = wl[0];
+  fft_x<T>(x, n, c->st, c->hook());
+  L.noise_fourier = true;
+  L.dc_pending = false;
+  L.psi_fourier = false;
+  FftY<T> y;
+  y.kmin = L.g.kmin();
+  y.nouter = wl[0];
+  y.win0 = w0[1];
+  y.wlen = wl[1];
+  y.add(A + planes, B, FFT_YZ_ONE);
+  y.add(A, B + rows, FFT_YZ_IKY, B + 2 * rows, FFT_YZ_IKZ);
+  fft_y<T>(y, n, c->st, c->hook());
+  fft_z_window<T>(B, O, 3 * long(wl[0]) * wl[1], w0[2], wl[2], n, c->st, c->hook());
+  hipLaunchKernelGGL(k_mask_square<T>, dim3(MASK_BLOCKS), dim3(256), 0, c->st, O, mask, n, w0[0], w0[1], w0[2], wl[0],
+                     wl[1], wl[2], part);
+  GIC_HIP(hipGetLastError());
+  if (grad) {
+    adjoint_table<T>(c, L, 2, 0.0, L.adj_tab);
+    fft_r2c_z_window<T>(O, B, 3 * long(wl[0]) * wl[1], w0[2], wl[2], n, c->st, c->hook());
+    FftYFwd<T> yf;
+    yf.kmin = L.g.kmin();
+    yf.nouter = wl[0];
+    yf.iwin0 = w0[1];
+    yf.iwlen = wl[1];
+    yf.add(B, nullptr, A + planes);
+    yf.add(B + rows, B + 2 * rows, A);
+    fft_y_forward<T>(yf, n, c->st, c->hook());
+    c->xhalf.ensure(L.g.padded_reals() * sizeof(T));
+    T *h = (T *)c->xhalf.p;
+    FftXAdj<T> xa;
+    xa.out = h;
+    xa.h1 = A + planes;
+    xa.h0 = A;
+    xa.tab = (const T *)L.adj_tab.p;
+    xa.kmin = L.g.kmin();
+    xa.iwin0 = w0[0];
+    xa.iwlen = wl[0];
+    fft_x_adjoint<T>(xa, n, c->st, c->hook());
+    FftY<T> yb;
+    yb.add(h, h, FFT_YZ_ONE);
+    fft_y<T>(yb, n, c->st, c->hook());
+    FftZ<T> zb;
+    zb.scale = 2;
+    zb.add(h, nullptr, grad, FFT_YZ_ONE);
+    fft_z<T>(zb, n, c->st, c->hook());
+  }
+  std::vector<double> sums(MASK_BLOCKS);
+  GIC_HIP(hipMemcpyAsync(sums.data(), part, MASK_BLOCKS * sizeof(double), hipMemcpyDeviceToHost, c->st));
+  GIC_HIP(hipStreamSynchronize(c->st));
+  double v = 0;
+  for (double s : sums) v += s;
+  return v;
+}
+
+template double do_masked_displacement<float>(gic_context *, const float *, const uint8_t *, float *);
+template double do_masked_displacement<double>(gic_context *, const double *, const uint8_t *, double *);
 template void do_displacement_forward<float>(gic_context *, const float *const *, float *const *);
 template void do_displacement_forward<double>(gic_context *, const double *const *, double *const *);
 template void do_displacement_adjoint<float>(gic_context *, const float *const *, float *const *);

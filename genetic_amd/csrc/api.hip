@@ -1164,6 +1164,14 @@ int gic_displacement_adjoint(gic_context *c, const void *const *psi_bar, void *c
   });
 }
 
+int gic_masked_displacement(gic_context *c, const void *noise, const uint8_t *mask, double *value, void *grad) {
+  return guarded(c, [&] {
+    if (!value) throw std::runtime_error("masked displacement: null pointer");
+    if (c->prec == 32) *value = do_masked_displacement<float>(c, (const float *)noise, mask, (float *)grad);
+    else *value = do_masked_displacement<double>(c, (const double *)noise, mask, (double *)grad);
+  });
+}
+
 int gic_variance_gradient(gic_context *c, const void *const *noise, double *value, void *const *grad) {
   return guarded(c, [&] {
     if (!noise || !value) throw std::runtime_error("variance gradient: null pointer");

@@ -321,11 +321,26 @@ template <typename T> void do_draw(gic_context *c);
 template <typename T> void ensure_noise_fourier(gic_context *c, Level &L);
 // dense (optional): 3 arrays per level that also receive the base level's
 // displacements; the levels' fields then hold noise transformed along z and y
+// The shortest cyclic run [b0, b0 + bl) mod n that holds every index with
+// used[] set (all but the longest gap); bl = 0 if there is none.
+inline void cyclic_hull(const uint8_t *used, int n, int &b0, int &bl) {
+  int best = 0, end = 0, run = 0;
+  for (int i = 0; i < 2 * n; ++i) {
+    run = used[i % n] ? 0 : std::min(run + 1, n);
+    if (run > best) {
+      best = run;
+      end = i + 1;
+    }
+  }
+  b0 = end % n;
+  bl = n - best;
+}
 template <typename T> void do_zeldovich(gic_context *c, T *const *dense);
 
 // ---- displacement map and its transpose (adjoint.hip) ----------------------------------
 // noise[l]: dense n_l^3 white noise; psi[3l+a]: dense displacement components
 template <typename T> void do_displacement_forward(gic_context *c, const T *const *noise, T *const *psi);
+template <typename T> double do_masked_displacement(gic_context *c, const T *noise, const uint8_t *mask, T *grad);
 template <typename T> void do_displacement_adjoint(gic_context *c, const T *const *psi_bar, T *const *noise_bar);
 
 // ---- constrained realisations (modif.hip) ------------------------------------------

@@ -204,24 +204,35 @@ template <typename T> struct FftZFwd {
 };
 template <typename T> void fft_z_forward(const FftZFwd<T> &z, int n, hipStream_t st, TimingHook *hook);
 
-// forward y passes: out = Y in, or with a second input -i k_y Y in - i k_z Y in2
+// forward y passes: out = Y in, or with a second input -i k_y Y in - i k_z Y in2.
+// With iwlen > 0 each of the nouter input planes holds the iwlen rows from
+// iwin0 on and is 0 elsewhere.
 template <typename T> struct FftYFwd {
   struct Job {
     const T *in, *in2;
     T *out;
   } job[FFT_JOBS] = {};
-  int njob = 0, nb = 1;
+  int njob = 0, nb = 1, nouter = 0, iwin0 = 0, iwlen = 0;
   long bs = 0;
   double kmin = 0;
   void add(const T *in, const T *in2, T *out) { job[njob++] = Job{in, in2, out}; }
 };
 template <typename T> void fft_y_forward(const FftYFwd<T> &y, int n, hipStream_t st, TimingHook *hook);
 
-// h1 <- inverse x transform of tab[|k|^2] n^-1.5 (-i k_x X h1 + X h0), plus the
-// same of g1, g0 with gtab if given (X the forward x transform)
+// out <- inverse x transform of tab[|k|^2] n^-1.5 (-i k_x X h1 + X h0), plus the
+// same of g1, g0 with gtab if given (X the forward x transform).  With
+// iwlen > 0 the inputs are the iwlen planes from iwin0 on of fields that are 0
+// elsewhere; without, out may be h1.
+template <typename T> struct FftXAdj {
+  T *out = nullptr;
+  const T *h1 = nullptr, *h0 = nullptr, *tab = nullptr, *g1 = nullptr, *g0 = nullptr, *gtab = nullptr;
+  int iwin0 = 0, iwlen = 0;
+  double kmin = 0;
+};
+template <typename T> void fft_x_adjoint(const FftXAdj<T> &x, int n, hipStream_t st, TimingHook *hook);
+// r2c along z of nrows rows given as their points [z0, z0 + wz) mod n, 0 elsewhere
 template <typename T>
-void fft_x_adjoint(T *h1, const T *h0, const T *tab, const T *g1, const T *g0, const T *gtab, int n, double kmin,
-                   hipStream_t st, TimingHook *hook);
+void fft_r2c_z_window(const T *win, T *out, long nrows, int z0, int wz, int n, hipStream_t st, TimingHook *hook);
 
 // The z passes of the second-order source S = xx yy + (xx + yy) zz - xy^2 -
 // xz^2 - yz^2, and with psi of the displacements over px, py, pz, from the

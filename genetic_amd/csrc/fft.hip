@@ -131,10 +131,13 @@ template <typename T> void fft_y_forward(const FftYFwd<T> &y, int n, hipStream_t
   if (y.njob < 1 || y.njob > FFT_JOBS) throw std::runtime_error("fft_y_forward: bad jobs");
   api<T>(n).y_forward(y, st, hook);
 }
+template <typename T> void fft_x_adjoint(const FftXAdj<T> &x, int n, hipStream_t st, TimingHook *hook) {
+  api<T>(n).x_adjoint(x, st, hook);
+}
 template <typename T>
-void fft_x_adjoint(T *h1, const T *h0, const T *tab, const T *g1, const T *g0, const T *gtab, int n, double kmin,
-                   hipStream_t st, TimingHook *hook) {
-  api<T>(n).x_adjoint(h1, h0, tab, g1, g0, gtab, kmin, st, hook);
+void fft_r2c_z_window(const T *win, T *out, long nrows, int z0, int wz, int n, hipStream_t st, TimingHook *hook) {
+  if (nrows < 1 || wz < 1 || wz > n || z0 < 0 || z0 >= n) throw std::runtime_error("fft_r2c_z_window: bad window");
+  api<T>(n).r2c_z_window(win, out, nrows, z0, wz, st, hook);
 }
 template <typename T>
 void fft_z_lpt(T *px, T *py, T *pz, const T *xx, const T *yy, const T *xy, T *S, bool psi, int n, double kmin,
@@ -149,8 +152,8 @@ void fft_z_lpt(T *px, T *py, T *pz, const T *xx, const T *yy, const T *xy, T *S,
   template void fft_z_window<T>(const T *, T *, long, int, int, int, hipStream_t, TimingHook *);             \
   template void fft_z_forward<T>(const FftZFwd<T> &, int, hipStream_t, TimingHook *);                       \
   template void fft_y_forward<T>(const FftYFwd<T> &, int, hipStream_t, TimingHook *);                       \
-  template void fft_x_adjoint<T>(T *, const T *, const T *, const T *, const T *, const T *, int, double,    \
-                                 hipStream_t, TimingHook *);                                                 \
+  template void fft_x_adjoint<T>(const FftXAdj<T> &, int, hipStream_t, TimingHook *);                       \
+  template void fft_r2c_z_window<T>(const T *, T *, long, int, int, int, hipStream_t, TimingHook *);         \
   template void fft_z_lpt<T>(T *, T *, T *, const T *, const T *, const T *, T *, bool, int, double,         \
                              hipStream_t, TimingHook *);                                                     \
   template void fft_r2c_post<T>(T *, int, const T *, hipStream_t, TimingHook *, const T *);                 \

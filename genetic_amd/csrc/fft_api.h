@@ -27,13 +27,13 @@ template <typename T> struct FftApi {
   void (*r2c_window)(const T *win, const int *w0, const int *wl, T *bufB, T *bufA, T *spec, const T *post, bool accum,
                      hipStream_t st, TimingHook *hook, const T *aux, const FilterInline *fil, double kmin);
   void (*r2c_window_zy)(const T *win, const int *w0, const int *wl, T *bufB, T *bufA, hipStream_t st, TimingHook *hook);
+  void (*r2c_z_window)(const T *win, T *out, long nrows, int z0, int wz, hipStream_t st, TimingHook *hook);
   void (*z_window)(const T *in, T *out, long nrows, int z0, int wz, hipStream_t st, TimingHook *hook);
   // fused passes
   void (*x)(const FftX<T> &q, hipStream_t st, TimingHook *hook);
   void (*y)(const FftY<T> &q, hipStream_t st, TimingHook *hook);
   void (*y_forward)(const FftYFwd<T> &q, hipStream_t st, TimingHook *hook);
-  void (*x_adjoint)(T *h1, const T *h0, const T *tab, const T *g1, const T *g0, const T *gtab, double kmin,
-                    hipStream_t st, TimingHook *hook);
+  void (*x_adjoint)(const FftXAdj<T> &q, hipStream_t st, TimingHook *hook);
   void (*z)(const FftZ<T> &q, hipStream_t st, TimingHook *hook);
   void (*z_forward)(const FftZFwd<T> &q, hipStream_t st, TimingHook *hook);
   void (*z_lpt)(T *px, T *py, T *pz, const T *xx, const T *yy, const T *xy, T *S, bool psi, double kmin,

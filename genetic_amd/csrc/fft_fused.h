@@ -303,13 +303,14 @@ __global__ __launch_bounds__((LineFft<T, L, C, 1, true>::TH), 2) void k_fft_x_fu
 // along z and y, the inverse x transform of
 //   tab[|k|^2] norm ( -i k_x X h1 + X h0 ),   X the forward x transform,
 // (0 for the first term at +Nyquist), plus the same of a second pair with a
-// table of its own, if given.  Written over h1.
+// table of its own, if given; inputs of the points [iwin0, iwin0 + iwlen).
+// Without h1 the first term is left out.
 template <typename T> struct XAdjArgs {
-  cx<T> *h1;
-  const cx<T> *h0, *g1, *g0;
+  cx<T> *out;
+  const cx<T> *h1, *h0, *g1, *g0;
   const T *tab, *gtab;
   T norm, kmin;
-  int nkzb;
+  int nkzb, iwin0, iwlen;
 };
 template <typename T, int L, int C>
 __global__ __launch_bounds__((LineFft<T, L, C, 1, true>::TH), 2) void k_fft_x_adjoint(XAdjArgs<T> a,
@@ -332,7 +333,8 @@ __global__ __launch_bounds__((LineFft<T, L, C, 1, true>::TH), 2) void k_fft_x_ad
     const cx<T> *h = s == 0 ? a.h1 : s == 1 ? a.h0 : s == 2 ? a.g1 : a.g0;
     const T *tab = s < 2 ? a.tab : a.gtab;
     if (!h) continue;
-    Fw::template load<Fw::first>(v, h + base, LS, nc);
+    if (a.iwlen < L) Fw::template load_window<Fw::first>(v, h + base, LS, nc, a.iwin0, a.iwlen);
+    else Fw::template load<Fw::first>(v, h + base, LS, nc);
     __syncthreads();   // LDS is free, the twiddles are there
     Fw::run(v, lds, ltw);
     const int t = Bw::fresh(int(threadIdx.x)), i0 = t / C, kz = min(col0 + t % C, NZ - 1);
@@ -352,7 +354,7 @@ __global__ __launch_bounds__((LineFft<T, L, C, 1, true>::TH), 2) void k_fft_x_ad
   }
   __syncthreads();
   Bw::run(acc, lds, ltw);
-  Bw::template store<Bw::last>(acc, a.h1 + base, LS, nc, 0, L);
+  Bw::template store<Bw::last>(acc, a.out + base, LS, nc, 0, L);
 }
 
 // ---- y passes ---------------------------------------------------------------------
@@ -441,7 +443,7 @@ template <typename T> struct YFwdArgs {
     cx<T> *out;
   } job[FUSED_JOBS];
   long bs;
-  int nkzb;
+  int nkzb, iwin0, iwlen;
   T kmin;
 };
 template <typename T, int L, int C>
@@ -456,8 +458,13 @@ k_fft_y_forward(YFwdArgs<T> a, const cx<T> *__restrict__ tw) {
   const int tile = xcd_tile(blockIdx.x, gridDim.x), outer = tile / a.nkzb, col0 = (tile - outer * a.nkzb) * C;
   const int nc = min(C, NZ - col0);
   const long at = long(blockIdx.z) * a.bs + long(outer) * L * NZ + col0;
+  const long in = long(blockIdx.z) * a.bs + long(outer) * a.iwlen * NZ + col0;
   cx<T> v[E];
-  Fw::template load<Fw::first>(v, job.in + at, NZ, nc);
+  auto load = [&](const cx<T> *p) {
+    if (a.iwlen < L) Fw::template load_window<Fw::first>(v, p + in, NZ, nc, a.iwin0, a.iwlen);
+    else Fw::template load<Fw::first>(v, p + in, NZ, nc);
+  };
+  load(job.in);
   __syncthreads();
   Fw::run(v, lds, ltw);
   if (job.in2) {
@@ -468,7 +475,7 @@ k_fft_y_forward(YFwdArgs<T> a, const cx<T> *__restrict__ tw) {
       for (int e = 0; e < E; ++e)
         r[e] = rot_mul<T>(3, v[e], k_power<T>(1, signed_k(i0 + Fw::template at<R>(e), L), L / 2, a.kmin));
     }
-    Fw::template load<Fw::first>(v, job.in2 + at, NZ, nc);
+    load(job.in2);
     __syncthreads();
     Fw::run(v, lds, ltw);
     const T gz = k_power<T>(1, col0 + Fw::fresh(int(threadIdx.x)) % C, L / 2, a.kmin);
@@ -805,21 +812,24 @@ template <typename T, int N> struct FftFused {
       a.job[j].in = c(q.job[j].in);
       a.job[j].in2 = c(q.job[j].in2);
       a.job[j].out = c(q.job[j].out);
-      fields += q.job[j].in2 ? 3 : 2;
+      fields += 1 + (q.job[j].in2 ? 2 : 1) * double(q.iwlen > 0 ? q.iwlen : N) / N;
     }
+    const int nouter = q.nouter > 0 ? q.nouter : N;
+    a.iwin0 = q.iwlen > 0 ? q.iwin0 : 0;
+    a.iwlen = q.iwlen > 0 ? q.iwlen : N;
     a.bs = q.bs / 2;
     a.nkzb = (NZ + CY - 1) / CY;
     a.kmin = T(q.kmin);
     constexpr int TH = LineFft<T, N, CY, 1, false>::TH;
-    launch(k_fft_y_forward<T, N, CY>, dim3(N * a.nkzb, q.njob, q.nb), TH, tile_lds(CY), "fft_y_fwd_multi",
-           q.nb * FIELD * fields, st, hook, a);
+    launch(k_fft_y_forward<T, N, CY>, dim3(nouter * a.nkzb, q.njob, q.nb), TH, tile_lds(CY), "fft_y_fwd_multi",
+           q.nb * FIELD * fields * nouter / N, st, hook, a);
   }
-  static void x_adjoint(T *h1, const T *h0, const T *tab, const T *g1, const T *g0, const T *gtab, double kmin,
-                        hipStream_t st, TimingHook *hook) {
-    XAdjArgs<T> a{c(h1), c(h0), c(g1), c(g0), tab, gtab, F::norm(), T(kmin), (NZ + CX - 1) / CX};
+  static void x_adjoint(const FftXAdj<T> &q, hipStream_t st, TimingHook *hook) {
+    XAdjArgs<T> a{c(q.out), c(q.h1), c(q.h0), c(q.g1), c(q.g0), q.tab, q.gtab, F::norm(), T(q.kmin), (NZ + CX - 1) / CX,
+                  q.iwlen > 0 ? q.iwin0 : 0, q.iwlen > 0 ? q.iwlen : N};
     constexpr int TH = LineFft<T, N, CX, 1, true>::TH;
-    launch(k_fft_x_adjoint<T, N, CX>, dim3(N * a.nkzb), TH, tile_lds(CX), "fft_x_adjoint", FIELD * (g1 ? 5 : 3), st,
-           hook, a);
+    launch(k_fft_x_adjoint<T, N, CX>, dim3(N * a.nkzb), TH, tile_lds(CX), "fft_x_adjoint",
+           FIELD * (1 + (q.g1 ? 4 : 2) * double(a.iwlen) / N), st, hook, a);
   }
   static void z(const FftZ<T> &q, hipStream_t st, TimingHook *hook) {
     ZArgs<T> a{};
@@ -873,6 +883,7 @@ template <typename T, int N> FftApi<T> fft_api_of() {
   a.c2r_window = F::c2r_window;
   a.r2c_window = F::r2c_window;
   a.r2c_window_zy = F::r2c_window_zy;
+  a.r2c_z_window = F::r2c_z_window;
   a.z_window = F::z_window;
   a.x = G::x;
   a.y = G::y;

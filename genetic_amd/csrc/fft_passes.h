@@ -1321,10 +1321,8 @@ template <typename T, int N> struct FftN {
     GIC_HIP(hipGetLastError());
     if (hook) hook->end(tag.c_str(), st);
   }
-  // the z and y passes of r2c_window: bufA <- wl[0] planes
-  static void r2c_window_zy(const T *win, const int *w0, const int *wl, T *bufB, T *bufA, hipStream_t st,
-                            TimingHook *hook) {
-    long nrows = long(wl[0]) * wl[1];
+  // r2c of nrows rows given as their points [z0, z0 + wz) (mod N)
+  static void r2c_z_window(const T *win, T *out, long nrows, int z0, int wz, hipStream_t st, TimingHook *hook) {
     int nblk = int((nrows + ROWS - 1) / ROWS);
     size_t shm = sizeof(cx<T>) * (ROWS * ZRow<M>::len + M);   // rows, then the M-point twiddles
     const cx<T> *tw = twtable<T>().get(N);
@@ -1333,11 +1331,16 @@ template <typename T, int N> struct FftN {
     std::string tag = "fft_z_r2c_win." + std::to_string(N);
     if (hook) {
       hook->begin(tag.c_str(), st);
-      hook->bytes(tag.c_str(), double(nrows) * ((N + 2) + wl[2]) * sizeof(T));
+      hook->bytes(tag.c_str(), double(nrows) * ((N + 2) + wz) * sizeof(T));
     }
-    hipLaunchKernelGGL(kern, dim3(nblk), dim3(THREADS), shm, st, win, bufB, nrows, w0[2], wl[2], T(1), tw);
+    hipLaunchKernelGGL(kern, dim3(nblk), dim3(THREADS), shm, st, win, out, nrows, z0, wz, T(1), tw);
     GIC_HIP(hipGetLastError());
     if (hook) hook->end(tag.c_str(), st);
+  }
+  // the z and y passes of r2c_window: bufA <- wl[0] planes
+  static void r2c_window_zy(const T *win, const int *w0, const int *wl, T *bufB, T *bufA, hipStream_t st,
+                            TimingHook *hook) {
+    r2c_z_window(win, bufB, long(wl[0]) * wl[1], w0[2], wl[2], st, hook);
     // y pass: tiles (x_local, kz block), lines over ky from the wl[1] window rows
     StridedArgs<T> ay{};
     ay.in = reinterpret_cast<const cx<T> *>(bufB);

@@ -1640,20 +1640,7 @@ template <typename T> struct VarianceBox {
       const uint64_t r = pow2 ? i >> sh : i / n, x = pow2 ? r >> sh : r / n;
       mx[x] = my[r - x * n] = mz[i - r * n] = 1;
     }
-    for (int d = 0; d < 3; ++d) {
-      // all but the longest cyclic run of indices without a flagged cell
-      const uint8_t *u = member.data() + d * n;
-      int best = 0, end = 0, run = 0;
-      for (int i = 0; i < 2 * int(n); ++i) {
-        run = u[i % int(n)] ? 0 : run + 1;
-        if (run > best && run < int(n)) {
-          best = run;
-          end = i + 1;
-        }
-      }
-      B.b0[d] = end % int(n);
-      B.bl[d] = int(n) - best;
-    }
+    for (int d = 0; d < 3; ++d) cyclic_hull(member.data() + d * n, g.n, B.b0[d], B.bl[d]);
     if (B.bl[0] > int(n) / 2) return false;
     nb = box_cells(B);
     upload_list(c, idx, cells);

@@ -58,6 +58,7 @@ SIGNATURES = {
     "gic_chi2": ([_v, _P(_d), _P(ctypes.c_uint64)], _i),
     "gic_displacement_forward": ([_v, _v, _v], _i),
     "gic_displacement_adjoint": ([_v, _v, _v], _i),
+    "gic_masked_displacement": ([_v, _v, _v, _P(_d), _v], _i),
     "gic_variance_gradient": ([_v, _v, _P(_d), _v], _i),
     "gic_batch_constrained": ([_v, _i, _v, _i, _v, _v, _i, _i, _P(_d)], _i),
     "gic_splice": ([_v, ctypes.c_ulong, _P(_i)], _i),
@@ -330,6 +331,13 @@ class ICGenerator:
     def displacement_adjoint(self, psi_bar_ptrs, noise_bar_ptrs):
         """noise_bar[l] <- (d psi / d w_l)^T psi_bar."""
         self._check(lib().gic_displacement_adjoint(self._h, self._ptrs(psi_bar_ptrs), self._ptrs(noise_bar_ptrs)))
+
+    def masked_displacement(self, noise_ptr, mask_ptr, grad_ptr=None):
+        """Sum of |psi|^2 over the cells of a byte mask for white noise of a
+        one-level context; with grad_ptr its gradient is written there."""
+        v = ctypes.c_double()
+        self._check(lib().gic_masked_displacement(self._h, noise_ptr, mask_ptr, ctypes.byref(v), grad_ptr))
+        return v.value
 
     def variance_gradient(self, noise_ptrs, grad_ptrs=None):
         """Filtered variance of the flagged region for the given white noise;

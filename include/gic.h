@@ -166,6 +166,11 @@ int gic_displacement_forward(gic_context *ctx, const void *const *noise, void *c
  * (d psi / d w_l)^T psi_bar, the gradient of a loss of psi with respect to the
  * white noise.  Independent of the context's fields. */
 int gic_displacement_adjoint(gic_context *ctx, const void *const *psi_bar, void *const *noise_bar);
+/* Sum of |psi|^2 over the cells of mask (n^3 bytes, 0 or not) for the white
+ * noise of a one-level context, and if grad is non-null its gradient with
+ * respect to the noise.  Replaces the context's overdensity as the forward
+ * map does; no displacement field is kept. */
+int gic_masked_displacement(gic_context *ctx, const void *noise, const uint8_t *mask, double *value, void *grad);
 /* Filtered variance V(w) of the flagged region for the white noise noise[l]
  * (calculate variance: QuadraticModification::calculateCurrentValue,
  * quadraticmodification.hpp:50-62, at the current filtering_scale) and, if
