@@ -95,14 +95,18 @@ long table_entries(const LevelGeom &g) {
 }
 
 // out[|k|^2] = sqrtP(k) filter(k) / k^2 with the filter of kind (0 low, 1
-// high, 2 unity) at kc, on level L
-template <typename T> void adjoint_table(gic_context *c, Level &L, int kind, double kc, DevBuf &out) {
+// high, 2 unity) at kc, on level L; kept while the spectrum's settings are
+template <typename T> void adjoint_table(gic_context *c, Level &L, int kind, double kc, DevBuf &out, TabKey &key) {
+  const TabKey want{c->spectrum, kind, L.g.n, kc, L.g.box};
+  if (key == want) return;
+  key = TabKey{};
   long nent = table_entries(L.g);
   out.ensure(nent * sizeof(T));
   filter_table<T>(kind, kc, L.g.kmin(), nent, (T *)out.p, c->st, true);
   hipLaunchKernelGGL(k_tab_mul<T>, dim3((nent + 255) / 256), dim3(256), 0, c->st, (T *)out.p, (const T *)L.sqrtp.p,
                      nent);
   GIC_HIP(hipGetLastError());
+  key = want;
 }
 
 void check_ready(gic_context *c) {
@@ -172,10 +176,11 @@ template <typename T> void do_displacement_adjoint(gic_context *c, const T *cons
   // pass towards the next finer level (for level 0 with sqrtP / k^2 folded in)
   for (size_t l = 0; l < nl; ++l) {
     Level &L = *c->levels[l];
-    adjoint_table<T>(c, L, l >= 1 ? 1 : 2, l >= 1 ? kcut_for_level(c, int(l) - 1) : 0.0, L.adj_tab);
+    adjoint_table<T>(c, L, l >= 1 ? 1 : 2, l >= 1 ? kcut_for_level(c, int(l) - 1) : 0.0, L.adj_tab,
+                     L.adj_tab_key);
     if (l + 1 < nl) {
       if (l == 0) {
-        adjoint_table<T>(c, L, 0, kcut_for_level(c, 0), L.adj_lp);
+        adjoint_table<T>(c, L, 0, kcut_for_level(c, 0), L.adj_lp, L.adj_lp_key);
       } else {
         L.adj_lp.ensure(table_entries(L.g) * sizeof(T));
         filter_table<T>(0, kcut_for_level(c, int(l)), L.g.kmin(), table_entries(L.g), (T *)L.adj_lp.p, c->st);
@@ -321,7 +326,7 @@ double do_masked_displacement(gic_context *c, const T *noise, const uint8_t *mas
                      wl[1], wl[2], part);
   GIC_HIP(hipGetLastError());
   if (grad) {
-    adjoint_table<T>(c, L, 2, 0.0, L.adj_tab);
+    adjoint_table<T>(c, L, 2, 0.0, L.adj_tab, L.adj_tab_key);
     fft_r2c_z_window<T>(O, B, 3 * long(wl[0]) * wl[1], w0[2], wl[2], n, c->st, c->hook());
     FftYFwd<T> yf;
     yf.kmin = L.g.kmin();

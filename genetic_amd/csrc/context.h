@@ -199,6 +199,17 @@ struct DevBuf {
   ~DevBuf() { release(); }
 };
 
+// What a level's |k|^2 table was built for: the spectrum's settings (the
+// context's count of them), the filter and the level's geometry.
+struct TabKey {
+  uint64_t spectrum = 0;   // 0: not built
+  int kind = -1, n = 0;
+  double kc = 0, box = 0;
+  bool operator==(const TabKey &o) const {
+    return spectrum == o.spectrum && kind == o.kind && n == o.n && kc == o.kc && box == o.box;
+  }
+};
+
 struct Level {
   LevelGeom g;
   DevBuf noise;            // white noise, then the overdensity
@@ -213,6 +224,7 @@ struct Level {
   bool have_psi2 = false;
   DevBuf adj_u[3];         // adjoint: gradient arriving from the finer level, per component
   DevBuf adj_tab, adj_lp;  // adjoint: |k|^2 tables of the level's operators
+  TabKey sqrtp_key, sqrtp_dm_key, adj_tab_key, adj_lp_key;
 };
 
 }  // namespace gic
@@ -239,6 +251,7 @@ struct gic_context {
   Cosmo cosmo;
   // frozen at the camb command
   bool have_camb = false;
+  uint64_t spectrum = 1;   // counts the settings of the power spectrum
   LogSpline tf_all, tf_dm;
   std::vector<double> kpts;
   double amplitude = 0, ns_frozen = 0;
