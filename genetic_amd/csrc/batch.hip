@@ -423,8 +423,7 @@ void do_batch(gic_context *c, int nreal, const uint64_t *seeds, int ncons, const
   int group = std::max(nlanes, std::min(GROUP_MAX, int(GROUP_BYTES / (double(ncons) * fs_reals * sizeof(T)))));
   group = std::min(group, nreal);
   if (boxes) group = std::min(group, int(2e9 / ((double(ncons) * wl * wl + 1024.0) * n)));
-  const int rows_mult = fft_box_rows_multiple<T>(n);
-  auto nrows_of = [&](int k) { return boxes ? (long(k) * ncons * wl * wl + rows_mult - 1) / rows_mult * rows_mult : 0; };
+  auto nrows_of = [&](int k) { return boxes ? long(k) * ncons * wl * wl : 0; };
   // the boxes' x origins of every constraint, then the y origins
   std::vector<int> win(boxes ? size_t(nreal) * ncons * 2 : 0);
   if (boxes) {

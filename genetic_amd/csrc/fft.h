@@ -23,7 +23,7 @@ struct TimingHook {
 template <typename T> void fft3d(T *d, int n, int dir, hipStream_t st, TimingHook *hook);
 
 // k-space operators applied inside the x pass
-enum { FFT_PRE_NONE = 0, FFT_PRE_TABLE = 1, FFT_PRE_ZA = 2, FFT_PRE_KK = 3 };
+enum { FFT_PRE_NONE = 0, FFT_PRE_TABLE = 1 };
 
 // A product of Fermi level filters, formed inside a transform's pass instead
 // of read from a |k|^2 table (used by FP32 transforms, whose table reads are
@@ -46,8 +46,6 @@ struct FilterInline {
 // fastest, no padding) and the spectrum lands in d.
 template <typename T>
 void fft_r2c_post(T *d, int n, const T *post, hipStream_t st, TimingHook *hook, const T *src = nullptr);
-// In-place c2r of d; with dst non-null the real result goes to the dense n^3
-// array dst instead (d is then scratch).
 // r2c of nb padded n^3 fields stored back to back, each mode times post[|k|^2] if post is given
 template <typename T> void fft_r2c_batch(T *d, int n, int nb, const T *post, hipStream_t st, TimingHook *hook);
 // builds the twiddle table of size n (a synchronous upload), so that later
@@ -56,50 +54,23 @@ template <typename T> void fft_prepare(int n);
 // r2c of nb fields that vanish outside boxes of wl x wl cells in (x, y), all
 // z: box b starts at (winx[b], winy[b]) mod n (device int arrays).  rows
 // holds the boxes' rows as dense rows of n reals, row (b wl + i) wl + j for
-// x = winx[b]+i, y = winy[b]+j; nrows is a multiple of
-// fft_box_rows_multiple(n) and rows past nb wl^2 are transformed but unused.
+// x = winx[b]+i, y = winy[b]+j; nrows >= nb wl^2, rows past those are
+// transformed but unused.
 // zbuf (nrows (n/2+1) complex) and ybuf (nb wl n (n/2+1) complex) are
 // scratch; field b's spectrum times post[|k|^2] goes to spec + b spec_stride.
 template <typename T>
 void fft_r2c_boxes(const T *rows, int n, long nrows, int nb, int wl, const int *winx, const int *winy, T *zbuf, T *ybuf,
                    T *spec, long spec_stride, const T *post, hipStream_t st, TimingHook *hook);
-template <typename T> int fft_box_rows_multiple(int n);
-template <typename T> void fft_c2r_to(T *d, T *dst, int n, hipStream_t st, TimingHook *hook);
-// Transpose of one Zel'dovich component (FFT_PRE_ZA followed by c2r): the r2c
-// of src (dense n^3, or d in place when null; d is overwritten) whose last
-// pass forms conj(i k_c tab[|k|^2]) times each mode, zero at k_c = +Nyquist,
-// and adds it to the spectrum acc (stores it when !accumulate).
-template <typename T>
-void fft_r2c_za_adjoint(const T *src, T *d, T *acc, int n, const T *tab, int comp, double kmin, bool accumulate,
-                        hipStream_t st, TimingHook *hook);
 // out <- c2r(op(spec)), out-of-place from a spectrum that is left untouched.
-// op: FFT_PRE_TABLE multiplies by tab[|k|^2]; FFT_PRE_ZA forms the Zel'dovich
-// component comp, i k_c tab[|k|^2], with tab = filter(k)/k^2 (0 at k=0) and
-// zero at k_c = +Nyquist.  FFT_PRE_KK forms k_a k_b tab[|k|^2] for comp = a + 3 b
-// (zero at a +Nyquist component when a != b).
+// op: FFT_PRE_TABLE multiplies by tab[|k|^2].
 // With dst non-null the real result goes to the dense n^3 array dst and out is scratch.
 // With tab null and inv_k2 non-zero the operator's factor is inv_k2 / (|k|^2 kmin^2)
 // (0 at k = 0), formed in FP64 as filter_table forms it for a unit filter.
 // fil (optional) replaces tab for FP32 transforms.
 template <typename T>
-void fft_c2r_from(const T *spec, T *out, int n, int pre, const T *tab, int comp, double kmin, hipStream_t st,
+void fft_c2r_from(const T *spec, T *out, int n, int pre, const T *tab, double kmin, hipStream_t st,
                   TimingHook *hook, T *dst = nullptr, double inv_k2 = 0, const FilterInline *fil = nullptr);
-// The same transforms split after their first pass, so that one x pass serves
-// several outputs (c2r is linear and a factor of k_y, k_z commutes with the
-// transform along x):
-//   half <- the x pass of c2r(op(spec)) alone (op, comp, tab, inv_k2 as for
-//           fft_c2r_from; half is a padded field holding complex x-k_y-k_z data);
-//   out  <- the y and z passes of c2r from half, the y pass multiplying each
-//           mode by m(k_y, k_z) as it reads it (FFT_YZ_*; dst as for
-//           fft_c2r_from);
-//   fft_c2r_yz_lpt: the same, its last pass folding the result into the 2LPT
-//           source instead of storing it (out is scratch): epi 1: S = A phi,
-//           A += phi;  2: S += A phi;  3: S -= phi^2 (S, A padded fields).
-// With X0 = x pass of tab spec, X1 = x pass of i k_x tab spec (FFT_PRE_ZA comp 0)
-// and X2 = x pass of k_x^2 tab spec (FFT_PRE_KK comp 0): the Zel'dovich
-// components are yz(X1, ONE), yz(X0, IKY), yz(X0, IKZ) and the second
-// derivatives yz(X2, ONE), yz(X1, MIKY), yz(X1, MIKZ), yz(X0, KYKY),
-// yz(X0, KYKZ), yz(X0, KZKZ), with the +Nyquist rules of FFT_PRE_ZA/KK.
+// Factors of (k_y, k_z) that the fused y and z passes multiply a field by
 enum {
   FFT_YZ_ONE = 0,    // 1
   FFT_YZ_IKY = 1,    // i k_y (0 at k_y = +Nyquist)
@@ -113,15 +84,6 @@ enum {
   FFT_YZ_KZ = 9,     // k_z (0 at k_z = +Nyquist)
   FFT_YZ_KY = 10     // k_y (0 at k_y = +Nyquist)
 };
-template <typename T>
-void fft_c2r_xpass(const T *spec, T *half, int n, int pre, const T *tab, int comp, double kmin, hipStream_t st,
-                   TimingHook *hook, double inv_k2 = 0);
-template <typename T>
-void fft_c2r_yz(const T *half, T *out, int n, int yop, double kmin, hipStream_t st, TimingHook *hook,
-                T *dst = nullptr);
-template <typename T>
-void fft_c2r_yz_lpt(const T *half, T *scratch, int n, int yop, double kmin, int epi, T *S, T *A, hipStream_t st,
-                    TimingHook *hook);
 // ---- fused passes (fft_fused.h) ----------------------------------------------------
 // Fields are padded (n * n * (n + 2) values of T); nb of them form a batch,
 // *_bs values apart.
@@ -261,13 +223,9 @@ void fft_r2c_window_zy(const T *win, int n, const int *w0, const int *wl, T *buf
                        TimingHook *hook);
 // Only the real-space window [w0, w0+wl) (per axis, wrapping mod n) of
 // c2r(op(spec)), via pruned passes: bufA holds wl[0]*n*(n/2+1) complex,
-// bufB wl[0]*wl[1]*(n/2+1) complex, out wl[0]*wl[1]*wl[2] reals.  yop
-// (FFT_YZ_*) multiplies the y pass's input as fft_c2r_yz does; with xpass
-// false bufA already holds the x pass of an earlier call on the same
-// spectrum, operator and window, and only the y and z passes run.
+// bufB wl[0]*wl[1]*(n/2+1) complex, out wl[0]*wl[1]*wl[2] reals.
 template <typename T>
-void fft_c2r_window(const T *spec, int n, int pre, const T *tab, int comp, double kmin, const int *w0, const int *wl,
-                    T *bufA, T *bufB, T *out, hipStream_t st, TimingHook *hook, const FilterInline *fil = nullptr,
-                    int yop = FFT_YZ_ONE, bool xpass = true);
+void fft_c2r_window(const T *spec, int n, int pre, const T *tab, double kmin, const int *w0, const int *wl,
+                    T *bufA, T *bufB, T *out, hipStream_t st, TimingHook *hook, const FilterInline *fil = nullptr);
 
 }  // namespace gic

@@ -29,7 +29,7 @@ template <typename T> void fft3d(T *d, int n, int dir, hipStream_t st, TimingHoo
   if (dir < 0) {
     api<T>(n).r2c(d, nullptr, st, hook, nullptr);
   } else {
-    api<T>(n).c2r(d, st, hook, nullptr);
+    api<T>(n).c2r(d, st, hook);
   }
 }
 template <typename T> void fft_r2c_post(T *d, int n, const T *post, hipStream_t st, TimingHook *hook, const T *src) {
@@ -43,41 +43,16 @@ template <typename T>
 void fft_r2c_boxes(const T *rows, int n, long nrows, int nb, int wl, const int *winx, const int *winy, T *zbuf, T *ybuf,
                    T *spec, long spec_stride, const T *post, hipStream_t st, TimingHook *hook) {
   if (nb < 1 || wl < 1 || wl >= n) throw std::runtime_error("fft_r2c_boxes: bad box count or size");
-  if (nrows < long(nb) * wl * wl || nrows % fft_box_rows_multiple<T>(n)) throw std::runtime_error("fft_r2c_boxes: bad row count");
+  if (nrows < long(nb) * wl * wl) throw std::runtime_error("fft_r2c_boxes: bad row count");
   api<T>(n).r2c_boxes(rows, nrows, nb, wl, winx, winy, zbuf, ybuf, spec, spec_stride, post, st, hook);
-}
-template <typename T> int fft_box_rows_multiple(int n) {
-  return api<T>(n).rows;
 }
 template <typename T> void fft_prepare(int n) {
   api<T>(n).prepare();
 }
-template <typename T> void fft_c2r_to(T *d, T *dst, int n, hipStream_t st, TimingHook *hook) {
-  api<T>(n).c2r(d, st, hook, dst);
-}
 template <typename T>
-void fft_r2c_za_adjoint(const T *src, T *d, T *acc, int n, const T *tab, int comp, double kmin, bool accumulate,
-                        hipStream_t st, TimingHook *hook) {
-  api<T>(n).r2c_za_adjoint(src, d, acc, tab, comp, T(kmin), accumulate, st, hook);
-}
-template <typename T>
-void fft_c2r_from(const T *spec, T *out, int n, int pre, const T *tab, int comp, double kmin, hipStream_t st,
+void fft_c2r_from(const T *spec, T *out, int n, int pre, const T *tab, double kmin, hipStream_t st,
                   TimingHook *hook, T *dst, double inv_k2, const FilterInline *fil) {
-  api<T>(n).c2r_from(spec, out, pre, tab, comp, kmin, st, hook, dst, inv_k2, fil);
-}
-template <typename T>
-void fft_c2r_xpass(const T *spec, T *half, int n, int pre, const T *tab, int comp, double kmin, hipStream_t st,
-                   TimingHook *hook, double inv_k2) {
-  api<T>(n).xpass_from(spec, half, pre, tab, comp, kmin, inv_k2, st, hook);
-}
-template <typename T>
-void fft_c2r_yz(const T *half, T *out, int n, int yop, double kmin, hipStream_t st, TimingHook *hook, T *dst) {
-  api<T>(n).yz_from(half, out, yop, kmin, st, hook, dst);
-}
-template <typename T>
-void fft_c2r_yz_lpt(const T *half, T *scratch, int n, int yop, double kmin, int epi, T *S, T *A, hipStream_t st,
-                    TimingHook *hook) {
-  api<T>(n).yz_from_epi(half, scratch, yop, kmin, epi, S, A, st, hook);
+  api<T>(n).c2r_from(spec, out, pre, tab, kmin, st, hook, dst, inv_k2, fil);
 }
 template <typename T>
 void fft_r2c_window_zy(const T *win, int n, const int *w0, const int *wl, T *bufB, T *bufA, hipStream_t st,
@@ -96,12 +71,11 @@ void fft_r2c_window(const T *win, int n, const int *w0, const int *wl, T *bufB, 
   api<T>(n).r2c_window(win, w0, wl, bufB, bufA, spec, post, accumulate, st, hook, aux, fil, kmin);
 }
 template <typename T>
-void fft_c2r_window(const T *spec, int n, int pre, const T *tab, int comp, double kmin, const int *w0, const int *wl,
-                    T *bufA, T *bufB, T *out, hipStream_t st, TimingHook *hook, const FilterInline *fil, int yop,
-                    bool xpass) {
+void fft_c2r_window(const T *spec, int n, int pre, const T *tab, double kmin, const int *w0, const int *wl,
+                    T *bufA, T *bufB, T *out, hipStream_t st, TimingHook *hook, const FilterInline *fil) {
   for (int a = 0; a < 3; ++a)
     if (wl[a] < 1 || wl[a] > n || w0[a] < 0 || w0[a] >= n) throw std::runtime_error("fft_c2r_window: bad window");
-  api<T>(n).c2r_window(spec, pre, tab, comp, T(kmin), w0, wl, bufA, bufB, out, st, hook, fil, yop, xpass);
+  api<T>(n).c2r_window(spec, pre, tab, kmin, w0, wl, bufA, bufB, out, st, hook, fil);
 }
 
 template <typename T> void fft_x(const FftX<T> &x, int n, hipStream_t st, TimingHook *hook) {
@@ -157,25 +131,17 @@ void fft_z_lpt(T *px, T *py, T *pz, const T *xx, const T *yy, const T *xy, T *S,
   template void fft_z_lpt<T>(T *, T *, T *, const T *, const T *, const T *, T *, bool, int, double,         \
                              hipStream_t, TimingHook *);                                                     \
   template void fft_r2c_post<T>(T *, int, const T *, hipStream_t, TimingHook *, const T *);                 \
-  template void fft_c2r_to<T>(T *, T *, int, hipStream_t, TimingHook *);                                    \
   template void fft_r2c_batch<T>(T *, int, int, const T *, hipStream_t, TimingHook *);                      \
   template void fft_prepare<T>(int);                                                                        \
-  template int fft_box_rows_multiple<T>(int);                                                               \
   template void fft_r2c_boxes<T>(const T *, int, long, int, int, const int *, const int *, T *, T *, T *, long,  \
                                  const T *, hipStream_t, TimingHook *);                                       \
-  template void fft_r2c_za_adjoint<T>(const T *, T *, T *, int, const T *, int, double, bool, hipStream_t,   \
-                                      TimingHook *);                                                          \
-  template void fft_c2r_from<T>(const T *, T *, int, int, const T *, int, double, hipStream_t, TimingHook *, T *, \
+  template void fft_c2r_from<T>(const T *, T *, int, int, const T *, double, hipStream_t, TimingHook *, T *, \
                                 double, const FilterInline *);                                               \
-  template void fft_c2r_xpass<T>(const T *, T *, int, int, const T *, int, double, hipStream_t, TimingHook *,  \
-                                 double);                                                                    \
-  template void fft_c2r_yz<T>(const T *, T *, int, int, double, hipStream_t, TimingHook *, T *);              \
-  template void fft_c2r_yz_lpt<T>(const T *, T *, int, int, double, int, T *, T *, hipStream_t, TimingHook *); \
   template void fft_r2c_window_zy<T>(const T *, int, const int *, const int *, T *, T *, hipStream_t, TimingHook *); \
   template void fft_r2c_window<T>(const T *, int, const int *, const int *, T *, T *, T *, const T *, bool,      \
                                   hipStream_t, TimingHook *, const T *, const FilterInline *, double);         \
-  template void fft_c2r_window<T>(const T *, int, int, const T *, int, double, const int *, const int *, T *, T *, \
-                                  T *, hipStream_t, TimingHook *, const FilterInline *, int, bool);
+  template void fft_c2r_window<T>(const T *, int, int, const T *, double, const int *, const int *, T *, T *, \
+                                  T *, hipStream_t, TimingHook *, const FilterInline *);
 GIC_FFT_INST(float)
 GIC_FFT_INST(double)
 

@@ -6,24 +6,16 @@
 namespace gic {
 
 template <typename T> struct FftApi {
-  int rows;   // z-pass rows per block
   void (*prepare)();
   void (*r2c)(T *d, const T *post, hipStream_t st, TimingHook *hook, const T *src);
   void (*r2c_batch)(T *d, int nb, const T *post, hipStream_t st, TimingHook *hook);
   void (*r2c_boxes)(const T *rows, long nrows, int nb, int wl, const int *winx, const int *winy, T *zbuf, T *ybuf,
                     T *spec, long spec_stride, const T *post, hipStream_t st, TimingHook *hook);
-  void (*c2r)(T *d, hipStream_t st, TimingHook *hook, T *dst);
-  void (*r2c_za_adjoint)(const T *src, T *d, T *acc, const T *tab, int comp, T kmin, bool accum, hipStream_t st,
-                         TimingHook *hook);
-  void (*c2r_from)(const T *spec, T *out, int pre, const T *tab, int comp, double kmin, hipStream_t st,
+  void (*c2r)(T *d, hipStream_t st, TimingHook *hook);
+  void (*c2r_from)(const T *spec, T *out, int pre, const T *tab, double kmin, hipStream_t st,
                    TimingHook *hook, T *dst, double inv_k2, const FilterInline *fil);
-  void (*xpass_from)(const T *spec, T *half, int pre, const T *tab, int comp, double kmin, double inv_k2,
-                     hipStream_t st, TimingHook *hook);
-  void (*yz_from)(const T *half, T *out, int yop, double kmin, hipStream_t st, TimingHook *hook, T *dst);
-  void (*yz_from_epi)(const T *half, T *out, int yop, double kmin, int epi, T *S, T *A, hipStream_t st,
-                      TimingHook *hook);
-  void (*c2r_window)(const T *spec, int pre, const T *tab, int comp, T kmin, const int *w0, const int *wl, T *bufA,
-                     T *bufB, T *out, hipStream_t st, TimingHook *hook, const FilterInline *fil, int yop, bool xpass);
+  void (*c2r_window)(const T *spec, int pre, const T *tab, double kmin, const int *w0, const int *wl, T *bufA,
+                     T *bufB, T *out, hipStream_t st, TimingHook *hook, const FilterInline *fil);
   void (*r2c_window)(const T *win, const int *w0, const int *wl, T *bufB, T *bufA, T *spec, const T *post, bool accum,
                      hipStream_t st, TimingHook *hook, const T *aux, const FilterInline *fil, double kmin);
   void (*r2c_window_zy)(const T *win, const int *w0, const int *wl, T *bufB, T *bufA, hipStream_t st, TimingHook *hook);

@@ -361,7 +361,6 @@ __global__ __launch_bounds__((LineFft<T, L, C, 1, true>::TH), 2) void k_fft_x_ad
 // Inverse: job j (blockIdx.y) transforms its input times FFT_YZ_* factors of
 // (k_y, k_z), up to three fields from one read; outputs keep the points
 // [win0, win0 + wlen).  An output may be the input's own memory.
-constexpr int FUSED_JOBS = 6;
 template <typename T> struct YArgs {
   struct Job {
     const cx<T> *in;
@@ -373,36 +372,6 @@ template <typename T> struct YArgs {
   int nkzb, win0, wlen;
   T kmin;
 };
-// FFT_YZ_* as i^rot k_y^py k_z^pz, the first powers 0 at +Nyquist
-struct YzOp {
-  int rot, py, pz;
-};
-__device__ __forceinline__ YzOp yz_op(int op) {
-  YzOp r{0, 0, 0};
-  switch (op) {
-    case FFT_YZ_IKY: return {1, 1, 0};
-    case FFT_YZ_IKZ: return {1, 0, 1};
-    case FFT_YZ_MIKY: return {3, 1, 0};
-    case FFT_YZ_MIKZ: return {3, 0, 1};
-    case FFT_YZ_KYKY: return {0, 2, 0};
-    case FFT_YZ_KYKZ: return {0, 1, 1};
-    case FFT_YZ_KZKZ: return {0, 0, 2};
-    case FFT_YZ_I: return {1, 0, 0};
-    case FFT_YZ_KZ: return {0, 0, 1};
-    case FFT_YZ_KY: return {0, 1, 0};
-  }
-  return r;
-}
-template <typename T> __device__ __forceinline__ T k_power(int p, int k, int nyq, T kmin) {
-  const T f = T(k) * kmin;
-  return p == 0 ? T(1) : p == 2 ? f * f : k == nyq ? T(0) : f;
-}
-template <typename T> __device__ __forceinline__ cx<T> rot_mul(int rot, cx<T> v, T f) {
-  if (rot == 0) return cx<T>{v.x * f, v.y * f};
-  if (rot == 3) f = -f;
-  return cx<T>{-v.y * f, v.x * f};
-}
-
 template <typename T, int L, int C>
 __global__ __launch_bounds__((LineFft<T, L, C, 1, false>::TH), (LineFft<T, L, C, 1, false>::TH > 512 ? 1 : 2)) void
 k_fft_y_fused(YArgs<T> a, const cx<T> *__restrict__ tw) {
@@ -485,236 +454,11 @@ k_fft_y_forward(YFwdArgs<T> a, const cx<T> *__restrict__ tw) {
   Fw::template store<R>(v, job.out + at, NZ, nc, 0, L);
 }
 
-// ---- z passes ---------------------------------------------------------------------
-// c2r of several fields (blockIdx.y) of a batch (blockIdx.z): complex rows
-// times a factor of k_z (FFT_YZ_ONE, IKZ, MIKZ, KZ, KZKZ or I), the real rows
-// to the padded field out (may be the input), a dense array, or both.
-template <typename T> struct ZArgs {
-  struct Job {
-    const T *in;
-    T *out, *dense;
-    int op;
-  } job[FUSED_JOBS];
-  long in_bs, out_bs, dense_bs;   // reals
-  T scale, kmin;
-};
-
-// the packed complex row of a c2r's half-length transform into LDS
-template <typename T, int N, int ROWS, int THREADS, class In>
-__device__ __forceinline__ void z_c2r_pack(cx<T> *lds, const cx<T> *__restrict__ twN, In in, int tid) {
-  constexpr int M = N / 2, H = M / 2 + 1;
-  for (int q = tid; q < ROWS * H; q += THREADS) {
-    int line = q / H, k = q - line * H;
-    cx<T> xk = in(line, k), xm = in(line, M - k);
-    if (k == 0) {   // c2r ignores the imaginary parts of the kz=0 and kz=N/2 entries
-      xk.y = 0;
-      xm.y = 0;
-    }
-    cx<T> Ev{xk.x + xm.x, xk.y - xm.y};
-    cx<T> D{xk.x - xm.x, xk.y + xm.y};
-    cx<T> w = twN[k];
-    w.y = -w.y;
-    cx<T> O = cmul(D, w);
-    lds[ZRow<M>::idx(line, k)] = cx<T>{Ev.x - O.y, Ev.y + O.x};
-    if (k != 0 && M - k != k) lds[ZRow<M>::idx(line, M - k)] = cx<T>{Ev.x + O.y, -Ev.y + O.x};
-  }
-}
-
-template <typename T, int N, int ROWS, int THREADS>
-__global__ __launch_bounds__(THREADS) void k_fft_z_c2r_fused(ZArgs<T> a, const cx<T> *__restrict__ twN) {
-  constexpr int M = N / 2;
-  extern __shared__ char smem_raw[];
-  cx<T> *lds = reinterpret_cast<cx<T> *>(smem_raw), *ltw = lds + ROWS * ZRow<M>::len;
-  for (int i = int(threadIdx.x); i < M; i += THREADS) ltw[i] = twN[2 * i];
-  const auto &job = a.job[blockIdx.y];
-  const long row0 = long(blockIdx.x) * ROWS;
-  const cx<T> *rows = reinterpret_cast<const cx<T> *>(job.in + long(blockIdx.z) * a.in_bs) + row0 * (M + 1);
-  const YzOp op = yz_op(job.op);
-  z_c2r_pack<T, N, ROWS, THREADS>(lds, twN, [&](int line, int k) {
-    return rot_mul<T>(op.rot, rows[long(line) * (M + 1) + k], k_power<T>(op.pz, k, M, a.kmin));
-  }, int(threadIdx.x));
-  __syncthreads();
-  cx<T> *out = job.out ? reinterpret_cast<cx<T> *>(job.out + long(blockIdx.z) * a.out_bs) + row0 * (M + 1) : nullptr;
-  cx<T> *dense = job.dense ? reinterpret_cast<cx<T> *>(job.dense + long(blockIdx.z) * a.dense_bs) + row0 * M : nullptr;
-  auto lidx = [](int line, int pt) { return ZRow<M>::idx(line, pt); };
-  auto lld = [&](int line, int pt) -> cx<T> { return lds[lidx(line, pt)]; };
-  auto gst = [&](int line, int pt, cx<T> v) {
-    cx<T> r{v.x * a.scale, v.y * a.scale};
-    if (out) out[long(line) * (M + 1) + pt] = r;
-    if (dense) dense[long(line) * M + pt] = r;
-  };
-  run_stages<T, M, ROWS, THREADS, +1, false, true, false, 0, false>(lds, ltw, 1, lld, gst, lidx);
-}
-
-// r2c of several fields: real rows from a padded field or a dense array (row
-// stride srs reals) to padded complex rows (may be the input).
-template <typename T> struct ZFwdArgs {
-  struct Job {
-    const T *src;
-    T *out;
-    long srs;
-  } job[FUSED_JOBS];
-  long src_bs, out_bs;
-};
-template <typename T, int N, int ROWS, int THREADS>
-__global__ __launch_bounds__(THREADS) void k_fft_z_r2c_fused(ZFwdArgs<T> a, const cx<T> *__restrict__ twN) {
-  constexpr int M = N / 2, H = M / 2 + 1;
-  extern __shared__ char smem_raw[];
-  cx<T> *lds = reinterpret_cast<cx<T> *>(smem_raw), *ltw = lds + ROWS * ZRow<M>::len;
-  for (int i = int(threadIdx.x); i < M; i += THREADS) ltw[i] = twN[2 * i];
-  const auto &job = a.job[blockIdx.y];
-  const long row0 = long(blockIdx.x) * ROWS, srs = job.srs / 2;
-  const cx<T> *src = reinterpret_cast<const cx<T> *>(job.src + long(blockIdx.z) * a.src_bs) + row0 * srs;
-  cx<T> *rows = reinterpret_cast<cx<T> *>(job.out + long(blockIdx.z) * a.out_bs) + row0 * (M + 1);
-  auto gld = [&](int line, int pt) -> cx<T> { return src[long(line) * srs + pt]; };
-  auto lidx = [](int line, int pt) { return ZRow<M>::idx(line, pt); };
-  auto lst = [&](int line, int pt, cx<T> v) { lds[lidx(line, pt)] = v; };
-  run_stages<T, M, ROWS, THREADS, -1, false, false, true, 0, false>(lds, ltw, 1, gld, lst, lidx);
-  __syncthreads();
-  for (int q = threadIdx.x; q < ROWS * H; q += THREADS) {
-    int line = q / H, k = q - line * H;
-    cx<T> zk = lds[lidx(line, k % M)], zm = lds[lidx(line, (M - k) % M)];
-    cx<T> F{(zk.x + zm.x) * T(0.5), (zk.y - zm.y) * T(0.5)};
-    cx<T> D{(zk.x - zm.x) * T(0.5), (zk.y + zm.y) * T(0.5)};
-    cx<T> wg = cmul(twN[k], cx<T>{D.y, -D.x});
-    cx<T> *o = rows + long(line) * (M + 1);
-    o[k] = cx<T>{F.x + wg.x, F.y + wg.y};
-    if (M - k != k) o[M - k] = cx<T>{F.x - wg.x, -(F.y - wg.y)};
-  }
-}
-
-// The stages of a row transform from LDS into registers: element b R + s of v
-// is point i + s M / R of butterfly q = tid + b THREADS = line (M / R) + i, R
-// the last stage's radix.  (A thread past the last butterfly repeats it.)
-template <typename T, int M, int ROWS, int THREADS, int S, int NV>
-__device__ __forceinline__ void rows_to_regs(cx<T> *lds, const cx<T> *ltw, cx<T> (&v)[NV], int tid) {
-  using P = RadixPlan<M, false>;
-  constexpr int R = P::radix(S), p = P::pbefore(S), NB = ROWS * (M / R), PER = (NB + THREADS - 1) / THREADS;
-  auto butterfly = [&](int b, cx<T> *x, int &line, int &i) {
-    const int q = min(tid + b * THREADS, NB - 1);
-    line = q / (M / R);
-    i = q % (M / R);
-    const int k = i % p;
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      x[r] = lds[ZRow<M>::idx(line, i + r * (M / R))];
-      if (p > 1 && r > 0) {
-        cx<T> w = ltw[r * k * (M / (p * R))];
-        w.y = -w.y;
-        x[r] = cmul(x[r], w);
-      }
-    }
-    Dft<R, +1, T>::run(x);
-  };
-  if constexpr (S < P::nstages - 1) {
-    cx<T> x[PER][R];
-    int line[PER], i[PER];
-#pragma unroll
-    for (int b = 0; b < PER; ++b) butterfly(b, x[b], line[b], i[b]);
-    __syncthreads();
-#pragma unroll
-    for (int b = 0; b < PER; ++b) {
-      const int k = i[b] % p, j = (i[b] - k) * R + k;
-      if (NB % THREADS == 0 || tid + b * THREADS < NB) {
-#pragma unroll
-        for (int s = 0; s < R; ++s) lds[ZRow<M>::idx(line[b], j + s * p)] = x[b][s];
-      }
-    }
-    __syncthreads();
-    rows_to_regs<T, M, ROWS, THREADS, S + 1>(lds, ltw, v, tid);
-  } else {
-    static_assert(NV == PER * R, "one register per element");
-    int line, i;
-#pragma unroll
-    for (int b = 0; b < PER; ++b) butterfly(b, v + b * R, line, i);
-  }
-}
-
-// The second-order source and the first-order displacements of one level
-// from six fields transformed along x and y:
-//   px: of i k_x f m   py: of k_y f m times X0   pz: of f m   (X0, X1 of the x pass)
-//   xx: of k_x^2 f m   yy: of k_y^2 f m           xy: of k_x k_y f m
-// psi_x = Z px, psi_y = Z i py, psi_z = Z i k_z pz, phi_xz = Z (-i k_z) px,
-// phi_yz = Z k_z py, phi_zz = Z k_z^2 pz, and
-//   S = xx yy + (xx + yy) zz - xy^2 - xz^2 - yz^2
-// so that each of the six is read once for the nine transforms made of it.
-// With PSI the displacements go over px, py, pz; S to a padded field.
-template <typename T> struct ZLptArgs {
-  T *px, *py, *pz;
-  const T *xx, *yy, *xy;
-  T *S;
-  T scale, kmin;
-};
-template <typename T, int N, int ROWS, int THREADS, bool PSI>
-__global__ __launch_bounds__(THREADS, (sizeof(T) == 4 ? 4 : 2)) void k_fft_z_lpt(ZLptArgs<T> a, const cx<T> *__restrict__ twN) {
-  constexpr int M = N / 2;
-  using P = RadixPlan<M, false>;
-  constexpr int RL = P::radix(P::nstages - 1);   // the last stage's radix
-  constexpr int NB = ROWS * (M / RL), PER = (NB + THREADS - 1) / THREADS;
-  extern __shared__ char smem_raw[];
-  cx<T> *lds = reinterpret_cast<cx<T> *>(smem_raw), *ltw = lds + ROWS * ZRow<M>::len;
-  for (int i = int(threadIdx.x); i < M; i += THREADS) ltw[i] = twN[2 * i];
-  const long row0 = long(blockIdx.x) * ROWS;
-  cx<T> S[PER * RL], A[PER * RL];
-  // one piece of code for the nine transforms; indexes formed anew in each
-  // (they would fill the registers that S and A need)
-#pragma unroll 1
-  for (int s = 0; s < (PSI ? 9 : 6); ++s) {
-    // xx, yy, zz, xy, xz, yz, then the displacements, each over its own rows,
-    // whose last reading this is
-    T *own = s == 6 ? a.px : s == 7 ? a.py : a.pz;
-    const T *src = s == 0 ? a.xx : s == 1 ? a.yy : s == 2 ? a.pz : s == 3 ? a.xy : s == 4 ? a.px : s == 5 ? a.py : own;
-    const YzOp f = s == 2 ? YzOp{0, 0, 2} : s == 4 ? YzOp{3, 0, 1} : s == 5 ? YzOp{0, 0, 1} : s == 7 ? YzOp{1, 0, 0}
-                   : s == 8 ? YzOp{1, 0, 1} : YzOp{0, 0, 0};
-    const cx<T> *rows = reinterpret_cast<const cx<T> *>(src) + row0 * (M + 1);
-    int tid = int(threadIdx.x);
-    asm volatile("" : "+v"(tid));
-    __syncthreads();   // LDS is free, the twiddles are there
-    z_c2r_pack<T, N, ROWS, THREADS>(lds, twN, [&](int line, int k) {
-      return rot_mul<T>(f.rot, rows[long(line) * (M + 1) + k], k_power<T>(f.pz, k, M, a.kmin));
-    }, tid);
-    __syncthreads();
-    cx<T> v[PER * RL];
-    rows_to_regs<T, M, ROWS, THREADS, 0>(lds, ltw, v, tid);
-#pragma unroll
-    for (int e = 0; e < PER * RL; ++e) {
-      const cx<T> x{v[e].x * a.scale, v[e].y * a.scale};
-      if (s == 0) {
-        A[e] = x;
-      } else if (s == 1) {
-        S[e] = cx<T>{A[e].x * x.x, A[e].y * x.y};
-        A[e] = cadd(A[e], x);
-      } else if (s == 2) {
-        S[e] = cx<T>{S[e].x + A[e].x * x.x, S[e].y + A[e].y * x.y};
-      } else if (s < 6) {
-        S[e] = cx<T>{S[e].x - x.x * x.x, S[e].y - x.y * x.y};
-      } else {
-        A[e] = x;
-      }
-    }
-    if (s >= 5) {
-      T *dst = s == 5 ? a.S : own;
-      cx<T> *o = reinterpret_cast<cx<T> *>(dst) + row0 * (M + 1);
-#pragma unroll
-      for (int b = 0; b < PER; ++b) {
-        const int q = tid + b * THREADS, line = q / (M / RL), i = q % (M / RL);
-        if (NB % THREADS == 0 || q < NB) {
-#pragma unroll
-          for (int r = 0; r < RL; ++r) {
-            // both read, then chosen: chosen by address they would live in memory
-            const cx<T> vs = S[b * RL + r], va = A[b * RL + r];
-            o[long(line) * (M + 1) + i + r * (M / RL)] = cx<T>{s == 5 ? vs.x : va.x, s == 5 ? vs.y : va.y};
-          }
-        }
-      }
-    }
-  }
-}
-
 // ---- launches ---------------------------------------------------------------------
 template <typename T, int N> struct FftFused {
   using F = FftN<T, N>;
-  static constexpr int NZ = N / 2 + 1, M = N / 2, ROWS = F::ROWS, ZTH = F::THREADS;
+  using Rows = RowLaunch<T, N>;
+  static constexpr int NZ = N / 2 + 1;
   static constexpr int CX = FusedCols<T, N>::x, CY = FusedCols<T, N>::y;
   static constexpr double FIELD = double(N) * N * NZ * sizeof(cx<T>);   // bytes of a spectrum
   static cx<T> *c(T *p) { return reinterpret_cast<cx<T> *>(p); }
@@ -735,11 +479,6 @@ template <typename T, int N> struct FftFused {
     if (hook) hook->end(tag.c_str(), st);
   }
   static size_t tile_lds(int cols) { return sizeof(cx<T>) * (cols + 1) * N; }
-  static size_t row_lds(int rows = ROWS) { return sizeof(cx<T>) * (rows * ZRow<M>::len + M); }
-  // rows per block of the 2LPT z pass: 8 (FP32) or 4 points a thread, of which
-  // three sets are held
-  static constexpr int LROWS0 = ZTH * (sizeof(T) == 4 ? 8 : 4) / M;
-  static constexpr int LROWS = LROWS0 > N * N ? N * N : LROWS0;
 
   static void x(const FftX<T> &q, hipStream_t st, TimingHook *hook) {
     XArgs<T> a{};
@@ -758,7 +497,7 @@ template <typename T, int N> struct FftFused {
     s.inv_k2 = q.inv_k2;
     if (q.fil) s.fil = *q.fil;
     F::prepare_factor(s);
-    a.f = PreArgs<T>{s.tab, 0, NZ, N, T(q.kmin), s.inv_k2, s.kmin_d, s.ff, s.inv_k2_f};
+    a.f = PreArgs<T>{s.tab, NZ, N, s.inv_k2, s.kmin_d, s.ff, s.inv_k2_f};
     a.tab0 = q.tab0;
     a.plain0 = q.plain0 ? 1 : 0;
     if ((q.out[1] || q.out[2] || q.out[3]) && !q.tab && q.inv_k2 == 0 && s.ff.nf < 0)
@@ -841,27 +580,29 @@ template <typename T, int N> struct FftFused {
     a.in_bs = q.in_bs;
     a.out_bs = q.out_bs;
     a.dense_bs = q.dense_bs;
+    a.nrows = long(N) * N;
+    a.iters = Rows::iters(a.nrows, long(q.njob) * q.nb);
     a.scale = F::norm() * T(q.scale);
     a.kmin = T(q.kmin);
-    launch(k_fft_z_c2r_fused<T, N, ROWS, ZTH>, dim3(N * N / ROWS, q.njob, q.nb), ZTH, row_lds(), "fft_z_c2r_multi",
-           q.nb * FIELD * fields, st, hook, a);
+    F::rows_launch(k_fft_z_c2r<T, N, Rows::TH, false>, a, q.njob, q.nb, "fft_z_c2r_multi", q.nb * FIELD * fields, st,
+                   hook);
   }
   static void z_forward(const FftZFwd<T> &q, hipStream_t st, TimingHook *hook) {
     ZFwdArgs<T> a{};
     for (int j = 0; j < q.njob; ++j) a.job[j] = {q.job[j].src, q.job[j].out, q.job[j].dense ? long(N) : long(N + 2)};
     a.src_bs = q.src_bs;
     a.out_bs = q.out_bs;
-    launch(k_fft_z_r2c_fused<T, N, ROWS, ZTH>, dim3(N * N / ROWS, q.njob, q.nb), ZTH, row_lds(), "fft_z_r2c_multi",
-           q.nb * FIELD * 2 * q.njob, st, hook, a);
+    a.nrows = long(N) * N;
+    a.iters = Rows::iters(a.nrows, long(q.njob) * q.nb);
+    F::rows_launch(k_fft_z_r2c<T, N, Rows::TH, false>, a, q.njob, q.nb, "fft_z_r2c_multi", q.nb * FIELD * 2 * q.njob, st,
+                   hook);
   }
   static void z_lpt(T *px, T *py, T *pz, const T *xx, const T *yy, const T *xy, T *S, bool psi, double kmin,
                     hipStream_t st, TimingHook *hook) {
-    ZLptArgs<T> a{px, py, pz, xx, yy, xy, S, F::norm(), T(kmin)};
-    dim3 grid(N * N / LROWS);
-    if (psi)
-      launch(k_fft_z_lpt<T, N, LROWS, ZTH, true>, grid, ZTH, row_lds(LROWS), "fft_z_lpt", FIELD * 10, st, hook, a);
-    else
-      launch(k_fft_z_lpt<T, N, LROWS, ZTH, false>, grid, ZTH, row_lds(LROWS), "fft_z_lpt", FIELD * 7, st, hook, a);
+    const long nrows = long(N) * N;
+    ZLptArgs<T> a{px, py, pz, xx, yy, xy, S, nrows, Rows::iters(nrows, 1), F::norm(), T(kmin)};
+    if (psi) F::rows_launch(k_fft_z_lpt<T, N, Rows::TH, true>, a, 1, 1, "fft_z_lpt", FIELD * 10, st, hook);
+    else F::rows_launch(k_fft_z_lpt<T, N, Rows::TH, false>, a, 1, 1, "fft_z_lpt", FIELD * 7, st, hook);
   }
 };
 
@@ -869,17 +610,12 @@ template <typename T, int N> FftApi<T> fft_api_of() {
   using F = FftN<T, N>;
   using G = FftFused<T, N>;
   FftApi<T> a;
-  a.rows = F::ROWS;
   a.prepare = [] { twtable<T>().get(N); };
   a.r2c = F::r2c;
   a.r2c_batch = F::r2c_batch;
   a.r2c_boxes = F::r2c_boxes;
   a.c2r = F::c2r;
-  a.r2c_za_adjoint = F::r2c_za_adjoint;
   a.c2r_from = F::c2r_from;
-  a.xpass_from = F::xpass_from;
-  a.yz_from = F::yz_from;
-  a.yz_from_epi = F::yz_from_epi;
   a.c2r_window = F::c2r_window;
   a.r2c_window = F::r2c_window;
   a.r2c_window_zy = F::r2c_window_zy;

@@ -111,10 +111,10 @@ template <typename T> void run(int n, int reps, double *ms, double *err) {
     gic::fft3d<T>(c, n, +1, st, nullptr);
   });
   ms[1] = timed([&] {
-    gic::fft_c2r_from<T>(a, c, n, gic::FFT_PRE_ZA, nullptr, 0, kmin, st, nullptr, b, 1.0, nullptr);
+    gic::fft_c2r_from<T>(a, c, n, gic::FFT_PRE_TABLE, nullptr, kmin, st, nullptr, b, 1.0, nullptr);
   });
   ms[2] = timed([&] {
-    gic::fft_c2r_window<T>(a, n, gic::FFT_PRE_TABLE, tab, 0, kmin, w0, wl, A, B, o, st, nullptr, &fil);
+    gic::fft_c2r_window<T>(a, n, gic::FFT_PRE_TABLE, tab, kmin, w0, wl, A, B, o, st, nullptr, &fil);
   });
   ms[3] = timed([&] {
     gic::fft_r2c_window<T>(o, n, w0, wl, B, A, c, tab, false, st, nullptr, a, &fil, kmin);

@@ -1226,7 +1226,7 @@ template <typename T> void add_transfer(gic_context *c, T *R, size_t lt, MLF<T> 
       T *bufA = (T *)scratch.p;
       T *bufB = (T *)((char *)scratch.p + a_b);
       T *out = (T *)((char *)scratch.p + a_b + b_b);
-      fft_c2r_window<T>(f.p(ls), gs.n, FFT_PRE_TABLE, tab, 0, gs.kmin(), w0, wl, bufA, bufB, out, c->st, c->hook(),
+      fft_c2r_window<T>(f.p(ls), gs.n, FFT_PRE_TABLE, tab, gs.kmin(), w0, wl, bufA, bufB, out, c->st, c->hook(),
                         &fil);
       v.p = out;
       for (int a = 0; a < 3; ++a) {
@@ -1237,7 +1237,7 @@ template <typename T> void add_transfer(gic_context *c, T *R, size_t lt, MLF<T> 
       v.sy = wl[2];
     } else {
       scratch = PBuf(c->mod->pool, gs.padded_reals() * sizeof(T));
-      fft_c2r_from<T>(f.p(ls), (T *)scratch.p, gs.n, FFT_PRE_TABLE, tab, 0, gs.kmin(), c->st, c->hook());
+      fft_c2r_from<T>(f.p(ls), (T *)scratch.p, gs.n, FFT_PRE_TABLE, tab, gs.kmin(), c->st, c->hook());
       v.p = scratch.p;
       for (int a = 0; a < 3; ++a) {
         v.org[a] = 0;
@@ -1250,7 +1250,7 @@ template <typename T> void add_transfer(gic_context *c, T *R, size_t lt, MLF<T> 
   } else {
     const T *tab = spec_table<T>(c, gs, s);
     PBuf tmp(c->mod->pool, gs.padded_reals() * sizeof(T));
-    fft_c2r_from<T>(f.p(ls), (T *)tmp.p, gs.n, FFT_PRE_TABLE, tab, 0, gs.kmin(), c->st, c->hook());
+    fft_c2r_from<T>(f.p(ls), (T *)tmp.p, gs.n, FFT_PRE_TABLE, tab, gs.kmin(), c->st, c->hook());
     AvgGeom a;
     a.r = (int)llround(gt.dx / gs.dx);
     a.cell_off[0] = (int)llround((gt.ox - gs.ox) / gs.dx);
@@ -1286,7 +1286,7 @@ template <typename T> bool cross_terms(gic_context *c, MLF<T> &f, size_t l, PBuf
       f.toF(s);
       const T *tab = spec_table<T>(c, gs, spec_levels(c, long(l), long(s), sq));
       PBuf tmp(c->mod->pool, gs.padded_reals() * sizeof(T));
-      fft_c2r_from<T>(f.p(s), (T *)tmp.p, gs.n, FFT_PRE_TABLE, tab, 0, gs.kmin(), c->st, c->hook());
+      fft_c2r_from<T>(f.p(s), (T *)tmp.p, gs.n, FFT_PRE_TABLE, tab, gs.kmin(), c->st, c->hook());
       hipLaunchKernelGGL(k_fine_to_coarse_box<T>, dim3(blocks(nb)), dim3(256), 0, c->st, (T *)Rbox.p,
                          (const T *)tmp.p, avg_geom(g, gs), B);
       GIC_HIP(hipGetLastError());
@@ -1734,7 +1734,7 @@ template <typename T> MLF<T> push_variance(MLF<T> &field, const std::vector<std:
     }
     VarianceBox<T> V;
     if (V.make(c, l, cells)) {
-      fft_c2r_window<T>(f.p(l), g.n, FFT_PRE_NONE, nullptr, 0, g.kmin(), V.B.b0, V.B.bl, V.A(), (T *)V.b.p, V.v(),
+      fft_c2r_window<T>(f.p(l), g.n, FFT_PRE_NONE, nullptr, g.kmin(), V.B.b0, V.B.bl, V.A(), (T *)V.b.p, V.v(),
                         c->st, c->hook());
       V.apply(hp);
       fft_r2c_window<T>(V.v(), g.n, V.B.b0, V.B.bl, (T *)V.b.p, V.A(), f.p(l), nullptr, false, c->st, c->hook());
@@ -1817,7 +1817,7 @@ template <typename T> double chi2_of(gic_context *c, MLF<T> &field) {
       {
         PBuf A(c->mod->pool, size_t(M.bl[0]) * g.n * nz * 2 * sizeof(T));
         PBuf Bb(c->mod->pool, size_t(M.bl[0]) * M.bl[1] * nz * 2 * sizeof(T));
-        fft_c2r_window<T>(field.p(l), g.n, FFT_PRE_NONE, nullptr, 0, g.kmin(), M.b0, M.bl, (T *)A.p, (T *)Bb.p,
+        fft_c2r_window<T>(field.p(l), g.n, FFT_PRE_NONE, nullptr, g.kmin(), M.b0, M.bl, (T *)A.p, (T *)Bb.p,
                           (T *)ubox.p, c->st, c->hook());
       }
       PBuf uspec(c->mod->pool, g.padded_reals() * sizeof(T));
@@ -1854,7 +1854,7 @@ template <typename T> double chi2_of(gic_context *c, MLF<T> &field) {
           xbox = PBuf(c->mod->pool, nb * sizeof(T));
           PBuf A(c->mod->pool, size_t(B.bl[0]) * g.n * nz * 2 * sizeof(T));
           PBuf Bb(c->mod->pool, size_t(B.bl[0]) * B.bl[1] * nz * 2 * sizeof(T));
-          fft_c2r_window<T>(field.p(l), g.n, FFT_PRE_NONE, nullptr, 0, g.kmin(), B.b0, B.bl, (T *)A.p, (T *)Bb.p,
+          fft_c2r_window<T>(field.p(l), g.n, FFT_PRE_NONE, nullptr, g.kmin(), B.b0, B.bl, (T *)A.p, (T *)Bb.p,
                             (T *)xbox.p, c->st, c->hook());
           xv = (const T *)xbox.p;
         }
