@@ -594,7 +594,7 @@ template <typename T> void do_copy_field(gic_context *c, int field, int level, i
     c->stage.ensure(ob);
     if (dtype == GIC_DTYPE_F32) unpad<T, float>((const T *)b->p, n, (float *)c->stage.p, c->st);
     else unpad<T, double>((const T *)b->p, n, (double *)c->stage.p, c->st);
-    GIC_HIP(hipMemcpyAsync(host, c->stage.p, ob, hipMemcpyDeviceToHost, c->st));
+    c->to_host.run({{host, c->stage.p, ob}}, c->st);
   } else {
     if (field == GIC_FIELD_OVERDENSITY) ensure_noise_fourier<T>(c, L);
     else if (!*flag) {
@@ -609,7 +609,7 @@ template <typename T> void do_copy_field(gic_context *c, int field, int level, i
     c->stage.ensure(ob);
     if (dtype == GIC_DTYPE_F32) convert<T, float>((const T *)b->p, nreal, (float *)c->stage.p, c->st);
     else convert<T, double>((const T *)b->p, nreal, (double *)c->stage.p, c->st);
-    GIC_HIP(hipMemcpyAsync(host, c->stage.p, ob, hipMemcpyDeviceToHost, c->st));
+    c->to_host.run({{host, c->stage.p, ob}}, c->st);
   }
   GIC_HIP(hipStreamSynchronize(c->st));
 }
@@ -722,9 +722,7 @@ void do_particles(gic_context *c, int level, const uint64_t *cells, size_t start
     particles<T>((const T *)L.psi[0].p, (const T *)L.psi[1].p, (const T *)L.psi[2].p, L.have_psi2 ? q2 : nullptr,
                  L.g.n, pg, dcells, start + s0, m,
                  dpos, dvel, c->st);
-    GIC_HIP(hipMemcpyAsync(pos + 3 * s0, dpos, m * 12, hipMemcpyDeviceToHost, c->st));
-    GIC_HIP(hipMemcpyAsync(vel + 3 * s0, dvel, m * 12, hipMemcpyDeviceToHost, c->st));
-    GIC_HIP(hipStreamSynchronize(c->st));
+    c->to_host.run({{pos + 3 * s0, dpos, m * 12}, {vel + 3 * s0, dvel, m * 12}}, c->st);
   }
 }
 

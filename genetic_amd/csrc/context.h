@@ -3,6 +3,7 @@
 #pragma once
 #include "../../include/gic.h"
 #include "gic_common.h"
+#include "host_copy.h"
 #include "fft.h"
 #include "rng.h"
 #include "kspace.h"
@@ -274,6 +275,7 @@ struct gic_context {
   // x pass serves several displacement or second-derivative fields; after the
   // Zel'dovich pass of a second-order run the first holds the base level's source
   DevBuf xhalf;
+  gic::HostCopier to_host;
   std::unique_ptr<EventTimer> timer;
   TimingHook *hook() { return timer.get(); }
   size_t tsize() const { return prec == 32 ? 4 : 8; }
