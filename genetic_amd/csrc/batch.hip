@@ -28,8 +28,6 @@ namespace {
 constexpr int MAXCONS = 32;        // constraints per realisation
 constexpr int GRAM_THREADS = 256;
 constexpr int GRAM_BLOCKS = 512;
-constexpr int GRAM_VMAX = 36;      // MAXCONS + 1 vectors rounded up to tiles of 4
-constexpr int GRAM_NWMAX = 45;     // tile pairs of 9 tiles
 
 __device__ __forceinline__ double stored_mode_weight(int x, int y, int z, int h) {
   // each conjugate pair once: the kz = 0 and kz = N/2 planes hold both halves
@@ -137,99 +135,132 @@ __global__ __launch_bounds__(256) void k_batch_box_rows(T *__restrict__ rows, un
   if (live) rows[e] = inside ? T(1) : T(0);
 }
 
-// Partial sums of the products of the vectors v_0..v_nm (v_i = c_i for i <
-// nm, v_nm = w), weighted by the stored-mode weights: chunks of K modes of
-// every vector are staged through LDS, and each thread forms a 4 x 4 tile of
-// products (vectors 4ti+u against 4tj+v, tj <= ti) over every G-th mode of
-// the chunk, so that each LDS value feeds four products.  The G mode-groups
-// of a tile are summed in order of the group at the end; block b writes the
-// 16 values of tile pair p = ti(ti+1)/2 + tj at part[(b nw + p) 16 + 4u + v].
-template <typename T>
-__global__ __launch_bounds__(GRAM_THREADS) void k_batch_gram(const cx<T> *__restrict__ cov, long fs,
-                                                             const cx<T> *__restrict__ w, int nm, int n,
-                                                             double *__restrict__ part) {
-  cov += size_t(blockIdx.y) * nm * fs;
-  w += size_t(blockIdx.y) * fs;
-  constexpr int K = sizeof(T) == 4 ? 128 : 64;
-  constexpr int S = K + 1;   // LDS row stride: rows of different vectors start in different banks
-  __shared__ cx<T> sv[GRAM_VMAX * S];
-  __shared__ double sw[K];
-  __shared__ double red[GRAM_NWMAX * 16];
-  const int nv = nm + 1;
-  const int nt = (nv + 3) / 4;
-  const int nw = nt * (nt + 1) / 2;
-  const int G = GRAM_THREADS / nw;
-  const int h = n / 2;
-  const size_t nmodes = size_t(n) * n * (h + 1);
-  const size_t nchunks = (nmodes + K - 1) / K;
-  const int t = threadIdx.x;
-  const int p = t % nw, g = t / nw;
-  const bool live = g < G;
-  int ti = 0;
-  while ((ti + 1) * (ti + 2) / 2 <= p) ++ti;
-  const int tj = p - ti * (ti + 1) / 2;
-  double acc[16];
-#pragma unroll
-  for (int e = 0; e < 16; ++e) acc[e] = 0;
-  for (size_t ch = blockIdx.x; ch < nchunks; ch += gridDim.x) {
-    size_t m0 = ch * K;
-    for (int e = t; e < nt * 4 * K; e += GRAM_THREADS) {
-      int v = e / K, q = e - v * K;
-      size_t m = m0 + q;
-      cx<T> val{T(0), T(0)};
-      if (m < nmodes && v < nv) val = v < nm ? cov[size_t(v) * fs + m] : w[m];
-      sv[v * S + q] = val;
-    }
-    if (t < K) {
-      size_t m = m0 + t;
-      double wt = 0;
-      if (m < nmodes) {
-        int z = int(m % size_t(h + 1));
-        size_t r = m / size_t(h + 1);
-        wt = stored_mode_weight(int(r / size_t(n)), int(r % size_t(n)), z, h);
-      }
-      sw[t] = wt;
-    }
-    __syncthreads();
-    if (live) {
-      const cx<T> *A = sv + 4 * ti * S;
-      const cx<T> *B = sv + 4 * tj * S;
-      for (int q = g; q < K; q += G) {
-        double wt = sw[q];
-        double ax[4], ay[4], bx[4], by[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          cx<T> va = A[u * S + q], vb = B[u * S + q];
-          ax[u] = wt * double(va.x);
-          ay[u] = wt * double(va.y);
-          bx[u] = double(vb.x);
-          by[u] = double(vb.y);
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-          for (int v = 0; v < 4; ++v) acc[u * 4 + v] += ax[u] * bx[v] + ay[u] * by[v];
-      }
-    }
-    __syncthreads();
-  }
-  for (int e = t; e < nw * 16; e += GRAM_THREADS) red[e] = 0;
-  __syncthreads();
-  for (int gg = 0; gg < G; ++gg) {
-    if (live && g == gg) {
-#pragma unroll
-      for (int e = 0; e < 16; ++e) red[p * 16 + e] += acc[e];
-    }
-    __syncthreads();
-  }
-  part += size_t(blockIdx.y) * gridDim.x * nw * 16;
-  for (int e = t; e < nw * 16; e += GRAM_THREADS) part[size_t(blockIdx.x) * nw * 16 + e] = red[e];
-}
-
 // where the product of v_i and v_j (i >= j) sits among the tile sums
 __device__ __forceinline__ int gram_slot(int i, int j) {
   int ti = i >> 2, tj = j >> 2;
   return ((ti * (ti + 1) / 2 + tj) << 4) + ((i & 3) << 2) + (j & 3);
+}
+
+// Partial sums of the products of the covectors c_i among themselves and with
+// the field w, weighted by the stored-mode weights, in FP64: a contraction
+// over modes with matrix instructions, covectors in NB blocks of 16 rows.
+// Lane l reads 16 bytes of covector l % 16 of a block (2 FP32 modes or 1 FP64
+// mode), l / 16 apart, straight from memory; each of their components is one
+// k of a 16 x 16 x 4 product, the same registers serving as both operands (A
+// times the weight).  A wavefront's loads are whole 64-byte pieces of each
+// covector, so nothing goes through LDS.  Block b of the grid writes the
+// products in gram_slot's order (0 where there is none) at part[b nw 16].
+//
+// It is bound by reading the covectors: 8 realisations of 16 at 128^3 FP32,
+// 1.16 GB, 298 us (3.9 TB/s); with tiles of 4 x 4 products in vector registers,
+// their operands widened from LDS for each, 726 us.  5 of 3 at 64^3 FP64: 27 us,
+// 270 before, when most threads had no tile.
+typedef double gram_acc __attribute__((ext_vector_type(4)));
+template <typename T> struct GramVec;
+template <> struct GramVec<float> {
+  typedef float type __attribute__((ext_vector_type(4)));
+};
+template <> struct GramVec<double> {
+  typedef double type __attribute__((ext_vector_type(2)));
+};
+
+template <typename T, int NB>
+__global__ __launch_bounds__(GRAM_THREADS) void k_batch_gram(const cx<T> *__restrict__ cov, long fs,
+                                                             const cx<T> *__restrict__ w, int nm, int n,
+                                                             double *__restrict__ part) {
+  using V = typename GramVec<T>::type;
+  constexpr int MPL = 16 / int(sizeof(cx<T>)), C = 2 * MPL;   // modes and components of a lane's load
+  constexpr int U = 2, STEP = 4 * MPL, PAIRS = NB * (NB + 1) / 2;
+  cov += size_t(blockIdx.y) * nm * fs;
+  w += size_t(blockIdx.y) * fs;
+  const int h = n / 2, lane = int(threadIdx.x) % 64, row = lane % 16, kk = lane / 16;
+  const unsigned nz = unsigned(h + 1), nmodes = unsigned(n) * unsigned(n) * nz;   // a multiple of STEP: n >= 4
+  const unsigned wave = blockIdx.x * (GRAM_THREADS / 64) + threadIdx.x / 64, waves = gridDim.x * (GRAM_THREADS / 64);
+  const cx<T> *v[NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) v[b] = cov + size_t(min(16 * b + row, nm - 1)) * fs;
+  gram_acc acc[PAIRS];
+  double dot[NB];
+#pragma unroll
+  for (int p = 0; p < PAIRS; ++p) acc[p] = gram_acc{0, 0, 0, 0};
+#pragma unroll
+  for (int b = 0; b < NB; ++b) dot[b] = 0;
+  for (unsigned m0 = wave * (U * STEP); m0 < nmodes; m0 += waves * (U * STEP)) {
+    V x[U][NB], y[U];
+    unsigned m[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      m[u] = m0 + u * STEP + kk * MPL;
+      const unsigned at = min(m[u], nmodes - MPL);   // past the end: weight 0
+#pragma unroll
+      for (int b = 0; b < NB; ++b) x[u][b] = *reinterpret_cast<const V *>(v[b] + at);
+      y[u] = *reinterpret_cast<const V *>(w + at);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      double wt[MPL];
+#pragma unroll
+      for (int q = 0; q < MPL; ++q) {
+        const unsigned mq = m[u] + q, r = mq / nz;
+        wt[q] = mq < nmodes ? stored_mode_weight(int(r / unsigned(n)), int(r % unsigned(n)), int(mq - r * nz), h) : 0.0;
+      }
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        double a[NB], aw[NB];
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+          a[b] = double(x[u][b][c]);
+          aw[b] = a[b] * wt[c / 2];
+          dot[b] += aw[b] * double(y[u][c]);
+        }
+#pragma unroll
+        for (int bi = 0; bi < NB; ++bi)
+#pragma unroll
+          for (int bj = 0; bj <= bi; ++bj) {
+            const int p = bi * (bi + 1) / 2 + bj;
+            acc[p] = __builtin_amdgcn_mfma_f64_16x16x4f64(aw[bi], a[bj], acc[p], 0, 0, 0);
+          }
+      }
+    }
+  }
+  // the wavefronts of the block one after the other: a fixed order of the sums
+  __shared__ double red[PAIRS * 256 + NB * 16];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    dot[b] += __shfl_xor(dot[b], 16);
+    dot[b] += __shfl_xor(dot[b], 32);
+  }
+  for (int e = int(threadIdx.x); e < PAIRS * 256 + NB * 16; e += GRAM_THREADS) red[e] = 0;
+  __syncthreads();
+  for (int g = 0; g < GRAM_THREADS / 64; ++g) {
+    if (int(threadIdx.x) / 64 == g) {
+      // register r of lane l holds row 4 r + l / 16, column l % 16
+#pragma unroll
+      for (int p = 0; p < PAIRS; ++p)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) red[p * 256 + (4 * r + kk) * 16 + row] += acc[p][r];
+      if (kk == 0) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b) red[PAIRS * 256 + 16 * b + row] += dot[b];
+      }
+    }
+    __syncthreads();
+  }
+  const int nt = (nm + 4) / 4, np = nt * (nt + 1) / 2 * 16;
+  part += (size_t(blockIdx.y) * gridDim.x + blockIdx.x) * np;
+  for (int e = int(threadIdx.x); e < np; e += GRAM_THREADS) {
+    int ti = 0;
+    while ((ti + 1) * (ti + 2) / 2 <= e / 16) ++ti;
+    const int i = 4 * ti + (e % 16) / 4, j = 4 * (e / 16 - ti * (ti + 1) / 2) + e % 4;
+    double s = 0;
+    if (i < nm && j < nm) {   // j's block is i's or one before
+      const int bi = i / 16, bj = j / 16;
+      s = red[(bi * (bi + 1) / 2 + bj) * 256 + (i % 16) * 16 + j % 16];
+    } else if (i == nm && j < nm) {
+      s = red[PAIRS * 256 + j];
+    }
+    part[e] = s;
+  }
 }
 
 // sums[p] = sum over blocks of part[b * np + p], one block per pair, fixed order
@@ -508,9 +539,9 @@ void do_batch(gic_context *c, int nreal, const uint64_t *seeds, int ncons, const
       fft_r2c_batch<T>(cv, n, nc, (const T *)L.sqrtp_dm.p, st, hook);
     }
     // Gram matrices and current values, FP64 solves, update with the transfer function
-    hipLaunchKernelGGL(k_batch_gram<T>, dim3(GRAM_BLOCKS, nb), dim3(GRAM_THREADS), 0, st,
-                       reinterpret_cast<const cx<T> *>(cv), fs, reinterpret_cast<const cx<T> *>(w), ncons, n,
-                       (double *)B.part.p);
+    auto gram = ncons <= 16 ? k_batch_gram<T, 1> : k_batch_gram<T, 2>;
+    hipLaunchKernelGGL(gram, dim3(GRAM_BLOCKS, nb), dim3(GRAM_THREADS), 0, st, reinterpret_cast<const cx<T> *>(cv), fs,
+                       reinterpret_cast<const cx<T> *>(w), ncons, n, (double *)B.part.p);
     GIC_HIP(hipGetLastError());
     hipLaunchKernelGGL(k_batch_reduce, dim3(np, nb), dim3(256), 0, st, (const double *)B.part.p, GRAM_BLOCKS, np,
                        (double *)B.sums.p);
