@@ -341,10 +341,9 @@ def batch_constraints(nreal=64, nmods=16, box=50.0, seed=20261202):
 def batch_throughput(nreal=64, n=128, box=50.0, nmods=16, precision=32, lanes=8, reps=3):
     """The batching workload: nreal independent n^3 realisations (real-space
     seeds 1..nreal), each with nmods overdensity constraints, then delta and
-    Zel'dovich psi; FP32 fields, FP64 Gram solve.  The batch runs as one HIP
-    graph per call (gic_batch_constrained, lanes concurrent chains), graph
-    recording included in the time; the same work one realisation at a time
-    through the ordinary calls is timed beside it."""
+    Zel'dovich psi; FP32 fields, FP64 Gram solve.  Every launch of a batch
+    works on a group of realisations (gic_batch_constrained); the same work
+    one realisation at a time through the ordinary calls is timed beside it."""
     import numpy as np
     import torch
     wl = dict(box=box, n=n, zooms=[])
@@ -386,7 +385,7 @@ def batch_throughput(nreal=64, n=128, box=50.0, nmods=16, precision=32, lanes=8,
                 one_at_a_time=dict(value=round(nreal * n ** 3 / dts / 1e6, 2),
                                    ms_per_realisation=round(dts / nreal * 1e3, 3)),
                 config="%d realisations of %d^3 in %.0f Mpc/h (seeds 1..%d), %d overdensity constraints each "
-                       "(splitmix64 seed 20261202), FP32 fields, FP64 Gram solve, one HIP graph per batch"
+                       "(splitmix64 seed 20261202), FP32 fields, FP64 Gram solve, grouped launches"
                        % (nreal, n, box, nreal, nmods))
 
 
@@ -418,7 +417,7 @@ def main():
     ap.add_argument("--copy-calibration", action="store_true",
                     help="run only a plain 1 GiB device copy (reference reading for the FETCH_SIZE/WRITE_SIZE counters)")
     ap.add_argument("--batch-only", action="store_true",
-                    help="run only the batching workload (64 constrained 128^3 realisations per HIP graph)")
+                    help="run only the batching workload (64 constrained 128^3 realisations per call)")
     args = ap.parse_args()
     if args.batch_only:
         print(json.dumps(batch_throughput()))

@@ -486,8 +486,9 @@ template <typename T> void level_displacements(gic_context *c, size_t l, bool fo
   fft_z_lpt<T>(psi[0], psi[1], psi[2], q[0], q[1], q[2], X0, true, g.n, g.kmin(), c->st, c->hook());
 }
 
-// io: the differentiable forward map, whose noise has been transformed along z
-// and y into the levels' fields; the displacements also go to its arrays
+// dense: the differentiable forward map, whose noise has been transformed
+// along z and y into the levels' fields; the base level's displacements also
+// go to its first three arrays
 template <typename T> void do_zeldovich(gic_context *c, T *const *dense) {
   if (!c->power_applied) do_apply_ps<T>(c);
   Phase ph(c, "phase:zeldovich");

@@ -52,8 +52,6 @@ void filter_table(int kind, double kc, double kmin, long nent, T *out, hipStream
 template <typename T> void mul_table(T *field, int n, const T *tab, hipStream_t st);
 // sum[m] += |spec_k|^2, cnt[m] += 1 over (ix,iy,iz) in [-N/2,N/2]^3, m = |k_int|^2
 template <typename T> void mode_power(const T *spec, int n, double *sum, double *cnt, hipStream_t st);
-template <typename T>
-void zeldovich(const T *delta, int n, double kmin, T *px, T *py, T *pz, const T *post, hipStream_t st);
 template <typename T> void interp_add(T *fine, int nf, const CoarseView &coarse, const InterpGeom &g, hipStream_t st);
 // transpose of interp_add with the coarse field whole and padded: coarse += I^T fine
 // (fine row stride frs: nf dense, nf+2 padded; tmp: interp_adjoint_bytes of scratch)
@@ -64,8 +62,6 @@ void interp_adjoint(const T *fine, int nf, long frs, T *coarse, const InterpGeom
 template <typename T>
 void particles(const T *px, const T *py, const T *pz, const T *const *psi2, int n, const ParticleGeom &g,
                const uint64_t *cells, size_t start, size_t count, float *pos, float *vel, hipStream_t st);
-// elementwise source accumulation: mode 0 S = A B, 1 S += A B, 2 S -= A A, 3 A += B
-template <typename T> void lpt_accum(T *S, T *A, const T *B, size_t n, int mode, hipStream_t st);
 template <typename T> void fill(T *p, size_t n, T v, hipStream_t st);
 // white noise adjustments: every stored mode to unit modulus; sign flip of the
 // modes with 0 < k^2 < kmax^2; p *= s over n values; out = 1/tab (0 where tab is 0)

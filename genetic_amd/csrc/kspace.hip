@@ -7,8 +7,6 @@
 //                        so one FP64 table indexed by kx^2+ky^2+kz^2 replaces the
 //                        reference's per-mode spline calls and its covariance field.
 //   apply transfer       Field::applyTransferFunction (field/field.hpp:394-412)
-//   Zel'dovich           ZeldovichParticleGenerator::calculateOffsetFields
-//                        (particles/zeldovich.hpp:155-181)
 //   filters              LowPassFermiFilter / ComplementaryCovarianceFilterAdaptor
 //                        (filters/filter.hpp:208-275), applied per mode
 //   level combination    Field::addFieldFromDifferentGrid + evaluateInterpolated
@@ -287,42 +285,6 @@ template <typename T> void mode_power(const T *spec, int n, double *sum, double 
   size_t w = size_t(n) + 1, tot = w * w * w;
   hipLaunchKernelGGL(k_mode_power<T>, dim3((tot + 255) / 256), dim3(256), 0, st,
                      reinterpret_cast<const cx<T> *>(spec), n, sum, cnt);
-  GIC_HIP(hipGetLastError());
-}
-
-// ---- Zel'dovich: psi_j(k) = i k_j delta(k) / k^2 -----------------------------------------
-// Computed in T with k_j = int * kMin as the reference does; the component
-// at k_j = +Nyquist and the k = 0 mode are zero.  An optional table factor
-// (the high-pass filter of a zoom level) is applied to the three outputs.
-template <typename T>
-__global__ void k_zeldovich(const cx<T> *__restrict__ d, int n, T kmin, cx<T> *__restrict__ px,
-                            cx<T> *__restrict__ py, cx<T> *__restrict__ pz, const T *__restrict__ post) {
-  size_t idx = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  size_t nm = size_t(n) * n * (n / 2 + 1);
-  if (idx >= nm) return;
-  int ix, iy, iz;
-  mode_ints(idx, n, ix, iy, iz);
-  T kx = T(ix) * kmin, ky = T(iy) * kmin, kz = T(iz) * kmin;
-  T nyq = T(n / 2) * kmin;
-  T kfft = kx * kx + ky * ky + kz * kz;
-  cx<T> v = d[idx];
-  cx<T> r{-v.y / kfft, v.x / kfft};
-  T f = post ? post[ix * ix + iy * iy + iz * iz] : T(1);
-  cx<T> rx{r.x * kx * f, r.y * kx * f}, ry{r.x * ky * f, r.y * ky * f}, rz{r.x * kz * f, r.y * kz * f};
-  if (kx == nyq || kfft == 0) rx = cx<T>{0, 0};
-  if (ky == nyq || kfft == 0) ry = cx<T>{0, 0};
-  if (kz == nyq || kfft == 0) rz = cx<T>{0, 0};
-  px[idx] = rx;
-  py[idx] = ry;
-  pz[idx] = rz;
-}
-
-template <typename T>
-void zeldovich(const T *delta, int n, double kmin, T *px, T *py, T *pz, const T *post, hipStream_t st) {
-  size_t nm = size_t(n) * n * (n / 2 + 1);
-  hipLaunchKernelGGL(k_zeldovich<T>, dim3((nm + 255) / 256), dim3(256), 0, st, reinterpret_cast<const cx<T> *>(delta),
-                     n, T(kmin), reinterpret_cast<cx<T> *>(px), reinterpret_cast<cx<T> *>(py),
-                     reinterpret_cast<cx<T> *>(pz), post);
   GIC_HIP(hipGetLastError());
 }
 
@@ -615,62 +577,6 @@ void particles(const T *px, const T *py, const T *pz, const T *const *psi2, int 
   GIC_HIP(hipGetLastError());
 }
 
-// ---- second-order source -------------------------------------------------------------
-// elementwise over a padded real field: mode 0 S = A B, 1 S += A B, 2 S -= A A, 3 A += B
-template <typename T>
-__global__ void k_lpt_accum(T *__restrict__ S, T *__restrict__ A, const T *__restrict__ B, size_t n, int mode) {
-  size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  if (mode == 0) S[i] = A[i] * B[i];
-  else if (mode == 1) S[i] += A[i] * B[i];
-  else if (mode == 2) S[i] -= A[i] * A[i];
-  else A[i] += B[i];
-}
-// four consecutive elements per thread (n is a multiple of 4 for even grids)
-template <typename T> struct alignas(4 * sizeof(T)) Vec4 {
-  T v[4];
-};
-template <typename T>
-__global__ void k_lpt_accum4(Vec4<T> *__restrict__ S, Vec4<T> *__restrict__ A, const Vec4<T> *__restrict__ B,
-                             size_t n4, int mode) {
-  size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n4) return;
-  Vec4<T> a = A[i];
-  if (mode == 3) {
-    Vec4<T> b = B[i];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) a.v[k] += b.v[k];
-    A[i] = a;
-    return;
-  }
-  Vec4<T> s;
-  if (mode == 0) {
-    Vec4<T> b = B[i];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) s.v[k] = a.v[k] * b.v[k];
-  } else if (mode == 1) {
-    Vec4<T> b = B[i];
-    s = S[i];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) s.v[k] += a.v[k] * b.v[k];
-  } else {
-    s = S[i];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) s.v[k] -= a.v[k] * a.v[k];
-  }
-  S[i] = s;
-}
-template <typename T> void lpt_accum(T *S, T *A, const T *B, size_t n, int mode, hipStream_t st) {
-  if (n % 4 == 0) {
-    size_t n4 = n / 4;
-    hipLaunchKernelGGL(k_lpt_accum4<T>, dim3((n4 + 255) / 256), dim3(256), 0, st, reinterpret_cast<Vec4<T> *>(S),
-                       reinterpret_cast<Vec4<T> *>(A), reinterpret_cast<const Vec4<T> *>(B), n4, mode);
-  } else {
-    hipLaunchKernelGGL(k_lpt_accum<T>, dim3((n + 255) / 256), dim3(256), 0, st, S, A, B, n, mode);
-  }
-  GIC_HIP(hipGetLastError());
-}
-
 // ---- white-noise adjustments ------------------------------------------------------------
 // enforcePowerSpectrumOneGrid (multilevelfield.hpp:498-510): every mode to
 // unit modulus, keeping its phase (0 stays 0)
@@ -780,13 +686,11 @@ template <typename S, typename D> void convert(const S *a, size_t n, D *b, hipSt
   template void mul_table<T>(T *, int, const T *, hipStream_t);                                               \
   template void mode_power<T>(const T *, int, double *, double *, hipStream_t);                               \
   template void fourier_draw_scatter<T>(const T *, int, T *, uint32_t *, int, hipStream_t);                   \
-  template void zeldovich<T>(const T *, int, double, T *, T *, T *, const T *, hipStream_t);                  \
   template void interp_add<T>(T *, int, const CoarseView &, const InterpGeom &, hipStream_t);                 \
   template size_t interp_adjoint_bytes<T>(int, const InterpGeom &);                                           \
   template void interp_adjoint<T>(const T *, int, long, T *, const InterpGeom &, T *, hipStream_t);           \
   template void particles<T>(const T *, const T *, const T *, const T *const *, int, const ParticleGeom &,    \
                              const uint64_t *, size_t, size_t, float *, float *, hipStream_t);                \
-  template void lpt_accum<T>(T *, T *, const T *, size_t, int, hipStream_t);                                  \
   template void fill<T>(T *, size_t, T, hipStream_t);                                                       \
   template void unit_modulus<T>(T *, int, hipStream_t);                                                     \
   template void reverse_small_k<T>(T *, int, double, double, hipStream_t);                                  \

@@ -54,9 +54,6 @@ void rng_draw_real(const RngPlan &plan, const std::vector<RngLevelOut> &levels, 
 size_t rng_dev_bytes(const RngPlan &plan);
 void rng_dev_pack(const RngPlan &plan, void *host_dst);
 size_t rng_workspace_bytes(const RngPlan &plan);
-// uploads the ziggurat and jump tables (once, synchronously) ahead of draws
-// that a graph records
-void rng_prepare();
 
 // Draws into a caller's device array with the fixed per-device workspace:
 // rng_scratch_setup(device) once per device with that device current, then

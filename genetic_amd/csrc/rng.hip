@@ -1013,7 +1013,6 @@ static void upload_tables() {
   g_tables_done[dev] = true;
 }
 
-void rng_prepare() { upload_tables(); }
 
 // a stream's device copy, written by a kernel from its arguments
 __global__ void k_rng_put_plan(RngDev d, RngDev *__restrict__ dst, uint32_t *__restrict__ flag) {

@@ -352,8 +352,9 @@ class ICGenerator:
         (real-space draws), cons[r, i] = (x, y, z, radius, target) top-hat
         mean-overdensity constraints with absolute targets; out_ptr (device,
         the context's precision) receives delta, psi_x, psi_y, psi_z per
-        realisation as dense n^3 arrays at out + r*4*n^3.  Returns the elapsed
-        milliseconds from the first recorded work to the end of the batch."""
+        realisation as dense n^3 arrays at out + r*4*n^3.  A launch works on a
+        group of at least lanes realisations; graph changes nothing.  Returns
+        the milliseconds from the first device work of the batch to its end."""
         seeds = np.ascontiguousarray(seeds, dtype=np.uint64).ravel()
         cons = np.ascontiguousarray(cons, dtype=np.float64)
         if cons.ndim != 3 or cons.shape[2] != 5 or cons.shape[0] != seeds.size:

@@ -193,10 +193,10 @@ int gic_set_quadratic_line_search(gic_context *ctx, int enable);
  * modificationmanager.hpp:160-312), then the transfer function and the
  * Zel'dovich displacement.  out (device, the context's precision) receives
  * per realisation four dense n^3 arrays: delta, psi_x, psi_y, psi_z at
- * out + r*4*n^3.  lanes (1..16) chains run concurrently on streams of their
- * own; use_graph != 0 records the whole batch into one HIP graph and launches
- * it once.  elapsed_ms (optional) receives the time from the first recorded
- * work to the end of the batch, graph recording included.  The context's own
+ * out + r*4*n^3.  Each launch works on a group of realisations, at least
+ * lanes (1..16) of them where the batch has as many; use_graph is accepted and
+ * changes nothing.  elapsed_ms (optional) receives the time from the first
+ * device work of the batch to its end.  The context's own
  * fields are untouched; no chi^2 is logged. */
 int gic_batch_constrained(gic_context *ctx, int nreal, const uint64_t *seeds, int ncons, const double *cons,
                           void *out, int lanes, int use_graph, double *elapsed_ms);
