@@ -1,35 +1,10 @@
 // Bit-exact parallel ranlxs2 stream and ziggurat Gaussians.
 #pragma once
 #include "gic_common.h"
+#include "rng_plan.h"
 #include <vector>
 
 namespace gic {
-
-// 576-bit numbers as 9 little-endian 64-bit limbs.
-struct U576 {
-  uint64_t w[9];
-};
-
-// One stream of a draw: its seed, the Gaussians wanted, and where the first
-// of them goes, counted in the order of the draw's targets.
-struct RngStream {
-  unsigned long seed;
-  size_t count;
-  size_t out0;
-};
-
-// Host-side set-up of one real-space draw: its streams, the chunk length and
-// how many wavefronts of 64 chunks each stream takes.
-struct RngPlan {
-  std::vector<RngStream> streams;
-  int kclog = 6;                             // log2 of the ranlxs2 blocks (24 numbers) per chunk: 0..6
-  int ch() const { return 24 << kclog; }     // raw numbers per chunk
-  std::vector<long> seg0;                    // each stream's first wavefront
-  long nseg = 0;                             // wavefronts in all
-};
-
-void rng_plan(const std::vector<RngStream> &streams, RngPlan &plan);
-void rng_plan(unsigned long seed, size_t n_gaussians, RngPlan &plan);   // one stream from the start of the targets
 
 // Draw the stream's Gaussians into the listed targets in order, as the
 // reference's serial loop does: a padded real field (n > 0, count n^3, cell
@@ -51,9 +26,6 @@ void rng_draw_real(const RngPlan &plan, const std::vector<RngLevelOut> &levels, 
 // dev_plan: the plan already in device memory (rng_dev_pack'd, rng_dev_bytes
 // long, copied there by the caller); otherwise the call puts it into the
 // workspace.
-size_t rng_dev_bytes(const RngPlan &plan);
-void rng_dev_pack(const RngPlan &plan, void *host_dst);
-size_t rng_workspace_bytes(const RngPlan &plan);
 
 // Draws into a caller's device array with the fixed per-device workspace:
 // rng_scratch_setup(device) once per device with that device current, then
@@ -65,8 +37,5 @@ void rng_gaussians_noalloc(int device, unsigned long seed, double *dev_out, size
 
 // Raw 24-bit stream (testing / bit-exactness checks): the first n numbers.
 void rng_raw(const RngPlan &plan, uint32_t *d_out, size_t n, hipStream_t st);
-
-// Host reference pieces used by tests of the jump arithmetic.
-void u576_mulmod_host(const U576 &a, const U576 &b, U576 &r);
 
 }  // namespace gic
