@@ -214,7 +214,7 @@ GIC_HD inline void decode_state(const uint64_t *V, uint64_t *x) {
 // squarings takes one per bit set in any lane's index).  They depend on
 // neither seed nor size.
 constexpr int RNG_KC_LOG = 7;    // kc = 1 .. 64
-constexpr int RNG_DIGITS = 4;    // 64^4 chunks
+constexpr int RNG_DIGITS = 5;    // 64^5 chunks a stream
 
 // One stream of a draw
 struct RngDev {
@@ -275,7 +275,7 @@ inline void u576_powmod(const uint64_t *base, u128 e_lo, uint64_t *r) {
 }
 
 // The constants of the jumps: b^12 and the device table d_jump, computed
-// once per process (about 1800 modular products)
+// once per process (about 2300 modular products)
 struct JumpTable {
   uint64_t b12[9];
   std::vector<uint64_t> w;   // as d_jump
@@ -367,10 +367,11 @@ inline void rng_plan(const std::vector<RngStream> &streams, RngPlan &plan) {
   plan.nseg = 0;
   for (auto &s : streams) {
     plan.seg0.push_back(plan.nseg);
-    long chunks = long(raw_needed(s.count) / plan.ch()) + 2;
-    plan.nseg += (chunks + 63) / 64;
+    // (the jump tables reach a chunk from its own stream's start)
+    const double chunks = raw_needed(s.count) / plan.ch() + 2;
+    if (chunks > double(1L << (6 * RNG_DIGITS)) - 64) throw std::runtime_error("RNG: stream too long");
+    plan.nseg += (long(chunks) + 63) / 64;
   }
-  if (plan.nseg > (1L << (6 * (RNG_DIGITS - 1)))) throw std::runtime_error("RNG: draw too large");
 }
 inline void rng_plan(unsigned long seed, size_t n_gaussians, RngPlan &plan) {
   rng_plan(std::vector<RngStream>{{seed, n_gaussians, 0}}, plan);

@@ -1,5 +1,5 @@
 // Plans of draws read from standard input, one a line: "nseeds seed count ...";
-// per plan and stream the first chunks' states are printed.  Built with the
+// per plan the first and last streams' chunk states are printed.  Built with the
 // host's sanitizers by test_cpu_rng_plan.py: the packed plan lies in an array
 // of exactly rng_dev_bytes.
 #include "../genetic_amd/csrc/rng_plan.h"
@@ -61,6 +61,7 @@ int main() {
       if (n > 1)
         for (uint64_t k = 0; k < d[i].nseg; ++k) must(of[seg + k] == uint32_t(i), "seg_stream");
       seg += d[i].nseg;
+      if (i >= 40 && i < n - 12) continue;
       const long last = long(d[i].nseg) * 64 - 1;
       for (long t : {1l, last / 2, last}) {
         uint64_t x[12], c;

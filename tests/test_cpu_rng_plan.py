@@ -49,3 +49,18 @@ def test_plans_pack_within_their_bytes(check):
         v = [int(x) for x in s.split()[1:]]
         want = po.ranlxs_raw_from_state(*rj.state_at_block(v[0], v[1]), 48)
         assert np.array_equal(po.ranlxs_raw_from_state(v[3:], v[2], 48), want), s
+
+
+@pytest.mark.parametrize("streams", [[(s, 16 ** 3) for s in range(1, 262146)],    # a wavefront of chunks each
+                                     [(s, 128 ** 3) for s in range(1, 5601)],
+                                     [(77, 12 * 10 ** 9)]])
+def test_reach_is_each_streams_own(check, streams):
+    """The jump tables reach a chunk of its own stream: draws of any number of
+    streams are planned, and a stream of more Gaussians than four base-64
+    digits of chunks hold; the furthest chunks are where the stream is."""
+    out = check(streams)
+    assert int(out[0].split()[2]) >= 262145
+    for s in out[1:4] + out[-3:]:
+        v = [int(x) for x in s.split()[1:]]
+        want = po.ranlxs_raw_from_state(*rj.state_at_block(v[0], v[1]), 48)
+        assert np.array_equal(po.ranlxs_raw_from_state(v[3:], v[2], 48), want), s
