@@ -149,7 +149,7 @@ __device__ __forceinline__ int gram_slot(int i, int j) {
 // k of a 16 x 16 x 4 product, the same registers serving as both operands (A
 // times the weight).  A wavefront's loads are whole 64-byte pieces of each
 // covector, so nothing goes through LDS.  Block b of the grid writes the
-// products in gram_slot's order (0 where there is none) at part[b nw 16].
+// products in gram_slot's order (0 where there is none) to its own piece of part.
 //
 // It is bound by reading the covectors: 8 realisations of 16 at 128^3 FP32,
 // 1.16 GB, 298 us (3.9 TB/s); with tiles of 4 x 4 products in vector registers,
@@ -395,7 +395,7 @@ template <typename T> __global__ void k_batch_dc(cx<T> *__restrict__ w, long fs,
 // Device memory of a batch's groups, kept for the next call
 struct BatchState {
   DevBuf cons, flags, win, plans, rng_ws;
-  DevBuf w, cov, x, part, sums, cnt, coef;
+  DevBuf w, cov, part, sums, cnt, coef;
   DevBuf rows, zbuf, ybuf;   // covectors from the constraints' boxes
 };
 
@@ -403,6 +403,12 @@ struct BatchState {
 // more than GROUP_BYTES; at least the concurrency the caller asks for.
 constexpr int GROUP_MAX = 16;
 constexpr double GROUP_BYTES = 192e6;
+// A realisation's fields in the groups' buffers: its noise, and the
+// covectors, over which the four fields of its output are made.
+static int batch_fields(int ncons) { return 1 + std::max(ncons, 4); }
+// Wavefronts of a draw (240 MB of chunk states, 32 for every SIMD); more
+// realisations than they hold are drawn one part after the other.
+constexpr long DRAW_SEGS = 32768;
 
 template <typename T>
 void do_batch(gic_context *c, int nreal, const uint64_t *seeds, int ncons, const double *cons, T *out, int nlanes,
@@ -435,13 +441,26 @@ void do_batch(gic_context *c, int nreal, const uint64_t *seeds, int ncons, const
   build_sqrtp_dm<T>(c, L);
   if (!c->batch) c->batch = std::make_shared<BatchState>();
   BatchState &B = *c->batch;
-  // one draw of every realisation's stream: each goes, dense, into the first
-  // of its output arrays, which its transform reads
-  std::vector<RngStream> streams;
-  for (int r = 0; r < nreal; ++r) streams.push_back({(unsigned long)seeds[r], n3, size_t(r) * 4 * n3});
-  RngPlan plan;
-  rng_plan(streams, plan);
-  B.rng_ws.ensure(rng_workspace_bytes(plan));
+  // The realisations' streams, in as few draws as DRAW_SEGS allows: each goes,
+  // dense, into the first of its output arrays, which its transform reads.
+  auto plan_of = [&](int r0, int k) {
+    std::vector<RngStream> streams;
+    for (int r = r0; r < r0 + k; ++r) streams.push_back({(unsigned long)seeds[r], n3, size_t(r) * 4 * n3});
+    RngPlan p;
+    rng_plan(streams, p);
+    return p;
+  };
+  std::vector<RngPlan> draws{plan_of(0, nreal)};
+  if (draws[0].nseg > DRAW_SEGS) {
+    const int k = std::max(1, int(double(nreal) * DRAW_SEGS / double(draws[0].nseg)));
+    draws.clear();
+    for (int r = 0; r < nreal; r += k) draws.push_back(plan_of(r, std::min(k, nreal - r)));
+  }
+  std::vector<size_t> plan_at(1, 0);
+  for (auto &p : draws) {
+    B.rng_ws.ensure(rng_workspace_bytes(p));
+    plan_at.push_back(plan_at.back() + rng_dev_bytes(p));
+  }
   // boxes around the spheres: x, y windows of wl cells from
   // floor((c - o - R)/dx - 1/2) (mod n), which hold every selected cell
   int wl = 0;
@@ -451,7 +470,10 @@ void do_batch(gic_context *c, int nreal, const uint64_t *seeds, int ncons, const
   }
   // (the row kernel indexes rows x n values in 32 bits)
   const bool boxes = wl < n && (double(ncons) * wl * wl + 1024.0) * n < 2e9;
-  int group = std::max(nlanes, std::min(GROUP_MAX, int(GROUP_BYTES / (double(ncons) * fs_reals * sizeof(T)))));
+  // (with fewer than four constraints the output's fields decide: no more
+  // memory than ncons + 3 fields for each of the caller's lanes)
+  const int lanes = std::max(1, std::min(nlanes, nlanes * (ncons + 3) / batch_fields(ncons)));
+  int group = std::max(lanes, std::min(GROUP_MAX, int(GROUP_BYTES / (double(ncons) * fs_reals * sizeof(T)))));
   group = std::min(group, nreal);
   if (boxes) group = std::min(group, int(2e9 / ((double(ncons) * wl * wl + 1024.0) * n)));
   auto nrows_of = [&](int k) { return boxes ? long(k) * ncons * wl * wl : 0; };
@@ -471,8 +493,7 @@ void do_batch(gic_context *c, int nreal, const uint64_t *seeds, int ncons, const
     B.ybuf.ensure(size_t(group) * ncons * wl * n * (n + 2) * sizeof(T));
   }
   B.w.ensure(size_t(group) * fs_reals * sizeof(T));
-  B.cov.ensure(size_t(group) * ncons * fs_reals * sizeof(T));
-  B.x.ensure(size_t(group) * 4 * fs_reals * sizeof(T));
+  B.cov.ensure(size_t(group) * (batch_fields(ncons) - 1) * fs_reals * sizeof(T));
   B.part.ensure(size_t(group) * GRAM_BLOCKS * np * sizeof(double));
   B.sums.ensure(size_t(group) * np * sizeof(double));
   B.cnt.ensure(size_t(group) * ncons * sizeof(uint32_t));
@@ -485,8 +506,8 @@ void do_batch(gic_context *c, int nreal, const uint64_t *seeds, int ncons, const
     GIC_HIP(hipMemcpyAsync(B.win.p, win.data(), win.size() * sizeof(int), hipMemcpyHostToDevice, c->st));
   }
   fill<uint32_t>((uint32_t *)B.flags.p, size_t(nreal), 0u, c->st);
-  std::vector<char> hplan(rng_dev_bytes(plan), 0);
-  rng_dev_pack(plan, hplan.data());
+  std::vector<char> hplan(plan_at.back(), 0);
+  for (size_t i = 0; i < draws.size(); ++i) rng_dev_pack(draws[i], hplan.data() + plan_at[i]);
   B.plans.ensure(hplan.size());
   GIC_HIP(hipMemcpyAsync(B.plans.p, hplan.data(), hplan.size(), hipMemcpyHostToDevice, c->st));
 
@@ -494,8 +515,12 @@ void do_batch(gic_context *c, int nreal, const uint64_t *seeds, int ncons, const
   TimingHook *hook = c->hook();
   const double *dcons = (const double *)B.cons.p;
   uint32_t *dflags = (uint32_t *)B.flags.p;
-  rng_draw_real<T>(plan, {{out, 0, size_t(nreal) * 4 * n3}}, B.rng_ws.p, B.rng_ws.bytes, st, hook, 1.0, dflags, 1,
-                   B.plans.p);
+  size_t drawn = 0;
+  for (size_t i = 0; i < draws.size(); ++i) {
+    rng_draw_real<T>(draws[i], {{out, 0, size_t(nreal) * 4 * n3}}, B.rng_ws.p, B.rng_ws.bytes, st, hook, 1.0,
+                     dflags + drawn, 1, (const char *)B.plans.p + plan_at[i]);
+    drawn += draws[i].streams.size();
+  }
   for (int r0 = 0; r0 < nreal; r0 += group) {
     const int nb = std::min(group, nreal - r0), nc = nb * ncons;
     T *w = (T *)B.w.p, *cv = (T *)B.cov.p, *o = out + size_t(r0) * 4 * n3;
@@ -554,7 +579,7 @@ void do_batch(gic_context *c, int nreal, const uint64_t *seeds, int ncons, const
                        (const double *)B.coef.p, (const T *)L.sqrtp.p, n);
     GIC_HIP(hipGetLastError());
     // delta and the Zel'dovich displacements, dense, into the caller's arrays
-    T *X = (T *)B.x.p;   // per realisation: of delta, delta/k^2 and i k_x delta/k^2, and one more
+    T *X = cv;   // per realisation: of delta, delta/k^2 and i k_x delta/k^2, and one more
     FftX<T> x;
     x.in = w;
     x.in_bs = fs_reals;

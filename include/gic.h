@@ -194,7 +194,8 @@ int gic_set_quadratic_line_search(gic_context *ctx, int enable);
  * Zel'dovich displacement.  out (device, the context's precision) receives
  * per realisation four dense n^3 arrays: delta, psi_x, psi_y, psi_z at
  * out + r*4*n^3.  Each launch works on a group of realisations, at least
- * lanes (1..16) of them where the batch has as many; use_graph is accepted and
+ * lanes (1..16) of them where the batch has as many (a fifth fewer with a
+ * single constraint); use_graph is accepted and
  * changes nothing.  elapsed_ms (optional) receives the time from the first
  * device work of the batch to its end.  The context's own
  * fields are untouched; no chi^2 is logged. */

@@ -140,3 +140,31 @@ def test_batch_large_spheres_match_one_at_a_time():
             np.testing.assert_allclose(got[r, f], want[f], atol=1e-9 * np.abs(want[f]).max(),
                                        err_msg="realisation %d field %d" % (r, f))
     ic.close()
+
+
+def test_many_small_realisations_in_bounded_memory():
+    """More wavefronts of streams than one draw takes: the realisations are
+    drawn in parts, the workspace stays that of one part (240 MB of chunk
+    states where all at once would take 740), and each realisation is the one
+    that its seed gives alone."""
+    import torch
+    n, nreal = 4, 100_000
+    print("batch of many", n, nreal, flush=True)
+    ic = _ctx(gic.FLOAT32, n)
+    cons = np.empty((nreal, 1, 5))
+    rng = np.random.default_rng(2)
+    cons[..., :3] = rng.uniform(0, BOX, (nreal, 1, 3))
+    cons[..., 3] = 15.0   # some cell's centroid is nearer than 12.5 sqrt(3) / 2
+    cons[..., 4] = rng.normal(0, 0.1, (nreal, 1))
+    out = torch.full((nreal, 4, n, n, n), float("nan"), dtype=torch.float32, device="cuda")
+    seeds = np.arange(1, nreal + 1)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    ic.batch_constrained(seeds, cons, out.data_ptr(), lanes=1)
+    assert free - torch.cuda.mem_get_info()[0] < 400e6
+    assert torch.isfinite(out).all()
+    one = torch.empty((1, 4, n, n, n), dtype=torch.float32, device="cuda")
+    for r in [0, 15, 16, 32767, 32768, 49_999, 65_536, 98_304, nreal - 1]:
+        ic.batch_constrained(seeds[r:r + 1], cons[r:r + 1], one.data_ptr())
+        assert torch.equal(one[0], out[r]), r
+    ic.close()
