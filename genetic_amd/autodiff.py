@@ -66,25 +66,47 @@ def displacement(gen, *noise):
     return [tuple(psi[3 * l:3 * l + 3]) for l in range(len(noise))]
 
 
+class _Gradient(torch.autograd.Function):
+    """A gradient that the library returned beside its value, as a function of
+    the noise: it depends on it, but has no derivative here."""
+
+    @staticmethod
+    def forward(ctx, grad, *noise):
+        return grad.view_as(grad)
+
+    @staticmethod
+    def backward(ctx, *_):
+        raise RuntimeError("no second derivatives with respect to the noise")
+
+
+def _times(ctx, grads, grad_v):
+    """The backward of a scalar whose gradients are saved.  Under create_graph
+    they are tied to the noise, so that a derivative of them is refused where
+    torch would take them for constants."""
+    if torch.is_grad_enabled():
+        grads = [_Gradient.apply(g, *ctx.noise) for g in grads]
+    return [g * grad_v.to(g.dtype) for g in grads]
+
+
 class MaskedSquares(torch.autograd.Function):
     """sum over the cells of a bool mask of |psi(w)|^2 on one level, a float64
     scalar.  Only the displacements of the mask's box are formed."""
 
     @staticmethod
-    def forward(ctx, gen, noise, mask):
-        noise, mask = noise.contiguous(), mask.contiguous()
+    def forward(ctx, gen, inp, mask):
+        noise, mask = inp.contiguous(), mask.contiguous()
         _check_levels(gen, (noise,), "displacement")
         grad = torch.empty_like(noise) if ctx.needs_input_grad[1] else None
         torch.cuda.current_stream().synchronize()
         v = gen.masked_displacement(noise.data_ptr(), mask.data_ptr(), None if grad is None else grad.data_ptr())
         if grad is not None:
             ctx.save_for_backward(grad)
+            ctx.noise = (inp,)
         return torch.tensor(v, dtype=torch.float64, device=noise.device)
 
     @staticmethod
     def backward(ctx, grad_v):
-        grad, = ctx.saved_tensors
-        return None, grad * grad_v.to(grad.dtype), None
+        return (None, *_times(ctx, ctx.saved_tensors, grad_v), None)
 
 
 class FilteredVariance(torch.autograd.Function):
@@ -92,20 +114,20 @@ class FilteredVariance(torch.autograd.Function):
     the context's filtering_scale) as a float64 scalar; d V / d w = 2 Q w."""
 
     @staticmethod
-    def forward(ctx, gen, *noise):
-        noise = [t.contiguous() for t in noise]
+    def forward(ctx, gen, *inp):
+        noise = [t.contiguous() for t in inp]
         _check_levels(gen, noise, "variance")
         grads = [torch.empty_like(t) for t in noise] if any(ctx.needs_input_grad[1:]) else None
         torch.cuda.current_stream().synchronize()
         v = gen.variance_gradient([t.data_ptr() for t in noise], grads and [g.data_ptr() for g in grads])
         if grads:
             ctx.save_for_backward(*grads)
+            ctx.noise = inp
         return torch.tensor(v, dtype=torch.float64, device=noise[0].device)
 
     @staticmethod
     def backward(ctx, grad_v):
-        grads = ctx.saved_tensors
-        return (None, *[g * grad_v.to(g.dtype) for g in grads])
+        return (None, *_times(ctx, ctx.saved_tensors, grad_v))
 
 
 def filtered_variance(gen, *noise):
