@@ -50,3 +50,17 @@ def test_one_cpu_and_pinned_memory(done):
     pinned = [torch.empty((128 ** 3, 3), dtype=torch.float32, pin_memory=True) for _ in range(2)]
     g._check(gic.lib().gic_particles(g._h, 0, None, 0, 128 ** 3, pinned[0].data_ptr(), pinned[1].data_ptr()))
     assert np.array_equal(pinned[0].numpy(), pos) and np.array_equal(pinned[1].numpy(), vel)
+
+
+@pytest.mark.parametrize("offset", [1, 3, 4, 8, 17])
+def test_arrays_of_any_alignment(done, offset):
+    """A level's field into an array that starts anywhere in memory."""
+    print("host copy to offset", offset, flush=True)
+    g = done[0]
+    n3 = 128 ** 3
+    want = g.field(gic.FIELD_PSI_X, 0, dtype=np.float32).ravel()
+    raw = np.full(4 * n3 + 4096, 0x5A, dtype=np.uint8)
+    at = -raw.ctypes.data % 2048 + offset
+    g._check(gic.lib().gic_copy_field(g._h, gic.FIELD_PSI_X, 0, gic.REAL_SPACE, raw.ctypes.data + at, gic.DTYPE_F32))
+    assert raw[at:at + 4 * n3].tobytes() == want.tobytes()
+    assert (raw[:at] == 0x5A).all() and (raw[at + 4 * n3:] == 0x5A).all()
