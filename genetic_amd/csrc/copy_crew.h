@@ -8,7 +8,6 @@
 #include <cstddef>
 #include <cstdint>
 #include <cstring>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -47,10 +46,11 @@ template <class Thread = std::thread> class CopyCrew {
     cpu_set_t set;
     if (sched_getaffinity(0, sizeof set, &set) == 0) n_ = std::max(1, std::min(n_, CPU_COUNT(&set)));
     for (auto &d : done_) d.store(0);
+    threads_.reserve(size_t(n_));   // (once threads run, nothing here may throw)
     for (int t = 0; t < n_; ++t) {
       try {
         threads_.emplace_back([this, t] { work(size_t(t)); });
-      } catch (const std::system_error &) {
+      } catch (...) {
         own_ |= 1u << t;   // without its thread the caller copies the slot's pieces (filled)
       }
     }

@@ -5,10 +5,25 @@
 #include "../genetic_amd/csrc/copy_crew.h"
 #include <cstdio>
 #include <cstdlib>
+#include <new>
 
 using namespace gic;
 
 constexpr size_t SLOT = 1 << 16;
+
+// a thread that may not be had
+static int refuse = 0;
+struct Scarce : std::thread {
+  template <class F> explicit Scarce(F f) : std::thread(start(std::move(f))) {}
+  template <class F> static std::thread start(F f) {
+    if (refuse & 1) {
+      refuse >>= 1;
+      throw std::bad_alloc();
+    }
+    refuse >>= 1;
+    return std::thread(std::move(f));
+  }
+};
 
 template <class Crew> static void copy(const std::vector<CopyPart> &parts) {
   const std::vector<CopyPart> pieces = copy_pieces(parts, SLOT);
@@ -29,6 +44,7 @@ int main() {
     std::vector<CopyPart> parts;
     std::vector<std::vector<char>> src, dst;
     char *s = line, *e;
+    int mode = int(std::strtol(s, &s, 10));
     for (;;) {
       const size_t bytes = std::strtoul(s, &e, 10);
       if (e == s) break;
@@ -40,7 +56,9 @@ int main() {
       d += (SLOT - reinterpret_cast<uintptr_t>(d) % SLOT) % SLOT + align;
       parts.push_back({d, src.back().data(), bytes});
     }
-    copy<CopyCrew<>>(parts);
+    refuse = mode;
+    if (mode) copy<CopyCrew<Scarce>>(parts);
+    else copy<CopyCrew<>>(parts);
     for (size_t p = 0; p < parts.size(); ++p)
       if (memcmp(parts[p].dst, parts[p].src, parts[p].bytes) != 0 ||
           ((const char *)parts[p].dst)[parts[p].bytes] != char(0x5a)) {

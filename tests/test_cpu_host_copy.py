@@ -1,6 +1,6 @@
 """The host's part of copies through pinned slots (copy_crew.h) without a GPU,
 under the host's sanitizers: every byte arrives, once, for arrays of any size
-and alignment, on one CPU too."""
+and alignment, on one CPU and with fewer threads than asked for."""
 import os
 import subprocess
 
@@ -24,9 +24,9 @@ def check(request, tmp_path_factory):
 
 
 # arrays of floats or doubles, their first byte anywhere in a page
-CASES = ["%d %d" % (b, a) for b in (4, SLOT - 4, SLOT, 5 * SLOT + 12, 40 * SLOT + 8)
+CASES = ["0 %d %d" % (b, a) for b in (4, SLOT - 4, SLOT, 5 * SLOT + 12, 40 * SLOT + 8)
          for a in (0, 1, 3, 4, 15, 16, 4097, SLOT - 15, SLOT - 1)]
-CASES += ["%d 1 %d 2 %d 0" % (3 * SLOT + 4, 9 * SLOT + 20, 12)]
+CASES += ["0 %d 1 %d 2 %d 0" % (3 * SLOT + 4, 9 * SLOT + 20, 12)]
 
 
 def test_any_size_and_alignment(check):
@@ -35,3 +35,9 @@ def test_any_size_and_alignment(check):
 
 def test_one_cpu(check):
     check(*CASES, cpus={min(os.sched_getaffinity(0))})
+
+
+@pytest.mark.parametrize("refused", [1, 2, 0x80, 0x5A, 0xFF])   # a bit for each thread
+def test_threads_that_cannot_be_had(check, refused):
+    """Whatever starting a thread throws, the caller does its share."""
+    check(*["%d%s" % (refused, c[1:]) for c in CASES[::4]])
