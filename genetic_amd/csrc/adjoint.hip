@@ -114,6 +114,33 @@ void check_ready(gic_context *c) {
   if (!c->have_camb) throw std::runtime_error("No power spectrum has been set (use the camb command)");
 }
 
+// The context's noise while a caller's takes its place: from the construction
+// on there is none, until done() says that the overdensity is the new one.  An
+// exception in between (no memory for a scratch array, say) leaves a context
+// that has to draw again, not one whose half-made field passes for a spectrum.
+class Replacing {
+ public:
+  explicit Replacing(gic_context *c) : c_(c) { none(); }
+  Replacing(const Replacing &) = delete;
+  Replacing &operator=(const Replacing &) = delete;
+  ~Replacing() {
+    if (!done_) none();
+  }
+  void done(bool zeldovich) {
+    done_ = true;
+    c_->seeded = c_->drawn = c_->power_applied = true;
+    c_->zeldovich_done = zeldovich;
+  }
+
+ private:
+  void none() {
+    c_->drawn = c_->power_applied = c_->zeldovich_done = false;
+    for (auto &L : c_->levels) L->noise_fourier = L->dc_pending = L->psi_fourier = L->have_psi = L->have_psi2 = false;
+  }
+  gic_context *c_;
+  bool done_ = false;
+};
+
 // L.noise <- the dense white noise transformed along z and y
 template <typename T> void load_noise_zy(gic_context *c, Level &L, const T *noise) {
   alloc_field(c, L.noise, L.g);
@@ -124,7 +151,6 @@ template <typename T> void load_noise_zy(gic_context *c, Level &L, const T *nois
   FftYFwd<T> y;
   y.add((const T *)L.noise.p, nullptr, (T *)L.noise.p);
   fft_y_forward<T>(y, L.g.n, c->st, c->hook());
-  L.have_psi = L.have_psi2 = false;
 }
 
 }  // namespace
@@ -138,8 +164,9 @@ template <typename T> void do_displacement_forward(gic_context *c, const T *cons
   // the noise along z and y, read straight from the caller's dense arrays;
   // the x pass of do_zeldovich makes delta_l = sqrtP r2c(w_l) and what the
   // displacements need of it
+  Replacing field(c);
   for (size_t l = 0; l < nl; ++l) load_noise_zy<T>(c, *c->levels[l], noise[l]);
-  c->seeded = c->drawn = c->power_applied = true;
+  c->drawn = c->power_applied = true;
   int order = c->lpt_order;
   c->lpt_order = 1;
   try {
@@ -149,7 +176,7 @@ template <typename T> void do_displacement_forward(gic_context *c, const T *cons
     throw;
   }
   c->lpt_order = order;
-  c->zeldovich_done = nl > 1;
+  field.done(nl > 1);
   for (size_t l = 1; l < nl; ++l) {
     Level &L = *c->levels[l];
     for (int a = 0; a < 3; ++a) unpad<T, T>((const T *)L.psi[a].p, L.g.n, psi[3 * l + a], c->st);
@@ -290,9 +317,8 @@ double do_masked_displacement(gic_context *c, const T *noise, const uint8_t *mas
       if (wl[d] == 0) wl[d] = 1;   // an empty mask: one cell, of weight 0
     }
   }
+  Replacing field(c);
   load_noise_zy<T>(c, L, noise);
-  c->seeded = c->drawn = c->power_applied = true;
-  c->zeldovich_done = false;
   // planes: f m and i k_x f m of the box's x; rows: of its x and y; the box
   const size_t planes = size_t(wl[0]) * n * nz * 2, rows = size_t(wl[0]) * wl[1] * nz * 2;
   const size_t nb = size_t(wl[0]) * wl[1] * wl[2];
@@ -311,8 +337,7 @@ double do_masked_displacement(gic_context *c, const T *noise, const uint8_t *mas
   x.wlen = wl[0];
   fft_x<T>(x, n, c->st, c->hook());
   L.noise_fourier = true;
-  L.dc_pending = false;
-  L.psi_fourier = false;
+  field.done(false);
   FftY<T> y;
   y.kmin = L.g.kmin();
   y.nouter = wl[0];

@@ -21,7 +21,9 @@ template <typename C> __device__ __host__ inline C csub(C a, C b) { return C{a.x
 template <typename C> __device__ __host__ inline C cconj(C a) { return C{a.x, -a.y}; }
 
 inline void hip_check(hipError_t e, const char *what) {
-  if (e != hipSuccess) throw std::runtime_error(std::string(what) + ": " + hipGetErrorString(e));
+  if (e == hipSuccess) return;
+  (void)hipGetLastError();   // or the next launch's check would find this error
+  throw std::runtime_error(std::string(what) + ": " + hipGetErrorString(e));
 }
 #define GIC_HIP(x) ::gic::hip_check((x), #x)
 
