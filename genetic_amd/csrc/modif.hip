@@ -548,6 +548,16 @@ __global__ void k_box_mask(const uint64_t *__restrict__ idx, size_t m, int n, in
   z += z < 0 ? n : 0;
   mask[(size_t(x) * by + y) * bz + z] = 1;
 }
+// the y and z with a listed cell (used: n bytes of each; set ones are left alone,
+// so that cells by the million do not all store to the same few lines)
+__global__ void k_list_axes(const uint64_t *__restrict__ idx, size_t m, int n, uint8_t *__restrict__ used) {
+  size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= m) return;
+  const uint64_t c = idx[i], r = c / uint64_t(n);
+  uint8_t *y = used + r % uint64_t(n), *z = used + n + c % uint64_t(n);
+  if (!*y) *y = 1;
+  if (!*z) *z = 1;
+}
 template <typename T>
 __global__ void k_box_keep(T *__restrict__ f, const uint8_t *__restrict__ mask, size_t n, T *__restrict__ copy) {
   size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -1656,25 +1666,45 @@ template <typename T> struct VarianceBox {
   // cut passes' scratch would exceed a field's (256^3 FP32, 14000 cells, value
   // and gradient: a box of 31 cells a side 0.50 ms, of 128 0.51 ms, of 129 and
   // more 1.30 ms with full transforms)
+  // The list is sorted (gic_set_flags).  Its planes are found by bisection, so
+  // that a set which spans too many is known without a look at each cell; up to
+  // HOST_CELLS the other axes are marked here, more cells (1.7 ns each) take the
+  // device and a read-back.  256^3 FP32, 8.5e6 cells of 129 planes: 3.9 ms for
+  // value and gradient, 18.4 with a pass over the list on the host for each try.
+  static constexpr size_t HOST_CELLS = 16384;
   bool make(gic_context *cc, size_t level, const std::vector<uint64_t> &idx) {
     c = cc;
     l = level;
     const LevelGeom &g = c->levels[l]->g;
-    const uint64_t n = uint64_t(g.n), n3 = g.n3();
-    if (idx.empty()) return false;
+    const uint64_t n = uint64_t(g.n), nn = n * n;
+    if (idx.empty() || idx.back() >= g.n3()) return false;
     std::vector<uint8_t> member(3 * n, 0);
-    uint8_t *mx = member.data(), *my = mx + n, *mz = my + n;
-    const bool pow2 = (n & (n - 1)) == 0;
-    const int sh = __builtin_ctzll(n);
-    for (uint64_t i : idx) {
-      if (i >= n3) return false;
-      const uint64_t r = pow2 ? i >> sh : i / n, x = pow2 ? r >> sh : r / n;
-      mx[x] = my[r - x * n] = mz[i - r * n] = 1;
+    uint64_t planes = 0;
+    for (size_t i = 0; i < idx.size();) {
+      const uint64_t x = idx[i] / nn;
+      member[x] = 1;
+      if (++planes > n / 2) return false;
+      const size_t end = std::min(idx.size(), i + size_t(nn));
+      i = size_t(std::lower_bound(idx.begin() + long(i), idx.begin() + long(end), (x + 1) * nn) - idx.begin());
     }
-    for (int d = 0; d < 3; ++d) cyclic_hull(member.data() + d * n, g.n, B.b0[d], B.bl[d]);
+    cyclic_hull(member.data(), g.n, B.b0[0], B.bl[0]);
     if (B.bl[0] > int(n) / 2) return false;
-    nb = box_cells(B);
     upload_list(c, idx, cells);
+    uint8_t *yz = member.data() + n;
+    if (idx.size() <= HOST_CELLS) {
+      const int sh = __builtin_ctzll(n);   // n is a power of two
+      for (uint64_t i : idx) yz[(i >> sh) & (n - 1)] = yz[n + (i & (n - 1))] = 1;
+    } else {
+      PBuf used(c->mod->pool, 2 * n);
+      fill<uint8_t>((uint8_t *)used.p, 2 * n, 0, c->st);
+      hipLaunchKernelGGL(k_list_axes, dim3(blocks(cells.n)), dim3(256), 0, c->st, (const uint64_t *)cells.idx.p,
+                         cells.n, g.n, (uint8_t *)used.p);
+      GIC_HIP(hipGetLastError());
+      GIC_HIP(hipMemcpyAsync(yz, used.p, 2 * n, hipMemcpyDeviceToHost, c->st));
+      GIC_HIP(hipStreamSynchronize(c->st));
+    }
+    for (int d = 1; d < 3; ++d) cyclic_hull(member.data() + d * n, g.n, B.b0[d], B.bl[d]);
+    nb = box_cells(B);
     mask = PBuf(c->mod->pool, nb);
     fill<uint8_t>((uint8_t *)mask.p, nb, 0, c->st);
     hipLaunchKernelGGL(k_box_mask, dim3(blocks(cells.n)), dim3(256), 0, c->st, (const uint64_t *)cells.idx.p, cells.n,

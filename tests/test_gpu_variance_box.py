@@ -91,3 +91,31 @@ def test_gradient_belongs_to_the_value(name, precision, tol):
     assert abs((vp - vm) - 2 * float((grad.double() * d.double()).sum())) <= tol * (vp + vm + v0)
     # and V(w) = <dV/dw, w> / 2
     assert abs(v0 - 0.5 * float((grad.double() * w.double()).sum())) <= tol * v0
+
+
+def _many_cells(name, n):
+    x, y, z = np.meshgrid(*[np.arange(n)] * 3, indexing="ij")
+    dx, dy, dz = (np.minimum((q - c) % n, (c - q) % n) for q, c in ((x, 1), (y, 30), (z, 60)))
+    m = {"ellipsoid": (dx / 15) ** 2 + (dy / 20) ** 2 + (dz / 20) ** 2 <= 1,
+         "wrapped slab": ((x >= 50) | (x < 10)) & (y != 4) & (z > 2),
+         "planes apart": (x % 16 == 3) & (y < 50),
+         "half": (x >= 32) & (y % 5 == 2),
+         "past half": x >= 31}[name]
+    return np.flatnonzero(m.ravel()).astype(np.uint64)
+
+
+@pytest.mark.parametrize("name", ["ellipsoid", "wrapped slab", "planes apart", "half", "past half"])
+def test_variance_of_many_cells_matches_oracle(name):
+    """Sets whose axes are marked on the device, and two that span too many
+    planes."""
+    print("variance of many cells", name, flush=True)
+    n, cells = 64, _many_cells(name, 64)
+    assert cells.size > 16384 or name == "planes apart"
+    ic, o = _gpu([(BOX, n)], gic.FLOAT64), _oracle([(BOX, n)])
+    for g in (ic, o):
+        (g.set_seed if g is ic else g.seed)(77)
+        g.set_flags(0, cells)
+    ic.set_variance_filter_scale(SCALE)
+    o.set_variance_scale(SCALE)
+    want = o.calculate("variance")
+    assert abs(ic.calculate("variance") - want) <= 1e-11 * abs(want)
