@@ -28,8 +28,9 @@ def done():
     return g, np.concatenate([p[0] for p in parts]), np.concatenate([p[1] for p in parts])
 
 
-# bytes of one array: just past two slots in all, an odd remainder, the level
-@pytest.mark.parametrize("start,count", [(0, 174763), (12345, 700001), (1, 128 ** 3 - 1), (0, 128 ** 3)])
+# just past two slots in all, the last that is copied straight and the next (24 bytes
+# a particle, 7 MB), an odd remainder, the level
+@pytest.mark.parametrize("start,count", [(0, 174763), (3, 305834), (3, 305835), (12345, 700001), (1, 128 ** 3 - 1), (0, 128 ** 3)])
 def test_particles_in_slots_equal_direct_copies(done, start, count):
     print("host copy of", count, "particles", flush=True)
     g, pos, vel = done
