@@ -4,7 +4,7 @@ to the oracle and the reference fixtures: reseed, draw, select_sphere +
 modify overdensity (absolute) per constraint, apply_modifications,
 apply_power_spectrum, zeldovich (ic.hpp:1458-1500,1613-1648).  Tolerances:
 FP64 1e-9 and FP32 2e-4 of each field's largest value; repeated batches,
-with or without a graph and on any number of chains, are bit-identical."""
+in groups of any size, are bit-identical."""
 import numpy as np
 import pytest
 
@@ -76,7 +76,9 @@ def test_batch_matches_one_at_a_time(precision, tol):
     ic.close()
 
 
-def test_batch_graph_and_chains_are_bit_identical():
+def test_batch_repeats_are_bit_identical():
+    """Whatever lanes and graph (which changes nothing) say, after other work
+    of the context and for other seeds in the same buffers."""
     import torch
     n, seeds = 64, [3, 1, 4, 1, 5]
     print("batch determinism", n, seeds, flush=True)
@@ -84,14 +86,14 @@ def test_batch_graph_and_chains_are_bit_identical():
     ic = _ctx(gic.FLOAT32, n)
     a = _batch(ic, n, seeds, cons, torch.float32, lanes=1, graph=False)
     b = _batch(ic, n, seeds, cons, torch.float32, lanes=3, graph=True)
-    # eager work on the context between two recorded batches
+    # other work of the context between two batches
     ic.reseed(9)
     ic.draw()
     ic.apply_power_spectrum()
     c = _batch(ic, n, seeds[:2], cons[:2], torch.float32, lanes=2, graph=True)
     np.testing.assert_array_equal(a, b)
     np.testing.assert_array_equal(c, a[:2])
-    # the recorded batch replayed for other seeds and constraints of the same shape
+    # other seeds and constraints of the same shape
     seeds2, cons2 = [7, 8, 9, 10, 11], _constraints(len(seeds), 8, 12)
     d = _batch(ic, n, seeds2, cons2, torch.float32, lanes=3, graph=True)
     e = _batch(ic, n, seeds2, cons2, torch.float32, lanes=3, graph=True)
@@ -139,6 +141,32 @@ def test_batch_large_spheres_match_one_at_a_time():
         for f in range(4):
             np.testing.assert_allclose(got[r, f], want[f], atol=1e-9 * np.abs(want[f]).max(),
                                        err_msg="realisation %d field %d" % (r, f))
+    ic.close()
+
+
+@pytest.mark.parametrize("n,precision,ncons,nreal,radius,lanes", [
+    (64, gic.FLOAT64, 32, 5, 4.0, [1, 2, 3, 16]),    # boxes; 69 MB of covectors each: groups of 2, 2 + 1, 3 + 2, all
+    (32, gic.FLOAT32, 2, 21, 4.0, [1, 16]),          # boxes; groups of 16 and 5
+    (32, gic.FLOAT32, 3, 21, 22.0, [1]),             # whole-field spheres among them, 16 and 5
+    (64, gic.FLOAT32, 1, 35, 4.0, [1]),              # one constraint: 16, 16 and 3
+])
+def test_each_realisation_of_uneven_groups_is_its_own(n, precision, ncons, nreal, radius, lanes):
+    """Groups with a short last one: every realisation is the one that its seed
+    and constraints give alone, bit by bit."""
+    import torch
+    print("batch in uneven groups", n, precision, ncons, nreal, flush=True)
+    ic = _ctx(precision, n)
+    dtype = torch.float64 if precision == gic.FLOAT64 else torch.float32
+    cons = _constraints(nreal, ncons, nreal)
+    cons[:, 0, 3] = radius
+    # centres on a lattice, so that the constraints of a realisation are independent
+    side = int(np.ceil(ncons ** (1 / 3)))
+    pts = (np.stack(np.meshgrid(*[np.arange(side)] * 3, indexing="ij"), -1).reshape(-1, 3)[:ncons] + 0.3) * (BOX / side)
+    cons[..., :3] = pts + np.random.default_rng(1).uniform(0, 2, (nreal, ncons, 3))
+    seeds = np.arange(nreal) * 7 + 3
+    alone = np.concatenate([_batch(ic, n, seeds[r:r + 1], cons[r:r + 1], dtype, 1, False) for r in range(nreal)])
+    for k in lanes:
+        np.testing.assert_array_equal(_batch(ic, n, seeds, cons, dtype, k, False), alone, err_msg="lanes %d" % k)
     ic.close()
 
 

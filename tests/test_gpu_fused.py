@@ -81,7 +81,7 @@ def test_displacement_and_transpose(n, precision):
 
 
 @pytest.mark.parametrize("precision", [32, 64])
-@pytest.mark.parametrize("n", SIZES[:-1])
+@pytest.mark.parametrize("n", SIZES)
 def test_second_order(n, precision):
     rng = np.random.default_rng(n)
     w = rng.standard_normal((n, n, n)).astype(np.float32 if precision == 32 else np.float64)
@@ -102,3 +102,68 @@ def test_second_order(n, precision):
         # S sums products of phi that cancel: a few times the error of one
         _near(torch.from_numpy(g.field(4 + a, 0)).cuda(), _inv(s * inv2 * (3.0 / 7.0) * (1j * odd[a]), n), precision, 10)
     g.close()
+
+
+# 1024: what the grids above check cell by cell, on one component, without the
+# fields' way through the host where there is another
+
+@pytest.mark.parametrize("precision", [32, 64])
+def test_displacement_and_transpose_at_1024(precision):
+    n = 1024
+    print("displacement at 1024, precision", precision, flush=True)
+    dt = torch.float32 if precision == 32 else torch.float64
+    rng = torch.Generator(device="cuda").manual_seed(n)
+    w = torch.randn((n, n, n), generator=rng, device="cuda", dtype=dt)
+    bar = [torch.randn((n, n, n), generator=rng, device="cuda", dtype=dt) for _ in range(3)]
+    psi = [torch.empty_like(w) for _ in range(3)]
+    wbar = torch.empty_like(w)
+    g = _gen(n, precision)
+    torch.cuda.synchronize()
+    g.displacement_forward([w.data_ptr()], [p.data_ptr() for p in psi])
+    g.displacement_adjoint([b.data_ptr() for b in bar], [wbar.data_ptr()])
+    g.close()
+
+    def dot(a, b):
+        return sum(float((x[i].double() * y[i].double()).sum()) for x, y in zip(a, b) for i in range(n))
+
+    size = (dot(psi, psi) * dot(bar, bar)) ** 0.5
+    assert abs(dot(psi, bar) - dot([w], [wbar])) < (2e-5 if precision == 32 else 1e-12) * size
+    del bar, wbar
+    _, odd, root, inv2 = _modes(n)
+    m = _fwd(w.double()) * root * inv2
+    del root, inv2
+    for a in (0, 2):
+        _near(psi[a], _inv(m * (1j * odd[a]), n), precision)
+
+
+@pytest.mark.parametrize("precision", [32, 64])
+def test_second_order_at_1024(precision):
+    n = 1024
+    print("second order at 1024, precision", precision, flush=True)
+    g = _gen(n, precision, lpt=2)
+    g.set_seed(1024)
+    g.zeldovich()
+    real = np.float32 if precision == 32 else np.float64
+    delta = torch.from_numpy(g.field(gic.FIELD_OVERDENSITY, 0, dtype=real)).cuda()
+    got = torch.from_numpy(g.field(5, 0, dtype=real)).cuda()   # psi2_y
+    g.close()
+    ks, odd, _, inv2 = _modes(n)
+    m = _fwd(delta.double()) * inv2
+    del delta
+
+    def phi(a, b):
+        return _inv(m * (ks[a] * ks[b] if a == b else odd[a] * odd[b]), n)
+
+    S = phi(0, 0)
+    trace = S.clone()
+    for a, first in ((1, True), (2, False)):
+        p = phi(a, a)
+        S = S * p if first else S + trace * p
+        trace += p
+    del trace, p
+    for a, b in ((0, 1), (0, 2), (1, 2)):
+        S -= phi(a, b) ** 2
+    del m
+    s = _fwd(S)
+    del S
+    _near(got, _inv(s * inv2 * (3.0 / 7.0) * (1j * odd[1]), n), precision, 10)

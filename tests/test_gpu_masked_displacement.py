@@ -36,10 +36,10 @@ def _mask(name, n):
             "none": x < 0}[name]
 
 
-# FP64: the same sums in other orders.  FP32: float rounding of transforms of
-# at most 2^18 points, as in the other displacement tests.
+# FP64: the same sums in other orders.  FP32: float rounding of the transforms,
+# as in the other displacement tests.
 @pytest.mark.parametrize("precision,tol", [(gic.FLOAT64, 1e-12), (gic.FLOAT32, 1e-5)])
-@pytest.mark.parametrize("n", [8, 64])
+@pytest.mark.parametrize("n", [8, 64, 128, 256])
 @pytest.mark.parametrize("name", ["corner_ball", "one_cell", "last_plane", "two_gaps", "all", "none"])
 def test_loss_of_a_mask_matches_weights(name, n, precision, tol):
     print("masked displacement", name, n, precision, flush=True)

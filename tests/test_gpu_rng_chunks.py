@@ -1,8 +1,8 @@
 """The chunked RNG at the sizes the workloads draw, against the serial
 stream.
 
-The device splits a draw into chunks of kc ranlxs2 blocks (kc = 4, 8, 16,
-32, 64 by draw size) and starts each chunk from a 576-bit modular jump;
+The device splits a draw into chunks of kc ranlxs2 blocks (kc = 1, 2, 4, ...
+64 by draw size) and starts each chunk from a 576-bit modular jump;
 draws of about 4.6e7 Gaussians and more (every level of 256^3 and above
 once combined, the 1024^3 workload at 1.1e9) use kc = 64 with chunk
 indices up to 2^20.  Windows far into a stream are checked against the
@@ -29,7 +29,7 @@ def _kc_of_gaussians(n):
     chunk; the plan halves 64 until it has about 65536 chunks)."""
     need = 2.2 * n + 4096.0
     kc = 64
-    while kc > 4 and need / (kc * 24.0) < 65536.0:
+    while kc > 1 and need / (kc * 24.0) < 65536.0:
         kc //= 2
     return kc
 

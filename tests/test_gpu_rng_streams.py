@@ -11,10 +11,11 @@ from genetic_amd import gic
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 11, 12, 13, 767, 768, 769, 20011, 700_001, 1_500_001, 3_000_001])
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 11, 12, 13, 767, 768, 769, 20011, 700_001, 1_428_013, 1_428_017,
+                               1_500_001, 2_857_889, 2_857_893, 3_000_001])
 def test_stream_of_any_length(n):
-    """One block per chunk up to about 7e5 values, then two, then four; the
-    values past the first are the same numbers in the same order."""
+    """One block per chunk up to 1 428 014 values, two up to 2 857 890, then
+    four; the values past the first are the same numbers in the same order."""
     seed = 4099 + n
     ic = gic.ICGenerator(precision=gic.FLOAT64)
     got = ic.gaussian_stream(seed, n)

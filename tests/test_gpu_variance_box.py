@@ -119,3 +119,36 @@ def test_variance_of_many_cells_matches_oracle(name):
     o.set_variance_scale(SCALE)
     want = o.calculate("variance")
     assert abs(ic.calculate("variance") - want) <= 1e-11 * abs(want)
+
+
+@pytest.mark.parametrize("n", [64, 128, 256])
+def test_cut_transforms_of_larger_grids(n):
+    """A wrapping ball's variance and gradient: in FP64 the gradient belongs to
+    the value (V is quadratic), in FP32 both are the FP64 ones to float
+    rounding."""
+    print("variance box at", n, flush=True)
+    q = np.minimum(np.arange(n), n - np.arange(n))
+    r2 = q[:, None, None] ** 2 + q[None, :, None] ** 2 + q[None, None, :] ** 2
+    cells = np.flatnonzero((r2 <= (n // 10) ** 2).ravel()).astype(np.uint64)
+    rng = torch.Generator(device="cuda").manual_seed(n)
+    w, d = (torch.randn((n, n, n), generator=rng, device="cuda", dtype=torch.float64) for _ in range(2))
+    got = {}
+    for precision, dt in ((gic.FLOAT64, torch.float64), (gic.FLOAT32, torch.float32)):
+        ic = _gpu([(BOX, n)], precision)
+        ic.set_flags(0, cells)
+        ic.set_variance_filter_scale(BOX / n * 4)
+
+        def value(t, g=None):
+            t = t.to(dt)
+            torch.cuda.synchronize()
+            return ic.variance_gradient([t.data_ptr()], None if g is None else [g.data_ptr()])
+
+        grad = torch.empty_like(w, dtype=dt)
+        got[precision] = value(w, grad), grad.double()
+        if precision == gic.FLOAT64:
+            vp, vm = value(w + d), value(w - d)
+            assert abs((vp - vm) - 2 * float((grad * d).sum())) <= 1e-11 * (vp + vm)
+        ic.close()
+    (v, g), (v32, g32) = got[gic.FLOAT64], got[gic.FLOAT32]
+    assert abs(v32 - v) <= 2e-5 * v
+    assert float((g32 - g).norm()) <= 2e-5 * float(g.norm())
