@@ -353,11 +353,11 @@ def batch_throughput(nreal=64, n=128, box=50.0, nmods=16, precision=32, lanes=8,
     seeds = np.arange(1, nreal + 1, dtype=np.uint64)
     out = torch.empty((nreal, 4, n, n, n), dtype=torch.float32 if precision == 32 else torch.float64,
                       device="cuda")
-    ic.batch_constrained(seeds, cons, out.data_ptr(), lanes=lanes, graph=True)   # warm-up: buffers, tables
+    ic.batch_constrained(seeds, cons, out.data_ptr(), lanes=lanes)   # warm-up: buffers, tables
     torch.cuda.synchronize()
     t0 = time.perf_counter()
     for _ in range(reps):
-        ic.batch_constrained(seeds, cons, out.data_ptr(), lanes=lanes, graph=True)
+        ic.batch_constrained(seeds, cons, out.data_ptr(), lanes=lanes)
     torch.cuda.synchronize()
     dt = (time.perf_counter() - t0) / reps
     ok = bool(torch.isfinite(out).all())
@@ -381,7 +381,7 @@ def batch_throughput(nreal=64, n=128, box=50.0, nmods=16, precision=32, lanes=8,
     del out
     return dict(value=round(nreal * n ** 3 / dt / 1e6, 2), unit="Mparticles/s",
                 ms_per_batch=round(dt * 1e3, 3), ms_per_realisation=round(dt / nreal * 1e3, 3),
-                lanes=lanes, graph=True, outputs_finite=ok,
+                lanes=lanes, outputs_finite=ok,
                 one_at_a_time=dict(value=round(nreal * n ** 3 / dts / 1e6, 2),
                                    ms_per_realisation=round(dts / nreal * 1e3, 3)),
                 config="%d realisations of %d^3 in %.0f Mpc/h (seeds 1..%d), %d overdensity constraints each "

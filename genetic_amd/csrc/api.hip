@@ -192,15 +192,8 @@ InterpGeom interp_geom(const LevelGeom &gf, const LevelGeom &gc) {
   ig.off[2] = (int)llround((gf.oz - gc.oz) / dxs);
   ig.sim = (int)llround(gf.periodic / dxs);
   ig.nsup = gc.n * ratio;
-  ig.dxs = dxs;
-  ig.dxc = gc.dx;
-  ig.co[0] = gc.ox;
-  ig.co[1] = gc.oy;
-  ig.co[2] = gc.oz;
-  ig.periodic = gc.periodic;
   ig.nc = gc.n;
-  ig.csim = (int)llround(gc.periodic / gc.dx);
-  ig.wrap = gc.n == ig.csim ? 1 : 0;
+  ig.wrap = gc.n == (int)llround(gc.periodic / gc.dx) ? 1 : 0;
   return ig;
 }
 
@@ -1154,10 +1147,10 @@ int gic_displacement_forward(gic_context *c, const void *const *noise, void *con
 }
 
 int gic_batch_constrained(gic_context *c, int nreal, const uint64_t *seeds, int ncons, const double *cons,
-                          void *out, int lanes, int use_graph, double *elapsed_ms) {
+                          void *out, int lanes, int /*use_graph*/, double *elapsed_ms) {
   return guarded(c, [&] {
-    if (c->prec == 32) do_batch<float>(c, nreal, seeds, ncons, cons, (float *)out, lanes, use_graph != 0, elapsed_ms);
-    else do_batch<double>(c, nreal, seeds, ncons, cons, (double *)out, lanes, use_graph != 0, elapsed_ms);
+    if (c->prec == 32) do_batch<float>(c, nreal, seeds, ncons, cons, (float *)out, lanes, elapsed_ms);
+    else do_batch<double>(c, nreal, seeds, ncons, cons, (double *)out, lanes, elapsed_ms);
   });
 }
 

@@ -84,13 +84,12 @@ __global__ __launch_bounds__(256) void k_batch_tophat(T *__restrict__ cov, long 
 
 // The rows of each constraint's box (wl x wl cells in x, y from (winx[f],
 // winy[f]) mod n, all z): 1 on the cells of the sphere, 0 elsewhere; row
-// (f wl + i) wl + j is x = winx[f]+i, y = winy[f]+j.  Rows past nm wl^2 (up
-// to nrows) are zero.  cnt[f] += the number of cells of constraint f.  The
-// box holds every selected cell: a cell is selected only if its centroid
+// (f wl + i) wl + j is x = winx[f]+i, y = winy[f]+j.
+// cnt[f] += the number of cells of constraint f.  The box holds every selected cell: a cell is selected only if its centroid
 // lies within the radius of the centre, and the box spans the centre's
 // +-radius with a cell to spare.
 template <typename T>
-__global__ __launch_bounds__(256) void k_batch_box_rows(T *__restrict__ rows, unsigned nrows, int nm, int wl, int n,
+__global__ __launch_bounds__(256) void k_batch_box_rows(T *__restrict__ rows, unsigned nrows, int wl, int n,
                                                         double dx, double ox, double oy, double oz, double periodic,
                                                         const double *__restrict__ cons, const int *__restrict__ winx,
                                                         const int *__restrict__ winy, uint32_t *__restrict__ cnt) {
@@ -102,7 +101,7 @@ __global__ __launch_bounds__(256) void k_batch_box_rows(T *__restrict__ rows, un
   unsigned ww = unsigned(wl) * unsigned(wl);
   int f = int(row / ww);
   bool inside = false;
-  if (live && f < nm) {
+  if (live) {
     unsigned r2 = row - unsigned(f) * ww;
     int i = int(r2 / unsigned(wl)), j = int(r2 - unsigned(i) * unsigned(wl));
     int x = (winx[f] + i) % n, y = (winy[f] + j) % n;
@@ -412,7 +411,7 @@ constexpr long DRAW_SEGS = 32768;
 
 template <typename T>
 void do_batch(gic_context *c, int nreal, const uint64_t *seeds, int ncons, const double *cons, T *out, int nlanes,
-              bool, double *ms) {
+              double *ms) {
   if (c->levels.size() != 1) throw std::runtime_error("batched realisations need exactly one grid level");
   if (!c->have_camb) throw std::runtime_error("No power spectrum has been set (use the camb command)");
   if (nreal < 1 || !seeds || !out) throw std::runtime_error("batch: no realisations, seeds or output");
@@ -469,13 +468,13 @@ void do_batch(gic_context *c, int nreal, const uint64_t *seeds, int ncons, const
     wl = std::max(wl, span >= double(n) ? n : int(span));
   }
   // (the row kernel indexes rows x n values in 32 bits)
-  const bool boxes = wl < n && (double(ncons) * wl * wl + 1024.0) * n < 2e9;
+  const bool boxes = wl < n && double(ncons) * wl * wl * n < 2e9;
   // (with fewer than four constraints the output's fields decide: no more
   // memory than ncons + 3 fields for each of the caller's lanes)
   const int lanes = std::max(1, std::min(nlanes, nlanes * (ncons + 3) / batch_fields(ncons)));
   int group = std::max(lanes, std::min(GROUP_MAX, int(GROUP_BYTES / (double(ncons) * fs_reals * sizeof(T)))));
   group = std::min(group, nreal);
-  if (boxes) group = std::min(group, int(2e9 / ((double(ncons) * wl * wl + 1024.0) * n)));
+  if (boxes) group = std::min(group, int(2e9 / (double(ncons) * wl * wl * n)));
   auto nrows_of = [&](int k) { return boxes ? long(k) * ncons * wl * wl : 0; };
   // the boxes' x origins of every constraint, then the y origins
   std::vector<int> win(boxes ? size_t(nreal) * ncons * 2 : 0);
@@ -553,7 +552,7 @@ void do_batch(gic_context *c, int nreal, const uint64_t *seeds, int ncons, const
       const long nrows = nrows_of(nb);
       unsigned ne = unsigned(nrows) * unsigned(n);
       hipLaunchKernelGGL(k_batch_box_rows<T>, dim3((ne + 255) / 256), dim3(256), 0, st, (T *)B.rows.p, unsigned(nrows),
-                         nc, wl, n, g.dx, g.ox, g.oy, g.oz, g.periodic, rc, wx, wy, (uint32_t *)B.cnt.p);
+                         wl, n, g.dx, g.ox, g.oy, g.oz, g.periodic, rc, wx, wy, (uint32_t *)B.cnt.p);
       GIC_HIP(hipGetLastError());
       fft_r2c_boxes<T>((const T *)B.rows.p, n, nrows, nc, wl, wx, wy, (T *)B.zbuf.p, (T *)B.ybuf.p, cv, fs,
                        (const T *)L.sqrtp_dm.p, st, hook);
@@ -629,8 +628,7 @@ void do_batch(gic_context *c, int nreal, const uint64_t *seeds, int ncons, const
   }
 }
 
-template void do_batch<float>(gic_context *, int, const uint64_t *, int, const double *, float *, int, bool, double *);
-template void do_batch<double>(gic_context *, int, const uint64_t *, int, const double *, double *, int, bool,
-                               double *);
+template void do_batch<float>(gic_context *, int, const uint64_t *, int, const double *, float *, int, double *);
+template void do_batch<double>(gic_context *, int, const uint64_t *, int, const double *, double *, int, double *);
 
 }  // namespace gic

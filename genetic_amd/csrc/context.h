@@ -334,8 +334,6 @@ template <typename T> void build_sqrtp(gic_context *c, Level &L);
 template <typename T> void build_sqrtp_dm(gic_context *c, Level &L);
 template <typename T> void do_draw(gic_context *c);
 template <typename T> void ensure_noise_fourier(gic_context *c, Level &L);
-// dense (optional): 3 arrays per level that also receive the base level's
-// displacements; the levels' fields then hold noise transformed along z and y
 // The shortest cyclic run [b0, b0 + bl) mod n that holds every index with
 // used[] set (all but the longest gap); bl = 0 if there is none.
 inline void cyclic_hull(const uint8_t *used, int n, int &b0, int &bl) {
@@ -350,6 +348,8 @@ inline void cyclic_hull(const uint8_t *used, int n, int &b0, int &bl) {
   b0 = end % n;
   bl = n - best;
 }
+// dense (optional): three arrays that also receive the base level's
+// displacements; the levels' fields then hold noise transformed along z and y
 template <typename T> void do_zeldovich(gic_context *c, T *const *dense);
 
 // ---- displacement map and its transpose (adjoint.hip) ----------------------------------
@@ -374,6 +374,6 @@ void mod_set_line_search(gic_context *c, bool on);
 template <typename T> void do_splice(gic_context *c, unsigned long new_seed, int *cg_iterations);
 template <typename T>
 void do_batch(gic_context *c, int nreal, const uint64_t *seeds, int ncons, const double *cons, T *out, int nlanes,
-              bool graph, double *ms);
+              double *ms);
 
 }  // namespace gic

@@ -48,9 +48,6 @@ template <typename T>
 void fft_r2c_post(T *d, int n, const T *post, hipStream_t st, TimingHook *hook, const T *src = nullptr);
 // r2c of nb padded n^3 fields stored back to back, each mode times post[|k|^2] if post is given
 template <typename T> void fft_r2c_batch(T *d, int n, int nb, const T *post, hipStream_t st, TimingHook *hook);
-// builds the twiddle table of size n (a synchronous upload), so that later
-// launches, also those recorded into a graph, need no host work
-template <typename T> void fft_prepare(int n);
 // r2c of nb fields that vanish outside boxes of wl x wl cells in (x, y), all
 // z: box b starts at (winx[b], winy[b]) mod n (device int arrays).  rows
 // holds the boxes' rows as dense rows of n reals, row (b wl + i) wl + j for
@@ -63,26 +60,16 @@ void fft_r2c_boxes(const T *rows, int n, long nrows, int nb, int wl, const int *
                    T *spec, long spec_stride, const T *post, hipStream_t st, TimingHook *hook);
 // out <- c2r(op(spec)), out-of-place from a spectrum that is left untouched.
 // op: FFT_PRE_TABLE multiplies by tab[|k|^2].
-// With dst non-null the real result goes to the dense n^3 array dst and out is scratch.
-// With tab null and inv_k2 non-zero the operator's factor is inv_k2 / (|k|^2 kmin^2)
-// (0 at k = 0), formed in FP64 as filter_table forms it for a unit filter.
-// fil (optional) replaces tab for FP32 transforms.
 template <typename T>
-void fft_c2r_from(const T *spec, T *out, int n, int pre, const T *tab, double kmin, hipStream_t st,
-                  TimingHook *hook, T *dst = nullptr, double inv_k2 = 0, const FilterInline *fil = nullptr);
+void fft_c2r_from(const T *spec, T *out, int n, int pre, const T *tab, double kmin, hipStream_t st, TimingHook *hook);
 // Factors of (k_y, k_z) that the fused y and z passes multiply a field by
 enum {
   FFT_YZ_ONE = 0,    // 1
   FFT_YZ_IKY = 1,    // i k_y (0 at k_y = +Nyquist)
   FFT_YZ_IKZ = 2,    // i k_z (0 at k_z = +Nyquist)
   FFT_YZ_MIKY = 3,   // -i k_y (0 at k_y = +Nyquist)
-  FFT_YZ_MIKZ = 4,   // -i k_z (0 at k_z = +Nyquist)
-  FFT_YZ_KYKY = 5,   // k_y^2
-  FFT_YZ_KYKZ = 6,   // k_y k_z (0 at either +Nyquist)
-  FFT_YZ_KZKZ = 7,   // k_z^2
-  FFT_YZ_I = 8,      // i
-  FFT_YZ_KZ = 9,     // k_z (0 at k_z = +Nyquist)
-  FFT_YZ_KY = 10     // k_y (0 at k_y = +Nyquist)
+  FFT_YZ_KYKY = 4,   // k_y^2
+  FFT_YZ_KY = 5      // k_y (0 at k_y = +Nyquist)
 };
 // ---- fused passes (fft_fused.h) ----------------------------------------------------
 // Fields are padded (n * n * (n + 2) values of T); nb of them form a batch,
@@ -94,8 +81,8 @@ enum {
 // spectrum m it makes the inverse x transforms
 //   out[0]: m (times the filter alone with plain0)   out[1]: f m
 //   out[2]: i k_x f m (0 at +Nyquist)                  out[3]: k_x^2 f m
-// (those not null) with f given as for fft_c2r_from: tab, fil (FP32) or
-// inv_k2.  plain0: fil holds a filter over k^2 and tab0 the filter's table.
+// (those not null), f the table tab[|k|^2], the filter product fil in its place
+// (FP32), or inv_k2 / (|k|^2 kmin^2) (0 at k = 0).  plain0: fil holds a filter over k^2 and tab0 the filter's table.
 // With wlen > 0 the outputs keep the points [win0, win0 + wlen) mod n, as
 // wlen planes; with iwlen > 0 (forward) the input is the iwlen planes from
 // iwin0 on of fields that are 0 elsewhere.  Outputs may be the input where
@@ -134,8 +121,8 @@ template <typename T> struct FftY {
 };
 template <typename T> void fft_y(const FftY<T> &y, int n, hipStream_t st, TimingHook *hook);
 
-// c2r along z, scaled by scale n^-1.5: each job's complex rows times a factor of
-// k_z (FFT_YZ_ONE, IKZ, MIKZ, KZ, KZKZ, I) to a padded field, a dense array or both
+// c2r along z, scaled by scale n^-1.5: each job's complex rows times FFT_YZ_ONE
+// or FFT_YZ_IKZ to a padded field, a dense array or both
 template <typename T> struct FftZ {
   struct Job {
     const T *in;

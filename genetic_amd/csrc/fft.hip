@@ -46,13 +46,10 @@ void fft_r2c_boxes(const T *rows, int n, long nrows, int nb, int wl, const int *
   if (nrows < long(nb) * wl * wl) throw std::runtime_error("fft_r2c_boxes: bad row count");
   api<T>(n).r2c_boxes(rows, nrows, nb, wl, winx, winy, zbuf, ybuf, spec, spec_stride, post, st, hook);
 }
-template <typename T> void fft_prepare(int n) {
-  api<T>(n).prepare();
-}
 template <typename T>
 void fft_c2r_from(const T *spec, T *out, int n, int pre, const T *tab, double kmin, hipStream_t st,
-                  TimingHook *hook, T *dst, double inv_k2, const FilterInline *fil) {
-  api<T>(n).c2r_from(spec, out, pre, tab, kmin, st, hook, dst, inv_k2, fil);
+                  TimingHook *hook) {
+  api<T>(n).c2r_from(spec, out, pre, tab, kmin, st, hook);
 }
 template <typename T>
 void fft_r2c_window_zy(const T *win, int n, const int *w0, const int *wl, T *bufB, T *bufA, hipStream_t st,
@@ -132,11 +129,9 @@ void fft_z_lpt(T *px, T *py, T *pz, const T *xx, const T *yy, const T *xy, T *S,
                              hipStream_t, TimingHook *);                                                     \
   template void fft_r2c_post<T>(T *, int, const T *, hipStream_t, TimingHook *, const T *);                 \
   template void fft_r2c_batch<T>(T *, int, int, const T *, hipStream_t, TimingHook *);                      \
-  template void fft_prepare<T>(int);                                                                        \
   template void fft_r2c_boxes<T>(const T *, int, long, int, int, const int *, const int *, T *, T *, T *, long,  \
                                  const T *, hipStream_t, TimingHook *);                                       \
-  template void fft_c2r_from<T>(const T *, T *, int, int, const T *, double, hipStream_t, TimingHook *, T *, \
-                                double, const FilterInline *);                                               \
+  template void fft_c2r_from<T>(const T *, T *, int, int, const T *, double, hipStream_t, TimingHook *);      \
   template void fft_r2c_window_zy<T>(const T *, int, const int *, const int *, T *, T *, hipStream_t, TimingHook *); \
   template void fft_r2c_window<T>(const T *, int, const int *, const int *, T *, T *, T *, const T *, bool,      \
                                   hipStream_t, TimingHook *, const T *, const FilterInline *, double);         \

@@ -6,14 +6,12 @@
 namespace gic {
 
 template <typename T> struct FftApi {
-  void (*prepare)();
   void (*r2c)(T *d, const T *post, hipStream_t st, TimingHook *hook, const T *src);
   void (*r2c_batch)(T *d, int nb, const T *post, hipStream_t st, TimingHook *hook);
   void (*r2c_boxes)(const T *rows, long nrows, int nb, int wl, const int *winx, const int *winy, T *zbuf, T *ybuf,
                     T *spec, long spec_stride, const T *post, hipStream_t st, TimingHook *hook);
   void (*c2r)(T *d, hipStream_t st, TimingHook *hook);
-  void (*c2r_from)(const T *spec, T *out, int pre, const T *tab, double kmin, hipStream_t st,
-                   TimingHook *hook, T *dst, double inv_k2, const FilterInline *fil);
+  void (*c2r_from)(const T *spec, T *out, int pre, const T *tab, double kmin, hipStream_t st, TimingHook *hook);
   void (*c2r_window)(const T *spec, int pre, const T *tab, double kmin, const int *w0, const int *wl, T *bufA,
                      T *bufB, T *out, hipStream_t st, TimingHook *hook, const FilterInline *fil);
   void (*r2c_window)(const T *win, const int *w0, const int *wl, T *bufB, T *bufA, T *spec, const T *post, bool accum,

@@ -610,7 +610,6 @@ template <typename T, int N> FftApi<T> fft_api_of() {
   using F = FftN<T, N>;
   using G = FftFused<T, N>;
   FftApi<T> a;
-  a.prepare = [] { twtable<T>().get(N); };
   a.r2c = F::r2c;
   a.r2c_batch = F::r2c_batch;
   a.r2c_boxes = F::r2c_boxes;

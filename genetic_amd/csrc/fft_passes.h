@@ -178,20 +178,20 @@ template <typename T, int N> struct FftN {
     GIC_HIP(hipGetLastError());
     if (hook) hook->end(tag.c_str(), st);
   }
-  // r2c (dir < 0) or c2r of nrows padded rows of d; ext (if non-null) holds
-  // the dense rows that the r2c reads, or takes those of the c2r
+  // r2c (dir < 0) or c2r of nrows padded rows of d; src (if non-null) holds
+  // the dense rows that the r2c reads
   static void zpass(T *d, T scale, int dir, long nrows, hipStream_t st, TimingHook *hook, const char *name,
-                    T *ext = nullptr) {
+                    const T *src = nullptr) {
     const double bytes = double(nrows) * (2 * N + 2) * sizeof(T);   // N reals one way, N+2 the other
     if (dir < 0) {
       ZFwdArgs<T> a{};
-      a.job[0] = {ext ? ext : d, d, ext ? long(N) : long(N + 2)};
+      a.job[0] = {src ? src : d, d, src ? long(N) : long(N + 2)};
       a.nrows = nrows;
       a.iters = Rows::iters(nrows, 1);
       rows_launch(k_fft_z_r2c<T, N, Rows::TH, false>, a, 1, 1, name, bytes, st, hook);
     } else {
       ZArgs<T> a{};
-      a.job[0] = {d, ext ? nullptr : d, ext, FFT_YZ_ONE};
+      a.job[0] = {d, d, nullptr, FFT_YZ_ONE};
       a.nrows = nrows;
       a.iters = Rows::iters(nrows, 1);
       a.scale = scale;
@@ -213,7 +213,7 @@ template <typename T, int N> struct FftN {
   }
   static void r2c(T *d, const T *post, hipStream_t st, TimingHook *hook, const T *src = nullptr) {
     cx<T> *c = reinterpret_cast<cx<T> *>(d);
-    zpass(d, T(1), -1, long(N) * N, st, hook, "fft_z_r2c", const_cast<T *>(src));
+    zpass(d, T(1), -1, long(N) * N, st, hook, "fft_z_r2c", src);
     strided<-1, PRE_NONE, POST_NONE, 1>(plain(c, false, T(1)), N, st, hook, "fft_y_fwd");
     StridedArgs<T> ax = plain(c, true, norm());
     if (post) {
@@ -251,7 +251,7 @@ template <typename T, int N> struct FftN {
   // spectrum, times post[|k|^2], goes to spec + b * spec_stride (complex).
   static void r2c_boxes(const T *rows, long nrows, int nb, int wl, const int *winx, const int *winy, T *zbuf,
                         T *ybuf, T *spec, long spec_stride, const T *post, hipStream_t st, TimingHook *hook) {
-    zpass(zbuf, T(1), -1, nrows, st, hook, "fft_z_r2c_boxes", const_cast<T *>(rows));
+    zpass(zbuf, T(1), -1, nrows, st, hook, "fft_z_r2c_boxes", rows);
     // y pass: per field, tiles (i, kz block), lines over ky from the wl rows j
     StridedArgs<T> ay{};
     ay.in = reinterpret_cast<const cx<T> *>(zbuf);
@@ -299,21 +299,18 @@ template <typename T, int N> struct FftN {
     zpass(d, norm(), +1, long(N) * N, st, hook, "fft_z_c2r");
   }
   // out <- c2r(op(spec)) with op applied while the x pass reads the spectrum
-  static void c2r_from(const T *spec, T *out, int pre, const T *tab, double kmin, hipStream_t st,
-                       TimingHook *hook, T *dst = nullptr, double inv_k2 = 0, const FilterInline *fil = nullptr) {
+  static void c2r_from(const T *spec, T *out, int pre, const T *tab, double kmin, hipStream_t st, TimingHook *hook) {
     const cx<T> *ci = reinterpret_cast<const cx<T> *>(spec);
     cx<T> *co = reinterpret_cast<cx<T> *>(out);
     StridedArgs<T> ax = plain(co, true, T(1));
     ax.in = ci;
     ax.tab = tab;
     ax.kmin_d = kmin;
-    ax.inv_k2 = inv_k2;
-    if (fil) ax.fil = *fil;
-    if (!tab && pre != PRE_NONE && inv_k2 == 0) throw std::runtime_error("c2r_from: operator without a table");
+    if (!tab && pre != PRE_NONE) throw std::runtime_error("c2r_from: operator without a table");
     if (pre == PRE_TABLE) strided<+1, PRE_TABLE, POST_NONE>(ax, N, st, hook, "fft_x_pre");
     else strided<+1, PRE_NONE, POST_NONE>(ax, N, st, hook, "fft_x");
     strided<+1, PRE_NONE, POST_NONE, 1>(plain(co, false, T(1)), N, st, hook, "fft_y");
-    zpass(out, norm(), +1, long(N) * N, st, hook, "fft_z_c2r", dst);
+    zpass(out, norm(), +1, long(N) * N, st, hook, "fft_z_c2r");
   }
   // real-space window [w0, w0+wl) (per axis, mod N) of c2r(op(spec)):
   // bufA holds wl[0] x-planes after the x pass, bufB wl[0]*wl[1] rows after

@@ -159,12 +159,7 @@ __device__ __forceinline__ YzOp yz_op(int op) {
     case FFT_YZ_IKY: return {1, 1, 0};
     case FFT_YZ_IKZ: return {1, 0, 1};
     case FFT_YZ_MIKY: return {3, 1, 0};
-    case FFT_YZ_MIKZ: return {3, 0, 1};
     case FFT_YZ_KYKY: return {0, 2, 0};
-    case FFT_YZ_KYKZ: return {0, 1, 1};
-    case FFT_YZ_KZKZ: return {0, 0, 2};
-    case FFT_YZ_I: return {1, 0, 0};
-    case FFT_YZ_KZ: return {0, 0, 1};
     case FFT_YZ_KY: return {0, 1, 0};
   }
   return r;
@@ -203,7 +198,7 @@ __device__ __forceinline__ void row_load(cx<T> (&v)[RowPlan<M>::E], const cx<T> 
 }
 
 // c2r of several fields (blockIdx.y) of a batch (blockIdx.z): complex rows
-// times a factor of k_z (FFT_YZ_ONE, IKZ, MIKZ, KZ, KZKZ or I), the real rows
+// times a factor of k_z (FFT_YZ_ONE or FFT_YZ_IKZ), the real rows
 // to the padded field out (may be the input), a dense array, or both.  WIN:
 // only the points [z0, z0 + wz) mod N, to dense rows of wz reals.
 constexpr int FUSED_JOBS = 6;

@@ -15,12 +15,7 @@ struct InterpGeom {
   int off[3];        // fine-grid origin in supersampled coarse cells
   int sim;           // box size in supersampled cells (wrap period)
   int nsup;          // coarse grid size in supersampled cells
-  double dxs;        // supersampled cell size
-  double dxc;        // coarse cell size
-  double co[3];      // coarse grid offsetLower
-  double periodic;   // box size
   int nc;            // coarse grid cells per side
-  int csim;          // box size in coarse cells
   int wrap;          // coarse grid covers the box: wrap, else clamp
 };
 

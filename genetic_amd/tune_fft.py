@@ -12,11 +12,10 @@ kernels at run time:
 `build` links csrc/fft.hip, compiled for one shape (GIC_TUNE_THREADS,
 GIC_TUNE_COLS), with the harness csrc/fft_tune.hip into _tune/libfft_t*_c*.so.
 `measure` loads each library in a process of its own and times, on a padded
-n^3 field, the forms of the transform the path uses: forward + inverse, the
-Zel'dovich inverse (i k/k^2, dense output), a windowed inverse with a
-low-pass filter and a windowed forward that adds a filtered spectrum.  The
-objective is their sum (medians of three timings of `reps` calls each); a
-shape whose round trip does not give the field back is discarded.  `apply`
+n^3 field, the forms of the transform the path uses: forward + inverse, an
+inverse with a |k|^2 table, a windowed inverse with a low-pass filter and a
+windowed forward that adds a filtered spectrum.  The objective is their sum
+(medians of three timings of `reps` calls each); a shape whose round trip does not give the field back is discarded.  `apply`
 keeps, per precision and size, the fastest shape if it beats the default
 (512 threads, 8 columns FP32 / 4 FP64) by more than 2 %, and the library is
 then rebuilt with the table (make -C genetic_amd/csrc).
