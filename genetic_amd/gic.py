@@ -353,7 +353,8 @@ class ICGenerator:
         mean-overdensity constraints with absolute targets; out_ptr (device,
         the context's precision) receives delta, psi_x, psi_y, psi_z per
         realisation as dense n^3 arrays at out + r*4*n^3.  A launch works on a
-        group of at least lanes realisations; graph changes nothing.  Returns
+        group of at least lanes realisations (a fifth fewer with a single
+        constraint); graph changes nothing.  Returns
         the milliseconds from the first device work of the batch to its end."""
         seeds = np.ascontiguousarray(seeds, dtype=np.uint64).ravel()
         cons = np.ascontiguousarray(cons, dtype=np.float64)
